@@ -8,8 +8,7 @@ shapes, so later runs of the same workload start from the tuned shape.
 Candidates span the knobs of the launch:
 
 * ``beam_tiles``: beams per wavefront (0 = 8 for <= 8 beams, else 16;
-  1 = always 8, as (beam, re/im) row pairs; 2 = always 16, where FP32 uses
-  the three-product form);
+  1 = always 8; 2 = always 16, where the operands fit);
 * ``chunks_per_item``: 256-sample time chunks per work item (load balance
   against per-item phasor staging);
 * ``workgroups_per_cu``: workgroups per compute unit in the grid (2-4 keep

@@ -3,7 +3,7 @@
 Two ``torch.autograd.Function``s back onto the hand-written kernels of the
 C-ABI (``blade_beamformer_adjoint``, ``blade_beamformer_stokes_i_grad``):
 
-* :class:`Beamform` -- ``y = beamformer(x, w)`` (FP32 matrix cores); its
+* :class:`Beamform` -- ``y = beamformer(x, w)`` (FP32 precision); its
   backward is the adjoint contraction ``grad_w = sum_t grad_y conj(x)``.
 * :class:`StokesIPower` -- ``L = -sum_b lambda_b sum |y_b|^2``, the negative
   detected (Stokes-I) power of weighted beams.  Forward and gradient come from

@@ -21,15 +21,23 @@
 // wavefront holds MW beam tiles (8 beams each) so that every voltage it loads
 // is multiplied by up to 16 beams.
 //
-// Two arithmetic variants:
-//  * FP32: v_mfma_f32_16x16x4_f32, FP32 accumulate.  With 16 beams per
+// Three arithmetic variants:
+//  * FP32, CI8 input: int8 -> bf16 is exact (8 significant bits), and every
+//    FP32 phasor component is the exact sum of three BF16 values (3 x 8 bits),
+//    so v_mfma_f32_16x16x32_bf16 forms exact products of the FP32 phasors and
+//    accumulates them in FP32.  Three BF16 products run 5x faster than the
+//    four FP32 ones (v_mfma_f32_16x16x4_f32, 1/16 of the rate), which takes
+//    the matrix cores off the critical path.  Against FP32 instructions in
+//    three-product (Gauss) form: production Mode-B block 122.9 -> 109.2 us
+//    (5.3 TB/s of algorithmic bytes), 8 uneven blocks batched 457 -> 373 us,
+//    error against FP64 1.5e-7 -> 1.0e-7 normwise.
+//  * FP32, CF32 input: v_mfma_f32_16x16x4_f32.  With 16 beams per
 //    wavefront (MW = 2) the tile rows are 16 beams and the complex product
 //    takes three real contractions instead of four (Gauss):
 //        P1 = Wr.Xr,  P2 = Wi.Xi,  P3 = (Wr + Wi).(Xr + Xi),
 //        Re y = P1 - P2,  Im y = P3 - P1 - P2,
-//    with Xr + Xi exact for CI8 input and Wr + Wi formed once in the pack
-//    kernel; with 8 beams (MW = 1) the rows are (beam, re/im) pairs of the
-//    embedding below.
+//    with Wr + Wi formed once while the phasors are packed; with 8 beams
+//    (MW = 1) the rows are (beam, re/im) pairs of the embedding below.
 //  * split FP16 (CI8 input only): int8 -> fp16 is exact; each phasor
 //    component is scaled by a per-(workgroup, pol) power of two, split into
 //    hi = fp16(w) and lo = fp16(w - hi), and both halves are multiplied on
@@ -53,6 +61,13 @@ constexpr int TILE = 16;      // rows and columns of one MFMA tile
 constexpr int KG = 4;         // lane groups (l / 16) along K
 constexpr int WAVES = 4;      // wavefronts per workgroup
 
+// Arithmetic of a variant (see above).
+constexpr int AR_F32 = 0;     // FP32 matrix instructions (CF32 voltages)
+constexpr int AR_F16X2 = 1;   // phasors as two FP16 parts
+constexpr int AR_BF16X3 = 2;  // phasors as three BF16 parts (FP32 precision, CI8 voltages)
+constexpr bool ar_split(int ar) { return ar != AR_F32; }
+constexpr int ar_parts(int ar) { return ar == AR_BF16X3 ? 3 : 2; }
+
 __device__ __forceinline__ floatx4 mfma_f32(float a, float b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -69,7 +84,7 @@ struct BfArgs {
     int incoherent, inc_sqrt;
     int rate;               // epilogue channelizer rate (1, 2, 4)
     int polarize;
-    int nsteps;             // K steps (FP32: 2 per antenna group; FP16: 1 per 16 antennas)
+    int nsteps;             // K steps (FP32: 2 per antenna group; split: 1 per 16 antennas)
     int n_tchunks;          // chunks of WAVES*TILE*NT samples along T
     int chunks_per_wg;      // chunks walked by one workgroup
     size_t wbytes;          // bytes of the phasor A operands in LDS
@@ -83,18 +98,19 @@ struct BfArgs {
 //   split FP16 [m][p][step][hl][lane] halfx8 (8 k values = 4 antennas x re/im),
 //              components scaled by a per-pol power of two so that all are < 1,
 //              hi = fp16(w), lo = fp16(w - hi).
+// (three-part BF16: bf_pack_bf16x3.)
 // G3 selects the three-product FP32 layout (16-beam tiles, see bf_body).
 //
 // bf_pack_fill writes the (beam tile m, pol p) part from staged phasors `sw`
 // ([SB][A] float2 of pol p: the 8 beams of tile m for FP32, all MW * 8 beams
 // of the group for split FP16, whose scale is shared by the group's pol).
-template <int MW, bool F16X2, bool G3>
+template <int MW, int AR, bool G3>
 __device__ __forceinline__ void bf_pack_fill(const BfArgs& a, const int m, const int p, const float2* sw,
                                              const float scale, unsigned char* dst) {
-    constexpr int AK = F16X2 ? 4 * KG : KG;
+    constexpr int AK = ar_split(AR) ? 4 * KG : KG;
     const int A = a.A;
     const int nsteps = a.nsteps;
-    if constexpr (F16X2) {
+    if constexpr (AR == AR_F16X2) {
         // beam (within the staged rows) of A-operand row `row` of tile m
         const int row_beam0 = m * (TILE / 2);
         // [m][p][step][hl][lane] halfx8, the (m, p) block
@@ -173,10 +189,60 @@ __device__ __forceinline__ void bf_pack_w0sq(const BfArgs& a, const float2* sw, 
     }
 }
 
+// Three-part BF16 operands of the (f, beam group), [m][p][step][part][lane]
+// bf16x8 (8 k values = 4 antennas x re/im), straight from memory: no scale is
+// shared, so nothing is staged, and every thread has the loads of its four
+// antennas (both pols in 16 bytes) in flight at once.  Ends with a barrier.
+template <int MW>
+__device__ __forceinline__ void bf_pack_bf16x3(const BfArgs& a, const int f, const int gz, unsigned char* dst,
+                                               float* w0sq) {
+    const int A = a.A, nsteps = a.nsteps;
+    const float4* w4 = reinterpret_cast<const float4*>(a.w) + f;
+    uint4* wb = reinterpret_cast<uint4*>(dst);
+    for (int e = threadIdx.x; e < MW * nsteps * 64; e += WAVES * 64) {
+        const int ln = e & 63, ms = e >> 6;
+        const int m = (MW == 2 && ms >= nsteps) ? 1 : 0, st = ms - m * nsteps;
+        const int row = ln & (TILE - 1), kg = ln >> 4;
+        const int b = gz * MW * (TILE / 2) + m * (TILE / 2) + (row >> 1);
+        const bool im = row & 1;
+        float4 w[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int an = st * 4 * KG + 4 * kg + q;
+            w[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (an < A && b < a.B) w[q] = w4[((size_t)b * A + an) * a.F];
+        }
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            uint32_t h[3][4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const float wr = p ? w[q].z : w[q].x, wi = p ? w[q].w : w[q].y;
+                // k = (antenna, c): c = 0 multiplies Re x, c = 1 multiplies Im x.
+                float v0[3], v1[3];
+                split_bf16x3(im ? wi : wr, v0);
+                split_bf16x3(im ? wr : -wi, v1);
+#pragma unroll
+                for (int k = 0; k < 3; k++) h[k][q] = bf16_pair(v0[k], v1[k]);
+            }
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                wb[(((m * 2 + p) * nsteps + st) * 3 + k) * 64 + ln] = make_uint4(h[k][0], h[k][1], h[k][2], h[k][3]);
+        }
+    }
+    if (gz == 0 && threadIdx.x < 128) {
+        float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (threadIdx.x < A) w = w4[(size_t)threadIdx.x * a.F];
+        w0sq[threadIdx.x] = w.x * w.x + w.y * w.y;
+        w0sq[128 + threadIdx.x] = w.z * w.z + w.w * w.w;
+    }
+    __syncthreads();
+}
+
 // The whole (f, beam group) straight into the workgroup's LDS: one round of
 // phasor loads for both pols and all MW * 8 beams (s_w: [2][MW * 8][A]),
 // then every (m, p) part.  Ends with a barrier.
-template <int MW, bool F16X2, bool G3>
+template <int MW, int AR, bool G3>
 __device__ __forceinline__ void bf_pack_lds(const BfArgs& a, const int f, const int gz, float2* s_w,
                                             unsigned int* s_max, unsigned char* dst, float* w0sq,
                                             float* unscale) {
@@ -186,8 +252,7 @@ __device__ __forceinline__ void bf_pack_lds(const BfArgs& a, const int f, const 
     float mx[2] = {0.f, 0.f};
     if (((uintptr_t)a.w & 15) == 0) {
         // Both pols of a (beam, antenna) are one 16-byte load: half the
-        // scattered phasor loads (FP32 124.6 -> 123.6 us, split FP16 114.7
-        // -> 113.0 us per Mode-B call).
+        // scattered phasor loads (split FP16 114.7 -> 113.0 us per Mode-B call).
         for (int r = threadIdx.x; r < NB * A; r += blockDim.x) {
             const int bl_ = r / A, an = r - bl_ * A, b = gz * NB + bl_;
             float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -211,7 +276,7 @@ __device__ __forceinline__ void bf_pack_lds(const BfArgs& a, const int f, const 
     }
     __syncthreads();
     float scale[2] = {1.f, 1.f}, uns[2] = {1.f, 1.f};
-    if constexpr (F16X2) {
+    if constexpr (AR == AR_F16X2) {
         atomicMax(&s_max[0], __float_as_uint(mx[0]));
         atomicMax(&s_max[1], __float_as_uint(mx[1]));
         __syncthreads();
@@ -226,8 +291,8 @@ __device__ __forceinline__ void bf_pack_lds(const BfArgs& a, const int f, const 
 #pragma unroll
     for (int mp = 0; mp < 2 * MW; mp++) {
         const int p = mp & 1, m = mp >> 1;
-        const float2* sw = s_w + (size_t)p * NB * A + (F16X2 ? 0 : m * (TILE / 2) * A);
-        bf_pack_fill<MW, F16X2, G3>(a, m, p, sw, scale[p], dst);
+        const float2* sw = s_w + (size_t)p * NB * A + (AR == AR_F16X2 ? 0 : m * (TILE / 2) * A);
+        bf_pack_fill<MW, AR, G3>(a, m, p, sw, scale[p], dst);
     }
     if (gz == 0) {
         bf_pack_w0sq(a, s_w, w0sq);
@@ -357,16 +422,18 @@ constexpr int EPI_MODEB = 4 | 8;          // rate 4, polarize, no incoherent bea
 constexpr int EPI_PLAIN = 1;              // rate 1
 constexpr int EPI_PLAIN_INC = 1 | 16;     // rate 1, incoherent beam
 
-// Mode-B epilogue through LDS (split FP16, 16-beam tiles): the four
+// Mode-B epilogue through LDS (split variants, 16-beam tiles): the four
 // wavefronts' spectra of one chunk are exchanged so that each store
 // instruction writes 1 KiB of one output row (64 consecutive spectra of one
 // (beam, fine channel)) instead of 256 B pieces of four rows.  Half of the
-// group's 16 beams at a time: [8 beams][4 fine channels][64 + 1] float4 in
-// LDS (the staged phasors' space, free once they are packed).
-template <int NT, bool F16X2, int MW, int EPI>
-constexpr bool staged_epilogue() { return F16X2 && MW == 2 && NT == 4 && EPI == EPI_MODEB; }
+// group's 16 beams at a time (a quarter with three BF16 parts, whose operands
+// take more LDS; 3 workgroups still fit a CU): [beams][4 fine channels][64 + 1]
+// float4 in LDS (the staged phasors' space, free once they are packed).
+template <int NT, int AR, int MW, int EPI>
+constexpr bool staged_epilogue() { return ar_split(AR) && MW == 2 && NT == 4 && EPI == EPI_MODEB; }
 constexpr int kStageRow = 65;                                   // float4 per staged row, padded
-constexpr size_t kStageBytes = (size_t)8 * 4 * kStageRow * 16;  // one half of the beams
+constexpr int stage_beams(int ar) { return ar == AR_BF16X3 ? 4 : 8; }
+constexpr size_t stage_bytes(int ar) { return (size_t)stage_beams(ar) * 4 * kStageRow * 16; }
 
 // One beam's 4 consecutive samples (one lane): DFT-4, fftshift, XY -> LR,
 // into the staged rows of local beam lb at column col (the spectrum's index
@@ -395,10 +462,10 @@ __device__ __forceinline__ void stage_beam(float4* stg, int lb, int col, float2 
 // One "unit" of voltage loads: what a lane needs for one K block.
 //  FP32, CI8  : one antenna x NT samples          -> NT words
 //  FP32, CF32 : one antenna x NT samples x 16 B   -> 4 NT words
-//  split FP16 : four antennas x NT samples        -> 4 NT words
-template <int NT, bool CI8, bool F16X2>
+//  split      : four antennas x NT samples        -> 4 NT words
+template <int NT, bool CI8, int AR>
 struct Unit {
-    static constexpr int WORDS = (F16X2 || !CI8) ? 4 * NT : NT;
+    static constexpr int WORDS = (ar_split(AR) || !CI8) ? 4 * NT : NT;
     uint32_t w[WORDS];
 };
 
@@ -419,6 +486,7 @@ __device__ __forceinline__ void load_words(uint32_t* dst, const uint32_t* src) {
 // LDS phasor layouts (A operands):
 //   FP32       wl[m][p][step][g][row]        float   (step = 2 * antenna group + component)
 //   split FP16 wh[m][p][step][hl][lane]      halfx8  (8 k values = 4 antennas x re/im)
+//   BF16 parts wb[m][p][step][part][lane]    bf16x8  (the same k values)
 //
 // Work split: blockIdx = (t-range, f, beam group of MW tiles).  A workgroup
 // walks up to `chunks_per_wg` chunks of WAVES*TILE*NT samples with the
@@ -433,12 +501,12 @@ __device__ __forceinline__ void load_words(uint32_t* dst, const uint32_t* src) {
 // chunk ranges.  The work item packs its phasors straight into LDS
 // (bf_pack_lds): lds_raw holds the A operands, then the staged phasors
 // [2][MW * 8][A] float2; s_unscale / s_w0sq the split-FP16 unscale and |w0|^2.
-template <int NT, int MW, bool CI8, bool F16X2, int D, bool NTS, int EPI, bool G3 = (!F16X2 && MW == 2)>
+template <int NT, int MW, bool CI8, int AR, int D, bool NTS, int EPI, bool G3 = (AR == AR_F32 && MW == 2)>
 __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int gz, const int cw0,
                                         unsigned char* lds_raw, float* s_unscale, float (*s_w0sq)[128],
                                         unsigned int* s_max, const int cstride = 1) {
-    constexpr int AK = F16X2 ? 4 * KG : KG;       // antennas per unit
-    typedef Unit<NT, CI8, F16X2> U_t;
+    constexpr int AK = ar_split(AR) ? 4 * KG : KG;       // antennas per unit
+    typedef Unit<NT, CI8, AR> U_t;
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -448,7 +516,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
     const int nsteps = a.nsteps;
     const bool do_inc = epi_inc<EPI>(a) && gz == 0;
 
-    const int n_units = F16X2 ? nsteps : nsteps / 2;
+    const int n_units = ar_split(AR) ? nsteps : nsteps / 2;
     const int upad = ((n_units + D - 1) / D) * D;
     const int nch = min(a.chunks_per_wg, (a.n_tchunks - cw0 + cstride - 1) / cstride);
     const int J = nch * upad;
@@ -470,7 +538,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
         t0 = (t0 < a.T) ? t0 : 0;
         const size_t off = (size_t)f * a.T + t0;
         constexpr int R = M::RUN;
-        if constexpr (F16X2) {
+        if constexpr (ar_split(AR)) {
             const uint32_t* x = static_cast<const uint32_t*>(a.x);
 #pragma unroll
             for (int q = 0; q < 4; q++) {
@@ -501,12 +569,15 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
     // ---- This (f, beam group)'s packed phasors into LDS. ---------------------
     // A operands, |w0|^2 per antenna and pol, and the power-of-two unscale of
     // the split-FP16 path.
-    bf_pack_lds<MW, F16X2, G3>(a, f, gz, reinterpret_cast<float2*>(lds_raw + a.wbytes), s_max, lds_raw,
-                               &s_w0sq[0][0], s_unscale);
-    const float unscale[2] = {s_unscale[0], s_unscale[1]};
+    if constexpr (AR == AR_BF16X3)
+        bf_pack_bf16x3<MW>(a, f, gz, lds_raw, &s_w0sq[0][0]);
+    else
+        bf_pack_lds<MW, AR, G3>(a, f, gz, reinterpret_cast<float2*>(lds_raw + a.wbytes), s_max, lds_raw,
+                                &s_w0sq[0][0], s_unscale);
+    const float unscale[2] = {AR == AR_F16X2 ? s_unscale[0] : 1.f, AR == AR_F16X2 ? s_unscale[1] : 1.f};
 
     // Three-product FP32 tiles (16 beams): accumulators P1, P2, P3.
-    static_assert(!G3 || (!F16X2 && MW == 2), "three products need FP32 and 16-beam tiles");
+    static_assert(!G3 || (AR == AR_F32 && MW == 2), "three products need FP32 and 16-beam tiles");
     constexpr int NACC = G3 ? 3 : MW;
     floatx4 acc[NACC][2][NT];
     float inc[2][NT];
@@ -528,7 +599,51 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
 
     // MFMAs (and incoherent power) of one unit.
     auto compute = [&](const U_t& u, int un) {
-        if constexpr (F16X2) {
+        if constexpr (ar_split(AR)) {
+            if (do_inc) {
+                // The unit's four antennas are summed in pairs (a shorter
+                // rounding chain than one after the other).
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    float w2[4];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int an = un * AK + 4 * g + q;
+                        w2[q] = an < a.A ? s_w0sq[p][min(an, a.A - 1)] : 0.f;
+                    }
+#pragma unroll
+                    for (int n = 0; n < NT; n++) {
+                        float pw[4];   // re^2 + im^2 of pol p, exact in 16 bits
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            const uint32_t d = u.w[q * NT + n];
+                            pw[q] = (float)__builtin_amdgcn_sdot4((int)d, (int)(d & (p ? 0xffff0000u : 0xffffu)), 0, false);
+                        }
+                        inc[p][n] += (pw[0] * w2[0] + pw[1] * w2[1]) + (pw[2] * w2[2] + pw[3] * w2[3]);
+                    }
+                }
+            }
+        }
+        if constexpr (AR == AR_BF16X3) {
+            const uint4* wb = reinterpret_cast<const uint4*>(lds_raw) + lane;
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                uint4 wv[MW][3];
+#pragma unroll
+                for (int m = 0; m < MW; m++)
+#pragma unroll
+                    for (int k = 0; k < 3; k++) wv[m][k] = wb[(((m * 2 + p) * nsteps + un) * 3 + k) * 64];
+#pragma unroll
+                for (int n = 0; n < NT; n++) {
+                    const uint4 xb = make_uint4(ci8_to_bf16(u.w[n], p), ci8_to_bf16(u.w[NT + n], p),
+                                                ci8_to_bf16(u.w[2 * NT + n], p), ci8_to_bf16(u.w[3 * NT + n], p));
+#pragma unroll
+                    for (int k = 0; k < 3; k++)
+#pragma unroll
+                        for (int m = 0; m < MW; m++) acc[m][p][n] = mfma_bf16(wv[m][k], xb, acc[m][p][n]);
+                }
+            }
+        } else if constexpr (AR == AR_F16X2) {
             const halfx8* wh = reinterpret_cast<const halfx8*>(lds_raw);
             halfx8 whi[2][MW], wlo[2][MW];
 #pragma unroll
@@ -557,23 +672,6 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
                         acc[m][p][n] = mfma_f16(whi[p][m], xb[p], acc[m][p][n]);
                         acc[m][p][n] = mfma_f16(wlo[p][m], xb[p], acc[m][p][n]);
                     }
-            }
-            if (do_inc) {
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int an = un * AK + 4 * g + q;
-                    const int ac = min(an, a.A - 1);
-#pragma unroll
-                    for (int p = 0; p < 2; p++) {
-                        const float w2 = an < a.A ? s_w0sq[p][ac] : 0.f;
-#pragma unroll
-                        for (int n = 0; n < NT; n++) {
-                            const float xr = ci8_byte(u.w[q * NT + n], 2 * p);
-                            const float xi = ci8_byte(u.w[q * NT + n], 2 * p + 1);
-                            inc[p][n] += (xr * xr + xi * xi) * w2;
-                        }
-                    }
-                }
             }
         } else {
             const float* wl = reinterpret_cast<const float*>(lds_raw);
@@ -640,7 +738,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
         // of the chunk loop (they would pin dozens of registers).
         int fo = f;
         asm volatile("" : "+s"(fo));
-        if constexpr (staged_epilogue<NT, F16X2, MW, EPI>()) {
+        if constexpr (staged_epilogue<NT, AR, MW, EPI>()) {
             // Every wavefront of the workgroup runs the same chunks, so the
             // barriers below are reached by all four.
             float4* stg = reinterpret_cast<float4*>(lds_raw + a.wbytes);
@@ -649,24 +747,30 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
             const int s = (cw0 + c * cstride) * (WAVES * TILE) + lane;
             float4* const base = reinterpret_cast<float4*>(a.y);
             float4* const sink = a.sink + lane;
+            // A round stages the beams of one tile (8), or every other one of
+            // them (4: tile m's beams 2g + rr), [beam][fine channel] rows.
+            constexpr int SB = stage_beams(AR);
+            constexpr int RPR = SB / 4;                            // beams per lane and round
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                __syncthreads();   // the previous half's (or chunk's) rows are stored
+            for (int h = 0; h < 16 / SB; h++) {
+                const int m = h * SB / 8, r0 = (h * RPR) & 1;
+                __syncthreads();   // the previous round's (or chunk's) rows are stored
 #pragma unroll
-                for (int r = 0; r < 4; r += 2) {
+                for (int q = 0; q < RPR; q++) {
+                    const int r = 2 * (r0 + q);
                     float2 v[2][4];
 #pragma unroll
                     for (int p = 0; p < 2; p++)
 #pragma unroll
                         for (int n = 0; n < 4; n++)
-                            v[p][n] = make_float2(acc[h][p][n][r] * unscale[p], acc[h][p][n][r + 1] * unscale[p]);
-                    stage_beam(stg, (4 * g + r) / 2, col, v);
+                            v[p][n] = make_float2(acc[m][p][n][r] * unscale[p], acc[m][p][n][r + 1] * unscale[p]);
+                    stage_beam(stg, RPR * g + q, col, v);
                 }
                 __syncthreads();
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int row = wave * 8 + j;
-                    const int b = b_wg + 8 * h + (row >> 2);
+                for (int j = 0; j < SB; j++) {
+                    const int row = wave * SB + j;
+                    const int b = b_wg + 8 * m + (RPR == 2 ? row >> 2 : 2 * (row >> 2) + r0);
                     const float4 q = stg[row * kStageRow + lane];
                     float4* dst = (s < S && b < a.B)
                                       ? base + (((size_t)b * a.F + fo) * 4 + (row & 3)) * S + s
@@ -702,7 +806,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
                 for (int p = 0; p < 2; p++)
 #pragma unroll
                     for (int n = 0; n < NT; n++) {
-                        if constexpr (F16X2)
+                        if constexpr (AR == AR_F16X2)
                             v[p][n] = make_float2(acc[m][p][n][r] * unscale[p], acc[m][p][n][r + 1] * unscale[p]);
                         else
                             v[p][n] = make_float2(acc[m][p][n][r], acc[m][p][n][r + 1]);
@@ -759,13 +863,13 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
 }
 
 // One block: blockIdx = (first chunk, f, beam group); chunks interleave.
-template <int NT, int MW, bool CI8, bool F16X2, int D, bool NTS, int EPI>
-__global__ __launch_bounds__(256, (staged_epilogue<NT, F16X2, MW, EPI>() ? 3 : 2)) void beamform_kernel(BfArgs a) {
+template <int NT, int MW, bool CI8, int AR, int D, bool NTS, int EPI>
+__global__ __launch_bounds__(256, (staged_epilogue<NT, AR, MW, EPI>() ? 3 : 2)) void beamform_kernel(BfArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     __shared__ float s_unscale[2];
     __shared__ float s_w0sq[2][128];
     __shared__ unsigned int s_max[2];
-    bf_body<NT, MW, CI8, F16X2, D, NTS, EPI, (!F16X2 && MW == 2)>(a, blockIdx.y, blockIdx.z, blockIdx.x, lds_raw,
+    bf_body<NT, MW, CI8, AR, D, NTS, EPI, (AR == AR_F32 && MW == 2)>(a, blockIdx.y, blockIdx.z, blockIdx.x, lds_raw,
                                                                 s_unscale, s_w0sq, s_max, gridDim.x);
 }
 
@@ -774,18 +878,42 @@ static int env_int(const char* name, int dflt) {
     return v ? atoi(v) : dflt;
 }
 
-// Bytes of the packed phasor A operands in LDS.  FP32 with two beam tiles
+// Bytes of the packed phasor A operands in LDS.  FP32 (CF32 input) with two beam tiles
 // stores three products per antenna group (Wr, Wi, Wr + Wi over 16 beams)
 // instead of the 2 x 2 embedding rows.
-static size_t operand_bytes(bool f16x2, int mw, int nsteps, bool g3) {
-    return f16x2 ? (size_t)mw * 2 * nsteps * 2 * 64 * 16
-                 : (g3 ? (size_t)3 * nsteps * 64 * 4 : (size_t)mw * 2 * nsteps * 64 * 4);
+static size_t operand_bytes(int ar, int mw, int nsteps) {
+    return ar_split(ar) ? (size_t)mw * 2 * nsteps * ar_parts(ar) * 64 * 16
+                        : (mw == 2 ? (size_t)3 * nsteps * 64 * 4 : (size_t)mw * 2 * nsteps * 64 * 4);
 }
 
 constexpr size_t kSinkBytes = 64 * sizeof(float4);
 
-static int nsteps_for(bool f16x2, int A) {
-    return f16x2 ? (A + 4 * KG - 1) / (4 * KG) : 2 * ((A + KG - 1) / KG);
+// Bytes of the phasors staged behind the A operands: both pols of the group's
+// beams (the three-part BF16 operands are packed without a stage).
+static size_t staged_bytes(int ar, int mw, int A) {
+    return ar == AR_BF16X3 ? 0 : (size_t)2 * mw * (TILE / 2) * A * sizeof(float2);
+}
+
+constexpr size_t kMaxLds = 150 * 1024;
+
+static int nsteps_for(int ar, int A) {
+    return ar_split(ar) ? (A + 4 * KG - 1) / (4 * KG) : 2 * ((A + KG - 1) / KG);
+}
+
+// Antenna limit of a call whose beams are taken `mw` tiles at a time: that of
+// the LDS image of FP32 operands and staged phasors (240 antennas at 16
+// beams, 400 at 8).  Every FP32 variant keeps it, whatever its own LDS need.
+static bool antennas_fit_f32(int mw, int A) {
+    return operand_bytes(AR_F32, mw, nsteps_for(AR_F32, A)) + staged_bytes(AR_F32, mw, A) <= kMaxLds;
+}
+
+// Beam tiles per wavefront: 16 beams (2 tiles) past 8 beams, where they fit in
+// LDS beside the Mode-B stage.  Three BF16 parts take 12 KiB per 16 antennas
+// at 16 beams (up to 176 antennas); above that 8-beam tiles (6 KiB) carry on.
+static int beam_tiles_for(int ar, int A, int B) {
+    if (B <= TILE / 2) return 1;
+    if (ar == AR_BF16X3 && operand_bytes(ar, 2, nsteps_for(ar, A)) + stage_bytes(ar) > kMaxLds) return 1;
+    return 2;
 }
 
 static int groups_for(int B, int mw) { return (B + mw * (TILE / 2) - 1) / (mw * (TILE / 2)); }
@@ -830,14 +958,14 @@ static int pick_chunks_per_wg(const void* fn, size_t lds, int n_tchunks, long pe
     return best;
 }
 
-template <int NT, int MW, bool CI8, bool F16X2, int D, bool NTS, int EPI = 0>
+template <int NT, int MW, bool CI8, int AR, int D, bool NTS, int EPI = 0>
 static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hipStream_t s) {
     BfArgs a = args;
-    a.nsteps = nsteps_for(F16X2, a.A);
-    a.wbytes = operand_bytes(F16X2, MW, a.nsteps, !F16X2 && MW == 2);
+    a.nsteps = nsteps_for(AR, a.A);
+    a.wbytes = operand_bytes(AR, MW, a.nsteps);
     // A operands, then the staged phasors of both pols (packed in the kernel).
-    size_t lds = a.wbytes + (size_t)2 * MW * (TILE / 2) * a.A * sizeof(float2);
-    if (staged_epilogue<NT, F16X2, MW, EPI>()) lds = std::max(lds, a.wbytes + kStageBytes);
+    size_t lds = a.wbytes + staged_bytes(AR, MW, a.A);
+    if (staged_epilogue<NT, AR, MW, EPI>()) lds = std::max(lds, a.wbytes + stage_bytes(AR));
     const int span = WAVES * TILE * NT;
     const int groups = groups_for(a.B, MW);
     // Device scratch: only the store sink of idle lanes (the phasors are
@@ -854,8 +982,8 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
     }
     a.sink = reinterpret_cast<float4*>(sink_mem);
     a.n_tchunks = (a.T + span - 1) / span;
-    const void* fn = reinterpret_cast<const void*>(&beamform_kernel<NT, MW, CI8, F16X2, D, NTS, EPI>);
-    if (lds > 150 * 1024) return fail("beamformer: too many antennas for the LDS phasor stage");
+    const void* fn = reinterpret_cast<const void*>(&beamform_kernel<NT, MW, CI8, AR, D, NTS, EPI>);
+    if (lds > kMaxLds) return fail("beamformer: too many antennas for the LDS phasor stage");
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
@@ -868,7 +996,7 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
     cpw = std::min(cpw, a.n_tchunks);
     a.chunks_per_wg = cpw;
     dim3 grid((unsigned)((a.n_tchunks + cpw - 1) / cpw), (unsigned)a.F, (unsigned)groups);
-    hipLaunchKernelGGL((beamform_kernel<NT, MW, CI8, F16X2, D, NTS, EPI>), grid, dim3(64 * WAVES), lds, s, a);
+    hipLaunchKernelGGL((beamform_kernel<NT, MW, CI8, AR, D, NTS, EPI>), grid, dim3(64 * WAVES), lds, s, a);
     return check_launch("beamformer");
 }
 
@@ -882,29 +1010,29 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
 // writes 16 bytes of every 32 or 64 and ordinary stores let L2 merge the lines
 // before they go out.
 
-template <int NT, int MW, bool CI8, bool F16X2, int D>
+template <int NT, int MW, bool CI8, int AR, int D>
 static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, hipStream_t s) {
     if constexpr (NT == 4) {
-        if (epi == EPI_MODEB) return launch_bf<NT, MW, CI8, F16X2, D, true, EPI_MODEB>(a, ws, wsb, s);
+        if (epi == EPI_MODEB) return launch_bf<NT, MW, CI8, AR, D, true, EPI_MODEB>(a, ws, wsb, s);
         // The rate-1 epilogues map a wave onto TILE * NT consecutive samples
         // (runs of one): T must not cut a wave.
         if (a.T % (TILE * NT) == 0) {
-            if (epi == EPI_PLAIN) return launch_bf<NT, MW, CI8, F16X2, D, true, EPI_PLAIN>(a, ws, wsb, s);
+            if (epi == EPI_PLAIN) return launch_bf<NT, MW, CI8, AR, D, true, EPI_PLAIN>(a, ws, wsb, s);
             if (epi == EPI_PLAIN_INC)
-                return launch_bf<NT, MW, CI8, F16X2, D, true, EPI_PLAIN_INC>(a, ws, wsb, s);
+                return launch_bf<NT, MW, CI8, AR, D, true, EPI_PLAIN_INC>(a, ws, wsb, s);
         }
     }
-    return launch_bf<NT, MW, CI8, F16X2, D, false, 0>(a, ws, wsb, s);
+    return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
 }
 
-template <bool CI8, bool F16X2>
+template <bool CI8, int AR>
 static int dispatch(const BfArgs& a, int nt, int mw, int epi, unsigned char* ws, size_t wsb, hipStream_t s) {
-    constexpr int D = (F16X2 || !CI8) ? 2 : 4;
+    constexpr int D = 2;
     if (nt == 4)
-        return mw == 2 ? launch_epi<4, 2, CI8, F16X2, D>(a, epi, ws, wsb, s)
-                       : launch_epi<4, 1, CI8, F16X2, D>(a, epi, ws, wsb, s);
-    return mw == 2 ? launch_epi<1, 2, CI8, F16X2, D>(a, epi, ws, wsb, s)
-                   : launch_epi<1, 1, CI8, F16X2, D>(a, epi, ws, wsb, s);
+        return mw == 2 ? launch_epi<4, 2, CI8, AR, D>(a, epi, ws, wsb, s)
+                       : launch_epi<4, 1, CI8, AR, D>(a, epi, ws, wsb, s);
+    return mw == 2 ? launch_epi<1, 2, CI8, AR, D>(a, epi, ws, wsb, s)
+                   : launch_epi<1, 1, CI8, AR, D>(a, epi, ws, wsb, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -946,44 +1074,30 @@ __device__ __forceinline__ BfArgs batch_block_args(const BatchArgs& ba, int k) {
     return a;
 }
 
-template <int NT, bool F16X2, int D>
+template <int NT, int AR, int D>
 __global__ __launch_bounds__(256, 2) void beamform_batched_kernel(BatchArgs ba) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     __shared__ float s_unscale[2];
     __shared__ float s_w0sq[2][128];
     __shared__ unsigned int s_max[2];
-    // A work item is a (channel, chunk range) of one block.  FP32: its beam
-    // groups run back to back in the item's workgroup (fewer, longer items:
-    // 5.3 against 5.6 ms on the seeded 32-block batch).  Split FP16: one
-    // item per beam group (4.5 against 4.6 ms).
-    constexpr bool GROUPS_IN_ITEM = !F16X2;
+    // A work item is a (channel, chunk range, beam group) of one block.
     for (int item = blockIdx.x; item < ba.total_items; item += gridDim.x) {
         int k = 0;
         while (k + 1 < ba.n_blocks && item >= ba.blk[k + 1].item_base) k++;
         const BatchBlock& b = ba.blk[k];
         int local = item - b.item_base;
-        int gz0 = 0, gz1 = b.groups;
-        if constexpr (!GROUPS_IN_ITEM) {
-            gz0 = local % b.groups;
-            gz1 = gz0 + 1;
-            local /= b.groups;
-        }
+        const int gz = local % b.groups;
+        local /= b.groups;
         const int f = local % b.F;
         const int tr = local / b.F;
         const BfArgs a = batch_block_args(ba, k);
-        for (int gz = gz0; gz < gz1; gz++) {
-            __syncthreads();   // the previous group's (or item's) readers of LDS are done
-            // FP32 16-beam tiles take the three-product form, as in the
-            // single-block kernel.  Each group packs its (channel, beam
-            // group)'s phasors into LDS itself, as the single-block kernel
-            // does.
-            if (b.mw == 2)
-                bf_body<NT, 2, true, F16X2, D, true, EPI_PLAIN, !F16X2>(a, f, gz, tr * b.cpw, lds_raw, s_unscale,
-                                                                        s_w0sq, s_max);
-            else
-                bf_body<NT, 1, true, F16X2, D, true, EPI_PLAIN>(a, f, gz, tr * b.cpw, lds_raw, s_unscale,
-                                                                s_w0sq, s_max);
-        }
+        __syncthreads();   // the previous item's readers of LDS are done
+        // Each item packs its (channel, beam group)'s phasors into LDS
+        // itself, as the single-block kernel does.
+        if (b.mw == 2)
+            bf_body<NT, 2, true, AR, D, true, EPI_PLAIN>(a, f, gz, tr * b.cpw, lds_raw, s_unscale, s_w0sq, s_max);
+        else
+            bf_body<NT, 1, true, AR, D, true, EPI_PLAIN>(a, f, gz, tr * b.cpw, lds_raw, s_unscale, s_w0sq, s_max);
     }
 }
 
@@ -995,11 +1109,16 @@ struct BatchPlan {
 };
 
 // Plans up to kBatchMax blocks; the workspace pointer may be null (sizing).
-static int plan_batch(bool f16x2, const blade_beamform_block* blocks, int n,
+static int plan_batch(int ar, const blade_beamform_block* blocks, int n,
                       const blade_batch_tuning* tuning, unsigned char* ws, BatchPlan* plan) {
     constexpr int NT = 4;
     const int span = WAVES * TILE * NT;
     const int mw_force = tuning ? tuning->beam_tiles : 0;
+    // A requested 16-beam tile gives way where its operands do not fit.
+    auto tiles_of = [&](const blade_beamform_block& bk) {
+        const int fit = beam_tiles_for(ar, (int)std::min<uint64_t>(bk.A, 4096), mw_force == 2 ? 16 : (int)bk.B);
+        return mw_force ? std::min(mw_force, std::max(fit, 1)) : fit;
+    };
     const int cpw_req = tuning ? tuning->chunks_per_item : 0;
     const int wpc = (tuning && tuning->workgroups_per_cu > 0) ? tuning->workgroups_per_cu : 3;
     if (tuning && tuning->time_samples_per_lane != 0 && tuning->time_samples_per_lane != NT)
@@ -1014,9 +1133,9 @@ static int plan_batch(bool f16x2, const blade_beamform_block* blocks, int n,
     long all_chunks = 0;
     for (int k = 0; k < n; k++) {
         const blade_beamform_block& bk = blocks[k];
-        // items: (channel, chunk range), and the beam group for split FP16
+        // items: (channel, chunk range, beam group)
         all_chunks += (long)ceil_div(bk.T, span) * bk.F *
-                      (f16x2 ? groups_for((int)bk.B, mw_force ? mw_force : (bk.B > 8 ? 2 : 1)) : 1);
+                      groups_for((int)bk.B, tiles_of(bk));
     }
     const long target = 2L * wpc * device_cus();
     const int cpw_auto = (int)std::max(1L, (all_chunks + target - 1) / target);
@@ -1030,24 +1149,26 @@ static int plan_batch(bool f16x2, const blade_beamform_block* blocks, int n,
         if (!bk.input || !bk.phasors || !bk.output) return fail("batched beamformer: null pointer");
         if ((uintptr_t)bk.input % 16 || (uintptr_t)bk.phasors % 16 || (uintptr_t)bk.output % 16)
             return fail("batched beamformer: buffers must be 16-byte aligned");
+        if (ar == AR_BF16X3 && !antennas_fit_f32(mw_force ? mw_force : (bk.B > TILE / 2 ? 2 : 1), (int)bk.A))
+            return fail("batched beamformer: too many antennas");
         BatchBlock& b = ba.blk[k];
-        b.mw = mw_force ? mw_force : (bk.B > 8 ? 2 : 1);
+        b.mw = tiles_of(bk);
         b.x = bk.input;
         b.w = static_cast<const float2*>(bk.phasors);
         b.y = static_cast<float2*>(bk.output);
         b.A = (int)bk.A; b.F = (int)bk.F; b.T = (int)bk.T; b.B = (int)bk.B;
-        b.nsteps = nsteps_for(f16x2, b.A);
-        b.wbytes = operand_bytes(f16x2, b.mw, b.nsteps, !f16x2 && b.mw == 2);
+        b.nsteps = nsteps_for(ar, b.A);
+        b.wbytes = operand_bytes(ar, b.mw, b.nsteps);
         b.groups = groups_for(b.B, b.mw);
         b.n_tchunks = (int)ceil_div(bk.T, span);
         b.cpw = std::min(b.n_tchunks, cpw_req > 0 ? cpw_req : cpw_auto);
         b.item_base = (int)items;
-        items += (long)ceil_div(b.n_tchunks, b.cpw) * b.F * (f16x2 ? b.groups : 1);
+        items += (long)ceil_div(b.n_tchunks, b.cpw) * b.F * b.groups;
         // A operands, then the staged phasors of both pols and the group's beams
-        lds = std::max(lds, b.wbytes + (size_t)2 * b.mw * (TILE / 2) * b.A * sizeof(float2));
+        lds = std::max(lds, b.wbytes + staged_bytes(ar, b.mw, b.A));
     }
     if (items > (1L << 30)) return fail("batched beamformer: too many work items");
-    if (lds > 150 * 1024) return fail("batched beamformer: too many antennas");
+    if (lds > kMaxLds) return fail("batched beamformer: too many antennas");
     ba.total_items = (int)items;
     ba.sink = ws ? reinterpret_cast<float4*>(ws) : nullptr;
     plan->ws_bytes = kSinkBytes;
@@ -1056,15 +1177,15 @@ static int plan_batch(bool f16x2, const blade_beamform_block* blocks, int n,
     return BLADE_SUCCESS;
 }
 
-template <bool F16X2>
+template <int AR>
 static int launch_batch(BatchPlan& plan, hipStream_t s) {
-    constexpr int D = F16X2 ? 2 : 4;
-    const void* fn = reinterpret_cast<const void*>(&beamform_batched_kernel<4, F16X2, D>);
+    constexpr int D = 2;
+    const void* fn = reinterpret_cast<const void*>(&beamform_batched_kernel<4, AR, D>);
     if (plan.lds > 65536) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.lds);
         if (e != hipSuccess) return fail(std::string("batched beamformer: LDS attribute: ") + hipGetErrorString(e));
     }
-    hipLaunchKernelGGL((beamform_batched_kernel<4, F16X2, D>), dim3((unsigned)plan.grid), dim3(64 * WAVES),
+    hipLaunchKernelGGL((beamform_batched_kernel<4, AR, D>), dim3((unsigned)plan.grid), dim3(64 * WAVES),
                        plan.lds, s, plan.args);
     return check_launch("batched beamformer");
 }
@@ -1075,19 +1196,19 @@ static int run_batched(int precision, const blade_beamform_block* blocks, uint64
     if (precision != BLADE_PREC_F32 && precision != BLADE_PREC_F16X2)
         return fail("batched beamformer: unknown precision");
     if (n > 0 && !blocks) return fail("batched beamformer: null block table");
-    const bool f16 = precision == BLADE_PREC_F16X2;
+    const int ar = precision == BLADE_PREC_F16X2 ? AR_F16X2 : AR_BF16X3;
     size_t total = 0;
     for (uint64_t k0 = 0; k0 < n; k0 += kBatchMax) {
         const int cnt = (int)std::min<uint64_t>(kBatchMax, n - k0);
         BatchPlan plan;
         unsigned char* base = ws ? ws + total : nullptr;
         if (base && (uintptr_t)base % 256) return fail("batched beamformer: workspace must be 256-byte aligned");
-        int rc = plan_batch(f16, blocks + k0, cnt, tuning, base, &plan);
+        int rc = plan_batch(ar, blocks + k0, cnt, tuning, base, &plan);
         if (rc) return rc;
         const size_t need = (plan.ws_bytes + 255) / 256 * 256;
         if (!size_out) {
             if (!ws || ws_bytes < total + need) return fail("batched beamformer: workspace too small");
-            rc = f16 ? launch_batch<true>(plan, s) : launch_batch<false>(plan, s);
+            rc = ar == AR_F16X2 ? launch_batch<AR_F16X2>(plan, s) : launch_batch<AR_BF16X3>(plan, s);
             if (rc) return rc;
         }
         total += need;
@@ -1129,13 +1250,15 @@ static int run_beamformer(int in_type, int precision, const void* input, const v
     a.chunks_per_wg = 1;
     a.wbytes = 0;
     a.sink = nullptr;
-    const int mw = B > 8 ? 2 : 1;
+    const int ar = precision == BLADE_PREC_F16X2 ? AR_F16X2 : (in_type == BLADE_CI8 ? AR_BF16X3 : AR_F32);
+    if (ar == AR_BF16X3 && !antennas_fit_f32(a.B > TILE / 2 ? 2 : 1, a.A))
+        return fail("beamformer: too many antennas for the LDS phasor stage");
+    const int mw = beam_tiles_for(ar, a.A, a.B);
     const int epi = (int)rate | (polarize ? 8 : 0) | (incoherent ? 16 : 0);
-    if (precision == BLADE_PREC_F16X2) return dispatch<true, true>(a, T % 4 == 0 ? 4 : 1, mw, epi, ws, wsb, s);
-    if (in_type == BLADE_CI8) {
-        return dispatch<true, false>(a, T % 4 == 0 ? 4 : 1, mw, epi, ws, wsb, s);
-    }
-    return dispatch<false, false>(a, T % 4 == 0 ? 4 : 1, mw, epi, ws, wsb, s);
+    const int nt = T % 4 == 0 ? 4 : 1;
+    if (ar == AR_F16X2) return dispatch<true, AR_F16X2>(a, nt, mw, epi, ws, wsb, s);
+    if (ar == AR_BF16X3) return dispatch<true, AR_BF16X3>(a, nt, mw, epi, ws, wsb, s);
+    return dispatch<false, AR_F32>(a, nt, mw, epi, ws, wsb, s);
 }
 
 // Scratch of blade_beamform_chain_noalloc: the store sink of idle lanes as

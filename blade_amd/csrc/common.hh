@@ -15,6 +15,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kWave = 64;
 
@@ -79,6 +80,39 @@ inline int type_bytes(int t) { return type_components(t) * type_scalar_bytes(t);
 
 __device__ __forceinline__ floatx4 mfma_f16(halfx8 a, halfx8 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ floatx4 mfma_bf16(uint4 a, uint4 b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// The high halves of two floats as one dword (lo in bits 0-15): the pair of
+// BF16 values (lo, hi) when both are exact in BF16.
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+
+// Exact CI8 -> BF16 (an int8 needs 8 significant bits, BF16 has 8): the
+// (re, im) pair of polarization p of one voltage dword.
+__device__ __forceinline__ uint32_t ci8_to_bf16(uint32_t d, int p) {
+    return bf16_pair((float)(int8_t)(d >> (16 * p)), (float)(int8_t)(d >> (16 * p + 8)));
+}
+
+// v = part[0] + part[1] + part[2] exactly, each part with the 8 significant
+// bits of BF16 (in the high half of its float): an FP32 value has 24, so
+// cutting 8 off the top three times leaves nothing (parts below FP32's normal
+// range aside).  Infinities and NaN stay in part 0.
+__device__ __forceinline__ void split_bf16x3(float v, float (&part)[3]) {
+    const uint32_t u = __float_as_uint(v);
+    if ((u & 0x7f800000u) == 0x7f800000u) {
+        part[0] = __uint_as_float((u & 0x007fffffu) ? (u | 0x00400000u) : u);
+        part[1] = part[2] = 0.f;
+        return;
+    }
+    part[0] = __uint_as_float(u & 0xffff0000u);
+    const float r = v - part[0];
+    part[1] = __uint_as_float(__float_as_uint(r) & 0xffff0000u);
+    part[2] = r - part[1];
 }
 
 // Exact CI8 -> FP16: int8 b becomes the biased byte u = b + 128, placed in the

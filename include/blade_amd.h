@@ -41,7 +41,8 @@ enum blade_type {
 
 /* Beamformer arithmetic. */
 enum blade_precision {
-    BLADE_PREC_F32 = 0,     /* FP32 MFMA (v_mfma_f32_*_f32), FP32 accumulate */
+    BLADE_PREC_F32 = 0,     /* FP32 phasors and accumulation: FP32 MFMA, or for CI8 input BF16 MFMA on
+                               phasors split exactly into three BF16 parts */
     BLADE_PREC_F16X2 = 1,   /* split FP16: phasor = hi + lo, 2 FP16 MFMAs, FP32 accumulate (CI8 input only) */
 };
 
@@ -140,7 +141,7 @@ typedef struct blade_beamform_block {
  * Tile shape and launch shape of the batched launch; 0 = automatic.
  *   time_samples_per_lane: 4
  *   beam_tiles: 16-row beam tiles per wavefront, 1 (8 beams) or 2 (16;
- *               FP32 then forms three real products per complex one)
+ *               16 gives way to 8 where its operands do not fit in LDS)
  *   chunks_per_item: time chunks of 256 samples per work item
  *   workgroups_per_cu: workgroups per compute unit in the grid (grid =
  *               min(work items, this x CUs); items beyond it are walked)

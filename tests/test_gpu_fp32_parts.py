@@ -1,0 +1,69 @@
+"""FP32 beamforming of CI8 voltages on three exact BF16 phasor parts.
+
+Elementwise bar: with exact products, only the FP32 accumulation of the 2A
+real terms rounds (unit roundoff 2^-24; the matrix core's own summation is
+allowed a factor of two), so |y - ref| <= 2 (2A + 2) 2^-24 sum_a |w| |x|,
+with (|Re w| + |Im w|) (|Re x| + |Im x|) bounding each antenna's terms.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from blade_amd import ops
+from blade_amd._lib import BladeError
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(A, F, T, B, seed):
+    rng = np.random.default_rng(seed)
+    x8 = rng.integers(-128, 128, size=(A, F, T, 2, 2), dtype=np.int8)
+    # phasor magnitudes from 1e-20 to 1e20 over the beams: no scale is shared
+    mag = 10.0 ** rng.uniform(-20, 20, size=(B, 1, 1, 1, 1))
+    w = (mag * (rng.normal(size=(B, A, F, 1, 2)) + 1j * rng.normal(size=(B, A, F, 1, 2)))).astype(np.complex64)
+    return x8, w
+
+
+def _check(y, x8, w, A, B):
+    ref = O.beamformer_ata(x8, w, False, False)
+    x = np.abs(x8[..., 0].astype(np.float64)) + np.abs(x8[..., 1].astype(np.float64))
+    ww = np.abs(w[:, :, :, 0].real.astype(np.float64)) + np.abs(w[:, :, :, 0].imag.astype(np.float64))
+    bound = 2 * (2 * A + 2) * 2.0 ** -24 * np.einsum("bafp,aftp->bftp", ww, x)
+    d = y[:B] - ref
+    assert (np.maximum(np.abs(d.real), np.abs(d.imag)) <= bound).all()
+
+
+@pytest.mark.parametrize("A,B", [(1, 1), (15, 8), (16, 9), (17, 16), (33, 5), (176, 16), (177, 16), (193, 9),
+                                 (240, 17), (400, 8)])
+@pytest.mark.parametrize("T", [64, 132, 70])
+def test_fp32_parts_match_oracle_elementwise(A, B, T):
+    x8, w = _case(A, 2, T, B, A * 100 + B)
+    y = ops.beamformer(torch.from_numpy(x8).cuda(), torch.from_numpy(w).cuda()).cpu().numpy()
+    _check(y, x8, w, A, B)
+
+
+def test_antenna_limits():
+    for A, B, ok in ((240, 9, True), (241, 9, False), (400, 8, True), (401, 8, False)):
+        x = torch.zeros((A, 1, 64, 2, 2), dtype=torch.int8, device="cuda")
+        w = torch.zeros((B, A, 1, 1, 2), dtype=torch.complex64, device="cuda")
+        y = torch.empty((B, 1, 64, 2), dtype=torch.complex64, device="cuda")
+        if ok:
+            ops.beamformer(x, w)
+            ops.BatchedBeamformer([(x, w, y)], tuning={"beam_tiles": 2 if B > 8 else 1})()
+        else:
+            with pytest.raises(BladeError, match="too many antennas"):
+                ops.beamformer(x, w)
+            with pytest.raises(BladeError, match="too many antennas"):
+                ops.BatchedBeamformer([(x, w, y)])()
+
+
+def test_nonfinite_phasors_stay_in_their_beam():
+    x8, w = _case(20, 1, 64, 4, 3)
+    w[1, 3, 0, 0, 0] = np.inf
+    w[2, 5, 0, 0, 1] = np.nan
+    with np.errstate(invalid="ignore"):
+        y = ops.beamformer(torch.from_numpy(x8).cuda(), torch.from_numpy(w).cuda()).cpu().numpy()
+    assert not np.isfinite(y[1, :, :, 0]).any() and not np.isfinite(y[2, :, :, 1]).any()
+    assert np.isfinite(y[[0, 3]]).all() and np.isfinite(y[1, :, :, 1]).all() and np.isfinite(y[2, :, :, 0]).all()

@@ -5,10 +5,7 @@
 // reference src/modules/beamformer/beamformer.cu:13-79) and an upstream
 // gradient gy = dL/dconj(y), the phasor gradient is the contraction over time
 //     gw[b,a,f,p] = dL/dconj(w[b,a,f,p]) = sum_t gy[b,f,t,p] conj(x[a,f,t,p]).
-// Per (f, p) this is a (B x T)(T x A) product, embedded as the real GEMM
-//     [Re gw; Im gw] = [[gy_r, gy_i], [gy_i, -gy_r]] . [x_r; x_i]
-// with rows (beam, re/im), K = (time, component) and columns = antennas, on
-// v_mfma_f32_16x16x4f32 (one 16-row tile = 8 beams).
+// Per (f, p) this is a (B x T)(T x A) product.
 //
 // Fused Stokes-I mode (stokes_grad_kernel): L = -sum_b lambda_b
 // sum_{f,t,p} |y_b|^2, so gy = -lambda_b y_b.  Each workgroup recomputes its
@@ -25,8 +22,7 @@
 // FP32 form runs stokes_grad_b4_kernel instead, on 4x4-block matrix
 // instructions whose columns are exactly the beams.
 //
-// Plain adjoint (adjoint_kernel, gy from memory): rows (beam, re/im),
-// K = (time, component), columns = antennas.
+// Plain adjoint (adjoint_kernel): gy from memory.
 //
 // Work split: blockIdx = (time split, f, beam tile of 8).  Partial gradients
 // are summed across waves in LDS and across time splits by
@@ -38,20 +34,13 @@
 
 namespace bl {
 
-constexpr int ADJ_TC = 128;        // time samples per LDS tile
+constexpr int ADJ_TC = 128;        // adjoint_kernel: time samples per step of a workgroup, 32 per wave
 constexpr int ADJ_WAVES = 4;
 constexpr int ADJ_MAXAT = 8;       // antenna tiles of 16: A <= 128
 constexpr int ADJ_MAXB = 64;       // beams of the fused loss
-constexpr int ADJ_GYS = 17;        // s_gy row stride: 16 values + 1 word of padding
 constexpr int ADJ_BATCH = 8;       // global loads in flight per thread while staging (16 costs a wave of occupancy)
 constexpr int SG_TC = 64;          // stokes_grad_kernel: time samples per tile, 16 per wave
 constexpr int SG_XPAD = 4;         // its LDS voltage row stride is apad + 4 words (see sg_xs)
-
-// Row stride (words) of the LDS voltage tile s_x[t][antenna]: the padded
-// antenna count plus one, so the 16 lanes of a group, which read 16
-// consecutive times of one antenna, hit 16 different banks (a stride of a
-// multiple of 16 words would put them in two).
-__host__ __device__ constexpr int adj_xs(int apad) { return apad + 1; }
 
 struct AdjArgs {
     const uint32_t* x;       // [A,F,T] dwords: CI8 (re0, im0, re1, im1)
@@ -79,14 +68,34 @@ __device__ __forceinline__ float ci8_component(uint32_t d, int idx) {
     return (float)(int8_t)((d >> (8 * idx)) & 0xFFu);
 }
 
-__global__ __launch_bounds__(256) void adjoint_kernel(AdjArgs a) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    const int apad = a.apad;
-    const int xs = adj_xs(apad);
-    uint32_t* s_x = reinterpret_cast<uint32_t*>(lds_raw);              // [TC][xs]
-    float* s_gy = reinterpret_cast<float*>(s_x + ADJ_TC * xs);          // [TC][ADJ_GYS]
-    float* s_G = s_gy + ADJ_TC * ADJ_GYS;                               // [2][16][apad]
+// Eight consecutive times of byte k of a voltage dword as a BF16 operand.
+__device__ __forceinline__ uint4 ci8_times_bf16(const uint4& lo, const uint4& hi, int k) {
+    auto pr = [k](uint32_t d0, uint32_t d1) {
+        return bf16_pair((float)(int8_t)(d0 >> (8 * k)), (float)(int8_t)(d1 >> (8 * k)));
+    };
+    return make_uint4(pr(lo.x, lo.y), pr(lo.z, lo.w), pr(hi.x, hi.y), pr(hi.z, hi.w));
+}
 
+// Plain adjoint of A <= 16 NAT antennas and 8 beams: the real products
+//     P[c][co] = sum_t x_c[a][t] gy_co[b][t]   (c, co = re, im)
+// with rows = antennas, columns = (beam, co) and K = 32 times per
+// instruction, combined at the end: Re gw = P[re][re] + P[im][im],
+// Im gw = P[re][im] - P[im][re].  A lane holds antenna row i (lane % 16) and
+// column i, times 8g .. 8g + 7 of the wave's 32, so both operands are whole
+// 16-byte pieces of memory in their native layout: nothing is staged in LDS
+// and the waves run without barriers.  CI8 is exact in BF16 and gy is the
+// exact sum of three BF16 parts, so the products are exact and v_mfma_f32_
+// 16x16x32_bf16 accumulates them in FP32.  The next 32 times' loads are
+// issued into the registers just converted.
+// HBM bound: A42 F384 T2048 B4 reads 182 MB (x and gy once); with the sums of
+// the splits it took 181 us through LDS tiles and FP32 instructions, 41 us so.
+// VEC: 16-byte
+// loads (T a multiple of 4, both buffers 16-byte aligned); otherwise single
+// dwords and float2.
+template <int NAT, bool VEC>
+__global__ __launch_bounds__(256, (NAT <= 3 ? 3 : NAT <= 5 ? 2 : 1)) void adjoint_kernel(AdjArgs a) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int APAD = 16 * NAT;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -95,94 +104,118 @@ __global__ __launch_bounds__(256) void adjoint_kernel(AdjArgs a) {
     const int sp = blockIdx.x;
     const int f = blockIdx.y;
     const int bt = blockIdx.z;
-    const int b0 = bt * 8;
     const int A = a.A, F = a.F, T = a.T, B = a.B;
     const int t_begin = sp * a.tsplit;
     const int t_end = min(T, t_begin + a.tsplit);
+    const bool im = i & 1;
+    // Rows past A and columns past B repeat the last one (never stored).
+    const float2* const gp = a.gy + ((size_t)min(bt * 8 + (i >> 1), B - 1) * F + f) * T * 2;
 
-    for (int e = tid; e < 2 * 16 * apad; e += blockDim.x) s_G[e] = 0.f;
+    uint4 xq[NAT][2];      // [antenna tile][times 0-3, 4-7 of the lane's 8]
+    float4 gq[8];          // one time each: (X re, X im, Y re, Y im)
+    auto load_x = [&](int t0, int at) {
+        const uint32_t* const xp = a.x + ((size_t)min(at * 16 + i, A - 1) * F + f) * T;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int t = t0 + 8 * g + 4 * h;
+            if constexpr (VEC) {
+                xq[at][h] = *reinterpret_cast<const uint4*>(xp + min(t, t_end - 4));
+            } else {
+                xq[at][h] = make_uint4(xp[min(t, t_end - 1)], xp[min(t + 1, t_end - 1)], xp[min(t + 2, t_end - 1)],
+                                       xp[min(t + 3, t_end - 1)]);
+            }
+        }
+    };
+    auto load_g = [&](int t0) {
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const int t = min(t0 + 8 * g + q, t_end - 1);
+            if constexpr (VEC) {
+                gq[q] = *reinterpret_cast<const float4*>(gp + 2 * t);
+            } else {
+                const float2 u = gp[2 * t], v = gp[2 * t + 1];
+                gq[q] = make_float4(u.x, u.y, v.x, v.y);
+            }
+        }
+    };
 
-    floatx4 acc2[2][ADJ_MAXAT];
+    floatx4 acc[2][NAT][2];    // [pol][antenna tile][component of x]
 #pragma unroll
     for (int p = 0; p < 2; p++)
 #pragma unroll
-        for (int at = 0; at < ADJ_MAXAT; at++) acc2[p][at] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int at = 0; at < NAT; at++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) acc[p][at][c] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    for (int t0 = t_begin; t0 < t_end; t0 += ADJ_TC) {
-        __syncthreads();   // the previous tile's readers are done
-        // Voltages of every antenna for this tile, s_x[t][a] (zero-padded).
-        // Loads in batches of ADJ_BATCH per thread, all issued before any is
-        // used, so a batch costs one memory round trip.
-        const int n_x = ADJ_TC * apad;
-        for (int e0 = tid; e0 < n_x; e0 += ADJ_BATCH * ADJ_WAVES * 64) {
-            uint32_t v[ADJ_BATCH];
+    int t0 = t_begin + wave * 32;
+    if (t0 < t_end) {          // otherwise there is nothing to read (T = 0 included)
+        load_g(t0);
 #pragma unroll
-            for (int k = 0; k < ADJ_BATCH; k++) {
-                const int e = e0 + k * ADJ_WAVES * 64;
-                const int an = e / ADJ_TC, tt = t0 + (e - an * ADJ_TC);
-                v[k] = (e < n_x && an < A && tt < t_end) ? a.x[((size_t)an * F + f) * T + tt] : 0u;
-            }
+        for (int at = 0; at < NAT; at++) load_x(t0, at);
+    }
+    for (; t0 < t_end; t0 += ADJ_TC) {
+        // gy of this lane's component, times past the split zeroed, in parts
+        uint4 gb[2][3];
+        {
+            uint32_t w[2][3][4];
 #pragma unroll
-            for (int k = 0; k < ADJ_BATCH; k++) {
-                const int e = e0 + k * ADJ_WAVES * 64;
-                const int an = e / ADJ_TC, t = e - an * ADJ_TC;
-                if (e < n_x) s_x[t * xs + an] = v[k];
-            }
-        }
-        __syncthreads();
-
+            for (int q = 0; q < 4; q++) {
+                const bool ok0 = t0 + 8 * g + 2 * q < t_end, ok1 = t0 + 8 * g + 2 * q + 1 < t_end;
 #pragma unroll
-        for (int p = 0; p < 2; p++) {
+                for (int p = 0; p < 2; p++) {
+                    const float4 u = gq[2 * q], v = gq[2 * q + 1];
+                    const float u0 = im ? (p ? u.w : u.y) : (p ? u.z : u.x);
+                    const float v0 = im ? (p ? v.w : v.y) : (p ? v.z : v.x);
+                    float pu[3], pv[3];
+                    split_bf16x3(ok0 ? u0 : 0.f, pu);
+                    split_bf16x3(ok1 ? v0 : 0.f, pv);
 #pragma unroll
-            for (int e = tid; e < ADJ_TC * 8; e += ADJ_WAVES * 64) {
-                const int bb = e / ADJ_TC, t = e - bb * ADJ_TC;
-                const int b = b0 + bb, tt = t0 + t;
-                float2 v = make_float2(0.f, 0.f);
-                if (b < B && tt < t_end) v = a.gy[(((size_t)b * F + f) * T + tt) * 2 + p];
-                s_gy[t * ADJ_GYS + 2 * bb] = v.x;
-                s_gy[t * ADJ_GYS + 2 * bb + 1] = v.y;
-            }
-            __syncthreads();
-
-            // Adjoint: K = (time, component), 4 samples per MFMA pair.
-#pragma unroll 2
-            for (int t4 = 0; t4 < 8; t4++) {
-                const int t = wave * 32 + t4 * 4 + g;
-                const float gr = s_gy[t * ADJ_GYS + 2 * (i >> 1)];
-                const float gi = s_gy[t * ADJ_GYS + 2 * (i >> 1) + 1];
-                const float a0 = (i & 1) == 0 ? gr : gi;     // multiplies x_r
-                const float a1 = (i & 1) == 0 ? gi : -gr;    // multiplies x_i
-#pragma unroll
-                for (int at = 0; at < ADJ_MAXAT; at++) {
-                    if (at < a.n_at) {
-                        const uint32_t d = s_x[t * xs + at * 16 + i];
-                        acc2[p][at] = adj_mfma(a0, ci8_component(d, 2 * p), acc2[p][at]);
-                        acc2[p][at] = adj_mfma(a1, ci8_component(d, 2 * p + 1), acc2[p][at]);
-                    }
+                    for (int k = 0; k < 3; k++) w[p][k][q] = bf16_pair(pu[k], pv[k]);
                 }
             }
-            __syncthreads();   // s_gy is rewritten by the next pol
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int k = 0; k < 3; k++) gb[p][k] = make_uint4(w[p][k][0], w[p][k][1], w[p][k][2], w[p][k][3]);
+        }
+        const int tn = min(t0 + ADJ_TC, t_end - 1);     // past the split: re-read its end
+        load_g(tn);
+#pragma unroll
+        for (int at = 0; at < NAT; at++) {
+            uint4 xo[2][2];
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int c = 0; c < 2; c++) xo[p][c] = ci8_times_bf16(xq[at][0], xq[at][1], 2 * p + c);
+            load_x(tn, at);
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+#pragma unroll
+                for (int p = 0; p < 2; p++)
+#pragma unroll
+                    for (int c = 0; c < 2; c++) acc[p][at][c] = mfma_bf16(xo[p][c], gb[p][k], acc[p][at][c]);
         }
     }
 
-    // Sum the four waves' partial gradients in LDS, then write this
-    // workgroup's [2][16][apad] block.
+    // Combine, then sum the four waves in order: [wave][p][col][antenna].
+    float* s_part = reinterpret_cast<float*>(lds_raw);
+    const float sg = im ? -1.f : 1.f;
 #pragma unroll
     for (int p = 0; p < 2; p++)
 #pragma unroll
-        for (int at = 0; at < ADJ_MAXAT; at++) {
-            if (at < a.n_at) {
+        for (int at = 0; at < NAT; at++)
 #pragma unroll
-                for (int r = 0; r < 4; r++)
-                    atomicAdd(&s_G[(p * 16 + 4 * g + r) * apad + at * 16 + i], acc2[p][at][r]);
-            }
-        }
+            for (int r = 0; r < 4; r++)
+                s_part[((wave * 2 + p) * 16 + i) * APAD + at * 16 + 4 * g + r] =
+                    acc[p][at][0][r] + sg * swap_pairs(acc[p][at][1][r]);
     __syncthreads();
-    float* out = a.partial + ((((size_t)sp * F + f) * 2) * a.btiles + bt) * 16 * apad;
-    const size_t pstride = (size_t)a.btiles * 16 * apad;   // between pols
-    for (int e = tid; e < 2 * 16 * apad; e += blockDim.x) {
-        const int p = e / (16 * apad), r = e - p * 16 * apad;
-        out[p * pstride + r] = s_G[e];
+    constexpr int NPART = 2 * 16 * APAD;
+    float* out = a.partial + ((((size_t)sp * F + f) * 2) * a.btiles + bt) * 16 * APAD;
+    const size_t pstride = (size_t)a.btiles * 16 * APAD;   // between pols
+    for (int e = tid; e < NPART; e += blockDim.x) {
+        const float v = ((s_part[e] + s_part[NPART + e]) + s_part[2 * NPART + e]) + s_part[3 * NPART + e];
+        const int p = e / (16 * APAD), r = e - p * 16 * APAD;
+        out[p * pstride + r] = v;
     }
 }
 
@@ -905,28 +938,25 @@ static int run_adjoint(bool fused, bool f16, const void* input, const void* phas
     // FP32 loss + gradient with at most 4 beams: the 4x4-block kernel.
     const bool b4 = fused && !f16 && B <= 4 && A <= 64 && T % 4 == 0 && (uintptr_t)input % 16 == 0 &&
                     A * F * T < (1ull << 31);
-    // Time splits, each a whole number of tiles.  Plain adjoint: about 2048
-    // workgroups.  Fused: the split length that minimises rounds of resident
-    // workgroups (per CU: 4 FP32 or 3 split FP16 up to 64 or 48 antennas,
-    // else 2; the 4x4-block kernel SG4_WGS) x tiles per wave (longest on
-    // ties, which keeps the partial sums few).
+    // Time splits, each a whole number of tiles: the split length that
+    // minimises rounds of resident workgroups (per CU: 4 FP32 or 3 split FP16
+    // up to 64 or 48 antennas, else 2; the 4x4-block kernel SG4_WGS; the plain
+    // adjoint 3, 2 or 1 by antenna tiles) x tiles per wave (longest on ties,
+    // which keeps the partial sums few).
     const int tc = b4 ? SG4_TC : fused ? SG_TC : ADJ_TC;
     const long tiles = (long)ceil_div(std::max<uint64_t>(T, 1), (uint64_t)tc);
     const long per_split = (long)F * a.btiles;
-    long tiles_per;
-    if (fused) {
-        const long slots = (long)device_cus() * (b4 ? SG4_WGS : f16 ? (a.n_at <= 3 ? 3 : 2) : (a.n_at <= 4 ? 4 : 2));
-        long best = -1;
-        tiles_per = tiles;
-        for (long tp = tiles; tp >= 1; tp--) {
-            const long ns = (tiles + tp - 1) / tp;
-            const long per_wave = b4 ? (tp + ADJ_WAVES - 1) / ADJ_WAVES : tp;   // b4: waves take tiles in turn
-            const long cost = ((ns * per_split + slots - 1) / slots) * per_wave;
-            if (best < 0 || cost < best) { best = cost; tiles_per = tp; }
-        }
-    } else {
-        const long ns = std::max(1L, std::min(tiles, (2048 + per_split - 1) / per_split));
-        tiles_per = (tiles + ns - 1) / ns;
+    long tiles_per = tiles, best = -1;
+    const long per_cu = !fused ? (a.n_at <= 3 ? 3 : a.n_at <= 5 ? 2 : 1)
+                        : b4   ? SG4_WGS
+                        : f16  ? (a.n_at <= 3 ? 3 : 2)
+                               : (a.n_at <= 4 ? 4 : 2);
+    const long slots = (long)device_cus() * per_cu;
+    for (long tp = tiles; tp >= 1; tp--) {
+        const long ns = (tiles + tp - 1) / tp;
+        const long per_wave = b4 ? (tp + ADJ_WAVES - 1) / ADJ_WAVES : tp;   // b4: waves take tiles in turn
+        const long cost = ((ns * per_split + slots - 1) / slots) * per_wave;
+        if (best < 0 || cost < best) { best = cost; tiles_per = tp; }
     }
     const long nsplit = (tiles + tiles_per - 1) / tiles_per;
     a.tsplit = (int)(tiles_per * tc);
@@ -941,43 +971,21 @@ static int run_adjoint(bool fused, bool f16, const void* input, const void* phas
     a.partial = reinterpret_cast<float*>(ws);
     a.loss_part = a.partial + part_floats;
 
-    const size_t lds = !fused ? ((size_t)ADJ_TC * adj_xs(a.apad) + ADJ_TC * ADJ_GYS + 2 * 16 * a.apad) * 4
+    const size_t lds = !fused ? (size_t)ADJ_WAVES * 2 * 16 * a.apad * 4
                        : b4    ? ((size_t)a.A * 4 * SG4_WS + (size_t)ADJ_WAVES * SG4_GY) * 4
                        : f16   ? (size_t)2 * SG_TC * sg_xs(a.apad) * 4 + (size_t)2 * a.n_at * 2 * 64 * 16
                                : ((size_t)2 * SG_TC * sg_xs(a.apad) + 2 * (size_t)a.nsteps * 64) * 4;
-    const void* fn = nullptr;
-    if (b4) {
-        switch (a.n_at) {
-            case 1: fn = reinterpret_cast<const void*>(&stokes_grad_b4_kernel<1>); break;
-            case 2: fn = reinterpret_cast<const void*>(&stokes_grad_b4_kernel<2>); break;
-            case 3: fn = reinterpret_cast<const void*>(&stokes_grad_b4_kernel<3>); break;
-            default: fn = reinterpret_cast<const void*>(&stokes_grad_b4_kernel<4>); break;
-        }
-    } else if (fused && f16) {
-        switch (a.n_at) {
-            case 1: fn = reinterpret_cast<const void*>(&stokes_grad_f16_kernel<1>); break;
-            case 2: fn = reinterpret_cast<const void*>(&stokes_grad_f16_kernel<2>); break;
-            case 3: fn = reinterpret_cast<const void*>(&stokes_grad_f16_kernel<3>); break;
-            case 4: fn = reinterpret_cast<const void*>(&stokes_grad_f16_kernel<4>); break;
-            case 5: fn = reinterpret_cast<const void*>(&stokes_grad_f16_kernel<5>); break;
-            case 6: fn = reinterpret_cast<const void*>(&stokes_grad_f16_kernel<6>); break;
-            case 7: fn = reinterpret_cast<const void*>(&stokes_grad_f16_kernel<7>); break;
-            default: fn = reinterpret_cast<const void*>(&stokes_grad_f16_kernel<8>); break;
-        }
-    } else if (fused) {
-        switch (a.n_at) {
-            case 1: fn = reinterpret_cast<const void*>(&stokes_grad_kernel<1>); break;
-            case 2: fn = reinterpret_cast<const void*>(&stokes_grad_kernel<2>); break;
-            case 3: fn = reinterpret_cast<const void*>(&stokes_grad_kernel<3>); break;
-            case 4: fn = reinterpret_cast<const void*>(&stokes_grad_kernel<4>); break;
-            case 5: fn = reinterpret_cast<const void*>(&stokes_grad_kernel<5>); break;
-            case 6: fn = reinterpret_cast<const void*>(&stokes_grad_kernel<6>); break;
-            case 7: fn = reinterpret_cast<const void*>(&stokes_grad_kernel<7>); break;
-            default: fn = reinterpret_cast<const void*>(&stokes_grad_kernel<8>); break;
-        }
-    } else {
-        fn = reinterpret_cast<const void*>(&adjoint_kernel);
-    }
+#define ADJ_FN(...) reinterpret_cast<const void*>(&__VA_ARGS__)
+    static const void* const fn_b4[4] = {ADJ_FN(stokes_grad_b4_kernel<1>), ADJ_FN(stokes_grad_b4_kernel<2>), ADJ_FN(stokes_grad_b4_kernel<3>), ADJ_FN(stokes_grad_b4_kernel<4>)};
+    static const void* const fn_f16[ADJ_MAXAT] = {ADJ_FN(stokes_grad_f16_kernel<1>), ADJ_FN(stokes_grad_f16_kernel<2>), ADJ_FN(stokes_grad_f16_kernel<3>), ADJ_FN(stokes_grad_f16_kernel<4>), ADJ_FN(stokes_grad_f16_kernel<5>), ADJ_FN(stokes_grad_f16_kernel<6>), ADJ_FN(stokes_grad_f16_kernel<7>), ADJ_FN(stokes_grad_f16_kernel<8>)};
+    static const void* const fn_f32[ADJ_MAXAT] = {ADJ_FN(stokes_grad_kernel<1>), ADJ_FN(stokes_grad_kernel<2>), ADJ_FN(stokes_grad_kernel<3>), ADJ_FN(stokes_grad_kernel<4>), ADJ_FN(stokes_grad_kernel<5>), ADJ_FN(stokes_grad_kernel<6>), ADJ_FN(stokes_grad_kernel<7>), ADJ_FN(stokes_grad_kernel<8>)};
+    static const void* const fn_adj[2][ADJ_MAXAT] = {
+        {ADJ_FN(adjoint_kernel<1, false>), ADJ_FN(adjoint_kernel<2, false>), ADJ_FN(adjoint_kernel<3, false>), ADJ_FN(adjoint_kernel<4, false>), ADJ_FN(adjoint_kernel<5, false>), ADJ_FN(adjoint_kernel<6, false>), ADJ_FN(adjoint_kernel<7, false>), ADJ_FN(adjoint_kernel<8, false>)},
+        {ADJ_FN(adjoint_kernel<1, true>), ADJ_FN(adjoint_kernel<2, true>), ADJ_FN(adjoint_kernel<3, true>), ADJ_FN(adjoint_kernel<4, true>), ADJ_FN(adjoint_kernel<5, true>), ADJ_FN(adjoint_kernel<6, true>), ADJ_FN(adjoint_kernel<7, true>), ADJ_FN(adjoint_kernel<8, true>)}};
+#undef ADJ_FN
+    const bool vec = T % 4 == 0 && (uintptr_t)input % 16 == 0 && (uintptr_t)grad_out % 16 == 0;
+    const int k_at = a.n_at - 1;
+    const void* fn = b4 ? fn_b4[k_at] : !fused ? fn_adj[vec][k_at] : f16 ? fn_f16[k_at] : fn_f32[k_at];
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
@@ -985,40 +993,9 @@ static int run_adjoint(bool fused, bool f16, const void* input, const void* phas
             return BLADE_HIP_ERROR;
         }
     }
-    dim3 grid((unsigned)nsplit, (unsigned)F, (unsigned)a.btiles);
-    const dim3 blk(64 * ADJ_WAVES);
-    if (b4) {
-        switch (a.n_at) {
-            case 1: hipLaunchKernelGGL(stokes_grad_b4_kernel<1>, grid, blk, lds, s, a); break;
-            case 2: hipLaunchKernelGGL(stokes_grad_b4_kernel<2>, grid, blk, lds, s, a); break;
-            case 3: hipLaunchKernelGGL(stokes_grad_b4_kernel<3>, grid, blk, lds, s, a); break;
-            default: hipLaunchKernelGGL(stokes_grad_b4_kernel<4>, grid, blk, lds, s, a); break;
-        }
-    } else if (fused && f16) {
-        switch (a.n_at) {
-            case 1: hipLaunchKernelGGL(stokes_grad_f16_kernel<1>, grid, blk, lds, s, a); break;
-            case 2: hipLaunchKernelGGL(stokes_grad_f16_kernel<2>, grid, blk, lds, s, a); break;
-            case 3: hipLaunchKernelGGL(stokes_grad_f16_kernel<3>, grid, blk, lds, s, a); break;
-            case 4: hipLaunchKernelGGL(stokes_grad_f16_kernel<4>, grid, blk, lds, s, a); break;
-            case 5: hipLaunchKernelGGL(stokes_grad_f16_kernel<5>, grid, blk, lds, s, a); break;
-            case 6: hipLaunchKernelGGL(stokes_grad_f16_kernel<6>, grid, blk, lds, s, a); break;
-            case 7: hipLaunchKernelGGL(stokes_grad_f16_kernel<7>, grid, blk, lds, s, a); break;
-            default: hipLaunchKernelGGL(stokes_grad_f16_kernel<8>, grid, blk, lds, s, a); break;
-        }
-    } else if (fused) {
-        switch (a.n_at) {
-            case 1: hipLaunchKernelGGL(stokes_grad_kernel<1>, grid, dim3(64 * ADJ_WAVES), lds, s, a); break;
-            case 2: hipLaunchKernelGGL(stokes_grad_kernel<2>, grid, dim3(64 * ADJ_WAVES), lds, s, a); break;
-            case 3: hipLaunchKernelGGL(stokes_grad_kernel<3>, grid, dim3(64 * ADJ_WAVES), lds, s, a); break;
-            case 4: hipLaunchKernelGGL(stokes_grad_kernel<4>, grid, dim3(64 * ADJ_WAVES), lds, s, a); break;
-            case 5: hipLaunchKernelGGL(stokes_grad_kernel<5>, grid, dim3(64 * ADJ_WAVES), lds, s, a); break;
-            case 6: hipLaunchKernelGGL(stokes_grad_kernel<6>, grid, dim3(64 * ADJ_WAVES), lds, s, a); break;
-            case 7: hipLaunchKernelGGL(stokes_grad_kernel<7>, grid, dim3(64 * ADJ_WAVES), lds, s, a); break;
-            default: hipLaunchKernelGGL(stokes_grad_kernel<8>, grid, dim3(64 * ADJ_WAVES), lds, s, a); break;
-        }
-    } else {
-        hipLaunchKernelGGL(adjoint_kernel, grid, dim3(64 * ADJ_WAVES), lds, s, a);
-    }
+    const dim3 grid((unsigned)nsplit, (unsigned)F, (unsigned)a.btiles);
+    void* args[] = {&a};
+    (void)hipLaunchKernel(fn, grid, dim3(64 * ADJ_WAVES), args, lds, s);   // check_launch below reports
     const size_t n = (size_t)F * 2 * a.btiles * 8 * A;
     hipLaunchKernelGGL(adjoint_reduce_kernel, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, s, a,
                        (int)nsplit, static_cast<float2*>(grad_phasors));

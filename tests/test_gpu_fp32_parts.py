@@ -67,3 +67,27 @@ def test_nonfinite_phasors_stay_in_their_beam():
         y = ops.beamformer(torch.from_numpy(x8).cuda(), torch.from_numpy(w).cuda()).cpu().numpy()
     assert not np.isfinite(y[1, :, :, 0]).any() and not np.isfinite(y[2, :, :, 1]).any()
     assert np.isfinite(y[[0, 3]]).all() and np.isfinite(y[1, :, :, 1]).all() and np.isfinite(y[2, :, :, 0]).all()
+
+
+@pytest.mark.parametrize("A,B", [(1, 1), (16, 8), (17, 9), (42, 4), (64, 3), (80, 2), (96, 5), (128, 17)])
+@pytest.mark.parametrize("T,offset", [(1, 0), (31, 0), (32, 0), (132, 0), (130, 0), (260, 1)])
+def test_adjoint_matches_oracle_elementwise(A, B, T, offset):
+    """sum_t gy conj(x): 2T exact products accumulated in FP32, the sums of the
+    four waves and of the time splits after them; ``offset`` float2s shift the
+    gradient off 16-byte alignment (single loads)."""
+    rng = np.random.default_rng(A + 10 * T)
+    x8 = rng.integers(-128, 128, size=(A, 3, T, 2, 2), dtype=np.int8)
+    gy = (10.0 ** rng.uniform(-6, 6, size=(B, 1, 1, 1)) *
+          (rng.normal(size=(B, 3, T, 2)) + 1j * rng.normal(size=(B, 3, T, 2)))).astype(np.complex64)
+    buf = torch.empty(gy.size + offset, dtype=torch.complex64, device="cuda")
+    gyd = buf[offset:].view(gy.shape)
+    gyd.copy_(torch.from_numpy(gy))
+    got = ops.beamformer_adjoint(torch.from_numpy(x8).cuda(), gyd).cpu().numpy()
+    ref = O.beamformer_adjoint(x8, gy)
+    g1 = np.abs(gy.real.astype(np.float64)) + np.abs(gy.imag.astype(np.float64))
+    x1 = np.abs(x8[..., 0].astype(np.float64)) + np.abs(x8[..., 1].astype(np.float64))
+    bound = 2 * (2 * T + 16) * 2.0 ** -24 * np.einsum("bftp,aftp->bafp", g1, x1)[:, :, :, None]
+    d = got - ref
+    assert (np.maximum(np.abs(d.real), np.abs(d.imag)) <= bound).all()
+    again = ops.beamformer_adjoint(torch.from_numpy(x8).cuda(), gyd).cpu().numpy()
+    assert (again == got).all()

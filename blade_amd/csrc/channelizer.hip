@@ -33,14 +33,28 @@ __global__ void twiddle_kernel(float2* tw, int C) {
 // kernel store into, so that every lane issues the same stores.
 constexpr size_t kTwiddleSinkBytes = 512 * sizeof(float4);
 
+// W_C^(n1 k2) as a matrix [n1][k2] with rows of N2 entries: between the two
+// passes of the four-step FFT lanes with consecutive k2 read consecutive
+// entries.  Stored under the negated rate.
+__global__ void twiddle_matrix_kernel(float2* tw, int C, int N2) {
+    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (m < C) {
+        double s, c;
+        sincospi(-2.0 * (double)((m / N2) * (m % N2)) / (double)C, &s, &c);
+        tw[m] = make_float2((float)c, (float)s);
+    }
+}
+
 static std::mutex g_tw_mutex;
 static std::map<std::pair<int, int>, float2*> g_tw;
 
-static int get_twiddles(int C, hipStream_t s, const float2** out) {
+// The table of rate C, or with N2 > 0 the matrix of C = N1 N2.
+static int get_twiddles(int C, hipStream_t s, const float2** out, int N2 = 0) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fail("channelizer: hipGetDevice failed");
     std::lock_guard<std::mutex> lock(g_tw_mutex);
-    auto it = g_tw.find({dev, C});
+    const std::pair<int, int> key(dev, N2 > 0 ? -C : C);
+    auto it = g_tw.find(key);
     if (it != g_tw.end()) {
         *out = it->second;
         return BLADE_SUCCESS;
@@ -51,10 +65,13 @@ static int get_twiddles(int C, hipStream_t s, const float2** out) {
         set_error(std::string("channelizer: twiddle allocation: ") + hipGetErrorString(e));
         return BLADE_HIP_ERROR;
     }
-    hipLaunchKernelGGL(twiddle_kernel, dim3((C + 255) / 256), dim3(256), 0, s, p, C);
+    if (N2 > 0)
+        hipLaunchKernelGGL(twiddle_matrix_kernel, dim3((C + 255) / 256), dim3(256), 0, s, p, C, N2);
+    else
+        hipLaunchKernelGGL(twiddle_kernel, dim3((C + 255) / 256), dim3(256), 0, s, p, C);
     int rc = check_launch("channelizer twiddles");
     if (rc) return rc;
-    g_tw[{dev, C}] = p;
+    g_tw[key] = p;
     *out = p;
     return BLADE_SUCCESS;
 }
@@ -1350,6 +1367,195 @@ static int launch_fft16(int C, const float2* in, void* out, uint64_t S, uint64_t
     return 0;
 }
 
+// ---------------------------------------------------------------------------
+// Two polarizations at C = 2^14, 2^15 and 2^16: the four-step FFT of
+// chan_big_pass1/2 with both passes on registers.  A pass transforms columns
+// of N = 128 or 256 points: a thread holds 16 points of both polarizations,
+// loaded straight from memory (all 16 loads in flight), takes a radix-16
+// butterfly, exchanges with its column through LDS one polarization at a time
+// (half the LDS: 4 workgroups per CU hide each other's loads), and finishes
+// with a radix-8 or 16 butterfly.  COLS = 16 or 32 neighbouring columns per
+// workgroup make every global access a run of 256 or 512 bytes.  Pass 1's
+// last butterfly is dealt to lanes along k2 instead of along the columns, so
+// that its stores into the scratch rows [n1][k2] are runs too.
+// LDS columns are N + N/16 + 2 float2 apart (18 or 10 mod 32): columns land on
+// even banks and neighbouring butterflies on odd ones.
+// Both passes stream at 5-6 TB/s.  Input and output bypass the caches
+// (nontemporal) and the spectra go through the passes in groups of 192 MiB of
+// scratch, part of which the 256 MB last-level cache then holds between the
+// passes: 376 us on [3,192,65536,2] at C = 65536 (1.2 GB in and out), against
+// 398 in one group, 456 with plain accesses, 400 at 128 and 454 at 64 MiB
+// (too few workgroups per launch), and 1459 with the runtime-radix passes of
+// chan_big_pass1/2.
+// ---------------------------------------------------------------------------
+template <int LN>
+struct FourStep {
+    static constexpr int N = 1 << LN;
+    static constexpr int TPC = N / 16;                 // threads per column
+    static constexpr int COLS = 256 / TPC;             // columns per workgroup of 256
+    static constexpr int CS = N + N / 16 + 2;          // LDS column stride, float2
+    static constexpr int R2 = N / 16;                  // radix of the second butterfly
+    static constexpr int G2 = 16 / R2;                 // second butterflies per thread
+    static constexpr size_t LDS = sizeof(float2) * ((size_t)COLS * CS + N);
+};
+
+// Columns of N points, points `stride` float4s apart.  FIRST: in = spectra
+// [n_spec][C], out = scratch [n_spec][N1][N2], times W_C^(n1 k2) (twm).
+// Second: in = scratch, out = fftshifted bins at [af, k2 + N2 k1, s].
+template <int LN, bool FIRST, bool NTS>
+__global__ __launch_bounds__(256, 4) void four_step_kernel(const float4* __restrict__ in, float4* __restrict__ out,
+                                                           int other, uint64_t sp0, uint64_t S,
+                                                           const float2* __restrict__ tw,
+                                                           const float2* __restrict__ twm) {
+    typedef FourStep<LN> K;
+    constexpr int N = K::N, TPC = K::TPC, COLS = K::COLS;
+    extern __shared__ float2 lds[];
+    float2* const twl = lds + COLS * K::CS;
+    // blockIdx.x = (spectrum of this group, tile of columns); `other` = the
+    // length of the other pass = columns per spectrum.
+    const unsigned tiles = (unsigned)other / COLS;
+    const unsigned b = (gridDim.x & 7u) ? blockIdx.x : xcd_order(blockIdx.x, gridDim.x);
+    // Second pass: neighbouring workgroups take the same tile of neighbouring
+    // spectra of one (antenna, channel), whose bins interleave at S.
+    const unsigned Su = (unsigned)S;
+    unsigned sp, tile;
+    if (FIRST || Su == 1) {
+        sp = b / tiles;
+        tile = b - sp * tiles;
+    } else {
+        const unsigned af = b / (tiles * Su), r = b - af * (tiles * Su);
+        tile = r / Su;
+        sp = af * Su + (r - tile * Su);
+    }
+    const unsigned c0 = tile * COLS;
+    const size_t C = (size_t)N * other;
+    for (int e = threadIdx.x; e < N; e += 256) twl[e] = tw[e];
+
+    const int c = threadIdx.x % COLS, j = threadIdx.x / COLS;
+    float2 v[2][16];
+    {
+        const float4* const src = in + (FIRST ? sp0 + sp : sp) * C + c0 + c;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const float* const q = reinterpret_cast<const float*>(src + (unsigned)((j + r * TPC) * other));
+            v[0][r] = make_float2(__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1));
+            v[1][r] = make_float2(__builtin_nontemporal_load(q + 2), __builtin_nontemporal_load(q + 3));
+        }
+    }
+    // Second butterflies: column c2, butterflies j2 + g TPC.
+    const int c2 = FIRST ? threadIdx.x / TPC : c;
+    const int j2 = FIRST ? threadIdx.x % TPC : j;
+    float2* const wr = lds + c * K::CS + j * 17;
+    const float2* const rd = lds + c2 * K::CS + j2;
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        dft16(v[p]);
+        if (p) __syncthreads();            // polarization 0 has been read
+#pragma unroll
+        for (int r = 0; r < 16; r++) wr[r] = v[p][r];
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < K::G2; g++) {
+            float2 x[K::R2];
+#pragma unroll
+            for (int r = 0; r < K::R2; r++) {
+                x[r] = rd[g * TPC + 17 * r];
+                if (r > 0) x[r] = cmul(x[r], twl[(j2 + g * TPC) * r]);
+            }
+            dft_pow2<K::R2>(x);
+#pragma unroll
+            for (int r = 0; r < K::R2; r++) v[p][g * K::R2 + r] = x[r];
+        }
+    }
+    if constexpr (FIRST) {
+        const unsigned n1 = c0 + c2;
+        float4* const dst = out + (size_t)sp * C + (size_t)n1 * N + j2;
+        const float2* const w = twm + (size_t)n1 * N + j2;
+#pragma unroll
+        for (int g = 0; g < K::G2; g++)
+#pragma unroll
+            for (int r = 0; r < K::R2; r++) {
+                const int k = g * TPC + 16 * r;
+                const float2 wk = w[k];
+                const float2 X = cmul(v[0][g * K::R2 + r], wk), Y = cmul(v[1][g * K::R2 + r], wk);
+                dst[k] = make_float4(X.x, X.y, Y.x, Y.y);
+            }
+    } else {
+        const uint64_t spg = sp0 + sp, af = spg / S, s = spg - af * S;
+        float4* const dst = out + (af * C + c0 + c) * S + s;
+#pragma unroll
+        for (int g = 0; g < K::G2; g++)
+#pragma unroll
+            for (int r = 0; r < K::R2; r++) {
+                const unsigned k1 = (unsigned)(j2 + g * TPC + 16 * r) ^ (N / 2);    // fftshift
+                const float2 X = v[0][g * K::R2 + r], Y = v[1][g * K::R2 + r];
+                float4* const o = dst + (size_t)(k1 * other) * S;
+                if constexpr (NTS) {
+                    float* const of = reinterpret_cast<float*>(o);
+                    __builtin_nontemporal_store(X.x, of);
+                    __builtin_nontemporal_store(X.y, of + 1);
+                    __builtin_nontemporal_store(Y.x, of + 2);
+                    __builtin_nontemporal_store(Y.y, of + 3);
+                } else {
+                    *o = make_float4(X.x, X.y, Y.x, Y.y);
+                }
+            }
+    }
+}
+
+constexpr size_t kFourStepScratch = 192ull << 20;
+
+static bool use_four_step(int C, int P) { return P == 2 && (C == 1 << 14 || C == 1 << 15 || C == 1 << 16); }
+
+// C = N1 N2 = 2^ln1 2^ln2.
+static void four_step_lengths(int C, int* ln1, int* ln2) {
+    *ln2 = C == 1 << 14 ? 7 : 8;
+    *ln1 = C == 1 << 16 ? 8 : 7;
+}
+
+static int launch_four_step(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec, hipStream_t s) {
+    int ln1, ln2;
+    four_step_lengths(C, &ln1, &ln2);
+    int N1 = 1 << ln1, N2 = 1 << ln2;
+    const float2 *twm = nullptr, *tw1 = nullptr, *tw2 = nullptr;
+    int rc = get_twiddles(C, s, &twm, N2);
+    if (!rc) rc = get_twiddles(N1, s, &tw1);
+    if (!rc) rc = get_twiddles(N2, s, &tw2);
+    if (rc) return rc;
+    // Spectra per group.  In place, a group's output must not reach input that
+    // is still to be read: whole (antenna, channel)s when input and output are
+    // the same, everything at once when they overlap otherwise.  Groups are
+    // whole (antenna, channel)s where bins of several spectra interleave.
+    const size_t bytes = sizeof(float4) * (size_t)C;
+    const char* pi = reinterpret_cast<const char*>(in);
+    const char* po = reinterpret_cast<const char*>(out);
+    const bool overlap = pi < po + bytes * n_spec && po < pi + bytes * n_spec;
+    uint64_t group = std::max<uint64_t>(S, kFourStepScratch / bytes / S * S);
+    if (overlap && pi != po) group = n_spec;
+    group = std::min<uint64_t>(group, n_spec);
+    unsigned char* scratch = nullptr;
+    rc = library_workspace(WS_CHANNELIZER_BIG, bytes * group, s, &scratch);
+    if (rc) return rc;
+    float4* y = reinterpret_cast<float4*>(scratch);
+    const float4* in4 = reinterpret_cast<const float4*>(in);
+    float4* out4 = reinterpret_cast<float4*>(out);
+#define FS_FN(...) reinterpret_cast<const void*>(&four_step_kernel<__VA_ARGS__>)
+    const void* first = ln2 == 8 ? FS_FN(8, true, false) : FS_FN(7, true, false);
+    const void* second = S == 1 ? (ln1 == 8 ? FS_FN(8, false, true) : FS_FN(7, false, true))
+                                : (ln1 == 8 ? FS_FN(8, false, false) : FS_FN(7, false, false));
+#undef FS_FN
+    for (uint64_t sp = 0; sp < n_spec; sp += group) {
+        const uint64_t n = std::min<uint64_t>(group, n_spec - sp);
+        const dim3 g1((unsigned)(n * N1 / (ln2 == 8 ? FourStep<8>::COLS : FourStep<7>::COLS)));
+        const dim3 g2((unsigned)(n * N2 / (ln1 == 8 ? FourStep<8>::COLS : FourStep<7>::COLS)));
+        void* args1[] = {&in4, &y, &N1, &sp, &S, &tw2, &twm};
+        void* args2[] = {&y, &out4, &N2, &sp, &S, &tw1, &twm};
+        (void)hipLaunchKernel(first, g1, dim3(256), args1, ln2 == 8 ? FourStep<8>::LDS : FourStep<7>::LDS, s);
+        (void)hipLaunchKernel(second, g2, dim3(256), args2, ln1 == 8 ? FourStep<8>::LDS : FourStep<7>::LDS, s);
+    }
+    return check_launch("channelizer");
+}
+
 // Direct O(C^2) DFT for rates with prime factors above 7.
 template <int P>
 __global__ __launch_bounds__(256) void chan_direct_kernel(const float2* __restrict__ in,
@@ -1531,6 +1737,7 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     if ((uint64_t)C * P > (uint64_t)kMaxLdsComplex) {
         // Past one workgroup's LDS: two passes through a scratch buffer (which
         // also makes any in-place call safe).
+        if (use_four_step(C, (int)P)) return launch_four_step(C, in, out, S, n_spec, s);
         BigPlan pl;
         if (!big_plan(C, (int)P, &pl))
             return fail("channelizer: rate must be even, at most 2^20, and factor into 2, 3, 5 and 7");
@@ -1598,6 +1805,14 @@ extern "C" int blade_channelizer_plan(uint64_t rate, blade_stream_t stream) {
     const float2* tw = nullptr;
     int rc = get_twiddles((int)rate, s, &tw);
     if (rc) return rc;
+    if (use_four_step((int)rate, 2)) {
+        int ln1, ln2;
+        four_step_lengths((int)rate, &ln1, &ln2);
+        rc = get_twiddles((int)rate, s, &tw, 1 << ln2);
+        if (!rc) rc = get_twiddles(1 << ln1, s, &tw);
+        if (!rc) rc = get_twiddles(1 << ln2, s, &tw);
+        if (rc) return rc;
+    }
     BigPlan pl;   // the two-pass FFT's tables (for two polarizations)
     if (rate * 2 > (uint64_t)kMaxLdsComplex && big_plan((int)rate, 2, &pl)) {
         rc = get_twiddles(pl.N1, s, &tw);

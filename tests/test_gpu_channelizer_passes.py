@@ -1,0 +1,59 @@
+"""Channelizer kernels at the edges of their plans, against the FP64 DFT.
+
+Bar: an FFT of C points rounds about 2 log2(C) times on the way of a value
+(one butterfly level and one twiddle each), so the normwise relative error is
+within 2 log2(C) * 2^-24 (random rounding leaves it well below).
+"""
+
+import math
+
+import pytest
+import torch
+
+from blade_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _spectra(x, C):
+    A, F, T, P = x.shape
+    v = x.to(torch.complex128).reshape(A, F, T // C, C, P)
+    return torch.fft.fftshift(torch.fft.fft(v, dim=3), dim=3).permute(0, 1, 3, 2, 4).reshape(A, F * C, T // C, P)
+
+
+def _rand(seed, *shape):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(shape, dtype=torch.complex64, device="cuda", generator=gen)
+
+
+def _err(y, ref):
+    return float((y.to(ref.dtype) - ref).abs().square().sum().sqrt() / ref.abs().square().sum().sqrt())
+
+
+def _bar(C):
+    return 2 * math.log2(C) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("A,F,S,C", [(1, 1, 1, 16384), (1, 3, 1, 16384), (1, 5, 2, 16384), (2, 1, 3, 32768),
+                                     (1, 1, 1, 65536), (1, 3, 2, 65536)])
+def test_four_step(A, F, S, C):
+    # odd spectrum counts leave a grid that is no multiple of 8 workgroups
+    x = _rand(C + S, A, F, S * C, 2)
+    assert _err(ops.channelizer(x, C), _spectra(x, C)) <= _bar(C)
+
+
+@pytest.mark.parametrize("alias", ["none", "same", "shifted"])
+def test_four_step_groups(alias):
+    """802 spectra (one group of the 192 MiB scratch and a short one), two per
+    channel: apart, in place, and with the output one channel behind the input
+    in the same buffer."""
+    C, S, F = 16384, 2, 401
+    n = F * S * C * 2
+    buf = _rand(9, n + S * C * 2)
+    off = S * C * 2 if alias == "shifted" else 0
+    x = buf[off:off + n].view(1, F, S * C, 2)
+    ref = _spectra(x[:, [0, 1, 382, 383, 384, 385, 400]], C)
+    out = torch.empty_like(buf[:n]) if alias == "none" else buf[:n]
+    y = ops.channelizer(x, C, out=out.view(1, F * C, S, 2))
+    y = y.view(F, C, S, 2)[[0, 1, 382, 383, 384, 385, 400]].reshape(1, 7 * C, S, 2)
+    assert _err(y, ref) <= _bar(C)

@@ -101,10 +101,12 @@ __device__ __forceinline__ uint32_t ci8_to_bf16(uint32_t d, int p) {
 // v = part[0] + part[1] + part[2] exactly, each part with the 8 significant
 // bits of BF16 (in the high half of its float): an FP32 value has 24, so
 // cutting 8 off the top three times leaves nothing (parts below FP32's normal
-// range aside).  Infinities and NaN stay in part 0.
+// range aside).  Infinities and NaN stay in part 0 (CHECKED; otherwise they
+// become NaN).
+template <bool CHECKED = true>
 __device__ __forceinline__ void split_bf16x3(float v, float (&part)[3]) {
     const uint32_t u = __float_as_uint(v);
-    if ((u & 0x7f800000u) == 0x7f800000u) {
+    if (CHECKED && (u & 0x7f800000u) == 0x7f800000u) {
         part[0] = __uint_as_float((u & 0x007fffffu) ? (u | 0x00400000u) : u);
         part[1] = part[2] = 0.f;
         return;

@@ -91,3 +91,46 @@ def test_adjoint_matches_oracle_elementwise(A, B, T, offset):
     assert (np.maximum(np.abs(d.real), np.abs(d.imag)) <= bound).all()
     again = ops.beamformer_adjoint(torch.from_numpy(x8).cuda(), gyd).cpu().numpy()
     assert (again == got).all()
+
+
+@pytest.mark.parametrize("A,B", [(1, 1), (16, 8), (17, 9), (42, 4), (48, 3), (64, 5), (65, 2), (96, 2), (128, 17)])
+@pytest.mark.parametrize("T,offset", [(1, 0), (63, 0), (64, 0), (68, 0), (260, 0), (261, 0), (512, 1)])
+def test_stokes_gradient_matches_oracle_elementwise(A, B, T, offset):
+    """y as in the forward test (error ey); gy = -lambda y rounds once; the
+    adjoint accumulates 2T terms and the partial sums.  ``offset`` shifts the
+    voltages off 16-byte alignment (single loads)."""
+    rng = np.random.default_rng(A + 10 * T)
+    x8 = rng.integers(-128, 128, size=(A, 2, T, 2, 2), dtype=np.int8)
+    w = (10.0 ** rng.uniform(-4, 4, size=(B, 1, 1, 1, 1)) *
+         (rng.normal(size=(B, A, 2, 1, 2)) + 1j * rng.normal(size=(B, A, 2, 1, 2)))).astype(np.complex64)
+    lam = [float(np.float32(v)) for v in rng.uniform(0.1, 1.0, size=B)]
+    buf = torch.empty(x8.size + 4 * offset, dtype=torch.int8, device="cuda")
+    xd = buf[4 * offset:].view(x8.shape)
+    xd.copy_(torch.from_numpy(x8))
+    loss, got = ops.stokes_i_loss_and_grad(xd, torch.from_numpy(w).cuda(), lam)
+    got = got.cpu().numpy()[:, :, :, 0]
+    x = x8[..., 0].astype(np.float64) + 1j * x8[..., 1]
+    y = np.einsum("bafp,aftp->bftp", w[:, :, :, 0].astype(np.complex128), x)
+    L = np.array(lam)[:, None, None, None]
+    ref = np.einsum("bftp,aftp->bafp", -L * y, x.conj())
+    x1 = np.abs(x.real) + np.abs(x.imag)
+    w1 = np.abs(w.real[:, :, :, 0].astype(np.float64)) + np.abs(w.imag[:, :, :, 0].astype(np.float64))
+    u = 2.0 ** -24
+    ey = 2 * (2 * A + 2) * u * np.einsum("bafp,aftp->bftp", w1, x1)
+    y1 = np.abs(y.real) + np.abs(y.imag) + 2 * ey
+    bound = np.einsum("bftp,aftp->bafp", L * (2 * ey + (2 * (2 * T + 16) + 2) * u * y1), x1)
+    d = got - ref
+    assert (np.maximum(np.abs(d.real), np.abs(d.imag)) <= bound).all()
+    power = float((L * np.abs(y) ** 2).sum())
+    assert abs(float(loss) + power) <= float((L * (2 * np.sqrt(2) * np.abs(y) * ey + ey ** 2 + 64 * u * np.abs(y) ** 2)).sum())
+
+
+def test_stokes_gradient_keeps_nonfinite_values_in_their_beam():
+    rng = np.random.default_rng(1)
+    x8 = rng.integers(-128, 128, size=(20, 1, 128, 2, 2), dtype=np.int8)
+    w = (rng.normal(size=(3, 20, 1, 1, 2)) + 1j * rng.normal(size=(3, 20, 1, 1, 2))).astype(np.complex64)
+    w[1, 4, 0, 0, 0] = np.inf
+    _, got = ops.stokes_i_loss_and_grad(torch.from_numpy(x8).cuda(), torch.from_numpy(w).cuda(), [1.0, 1.0, 1.0])
+    got = got.cpu().numpy()
+    assert np.isfinite(got[[0, 2]]).all() and np.isfinite(got[1, ..., 1]).all()
+    assert not np.isfinite(got[1, ..., 0]).any()

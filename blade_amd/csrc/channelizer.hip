@@ -416,11 +416,10 @@ __global__ __launch_bounds__(1024) void chan_big_pass2(const float2* __restrict_
 }
 
 // Channelizer with the detector fused on the output: one workgroup per
-// (a, f) walks its S = T/C spectra, transforms both pols in LDS and
-// integrates |X|^2+|Y|^2 (or XX*, YY*, Re XY*, Im XY*) of every fine channel
-// over N consecutive spectra in registers, writing
-//   out[a, f*C + k', s/N, q]   (N <= S, N | S)
-//   out[a, f*C + k', 0, q]    (+=) when N spans several blocks (accumulate).
+// integration walks its S spectra, transforms both pols in LDS and sums
+// |X|^2+|Y|^2 (or XX*, YY*, Re XY*, Im XY*) of every fine channel over them in
+// registers, writing (or adding to, with accumulate)
+//   out[a, f*C + k', group, q].
 // The CF32 spectra never reach HBM.
 // Detector sums of (X, Y) turned into those of (L, R) = (X + jY, X - jY),
 // the polarizer (polarizer.cu:5-25) applied before the detector: sums are
@@ -443,23 +442,22 @@ __device__ inline void circular_sums(float (&a)[NPOL]) {
 template <int NPOL, int KPT>
 __global__ __launch_bounds__(1024) void chan_detect_kernel(const float2* __restrict__ in,
                                                            float* __restrict__ out, int C,
-                                                           int S, int N, uint64_t n_af,
+                                                           int S, int groups, uint64_t n_items,
                                                            const float2* __restrict__ tw,
                                                            Radices rad, int flags) {
     extern __shared__ float2 data[];
     const int accumulate = flags & 1;
     const bool circular = flags & 2;
     const int PC = 2 * C;
-    const int groups = (N <= S) ? S / N : 1;
     const int half = C / 2;
-    for (uint64_t af = blockIdx.x; af < n_af; af += gridDim.x) {
+    for (uint64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
         float acc[KPT][NPOL];
 #pragma unroll
         for (int j = 0; j < KPT; j++)
 #pragma unroll
             for (int q = 0; q < NPOL; q++) acc[j][q] = 0.f;
         for (int s = 0; s < S; s++) {
-            const float4* src = reinterpret_cast<const float4*>(in + ((af * S + s) * (uint64_t)C) * 2);
+            const float4* src = reinterpret_cast<const float4*>(in + ((item * S + s) * (uint64_t)C) * 2);
             for (int n = threadIdx.x; n < C; n += blockDim.x) {
                 const float4 q = src[n];
                 data[n] = make_float2(q.x, q.y);
@@ -493,9 +491,9 @@ __global__ __launch_bounds__(1024) void chan_detect_kernel(const float2* __restr
                 }
             }
             __syncthreads();
-            const bool flush = (N <= S) ? ((s + 1) % N == 0) : (s == S - 1);
-            if (flush) {
-                const int grp = (N <= S) ? s / N : 0;
+            if (s == S - 1) {
+                const uint64_t af = item / (unsigned)groups;
+                const unsigned grp = (unsigned)(item - af * (unsigned)groups);
                 if (circular) {
 #pragma unroll
                     for (int j = 0; j < KPT; j++) circular_sums<NPOL>(acc[j]);
@@ -534,7 +532,7 @@ __global__ __launch_bounds__(1024) void chan_detect_kernel(const float2* __restr
 template <int MODE, int RL>
 __global__ __launch_bounds__(1024) void fft2_kernel(const float4* __restrict__ in, void* __restrict__ outv,
                                                     int C, int nmid, uint64_t S, uint64_t n_items,
-                                                    int N, int flags,
+                                                    int groups, int flags,
                                                     const float2* __restrict__ tw) {
     extern __shared__ float2 data[];
     const int accumulate = flags & 1;
@@ -549,7 +547,6 @@ __global__ __launch_bounds__(1024) void fft2_kernel(const float4* __restrict__ i
     const uint64_t per_round = (uint64_t)gridDim.x * spw;
     const uint64_t rounds = (n_items + per_round - 1) / per_round;
     const int nspec = MODE == 0 ? 1 : (int)S;
-    const int groups = MODE == 0 ? 1 : ((N <= (int)S) ? (int)S / N : 1);
     const int lastR = C / RL;                   // stride of the last pass
 
     auto item_of = [&](uint64_t round) { return (round * gridDim.x + blockIdx.x) * spw + slot; };
@@ -639,9 +636,14 @@ __global__ __launch_bounds__(1024) void fft2_kernel(const float4* __restrict__ i
                 }
             }
             if constexpr (MODE != 0) {
-                const bool flush = (N <= (int)S) ? ((s + 1) % N == 0) : (s == (int)S - 1);
-                if (flush) {
-                    const int grp = (N <= (int)S) ? s / N : 0;
+                if (s == nspec - 1) {
+                    // items fit 32 bits (host check); one integration per
+                    // channel needs no division
+                    unsigned af = (unsigned)item, grp = 0;
+                    if (groups != 1) {
+                        af = (unsigned)item / (unsigned)groups;
+                        grp = (unsigned)item - af * (unsigned)groups;
+                    }
                     float* out = static_cast<float*>(outv);
                     if (circular) {
 #pragma unroll
@@ -656,7 +658,7 @@ __global__ __launch_bounds__(1024) void fft2_kernel(const float4* __restrict__ i
                             if (valid) {
                                 const int k = j + g * tps + r * lastR;
                                 const int ko = (k + (C >> 1)) & (C - 1);
-                                float* o = out + ((item * C + ko) * groups + grp) * NPOL;
+                                float* o = out + (((uint64_t)af * C + ko) * groups + grp) * NPOL;
 #pragma unroll
                                 for (int c = 0; c < NPOL; c++) o[c] = accumulate ? o[c] + acc[g][r][c] : acc[g][r][c];
                             }
@@ -692,7 +694,7 @@ static bool fft2_plan(int C, Fft2Plan* pl) {
 
 template <int MODE>
 static int launch_fft2(const Fft2Plan& pl, const float2* in, void* out, int C, uint64_t S, uint64_t n_items,
-                       int N, int accumulate, const float2* tw, hipStream_t s) {
+                       int groups, int accumulate, const float2* tw, hipStream_t s) {
     const size_t lds = sizeof(float2) * 2 * (size_t)C * pl.spw;
     // One workgroup per SPW spectra: the hardware refills each CU as
     // workgroups finish, which beats persistent rounds here by 2-6%.
@@ -711,11 +713,11 @@ static int launch_fft2(const Fft2Plan& pl, const float2* in, void* out, int C, u
     const float4* in4 = reinterpret_cast<const float4*>(in);
     const dim3 grid((unsigned)blocks), block((unsigned)pl.threads);
     if (pl.rl == 2)
-        hipLaunchKernelGGL((fft2_kernel<MODE, 2>), grid, block, lds, s, in4, out, C, pl.nmid, S, n_items, N, accumulate, tw);
+        hipLaunchKernelGGL((fft2_kernel<MODE, 2>), grid, block, lds, s, in4, out, C, pl.nmid, S, n_items, groups, accumulate, tw);
     else if (pl.rl == 4)
-        hipLaunchKernelGGL((fft2_kernel<MODE, 4>), grid, block, lds, s, in4, out, C, pl.nmid, S, n_items, N, accumulate, tw);
+        hipLaunchKernelGGL((fft2_kernel<MODE, 4>), grid, block, lds, s, in4, out, C, pl.nmid, S, n_items, groups, accumulate, tw);
     else
-        hipLaunchKernelGGL((fft2_kernel<MODE, 8>), grid, block, lds, s, in4, out, C, pl.nmid, S, n_items, N, accumulate, tw);
+        hipLaunchKernelGGL((fft2_kernel<MODE, 8>), grid, block, lds, s, in4, out, C, pl.nmid, S, n_items, groups, accumulate, tw);
     return check_launch("channelizer");
 }
 
@@ -931,9 +933,12 @@ __device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned G) { return (
 // SM (MODE 0 stores): 0 strided, 1 nontemporal with one spectrum per
 // (antenna, channel), 2 transposed through LDS so that the workgroup's SPW
 // consecutive spectra of one (antenna, channel) land as whole lines.
+// Detector items: SM 0 one integration each (S spectra, `ng` = integrations per
+// channel), SM 3 one (antenna, channel) each (S spectra, `ng` = spectra per
+// integration).
 template <int LC, int NT, int MODE, int SM>
 __global__ __launch_bounds__(NT, 2) void fft16_kernel(const float4* __restrict__ in, void* __restrict__ outv,
-                                                      uint64_t S, uint64_t n_items, int N, int flags,
+                                                      uint64_t S, uint64_t n_items, int ng, int flags,
                                                       const float2* __restrict__ tw, float4* __restrict__ sink) {
     const int accumulate = flags & 1;
     const bool circular = flags & 2;
@@ -991,7 +996,6 @@ __global__ __launch_bounds__(NT, 2) void fft16_kernel(const float4* __restrict__
     const uint64_t per_round = (uint64_t)gridDim.x * SPW;
     const uint64_t rounds = (n_items + per_round - 1) / per_round;
     const int nspec = MODE == 0 ? 1 : (int)S;
-    const int groups = MODE == 0 ? 1 : ((N <= (int)S) ? (int)S / N : 1);
 
     // The spectra of a workgroup in one round are consecutive (items first ..
     // first + SPW - 1): addresses are a workgroup-uniform base plus a 32-bit
@@ -1231,15 +1235,21 @@ __global__ __launch_bounds__(NT, 2) void fft16_kernel(const float4* __restrict__
                         acc[i][NPOL > 3 ? 3 : 0] += X.y * Y.x - X.x * Y.y;
                     }
                 }
-                const bool flush = (N <= (int)S) ? ((s + 1) % N == 0) : (s == (int)S - 1);
+                const bool flush = SM == 3 ? ((ng <= (int)S) ? ((s + 1) % ng == 0) : (s == (int)S - 1)) : s == nspec - 1;
                 if (flush) {
-                    const int grp = (N <= (int)S) ? s / N : 0;
+                    const int groups = SM == 3 ? ((ng <= (int)S) ? (int)S / ng : 1) : ng;
+                    uint64_t af = item;
+                    unsigned grp = SM == 3 && ng <= (int)S ? s / ng : 0;
+                    if (SM != 3 && groups != 1) {          // items fit 32 bits (host check)
+                        af = (unsigned)item / (unsigned)groups;
+                        grp = (unsigned)item - (unsigned)af * (unsigned)groups;
+                    }
                     if (circular) {
 #pragma unroll
                         for (int i = 0; i < 16; i++) circular_sums<NPOL>(acc[i]);
                     }
                     const unsigned gn = (unsigned)groups * NPOL;
-                    float* const lb = valid ? static_cast<float*>(outv) + (item * C + ch0) * gn + grp * NPOL
+                    float* const lb = valid ? static_cast<float*>(outv) + (af * C + ch0) * gn + grp * NPOL
                                             : reinterpret_cast<float*>(sink + threadIdx.x);
                     unsigned step = valid ? gn : 0;
                     // Opaque: keeps the 16 output addresses from being hoisted
@@ -1300,7 +1310,7 @@ __global__ __launch_bounds__(NT, 2) void fft16_kernel(const float4* __restrict__
 // Launch of fft16_kernel for C = 2^LC; NT threads use NT * 272 bytes of LDS
 // (one 512-thread workgroup per CU).
 template <int LC, int NT, int MODE, int SM>
-static int launch_fft16_t(const float2* in, void* out, uint64_t S, uint64_t n_items, int N, int accumulate,
+static int launch_fft16_t(const float2* in, void* out, uint64_t S, uint64_t n_items, int groups, int accumulate,
                           const float2* tw, hipStream_t s) {
     constexpr int C = 1 << LC;
     constexpr int SPW = NT / (C / 16);
@@ -1321,7 +1331,7 @@ static int launch_fft16_t(const float2* in, void* out, uint64_t S, uint64_t n_it
     if (MODE == 0 && SM == 0) blocks = ceil_div(blocks, 8) * 8;   // xcd_order needs G % 8 == 0
     float4* sink = reinterpret_cast<float4*>(const_cast<float2*>(tw) + C);
     hipLaunchKernelGGL((fft16_kernel<LC, NT, MODE, SM>), dim3((unsigned)blocks), dim3(NT), lds, s,
-                       reinterpret_cast<const float4*>(in), out, S, n_items, N, accumulate, tw, sink);
+                       reinterpret_cast<const float4*>(in), out, S, n_items, groups, accumulate, tw, sink);
     return check_launch("channelizer");
 }
 
@@ -1329,7 +1339,7 @@ static int launch_fft16_t(const float2* in, void* out, uint64_t S, uint64_t n_it
 static bool use_fft16(int C) { return C >= 256 && C <= 8192 && !(C & (C - 1)); }
 
 template <int LC, int MODE>
-static int launch_fft16_lc(const float2* in, void* out, uint64_t S, uint64_t n_items, int N, int accumulate,
+static int launch_fft16_lc(const float2* in, void* out, uint64_t S, uint64_t n_items, int groups, int accumulate,
                            const float2* tw, hipStream_t s) {
     // Nontemporal stores pay off only where the stores are whole lines: one
     // spectrum per (antenna, channel), or several staged through LDS when a
@@ -1340,29 +1350,43 @@ static int launch_fft16_lc(const float2* in, void* out, uint64_t S, uint64_t n_i
     // much slower than plain stores.
     if constexpr (MODE == 0) {
         constexpr uint64_t SPW = 512 / ((1 << LC) / 16);
-        if (S == 1) return launch_fft16_t<LC, 512, MODE, 1>(in, out, S, n_items, N, accumulate, tw, s);
+        if (S == 1) return launch_fft16_t<LC, 512, MODE, 1>(in, out, S, n_items, groups, accumulate, tw, s);
         if constexpr (SPW >= 4) {
-            if (S % SPW == 0) return launch_fft16_t<LC, 512, MODE, 2>(in, out, S, n_items, N, accumulate, tw, s);
+            if (S % SPW == 0) return launch_fft16_t<LC, 512, MODE, 2>(in, out, S, n_items, groups, accumulate, tw, s);
         }
     }
-    return launch_fft16_t<LC, 512, MODE, 0>(in, out, S, n_items, N, accumulate, tw, s);
+    // Detector, C up to 2048: two workgroups of 256 threads per CU overlap each
+    // other's loads and passes.  [8,192,8192,2], 4 pols, against one of 512:
+    // C = 256 56 / 60 us, 512 60 / 69, 1024 72 / 90; Stokes I 512 55 / 57,
+    // 1024 51 / 57, but 256 53 / 47 and C = 4096 109 / 103 (178 / 155 with 4
+    // pols), which keep 512.
+    // At C = 8192 (one spectrum per workgroup) items are whole (antenna,
+    // channel)s where these fill the chip: 2.5% faster in the Mode-A case.
+    if constexpr (MODE != 0 && LC == 13) {
+        if (n_items / groups >= (uint64_t)device_cus() || groups == 1)
+            return launch_fft16_t<LC, 512, MODE, 3>(in, out, S * groups, n_items / groups, (int)S, accumulate, tw, s);
+    }
+    if constexpr ((MODE == 4 && LC <= 11) || (MODE == 1 && LC >= 9 && LC <= 11))
+        return launch_fft16_t<LC, 256, MODE, 0>(in, out, S, n_items, groups, accumulate, tw, s);
+    else
+        return launch_fft16_t<LC, 512, MODE, 0>(in, out, S, n_items, groups, accumulate, tw, s);
 }
 
 constexpr uint64_t NT_MAX_SPECTRA = 32;    // spectra per workgroup at C = 256, 512 threads
 
 // Returns 1 and launches when fft16_kernel covers C, else 0.
 template <int MODE>
-static int launch_fft16(int C, const float2* in, void* out, uint64_t S, uint64_t n_items, int N, int accumulate,
+static int launch_fft16(int C, const float2* in, void* out, uint64_t S, uint64_t n_items, int groups, int accumulate,
                         const float2* tw, hipStream_t s, int* rc) {
     // Lane offsets within a workgroup's spectra are 32-bit.
     if ((uint64_t)(NT_MAX_SPECTRA + 2) * S * (uint64_t)C >= (1ull << 31)) return 0;
     switch (C) {
-        case 1 << 8: *rc = launch_fft16_lc<8, MODE>(in, out, S, n_items, N, accumulate, tw, s); return 1;
-        case 1 << 9: *rc = launch_fft16_lc<9, MODE>(in, out, S, n_items, N, accumulate, tw, s); return 1;
-        case 1 << 10: *rc = launch_fft16_lc<10, MODE>(in, out, S, n_items, N, accumulate, tw, s); return 1;
-        case 1 << 11: *rc = launch_fft16_lc<11, MODE>(in, out, S, n_items, N, accumulate, tw, s); return 1;
-        case 1 << 12: *rc = launch_fft16_lc<12, MODE>(in, out, S, n_items, N, accumulate, tw, s); return 1;
-        case 1 << 13: *rc = launch_fft16_lc<13, MODE>(in, out, S, n_items, N, accumulate, tw, s); return 1;
+        case 1 << 8: *rc = launch_fft16_lc<8, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
+        case 1 << 9: *rc = launch_fft16_lc<9, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
+        case 1 << 10: *rc = launch_fft16_lc<10, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
+        case 1 << 11: *rc = launch_fft16_lc<11, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
+        case 1 << 12: *rc = launch_fft16_lc<12, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
+        case 1 << 13: *rc = launch_fft16_lc<13, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
     }
     return 0;
 }
@@ -1840,31 +1864,35 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     const int C = (int)rate;
     // bit 0: add into the output (stepped integration); bit 1: XY -> LR first
     const int flags = (accumulate ? 1 : 0) | (polarize ? 2 : 0);
+    // An item is one integration: Sg spectra in a row of one (antenna, channel)
+    // (all S of the block when the integration spans blocks), whose sums stay
+    // in one thread's registers.  Every (antenna, channel) gives `groups`.
+    const uint64_t Sg = std::min(integration, S);
+    const int groups = (int)(S / Sg);
+    const uint64_t n_items = A * F * groups;
     Radices rad;
     if (!factorize(C, &rad)) return fail("channelizer-detector: rate must factor into 2, 3, 5 and 7");
     const float2* tw = nullptr;
     int rc = get_twiddles(C, s, &tw);
     if (rc) return rc;
-    if (use_fft16(C)) {
+    const bool small = n_items < (1ull << 31);      // the pow-2 kernels count items in 32 bits
+    if (small && use_fft16(C)) {
         int rc16 = 0;
         const float2* in16 = static_cast<const float2*>(input);
-        if (out_pols == 1 ? launch_fft16<1>(C, in16, output, S, A * F, (int)integration, flags, tw, s, &rc16)
-                          : launch_fft16<4>(C, in16, output, S, A * F, (int)integration, flags, tw, s, &rc16))
+        if (out_pols == 1 ? launch_fft16<1>(C, in16, output, Sg, n_items, groups, flags, tw, s, &rc16)
+                          : launch_fft16<4>(C, in16, output, Sg, n_items, groups, flags, tw, s, &rc16))
             return rc16;
     }
     Fft2Plan pl;
-    if (fft2_plan(C, &pl)) {
+    if (small && fft2_plan(C, &pl)) {
         if (out_pols == 1)
-            return launch_fft2<1>(pl, static_cast<const float2*>(input), output, C, S, A * F, (int)integration,
-                                  flags, tw, s);
-        return launch_fft2<4>(pl, static_cast<const float2*>(input), output, C, S, A * F, (int)integration,
-                              flags, tw, s);
+            return launch_fft2<1>(pl, static_cast<const float2*>(input), output, C, Sg, n_items, groups, flags, tw, s);
+        return launch_fft2<4>(pl, static_cast<const float2*>(input), output, C, Sg, n_items, groups, flags, tw, s);
     }
     int threads = 64;
     while (threads < 1024 && threads * 8 < 2 * C) threads *= 2;
     const size_t lds = sizeof(float2) * 2 * (size_t)C;
-    const uint64_t n_af = A * F;
-    uint64_t blocks = n_af;
+    uint64_t blocks = n_items;
     if (blocks > 256 * 64) blocks = 256 * 64;
     const void* fn = out_pols == 1 ? reinterpret_cast<const void*>(&chan_detect_kernel<1, 8>)
                                    : reinterpret_cast<const void*>(&chan_detect_kernel<4, 8>);
@@ -1879,9 +1907,9 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     float* out = static_cast<float*>(output);
     if (out_pols == 1)
         hipLaunchKernelGGL((chan_detect_kernel<1, 8>), dim3((unsigned)blocks), dim3(threads), lds, s, in, out, C,
-                           (int)S, (int)integration, n_af, tw, rad, flags);
+                           (int)Sg, groups, n_items, tw, rad, flags);
     else
         hipLaunchKernelGGL((chan_detect_kernel<4, 8>), dim3((unsigned)blocks), dim3(threads), lds, s, in, out, C,
-                           (int)S, (int)integration, n_af, tw, rad, flags);
+                           (int)Sg, groups, n_items, tw, rad, flags);
     return check_launch("channelizer-detector");
 }

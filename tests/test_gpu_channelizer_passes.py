@@ -57,3 +57,32 @@ def test_four_step_groups(alias):
     y = ops.channelizer(x, C, out=out.view(1, F * C, S, 2))
     y = y.view(F, C, S, 2)[[0, 1, 382, 383, 384, 385, 400]].reshape(1, 7 * C, S, 2)
     assert _err(y, ref) <= _bar(C)
+
+
+def _detect(spec, n, pols):
+    X, Y = spec[..., 0], spec[..., 1]
+    if pols == 1:
+        d = (X.abs().square() + Y.abs().square())[..., None]
+    else:
+        xy = X * Y.conj()
+        d = torch.stack((X.abs().square(), Y.abs().square(), xy.real, xy.imag), dim=-1)
+    a, f, t, q = d.shape
+    return d.reshape(a, f, t // n, n, q).sum(3)
+
+
+@pytest.mark.parametrize("C", [32, 64, 128, 256, 512, 1024, 2048, 4096, 8192, 96, 1000])
+@pytest.mark.parametrize("A,F,S,N", [(1, 1, 1, 1), (1, 1, 6, 2), (1, 3, 7, 1), (2, 5, 9, 3), (1, 37, 4, 4)])
+@pytest.mark.parametrize("pols", [1, 4])
+def test_integrations_of_a_block(C, A, F, S, N, pols):
+    """Every integration is an item of its own: counts that leave slots of the
+    last workgroup idle, several integrations per channel, then the same block
+    added again.  Sums of N powers round N more times."""
+    x = _rand(C + S + N, A, F, S * C, 2)
+    ref = _detect(_spectra(x, C), N, pols)
+    bar = 2 * _bar(C) + (N + 4) * 2.0 ** -24
+    y = ops.channelizer_detector(x, C, N, pols)
+    assert y.shape == ref.shape and _err(y, ref) <= bar
+    if N == S:                                  # stepped over two blocks
+        ops.channelizer_detector(x, C, 2 * N, pols, out=y)
+        ops.channelizer_detector(x, C, 2 * N, pols, out=y, accumulate=True)
+        assert _err(y, 2 * ref) <= 2 * bar

@@ -6,7 +6,8 @@
 // in natural order without a bit-reversal pass.  fftshift is an index remap on
 // the store.  Twiddles come from a per-C table built in FP64 and rounded
 // once to FP32.
-#include "common.hh"
+#include "fft_regs.hh"
+#include "mixed_fft.hh"
 
 #include <algorithm>
 #include <cmath>
@@ -79,55 +80,6 @@ static int get_twiddles(int C, hipStream_t s, const float2** out, int N2 = 0) {
 // ---------------------------------------------------------------------------
 // Small DFT in registers.
 // ---------------------------------------------------------------------------
-
-__device__ __forceinline__ float2 mul_neg_j(float2 a) { return make_float2(a.y, -a.x); }
-
-template <int R>
-__device__ __forceinline__ void dft_reg(float2 (&v)[R], const float2* __restrict__ tw, int twstep) {
-    if constexpr (R == 1) {
-        return;
-    } else if constexpr (R == 2) {
-        const float2 a = v[0], b = v[1];
-        v[0] = cadd(a, b);
-        v[1] = csub(a, b);
-    } else if constexpr (R == 4) {
-        const float2 s02 = cadd(v[0], v[2]), d02 = csub(v[0], v[2]);
-        const float2 s13 = cadd(v[1], v[3]), d13 = mul_neg_j(csub(v[1], v[3]));
-        v[0] = cadd(s02, s13);
-        v[2] = csub(s02, s13);
-        v[1] = cadd(d02, d13);
-        v[3] = csub(d02, d13);
-    } else if constexpr (R == 8) {
-        float2 e[4] = {v[0], v[2], v[4], v[6]};
-        float2 o[4] = {v[1], v[3], v[5], v[7]};
-        dft_reg<4>(e, tw, 0);
-        dft_reg<4>(o, tw, 0);
-        const float c = 0.70710678118654752440f;
-        const float2 o1 = make_float2(c * (o[1].x + o[1].y), c * (o[1].y - o[1].x));   // * e^{-j pi/4}
-        const float2 o2 = mul_neg_j(o[2]);                                            // * e^{-j pi/2}
-        const float2 o3 = make_float2(c * (o[3].y - o[3].x), -c * (o[3].x + o[3].y)); // * e^{-j 3pi/4}
-        v[0] = cadd(e[0], o[0]); v[4] = csub(e[0], o[0]);
-        v[1] = cadd(e[1], o1);   v[5] = csub(e[1], o1);
-        v[2] = cadd(e[2], o2);   v[6] = csub(e[2], o2);
-        v[3] = cadd(e[3], o3);   v[7] = csub(e[3], o3);
-    } else {
-        // Direct DFT of size R with W_R^q = tw[q * twstep].
-        float2 r[R];
-#pragma unroll
-        for (int k = 0; k < R; k++) {
-            float2 acc = v[0];
-#pragma unroll
-            for (int n = 1; n < R; n++) {
-                const float2 w = tw[((n * k) % R) * twstep];
-                acc.x += v[n].x * w.x - v[n].y * w.y;
-                acc.y += v[n].x * w.y + v[n].y * w.x;
-            }
-            r[k] = acc;
-        }
-#pragma unroll
-        for (int k = 0; k < R; k++) v[k] = r[k];
-    }
-}
 
 // Constant-twiddle DFT for the register kernel (W computed at compile time
 // from the table argument in a small struct).
@@ -421,24 +373,6 @@ __global__ __launch_bounds__(1024) void chan_big_pass2(const float2* __restrict_
 // registers, writing (or adding to, with accumulate)
 //   out[a, f*C + k', group, q].
 // The CF32 spectra never reach HBM.
-// Detector sums of (X, Y) turned into those of (L, R) = (X + jY, X - jY),
-// the polarizer (polarizer.cu:5-25) applied before the detector: sums are
-// linear in [XX*, YY*, Re XY*, Im XY*], so the map applies after integration.
-//   Stokes I doubles; |L|^2 = XX + YY + 2 Im, |R|^2 = XX + YY - 2 Im,
-//   Re LR* = XX - YY, Im LR* = 2 Re.
-template <int NPOL>
-__device__ inline void circular_sums(float (&a)[NPOL]) {
-    if constexpr (NPOL == 1) {
-        a[0] *= 2.f;
-    } else {
-        const float xx = a[0], yy = a[1], re = a[2], im = a[3];
-        a[0] = (xx + yy) + 2.f * im;
-        a[1] = (xx + yy) - 2.f * im;
-        a[2] = xx - yy;
-        a[3] = 2.f * re;
-    }
-}
-
 template <int NPOL, int KPT>
 __global__ __launch_bounds__(1024) void chan_detect_kernel(const float2* __restrict__ in,
                                                            float* __restrict__ out, int C,
@@ -518,210 +452,6 @@ __global__ __launch_bounds__(1024) void chan_detect_kernel(const float2* __restr
 }
 
 // ---------------------------------------------------------------------------
-// Power-of-two rates 16 < C < 256 with both polarizations (fft16_kernel
-// below takes 256 <= C <= 8192).
-//
-// A spectrum is handled by C/8 threads; a workgroup holds SPW = max(1,
-// 2048/C) spectra.  Pass 1 (radix 8) runs on registers loaded straight from
-// HBM (eight 16-byte loads per thread, both pols, all in flight at once);
-// the radix-8 middle passes run in LDS.  The last pass (radix RL = 2, 4 or 8)
-// reads LDS and writes the fftshifted spectrum (MODE 0) or integrates the
-// detector (MODE 1: Stokes I, MODE 4: XX*, YY*, Re XY*, Im XY*) in registers,
-// so the spectra of the fused channelizer + detector never reach HBM.
-// ---------------------------------------------------------------------------
-template <int MODE, int RL>
-__global__ __launch_bounds__(1024) void fft2_kernel(const float4* __restrict__ in, void* __restrict__ outv,
-                                                    int C, int nmid, uint64_t S, uint64_t n_items,
-                                                    int groups, int flags,
-                                                    const float2* __restrict__ tw) {
-    extern __shared__ float2 data[];
-    const int accumulate = flags & 1;
-    const bool circular = flags & 2;
-    constexpr int G = 8 / RL;                   // last-pass butterflies per thread and pol
-    const int tps = C >> 3;                     // threads per spectrum
-    const int spw = blockDim.x / tps;
-    const int slot = threadIdx.x / tps;
-    const int j = threadIdx.x - slot * tps;
-    const int PC = spw * 2 * C;
-    float2* const blk = data + (size_t)slot * 2 * C;    // pol 0; pol 1 at + C
-    const uint64_t per_round = (uint64_t)gridDim.x * spw;
-    const uint64_t rounds = (n_items + per_round - 1) / per_round;
-    const int nspec = MODE == 0 ? 1 : (int)S;
-    const int lastR = C / RL;                   // stride of the last pass
-
-    auto item_of = [&](uint64_t round) { return (round * gridDim.x + blockIdx.x) * spw + slot; };
-    auto spec_of = [&](uint64_t round, int s) {
-        const uint64_t it = item_of(round);
-        const uint64_t sp = MODE == 0 ? it : it * S + s;
-        return it < n_items ? sp : 0;           // idle slots re-read spectrum 0
-    };
-    float4 q[8];
-    auto load = [&](uint64_t sp) {
-        const float4* src = in + sp * (uint64_t)C;
-#pragma unroll
-        for (int r = 0; r < 8; r++) q[r] = src[j + r * tps];
-    };
-
-    constexpr int NPOL = MODE == 0 ? 1 : MODE;
-    float acc[G][RL][NPOL];
-#pragma unroll
-    for (int g = 0; g < G; g++)
-#pragma unroll
-        for (int r = 0; r < RL; r++)
-#pragma unroll
-            for (int c = 0; c < NPOL; c++) acc[g][r][c] = 0.f;
-
-    for (uint64_t round = 0; round < rounds; round++) {
-        const uint64_t item = item_of(round);
-        const bool valid = item < n_items;
-        for (int s = 0; s < nspec; s++) {
-            load(spec_of(round, s));
-            // ---- pass 1: radix 8 on registers -> LDS (Stockham, Ns = 1)
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                float2 v[8];
-#pragma unroll
-                for (int r = 0; r < 8; r++)
-                    v[r] = p == 0 ? make_float2(q[r].x, q[r].y) : make_float2(q[r].z, q[r].w);
-                dft_reg<8>(v, tw, 0);
-#pragma unroll
-                for (int r = 0; r < 8; r++) blk[p * C + j * 8 + r] = v[r];
-            }
-            __syncthreads();
-            int Ns = 8;
-            for (int i = 0; i < nmid; i++) {
-                stockham_pass<8>(data, C, PC, Ns, tw);
-                Ns *= 8;
-            }
-            // ---- last pass: radix RL, LDS -> output (Ns = C / RL)
-            const uint64_t sp = MODE == 0 ? item : item * S + s;
-#pragma unroll
-            for (int g = 0; g < G; g++) {
-                const int jb = j + g * tps;
-                float2 x[2][RL];
-#pragma unroll
-                for (int p = 0; p < 2; p++) {
-#pragma unroll
-                    for (int r = 0; r < RL; r++) {
-                        float2 v = blk[p * C + jb + r * lastR];
-                        if (r > 0 && jb > 0) v = cmul(v, tw[jb * r]);
-                        x[p][r] = v;
-                    }
-                    dft_reg<RL>(x[p], tw, C / RL);
-                }
-                if constexpr (MODE == 0) {
-                    if (valid) {
-                        const uint64_t af = sp / S, si = sp - af * S;
-                        float4* out = static_cast<float4*>(outv);
-#pragma unroll
-                        for (int r = 0; r < RL; r++) {
-                            const int k = jb + r * lastR;
-                            const int ko = (k + (C >> 1)) & (C - 1);
-                            out[(af * C + ko) * S + si] = make_float4(x[0][r].x, x[0][r].y, x[1][r].x, x[1][r].y);
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int r = 0; r < RL; r++) {
-                        const float2 X = x[0][r], Y = x[1][r];
-                        if constexpr (MODE == 1) {
-                            acc[g][r][0] += X.x * X.x + X.y * X.y + Y.x * Y.x + Y.y * Y.y;
-                        } else {
-                            acc[g][r][0] += X.x * X.x + X.y * X.y;
-                            acc[g][r][NPOL > 1 ? 1 : 0] += Y.x * Y.x + Y.y * Y.y;
-                            acc[g][r][NPOL > 2 ? 2 : 0] += X.x * Y.x + X.y * Y.y;
-                            acc[g][r][NPOL > 3 ? 3 : 0] += X.y * Y.x - X.x * Y.y;
-                        }
-                    }
-                }
-            }
-            if constexpr (MODE != 0) {
-                if (s == nspec - 1) {
-                    // items fit 32 bits (host check); one integration per
-                    // channel needs no division
-                    unsigned af = (unsigned)item, grp = 0;
-                    if (groups != 1) {
-                        af = (unsigned)item / (unsigned)groups;
-                        grp = (unsigned)item - af * (unsigned)groups;
-                    }
-                    float* out = static_cast<float*>(outv);
-                    if (circular) {
-#pragma unroll
-                        for (int g = 0; g < G; g++)
-#pragma unroll
-                            for (int r = 0; r < RL; r++) circular_sums<NPOL>(acc[g][r]);
-                    }
-#pragma unroll
-                    for (int g = 0; g < G; g++)
-#pragma unroll
-                        for (int r = 0; r < RL; r++) {
-                            if (valid) {
-                                const int k = j + g * tps + r * lastR;
-                                const int ko = (k + (C >> 1)) & (C - 1);
-                                float* o = out + (((uint64_t)af * C + ko) * groups + grp) * NPOL;
-#pragma unroll
-                                for (int c = 0; c < NPOL; c++) o[c] = accumulate ? o[c] + acc[g][r][c] : acc[g][r][c];
-                            }
-#pragma unroll
-                            for (int c = 0; c < NPOL; c++) acc[g][r][c] = 0.f;
-                        }
-                }
-            }
-            __syncthreads();   // LDS is rewritten by the next spectrum's pass 1
-        }
-    }
-}
-
-// Passes of fft2_kernel for C = 2^k: radix 8 first, nmid radix-8 middle
-// passes, last radix RL with 3 + 3 nmid + log2(RL) = k.
-struct Fft2Plan {
-    int rl, nmid, threads, spw;
-};
-
-static bool fft2_plan(int C, Fft2Plan* pl) {
-    if (C < 16 || C > 8192 || (C & (C - 1))) return false;
-    int k = 0;
-    while ((1 << k) < C) k++;
-    const int rem = (k - 3) % 3;
-    pl->rl = rem == 0 ? 8 : (rem == 1 ? 2 : 4);
-    const int lr = rem == 0 ? 3 : rem;
-    pl->nmid = (k - 3 - lr) / 3;
-    const int tps = C / 8;
-    pl->threads = tps >= 256 ? tps : 256;
-    pl->spw = pl->threads / tps;
-    return true;
-}
-
-template <int MODE>
-static int launch_fft2(const Fft2Plan& pl, const float2* in, void* out, int C, uint64_t S, uint64_t n_items,
-                       int groups, int accumulate, const float2* tw, hipStream_t s) {
-    const size_t lds = sizeof(float2) * 2 * (size_t)C * pl.spw;
-    // One workgroup per SPW spectra: the hardware refills each CU as
-    // workgroups finish, which beats persistent rounds here by 2-6%.
-    const uint64_t blocks = std::min<uint64_t>(ceil_div(n_items, pl.spw), 0x7fffffffull);
-    const void* fns[3] = {reinterpret_cast<const void*>(&fft2_kernel<MODE, 2>),
-                          reinterpret_cast<const void*>(&fft2_kernel<MODE, 4>),
-                          reinterpret_cast<const void*>(&fft2_kernel<MODE, 8>)};
-    const void* fn = fns[pl.rl == 2 ? 0 : (pl.rl == 4 ? 1 : 2)];
-    if (lds > 65536) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) {
-            set_error(std::string("channelizer: LDS attribute: ") + hipGetErrorString(e));
-            return BLADE_HIP_ERROR;
-        }
-    }
-    const float4* in4 = reinterpret_cast<const float4*>(in);
-    const dim3 grid((unsigned)blocks), block((unsigned)pl.threads);
-    if (pl.rl == 2)
-        hipLaunchKernelGGL((fft2_kernel<MODE, 2>), grid, block, lds, s, in4, out, C, pl.nmid, S, n_items, groups, accumulate, tw);
-    else if (pl.rl == 4)
-        hipLaunchKernelGGL((fft2_kernel<MODE, 4>), grid, block, lds, s, in4, out, C, pl.nmid, S, n_items, groups, accumulate, tw);
-    else
-        hipLaunchKernelGGL((fft2_kernel<MODE, 8>), grid, block, lds, s, in4, out, C, pl.nmid, S, n_items, groups, accumulate, tw);
-    return check_launch("channelizer");
-}
-
-// ---------------------------------------------------------------------------
 // Power-of-two rates 256 <= C <= 8192 with both polarizations, radix 16.
 //
 // Every thread holds 16 points of each polarization, so a spectrum takes
@@ -744,45 +474,6 @@ static int launch_fft2(const Fft2Plan& pl, const float2* in, void* out, int C, u
 // ---------------------------------------------------------------------------
 
 __device__ __forceinline__ int lpad(int pos) { return pos + (pos >> 4); }
-
-// a * W_16^E with W_16 = exp(-j 2 pi / 16); cos(2 pi e / 16) by table,
-// -sin(2 pi e / 16) = cos(2 pi (e + 4) / 16).
-template <int E>
-__device__ __forceinline__ float2 mul_w16(float2 a) {
-    constexpr int e = E & 15;
-    constexpr float c1 = 0.92387953251128675613f;   // cos(pi/8)
-    constexpr float s1 = 0.38268343236508977173f;   // sin(pi/8)
-    constexpr float h = 0.70710678118654752440f;    // cos(pi/4)
-    constexpr float cs[16] = {1.f, c1, h, s1, 0.f, -s1, -h, -c1, -1.f, -c1, -h, -s1, 0.f, s1, h, c1};
-    if constexpr (e == 0) return a;
-    else if constexpr (e == 4) return make_float2(a.y, -a.x);
-    else if constexpr (e == 8) return make_float2(-a.x, -a.y);
-    else if constexpr (e == 12) return make_float2(-a.y, a.x);
-    else return cmul(a, make_float2(cs[e], cs[(e + 4) & 15]));
-}
-
-// 16-point DFT in natural order: n = 4 n1 + n2, k = k1 + 4 k2,
-// X[k1 + 4 k2] = sum_n2 W4^(n2 k2) W16^(n2 k1) sum_n1 W4^(n1 k1) x[4 n1 + n2].
-__device__ __forceinline__ void dft16(float2 (&v)[16]) {
-    float2 y[4][4];
-#pragma unroll
-    for (int n2 = 0; n2 < 4; n2++) {
-        float2 t[4] = {v[n2], v[n2 + 4], v[n2 + 8], v[n2 + 12]};
-        dft_reg<4>(t, nullptr, 0);
-#pragma unroll
-        for (int k1 = 0; k1 < 4; k1++) y[n2][k1] = t[k1];
-    }
-    y[1][1] = mul_w16<1>(y[1][1]); y[1][2] = mul_w16<2>(y[1][2]); y[1][3] = mul_w16<3>(y[1][3]);
-    y[2][1] = mul_w16<2>(y[2][1]); y[2][2] = mul_w16<4>(y[2][2]); y[2][3] = mul_w16<6>(y[2][3]);
-    y[3][1] = mul_w16<3>(y[3][1]); y[3][2] = mul_w16<6>(y[3][2]); y[3][3] = mul_w16<9>(y[3][3]);
-#pragma unroll
-    for (int k1 = 0; k1 < 4; k1++) {
-        float2 t[4] = {y[0][k1], y[1][k1], y[2][k1], y[3][k1]};
-        dft_reg<4>(t, nullptr, 0);
-#pragma unroll
-        for (int k2 = 0; k2 < 4; k2++) v[k1 + 4 * k2] = t[k2];
-    }
-}
 
 template <int R>
 __device__ __forceinline__ void dft_pow2(float2 (&v)[R]) {
@@ -923,12 +614,6 @@ __device__ __forceinline__ void halves(float x, float& u, float& v) {
     u = __uint_as_float(p[0]);
     v = __uint_as_float(p[1]);
 }
-
-// Workgroup order with consecutive values on one XCD: the dispatcher deals
-// workgroups to the 8 XCDs round-robin (b mod 8), so b -> (b mod 8) G/8 + b/8
-// hands workgroups that take consecutive spectra to one XCD, whose L2 then
-// merges their interleaved pieces of each output line.  G is a multiple of 8.
-__device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned G) { return (b & 7u) * (G >> 3) + (b >> 3); }
 
 // SM (MODE 0 stores): 0 strided, 1 nontemporal with one spectrum per
 // (antenna, channel), 2 transposed through LDS so that the workgroup's SPW
@@ -1774,6 +1459,13 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
                                 : dispatch_small<1>(C, in, out, n_spec, S, s);
         if (ok) return check_launch("channelizer");
     }
+    // Mixed-radix kernel: every rate made of 2, 3, 5 and 7 but the powers of two
+    // of the radix-16 kernel, and of these C = 4096 where several spectra
+    // interleave: its stores write runs of them ([8,.,4 C,2]: 123 us against
+    // 156 us at S = 4, 102 against 108 at S = 2; 512 to 2048 are staged there
+    // and 10-30% faster, 8192 106 against 129 us).
+    if (P == 2 && (!use_fft16(C) || (C == 4096 && S > 1)) && T < (1ull << 31) && mixed_fft_covers(rate))
+        return mixed_fft(C, in, out, S, n_spec, s);
     const float2* tw = nullptr;
     int rc = get_twiddles(C, s, &tw);
     if (rc) return rc;
@@ -1781,9 +1473,6 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
         int rc16 = 0;
         if (launch_fft16<0>(C, in, out, S, n_spec, 1, 0, tw, s, &rc16)) return rc16;
     }
-    Fft2Plan pl;
-    if (P == 2 && fft2_plan(C, &pl))
-        return launch_fft2<0>(pl, in, out, C, S, n_spec, 1, 0, tw, s);
     Radices rad;
     const size_t lds = sizeof(float2) * (size_t)C * P;
     uint64_t blocks = n_spec;
@@ -1828,6 +1517,7 @@ extern "C" int blade_channelizer_plan(uint64_t rate, blade_stream_t stream) {
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const float2* tw = nullptr;
     int rc = get_twiddles((int)rate, s, &tw);
+    if (!rc && mixed_fft_covers(rate)) rc = mixed_fft_plan((int)rate, s);
     if (rc) return rc;
     if (use_four_step((int)rate, 2)) {
         int ln1, ln2;
@@ -1872,22 +1562,24 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     const uint64_t n_items = A * F * groups;
     Radices rad;
     if (!factorize(C, &rad)) return fail("channelizer-detector: rate must factor into 2, 3, 5 and 7");
+    // Mixed-radix kernel: as for the channelizer, and full Stokes at 2048 and
+    // 4096 with several integrations per channel, whose 16-byte outputs it writes
+    // in runs (one spectrum each: 117 against 151 and 136 against 190 us for
+    // 200 MB; Stokes I 95 against 82 and 109 against 71 us the other way).
+    const bool small = n_items < (1ull << 31);      // these kernels count items in 32 bits
+    const bool runs = out_pols == 4 && groups > 1 && (C == 2048 || C == 4096);
+    if (small && Sg < (1ull << 31) && (!use_fft16(C) || runs) && mixed_fft_covers(rate))
+        return mixed_fft_detect(C, static_cast<const float2*>(input), static_cast<float*>(output), Sg, groups, n_items,
+                                (int)out_pols, flags, s);
     const float2* tw = nullptr;
     int rc = get_twiddles(C, s, &tw);
     if (rc) return rc;
-    const bool small = n_items < (1ull << 31);      // the pow-2 kernels count items in 32 bits
     if (small && use_fft16(C)) {
         int rc16 = 0;
         const float2* in16 = static_cast<const float2*>(input);
         if (out_pols == 1 ? launch_fft16<1>(C, in16, output, Sg, n_items, groups, flags, tw, s, &rc16)
                           : launch_fft16<4>(C, in16, output, Sg, n_items, groups, flags, tw, s, &rc16))
             return rc16;
-    }
-    Fft2Plan pl;
-    if (small && fft2_plan(C, &pl)) {
-        if (out_pols == 1)
-            return launch_fft2<1>(pl, static_cast<const float2*>(input), output, C, Sg, n_items, groups, flags, tw, s);
-        return launch_fft2<4>(pl, static_cast<const float2*>(input), output, C, Sg, n_items, groups, flags, tw, s);
     }
     int threads = 64;
     while (threads < 1024 && threads * 8 < 2 * C) threads *= 2;

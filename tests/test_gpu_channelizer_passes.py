@@ -59,6 +59,23 @@ def test_four_step_groups(alias):
     assert _err(y, ref) <= _bar(C)
 
 
+MIXED = [18, 20, 24, 28, 30, 32, 36, 42, 50, 54, 60, 64, 70, 84, 90, 98, 126, 128, 150, 162, 196, 210, 250, 360, 486, 490,
+         686, 1000, 1176, 1458, 2058, 2500, 3430, 4096, 4374, 4802, 5000, 6250, 7680, 8064, 8100]
+
+
+@pytest.mark.parametrize("C", MIXED)
+def test_mixed_radices(C):
+    """Every radix in every position; spectra that fill no workgroup, one and
+    several per channel, and in place."""
+    for A, F, S in ((1, 3, 1), (2, 7, 5), (1, 5, 8)):
+        x = _rand(C + S, A, F, S * C, 2)
+        ref = _spectra(x, C)
+        assert _err(ops.channelizer(x, C), ref) <= _bar(C)
+        if S == 1:
+            ops.channelizer(x, C, out=x)
+            assert _err(x.view(ref.shape), ref) <= _bar(C)
+
+
 def _detect(spec, n, pols):
     X, Y = spec[..., 0], spec[..., 1]
     if pols == 1:
@@ -70,8 +87,8 @@ def _detect(spec, n, pols):
     return d.reshape(a, f, t // n, n, q).sum(3)
 
 
-@pytest.mark.parametrize("C", [32, 64, 128, 256, 512, 1024, 2048, 4096, 8192, 96, 1000])
-@pytest.mark.parametrize("A,F,S,N", [(1, 1, 1, 1), (1, 1, 6, 2), (1, 3, 7, 1), (2, 5, 9, 3), (1, 37, 4, 4)])
+@pytest.mark.parametrize("C", [4, 6, 18, 32, 64, 128, 256, 512, 1024, 2048, 4096, 8192, 96, 490, 1000, 4802, 8100])
+@pytest.mark.parametrize("A,F,S,N", [(1, 1, 1, 1), (1, 1, 6, 2), (1, 3, 7, 1), (2, 5, 9, 3), (1, 37, 4, 4), (1, 2, 40, 40)])
 @pytest.mark.parametrize("pols", [1, 4])
 def test_integrations_of_a_block(C, A, F, S, N, pols):
     """Every integration is an item of its own: counts that leave slots of the

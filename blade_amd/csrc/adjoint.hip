@@ -39,7 +39,7 @@ struct AdjArgs {
     const float2* w;         // [B,A,F,1,P] phasors (fused mode)
     const float2* gy;        // [B,F,T,P] upstream gradient (adjoint mode)
     float* partial;          // [nsplit][F][P][btiles][16][apad]
-    float* loss_part;        // [nsplit][F][btiles]
+    double* loss_part;       // [nsplit][F][btiles]
     int A, F, T, B;
     int apad, n_at;          // padded antennas, antenna tiles
     int tsplit;              // time samples per workgroup (a multiple of ADJ_TC or SG_TC)
@@ -235,7 +235,7 @@ template <int NAT, bool VEC>
 __global__ __launch_bounds__(256, (NAT <= 2 ? 3 : NAT <= 4 ? 2 : 1)) void stokes_grad_kernel(AdjArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     uint4* const s_w = reinterpret_cast<uint4*>(lds_raw);                 // [unit][p][part][64]
-    __shared__ float s_loss[ADJ_WAVES];
+    __shared__ double s_loss[ADJ_WAVES];
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(256, (NAT <= 2 ? 3 : NAT <= 4 ? 2 : 1)) void stokes
         for (int at = 0; at < NAT; at++)
 #pragma unroll
             for (int c = 0; c < 2; c++) acc[p][at][c] = zero4;
-    float loss = 0.f;
+    double loss = 0.0;      // FP64 past the 32 squares of a lane's tile
 
     for (; t0 < t_end; t0 += ADJ_WAVES * SG_TC) {
         // ---- forward: y[p][n], register r of lane (g, column): time
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(256, (NAT <= 2 ? 3 : NAT <= 4 ? 2 : 1)) void stokes
                 for (int r = 0; r < 4; r++) e += y[p][n][r] * y[p][n][r];
             tl += e;
         }
-        loss += lam * tl;
+        loss += (double)lam * (double)tl;
         // Infinities and NaN (they show in tl) take the split that keeps them.
         const bool plain = __all(fabsf(tl) <= 3.0e38f);
         // ---- adjoint, half of the times at a time (half the operands of gy
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256) void adjoint_reduce_kernel(AdjArgs a, int nspl
     if (loss && blockIdx.x == gridDim.x - 1) {
         __shared__ double s[256];
         double v = 0.0;
-        for (size_t e = threadIdx.x; e < n_loss; e += blockDim.x) v += (double)a.loss_part[e];
+        for (size_t e = threadIdx.x; e < n_loss; e += blockDim.x) v += a.loss_part[e];
         s[threadIdx.x] = v;
         __syncthreads();
         for (int off = 128; off > 0; off >>= 1) {
@@ -525,14 +525,14 @@ static int run_adjoint(bool fused, const void* input, const void* phasors, const
     a.tsplit = (int)(tiles_per * tc);
 
     const size_t part_floats = (size_t)nsplit * F * 2 * a.btiles * 16 * a.apad;
-    const size_t loss_floats = (size_t)nsplit * F * a.btiles;
+    const size_t n_loss = (size_t)nsplit * F * a.btiles;
     unsigned char* ws = nullptr;
-    const size_t ws_bytes = (part_floats + loss_floats) * sizeof(float);
+    const size_t ws_bytes = part_floats * sizeof(float) + n_loss * sizeof(double);
     if (F == 0) return BLADE_SUCCESS;
     int rc = library_workspace(WS_ADJOINT, ws_bytes, s, &ws);
     if (rc) return rc;
     a.partial = reinterpret_cast<float*>(ws);
-    a.loss_part = a.partial + part_floats;
+    a.loss_part = reinterpret_cast<double*>(a.partial + part_floats);     // part_floats is even
 
     const size_t lds_sum = (size_t)ADJ_WAVES * 2 * 16 * a.apad * 4;
     const size_t lds = fused ? std::max(lds_sum, (size_t)a.n_at * 6 * 64 * 16 + ADJ_WAVES * 16 * SG_XS * 4) : lds_sum;
@@ -558,7 +558,7 @@ static int run_adjoint(bool fused, const void* input, const void* phasors, const
     (void)hipLaunchKernel(fn, grid, dim3(64 * ADJ_WAVES), args, lds, s);   // check_launch below reports
     const size_t n = (size_t)F * 2 * a.btiles * 8 * A;
     hipLaunchKernelGGL(adjoint_reduce_kernel, dim3((unsigned)ceil_div(n, 256) + (fused ? 1 : 0)), dim3(256), 0, s, a,
-                       (int)nsplit, static_cast<float2*>(grad_phasors), loss_floats, loss);
+                       (int)nsplit, static_cast<float2*>(grad_phasors), n_loss, loss);
     return check_launch(who);
 }
 

@@ -56,7 +56,7 @@ class Beamform(torch.autograd.Function):
 class StokesIPower(torch.autograd.Function):
     """``L = -sum_b beam_weights[b] sum_{f,t,p} |y_b|^2`` (FP64 scalar).
 
-    ``precision``: "f32" or "f16x2" (FP16 matrix cores with hi + lo halves)."""
+    ``precision``: "f32" or "f16x2" (the same kernel, FP32 precision)."""
 
     @staticmethod
     def forward(ctx, x, w, beam_weights, precision="f32"):
@@ -67,8 +67,9 @@ class StokesIPower(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_loss):
         (grad,) = ctx.saved_tensors
-        # PyTorch's complex gradient is twice dL/dconj(w).
-        return None, grad * (2.0 * grad_loss.to(torch.float32)), None, None
+        # PyTorch's complex gradient is twice dL/dconj(w); the 0-dim factor
+        # takes the gradient's precision in the product itself.
+        return None, grad * (2.0 * grad_loss), None, None
 
 
 class SteeredStokesIPower(torch.autograd.Function):
@@ -90,7 +91,7 @@ class SteeredStokesIPower(torch.autograd.Function):
     def backward(ctx, grad_loss):
         (grad_g,) = ctx.saved_tensors
         # PyTorch's complex gradient is twice dL/dconj(g).
-        return None, None, grad_g * (2.0 * grad_loss.to(torch.float32)), None, None
+        return None, None, grad_g * (2.0 * grad_loss), None, None
 
 
 def beamform(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -195,7 +196,7 @@ def calibrate(x: torch.Tensor, w: torch.Tensor, steps: int = 200, lr: float = 0.
     stay on the device until the end (one read).  With ``graph`` the step
     (steering, fused loss and gradient, chain rule, Adam) is captured once in
     a CUDA graph after a few eager steps on the same stream and replayed.
-    ``precision`` selects the loss + gradient kernel ("f32" or "f16x2").
+    ``precision``: "f32" or "f16x2" (the same loss + gradient kernel).
     With ``fused_adam`` every step is the library's kernels, the Adam updates
     included (``blade_gain_adam``, ``blade_delay_adam``); otherwise
     torch.optim.Adam (capturable) after autograd.

@@ -23,8 +23,14 @@ __all__ = ["type_of", "stream_handle", "cast", "beamformer", "beamform_chain", "
 
 
 def stream_handle(stream=None):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ct.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return ct.c_void_p(stream.cuda_stream)
+    # The raw handle of the current device's current stream.  Going through a
+    # torch.cuda.Stream object costs 3 us a call, and 25 us in autograd's
+    # backward thread.
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return ct.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _ptr(t: torch.Tensor):

@@ -88,6 +88,7 @@ struct BfArgs {
     int n_tchunks;          // chunks of WAVES*TILE*NT samples along T
     int chunks_per_wg;      // chunks walked by one workgroup
     size_t wbytes;          // bytes of the phasor A operands in LDS
+    int stage;              // EPI 0 and EPI_BATCH: LDS for the wavefronts' staged rows behind them
     float4* sink;           // 64 x 16 B: target of the stores of lanes with nothing to store
 };
 
@@ -353,14 +354,16 @@ __device__ __forceinline__ constexpr int epi_code(int rate, bool pol, bool inc) 
     return rate | (pol ? 8 : 0) | (inc ? 16 : 0);
 }
 template <int EPI> __device__ __forceinline__ int epi_rate(const BfArgs& a) { return EPI ? (EPI & 7) : a.rate; }
-template <int NT, int EPI> constexpr int epi_run() { return (EPI && (EPI & 7) == 1) ? 1 : (NT < 4 ? NT : 4); }
+template <int NT, int EPI, int AR> constexpr int epi_run() {
+    return (EPI && (EPI & 7) == 1 && !ar_split(AR)) ? 1 : (NT < 4 ? NT : 4);
+}
 template <int EPI> __device__ __forceinline__ bool epi_pol(const BfArgs& a) { return EPI ? (EPI & 8) != 0 : a.polarize != 0; }
 template <int EPI> __device__ __forceinline__ bool epi_inc(const BfArgs& a) { return EPI ? (EPI & 16) != 0 : a.incoherent != 0; }
 
-template <int NT, bool NTS, int EPI>
+template <int NT, bool NTS, int EPI, int AR>
 __device__ __forceinline__ void store_beam(const BfArgs& a, int b, int f, int t0,
                                            float2 (&v)[2][NT], bool ok) {
-    typedef TimeMap<NT, epi_run<NT, EPI>()> M;
+    typedef TimeMap<NT, epi_run<NT, EPI, AR>()> M;
     float4* const sink = a.sink + (threadIdx.x & 63);
     const int rate = epi_rate<EPI>(a);
     const bool pol = epi_pol<EPI>(a);
@@ -421,6 +424,8 @@ __device__ __forceinline__ void store_beam(const BfArgs& a, int b, int f, int t0
 constexpr int EPI_MODEB = 4 | 8;          // rate 4, polarize, no incoherent beam
 constexpr int EPI_PLAIN = 1;              // rate 1
 constexpr int EPI_PLAIN_INC = 1 | 16;     // rate 1, incoherent beam
+constexpr int EPI_STAGE_FLAG = 32;        // with a fixed variant: staged rows only where BfArgs::stage says so
+constexpr int EPI_BATCH = EPI_PLAIN | EPI_STAGE_FLAG;
 
 // Mode-B epilogue through LDS (split variants, 16-beam tiles): the four
 // wavefronts' spectra of one chunk are exchanged so that each store
@@ -434,6 +439,63 @@ constexpr bool staged_epilogue() { return ar_split(AR) && MW == 2 && NT == 4 && 
 constexpr int kStageRow = 65;                                   // float4 per staged row, padded
 constexpr int stage_beams(int ar) { return ar == AR_BF16X3 ? 4 : 8; }
 constexpr size_t stage_bytes(int ar) { return (size_t)stage_beams(ar) * 4 * kStageRow * 16; }
+
+// Epilogue through LDS within a wavefront (split variants, every other
+// epilogue with 4 samples per lane): a lane's 4 consecutive samples of one beam,
+// channelized and polarized, go to its beam's row of 64 results in LDS, and
+// each store instruction then writes one row: runs of 1 KiB (rate 1), 512 or
+// 256 bytes instead of 16 bytes of every 64, 32 or 256.  The loads keep runs of
+// 4 samples (16 bytes per lane).  4 rows (every other beam of a tile) at a time,
+// private to the wavefront: LDS operations of a wavefront complete in order, so
+// there is no barrier.  Rows carry one entry of padding per 4, which puts the 16
+// lanes' 64-byte pieces on different banks.
+template <int NT, int AR, int MW, int EPI>
+constexpr bool wave_stage() { return ar_split(AR) && NT == 4 && !staged_epilogue<NT, AR, MW, EPI>(); }
+constexpr int kWaveRow = 80;                                    // float4 per row
+constexpr size_t kWaveStageBytes = (size_t)WAVES * 4 * kWaveRow * 16;
+
+// One beam's 4 consecutive samples (lane i of its group) into its row.
+__device__ __forceinline__ void wave_stage_beam(float4* row, int i, int rate, bool pol, float2 (&v)[2][4]) {
+    float2 o[2][4];
+    int c[4];           // column of result j: (fine channel, spectrum)
+    if (rate == 4) {
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const float2* x = &v[p][0];
+            const float2 s02 = cadd(x[0], x[2]), d02 = csub(x[0], x[2]);
+            const float2 s13 = cadd(x[1], x[3]), dd = csub(x[1], x[3]);
+            const float2 d13 = make_float2(dd.y, -dd.x);   // -j (x1 - x3)
+            o[p][0] = cadd(s02, s13);
+            o[p][1] = cadd(d02, d13);
+            o[p][2] = csub(s02, s13);
+            o[p][3] = csub(d02, d13);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) c[j] = 16 * j + i;
+    } else if (rate == 2) {
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                o[p][h] = cadd(v[p][2 * h], v[p][2 * h + 1]);
+                o[p][2 + h] = csub(v[p][2 * h], v[p][2 * h + 1]);
+            }
+#pragma unroll
+        for (int j = 0; j < 4; j++) c[j] = 32 * (j >> 1) + 2 * i + (j & 1);
+    } else {
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[p][j] = v[p][j];
+#pragma unroll
+        for (int j = 0; j < 4; j++) c[j] = 4 * i + j;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (pol) polarize2(o[0][j], o[1][j]);
+        row[c[j] + (c[j] >> 2)] = make_float4(o[0][j].x, o[0][j].y, o[1][j].x, o[1][j].y);
+    }
+}
 
 // One beam's 4 consecutive samples (one lane): DFT-4, fftshift, XY -> LR,
 // into the staged rows of local beam lb at column col (the spectrum's index
@@ -522,7 +584,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
     const int J = nch * upad;
     const size_t ant_stride = (size_t)a.F * a.T;   // complex samples between antennas
 
-    typedef TimeMap<NT, epi_run<NT, EPI>()> M;
+    typedef TimeMap<NT, epi_run<NT, EPI, AR>()> M;
     // First sample of this lane in chunk c (runs of M::RUN samples, TimeMap).
     auto chunk_t0 = [&](int c) { return ((cw0 + c * cstride) * WAVES + wave) * (TILE * NT) + M::RUN * i; };
 
@@ -780,6 +842,61 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
             }
             return;
         }
+        if constexpr (wave_stage<NT, AR, MW, EPI>()) {
+            if ((EPI && !(EPI & EPI_STAGE_FLAG)) || a.stage) {
+            float4* const stg = reinterpret_cast<float4*>(lds_raw + a.wbytes) + wave * 4 * kWaveRow;
+            const int rate = epi_rate<EPI>(a), lr = rate >> 1;       // log2 of 1, 2, 4
+            const bool pol = epi_pol<EPI>(a);
+            // This lane's result of a row: fine channel k, spectrum s.
+            const int tw = ((cw0 + c * cstride) * WAVES + wave) * (TILE * 4);
+            const int k = lane >> (6 - lr), sc = (tw >> lr) + (lane & ((64 >> lr) - 1));
+            const int S = a.T >> lr, kp = k ^ (rate >> 1);           // fftshift
+            const bool s_ok = sc < S;
+            float4* const base = reinterpret_cast<float4*>(a.y) + ((size_t)fo * rate + kp) * S + sc;
+            const size_t bstride = (size_t)a.F * a.T;
+            float4* const sink = a.sink + lane;
+            const int rd = lane + (lane >> 2);
+#pragma unroll
+            for (int m = 0; m < MW; m++)
+#pragma unroll
+                for (int rr = 0; rr < 2; rr++) {
+                    float2 v[2][4];
+#pragma unroll
+                    for (int p = 0; p < 2; p++)
+#pragma unroll
+                        for (int n = 0; n < 4; n++)
+                            v[p][n] = make_float2(acc[m][p][n][2 * rr] * unscale[p], acc[m][p][n][2 * rr + 1] * unscale[p]);
+                    wave_stage_beam(stg + g * kWaveRow, i, rate, pol, v);
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int b = b_wg + 8 * m + 2 * q + rr;
+                        const float4 z = stg[q * kWaveRow + rd];
+                        store4<NTS>(s_ok && b < a.B ? base + b * bstride : sink, make_float2(z.x, z.y),
+                                    make_float2(z.z, z.w));
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                }
+            if (epi_inc<EPI>(a)) {
+                float2 v[2][4];
+#pragma unroll
+                for (int p = 0; p < 2; p++)
+#pragma unroll
+                    for (int n = 0; n < 4; n++) {
+                        float e = inc[p][n];
+                        e += __shfl_xor(e, 16, 64);
+                        e += __shfl_xor(e, 32, 64);
+                        v[p][n] = make_float2(a.inc_sqrt ? sqrtf(e) : e, 0.f);
+                    }
+                wave_stage_beam(stg + g * kWaveRow, i, rate, pol, v);     // four equal rows
+                __builtin_amdgcn_wave_barrier();
+                const float4 z = stg[rd];
+                store4<NTS>(do_inc && s_ok ? base + a.B * bstride : sink, make_float2(z.x, z.y), make_float2(z.z, z.w));
+                __builtin_amdgcn_wave_barrier();
+            }
+            return;
+            }
+        }
         if constexpr (G3) {
             // Rows are beams: lane group g holds beams 4g .. 4g + 3.
 #pragma unroll
@@ -793,7 +910,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
                         const float p1 = acc[0][p][n][r], p2 = acc[1][p][n][r], p3 = acc[2][p][n][r];
                         v[p][n] = make_float2(p1 - p2, p3 - p1 - p2);
                     }
-                store_beam<NT, NTS, EPI>(a, min(b, a.B - 1), fo, t0, v, t_ok && b < a.B);
+                store_beam<NT, NTS, EPI, AR>(a, min(b, a.B - 1), fo, t0, v, t_ok && b < a.B);
             }
         } else
 #pragma unroll
@@ -811,7 +928,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
                         else
                             v[p][n] = make_float2(acc[m][p][n][r], acc[m][p][n][r + 1]);
                     }
-                store_beam<NT, NTS, EPI>(a, min(b, a.B - 1), fo, t0, v, t_ok && b < a.B);
+                store_beam<NT, NTS, EPI, AR>(a, min(b, a.B - 1), fo, t0, v, t_ok && b < a.B);
             }
         }
         // The incoherent beam's stores are issued by every workgroup (to the
@@ -832,7 +949,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
 #pragma unroll
                 for (int n = 0; n < NT; n++)
                     v[p][n] = make_float2(a.inc_sqrt ? sqrtf(inc[p][n]) : inc[p][n], 0.f);
-            store_beam<NT, false, EPI>(a, a.B, fo, t0, v, do_inc && t_ok && g == 0);
+            store_beam<NT, false, EPI, AR>(a, a.B, fo, t0, v, do_inc && t_ok && g == 0);
         }
     };
 
@@ -966,6 +1083,10 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
     // A operands, then the staged phasors of both pols (packed in the kernel).
     size_t lds = a.wbytes + staged_bytes(AR, MW, a.A);
     if (staged_epilogue<NT, AR, MW, EPI>()) lds = std::max(lds, a.wbytes + stage_bytes(AR));
+    if (wave_stage<NT, AR, MW, EPI>() && (EPI || a.wbytes + kWaveStageBytes <= kMaxLds)) {
+        a.stage = 1;
+        lds = std::max(lds, a.wbytes + kWaveStageBytes);
+    }
     const int span = WAVES * TILE * NT;
     const int groups = groups_for(a.B, MW);
     // Device scratch: only the store sink of idle lanes (the phasors are
@@ -1013,9 +1134,14 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
 template <int NT, int MW, bool CI8, int AR, int D>
 static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, hipStream_t s) {
     if constexpr (NT == 4) {
+        // The largest arrays leave no LDS for staged rows: generic variant.
+        const size_t wb = operand_bytes(AR, MW, nsteps_for(AR, a.A));
+        if (ar_split(AR) && wb + std::max(stage_bytes(AR), kWaveStageBytes) > kMaxLds)
+            return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
         if (epi == EPI_MODEB) return launch_bf<NT, MW, CI8, AR, D, true, EPI_MODEB>(a, ws, wsb, s);
-        // The rate-1 epilogues map a wave onto TILE * NT consecutive samples
-        // (runs of one): T must not cut a wave.
+        // The rate-1 epilogues of CF32 input map a wave onto TILE * NT
+        // consecutive samples (runs of one): T must not cut a wave.  Nontemporal
+        // stores want whole lines besides.
         if (a.T % (TILE * NT) == 0) {
             if (epi == EPI_PLAIN) return launch_bf<NT, MW, CI8, AR, D, true, EPI_PLAIN>(a, ws, wsb, s);
             if (epi == EPI_PLAIN_INC)
@@ -1052,7 +1178,7 @@ struct BatchBlock {
     float2* y;
     size_t wbytes;          // bytes of the phasor A operands in LDS
     int A, F, T, B;
-    int nsteps, n_tchunks, cpw, groups, mw;
+    int nsteps, n_tchunks, cpw, groups, mw, stage;
     int item_base;          // first work item of the block
 };
 
@@ -1070,6 +1196,7 @@ __device__ __forceinline__ BfArgs batch_block_args(const BatchArgs& ba, int k) {
     a.incoherent = 0; a.inc_sqrt = 0; a.rate = 1; a.polarize = 0;
     a.nsteps = b.nsteps; a.n_tchunks = b.n_tchunks; a.chunks_per_wg = b.cpw;
     a.wbytes = b.wbytes;
+    a.stage = b.stage;
     a.sink = ba.sink;
     return a;
 }
@@ -1095,9 +1222,9 @@ __global__ __launch_bounds__(256, 2) void beamform_batched_kernel(BatchArgs ba) 
         // Each item packs its (channel, beam group)'s phasors into LDS
         // itself, as the single-block kernel does.
         if (b.mw == 2)
-            bf_body<NT, 2, true, AR, D, true, EPI_PLAIN>(a, f, gz, tr * b.cpw, lds_raw, s_unscale, s_w0sq, s_max);
+            bf_body<NT, 2, true, AR, D, true, EPI_BATCH>(a, f, gz, tr * b.cpw, lds_raw, s_unscale, s_w0sq, s_max);
         else
-            bf_body<NT, 1, true, AR, D, true, EPI_PLAIN>(a, f, gz, tr * b.cpw, lds_raw, s_unscale, s_w0sq, s_max);
+            bf_body<NT, 1, true, AR, D, true, EPI_BATCH>(a, f, gz, tr * b.cpw, lds_raw, s_unscale, s_w0sq, s_max);
     }
 }
 
@@ -1165,7 +1292,8 @@ static int plan_batch(int ar, const blade_beamform_block* blocks, int n,
         b.item_base = (int)items;
         items += (long)ceil_div(b.n_tchunks, b.cpw) * b.F * b.groups;
         // A operands, then the staged phasors of both pols and the group's beams
-        lds = std::max(lds, b.wbytes + staged_bytes(ar, b.mw, b.A));
+        b.stage = b.wbytes + kWaveStageBytes <= kMaxLds;
+        lds = std::max(lds, b.wbytes + std::max(staged_bytes(ar, b.mw, b.A), b.stage ? kWaveStageBytes : 0));
     }
     if (items > (1L << 30)) return fail("batched beamformer: too many work items");
     if (lds > kMaxLds) return fail("batched beamformer: too many antennas");
@@ -1249,6 +1377,7 @@ static int run_beamformer(int in_type, int precision, const void* input, const v
     a.n_tchunks = 0;
     a.chunks_per_wg = 1;
     a.wbytes = 0;
+    a.stage = 0;
     a.sink = nullptr;
     const int ar = precision == BLADE_PREC_F16X2 ? AR_F16X2 : (in_type == BLADE_CI8 ? AR_BF16X3 : AR_F32);
     if (ar == AR_BF16X3 && !antennas_fit_f32(a.B > TILE / 2 ? 2 : 1, a.A))

@@ -92,59 +92,15 @@ struct BfArgs {
     float4* sink;           // 64 x 16 B: target of the stores of lanes with nothing to store
 };
 
-// Packs the phasors of one (f, beam group) into the A-operand layout the
-// beamformer reads from LDS, followed by |w0|^2[p][a] (256 floats) and the
-// split-FP16 unscale factors (2 floats).
-//   FP32       [m][p][step][g][row] float, step = 2 * antenna group + component
-//   split FP16 [m][p][step][hl][lane] halfx8 (8 k values = 4 antennas x re/im),
-//              components scaled by a per-pol power of two so that all are < 1,
-//              hi = fp16(w), lo = fp16(w - hi).
-// (three-part BF16: bf_pack_bf16x3.)
-// G3 selects the three-product FP32 layout (16-beam tiles, see bf_body).
-//
-// bf_pack_fill writes the (beam tile m, pol p) part from staged phasors `sw`
-// ([SB][A] float2 of pol p: the 8 beams of tile m for FP32, all MW * 8 beams
-// of the group for split FP16, whose scale is shared by the group's pol).
-template <int MW, int AR, bool G3>
+// FP32 operands of (beam tile m, pol p) from the staged phasors `sw` ([8][A]
+// float2 of pol p):  [m][p][step][g][row] float, step = 2 * antenna group +
+// component.  G3 selects the three-product layout (16-beam tiles, see bf_body).
+template <int MW, bool G3>
 __device__ __forceinline__ void bf_pack_fill(const BfArgs& a, const int m, const int p, const float2* sw,
-                                             const float scale, unsigned char* dst) {
-    constexpr int AK = ar_split(AR) ? 4 * KG : KG;
+                                             unsigned char* dst) {
     const int A = a.A;
     const int nsteps = a.nsteps;
-    if constexpr (AR == AR_F16X2) {
-        // beam (within the staged rows) of A-operand row `row` of tile m
-        const int row_beam0 = m * (TILE / 2);
-        // [m][p][step][hl][lane] halfx8, the (m, p) block
-        halfx8* wh = reinterpret_cast<halfx8*>(dst) + (size_t)((m * 2 + p) * nsteps) * 128;
-        for (int e = threadIdx.x; e < nsteps * 128; e += blockDim.x) {
-            const int st = e >> 7, hl = (e >> 6) & 1, ln = e & 63;
-            const int row = ln & (TILE - 1), kg = ln >> 4;
-            const int bl_ = row_beam0 + (row >> 1), co = row & 1;
-            halfx8 h;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int an = st * AK + 4 * kg + q;
-                float wr = 0.f, wi = 0.f;
-                if (an < A) {
-                    const float2 w = sw[bl_ * A + an];
-                    wr = w.x * scale;
-                    wi = w.y * scale;
-                }
-                // k = (antenna, c): c = 0 multiplies Re x, c = 1 multiplies Im x.
-                const float v0 = co == 0 ? wr : wi;
-                const float v1 = co == 0 ? -wi : wr;
-                const _Float16 h0 = (_Float16)v0, h1 = (_Float16)v1;
-                if (hl == 0) {
-                    h[2 * q] = h0;
-                    h[2 * q + 1] = h1;
-                } else {
-                    h[2 * q] = (_Float16)(v0 - (float)h0);
-                    h[2 * q + 1] = (_Float16)(v1 - (float)h1);
-                }
-            }
-            wh[e] = h;
-        }
-    } else if constexpr (G3) {
+    if constexpr (G3) {
         // Three-product layout [p][unit][q][g][row] float, q = (Wr, Wi, Wr + Wi),
         // row = beam of the 16-beam tile; this part is rows 8m .. 8m + 7.
         const int nunits = nsteps / 2;
@@ -190,94 +146,46 @@ __device__ __forceinline__ void bf_pack_w0sq(const BfArgs& a, const float2* sw, 
     }
 }
 
-// Three-part BF16 operands of the (f, beam group), [m][p][step][part][lane]
-// bf16x8 (8 k values = 4 antennas x re/im), straight from memory: no scale is
-// shared, so nothing is staged, and every thread has the loads of its four
-// antennas (both pols in 16 bytes) in flight at once.  Ends with a barrier.
-template <int MW>
-__device__ __forceinline__ void bf_pack_bf16x3(const BfArgs& a, const int f, const int gz, unsigned char* dst,
-                                               float* w0sq) {
+// Split operands of the (f, beam group), [m][p][step][part][lane] (16 bytes:
+// 8 k values = 4 antennas x re/im), straight from memory: every thread has the
+// loads of its four antennas (both pols in 16 bytes) in flight at once and
+// nothing is staged.  Split FP16 first takes the largest component per pol for
+// its power-of-two scale; the first entry's phasors (all of them up to 32
+// antennas at 16 beams) stay in registers across that barrier, later ones are
+// read again.  Ends with a barrier.
+template <int MW, int AR>
+__device__ __forceinline__ void bf_pack_split(const BfArgs& a, const int f, const int gz, unsigned char* dst,
+                                              unsigned int* s_max, float* w0sq, float* unscale) {
+    constexpr int PARTS = ar_parts(AR);
     const int A = a.A, nsteps = a.nsteps;
     const float4* w4 = reinterpret_cast<const float4*>(a.w) + f;
     uint4* wb = reinterpret_cast<uint4*>(dst);
-    for (int e = threadIdx.x; e < MW * nsteps * 64; e += WAVES * 64) {
+    const int n_e = MW * nsteps * 64;
+    auto load = [&](int e, float4 (&w)[4]) {
         const int ln = e & 63, ms = e >> 6;
         const int m = (MW == 2 && ms >= nsteps) ? 1 : 0, st = ms - m * nsteps;
-        const int row = ln & (TILE - 1), kg = ln >> 4;
-        const int b = gz * MW * (TILE / 2) + m * (TILE / 2) + (row >> 1);
-        const bool im = row & 1;
-        float4 w[4];
+        const int b = gz * MW * (TILE / 2) + m * (TILE / 2) + ((ln & (TILE - 1)) >> 1);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int an = st * 4 * KG + 4 * kg + q;
+            const int an = st * 4 * KG + 4 * (ln >> 4) + q;
             w[q] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (an < A && b < a.B) w[q] = w4[((size_t)b * A + an) * a.F];
         }
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            uint32_t h[3][4];
+    };
+    float4 w[4];
+    float scale[2] = {1.f, 1.f};
+    if constexpr (AR == AR_F16X2) {
+        if (threadIdx.x < 2) s_max[threadIdx.x] = 0u;
+        __syncthreads();
+        float mx[2] = {0.f, 0.f};
+        for (int e = n_e - 1 - (int)((n_e - 1 - threadIdx.x) % (WAVES * 64)); e >= 0; e -= WAVES * 64) {   // last: e = threadIdx.x
+            load(e, w);
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const float wr = p ? w[q].z : w[q].x, wi = p ? w[q].w : w[q].y;
-                // k = (antenna, c): c = 0 multiplies Re x, c = 1 multiplies Im x.
-                float v0[3], v1[3];
-                split_bf16x3(im ? wi : wr, v0);
-                split_bf16x3(im ? wr : -wi, v1);
-#pragma unroll
-                for (int k = 0; k < 3; k++) h[k][q] = bf16_pair(v0[k], v1[k]);
+                mx[0] = fmaxf(mx[0], fmaxf(fabsf(w[q].x), fabsf(w[q].y)));
+                mx[1] = fmaxf(mx[1], fmaxf(fabsf(w[q].z), fabsf(w[q].w)));
             }
-#pragma unroll
-            for (int k = 0; k < 3; k++)
-                wb[(((m * 2 + p) * nsteps + st) * 3 + k) * 64 + ln] = make_uint4(h[k][0], h[k][1], h[k][2], h[k][3]);
         }
-    }
-    if (gz == 0 && threadIdx.x < 128) {
-        float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (threadIdx.x < A) w = w4[(size_t)threadIdx.x * a.F];
-        w0sq[threadIdx.x] = w.x * w.x + w.y * w.y;
-        w0sq[128 + threadIdx.x] = w.z * w.z + w.w * w.w;
-    }
-    __syncthreads();
-}
-
-// The whole (f, beam group) straight into the workgroup's LDS: one round of
-// phasor loads for both pols and all MW * 8 beams (s_w: [2][MW * 8][A]),
-// then every (m, p) part.  Ends with a barrier.
-template <int MW, int AR, bool G3>
-__device__ __forceinline__ void bf_pack_lds(const BfArgs& a, const int f, const int gz, float2* s_w,
-                                            unsigned int* s_max, unsigned char* dst, float* w0sq,
-                                            float* unscale) {
-    constexpr int NB = MW * (TILE / 2);
-    const int A = a.A;
-    if (threadIdx.x < 2) s_max[threadIdx.x] = 0u;
-    float mx[2] = {0.f, 0.f};
-    if (((uintptr_t)a.w & 15) == 0) {
-        // Both pols of a (beam, antenna) are one 16-byte load: half the
-        // scattered phasor loads (split FP16 114.7 -> 113.0 us per Mode-B call).
-        for (int r = threadIdx.x; r < NB * A; r += blockDim.x) {
-            const int bl_ = r / A, an = r - bl_ * A, b = gz * NB + bl_;
-            float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (b < a.B) w = reinterpret_cast<const float4*>(a.w)[((size_t)b * A + an) * a.F + f];
-            s_w[r] = make_float2(w.x, w.y);
-            s_w[NB * A + r] = make_float2(w.z, w.w);
-            mx[0] = fmaxf(mx[0], fmaxf(fabsf(w.x), fabsf(w.y)));
-            mx[1] = fmaxf(mx[1], fmaxf(fabsf(w.z), fabsf(w.w)));
-        }
-    } else {
-        for (int e = threadIdx.x; e < 2 * NB * A; e += blockDim.x) {
-            const int p = e / (NB * A), r = e - p * (NB * A);
-            const int bl_ = r / A, an = r - bl_ * A, b = gz * NB + bl_;
-            float2 w = make_float2(0.f, 0.f);
-            if (b < a.B) w = a.w[(((size_t)b * A + an) * a.F + f) * 2 + p];
-            s_w[e] = w;
-            const float v = fmaxf(fabsf(w.x), fabsf(w.y));
-            mx[0] = p == 0 ? fmaxf(mx[0], v) : mx[0];
-            mx[1] = p == 1 ? fmaxf(mx[1], v) : mx[1];
-        }
-    }
-    __syncthreads();
-    float scale[2] = {1.f, 1.f}, uns[2] = {1.f, 1.f};
-    if constexpr (AR == AR_F16X2) {
         atomicMax(&s_max[0], __float_as_uint(mx[0]));
         atomicMax(&s_max[1], __float_as_uint(mx[1]));
         __syncthreads();
@@ -286,20 +194,75 @@ __device__ __forceinline__ void bf_pack_lds(const BfArgs& a, const int f, const 
             int ex = 0;
             frexpf(__uint_as_float(s_max[p]), &ex);
             scale[p] = ldexpf(1.0f, -ex);
-            uns[p] = ldexpf(1.0f, ex);
+            if (threadIdx.x == 0) unscale[p] = ldexpf(1.0f, ex);
         }
     }
+    for (int e = threadIdx.x; e < n_e; e += WAVES * 64) {
+        if (AR != AR_F16X2 || e >= WAVES * 64) load(e, w);
+        const int ln = e & 63, ms = e >> 6;
+        const int m = (MW == 2 && ms >= nsteps) ? 1 : 0, st = ms - m * nsteps;
+        const bool im = ln & 1;
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            uint32_t h[PARTS][4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const float wr = p ? w[q].z : w[q].x, wi = p ? w[q].w : w[q].y;
+                // k = (antenna, c): c = 0 multiplies Re x, c = 1 multiplies Im x.
+                const float v0 = im ? wi : wr, v1 = im ? wr : -wi;
+                if constexpr (AR == AR_BF16X3) {
+                    float p0[3], p1[3];
+                    split_bf16x3(v0, p0);
+                    split_bf16x3(v1, p1);
+#pragma unroll
+                    for (int k = 0; k < 3; k++) h[k][q] = bf16_pair(p0[k], p1[k]);
+                } else {
+                    const float u0 = v0 * scale[p], u1 = v1 * scale[p];
+                    const halfx2 hi = {(_Float16)u0, (_Float16)u1};
+                    const halfx2 lo = {(_Float16)(u0 - (float)hi[0]), (_Float16)(u1 - (float)hi[1])};
+                    h[0][q] = __builtin_bit_cast(uint32_t, hi);
+                    h[1][q] = __builtin_bit_cast(uint32_t, lo);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < PARTS; k++)
+                wb[(((m * 2 + p) * nsteps + st) * PARTS + k) * 64 + ln] = make_uint4(h[k][0], h[k][1], h[k][2], h[k][3]);
+        }
+    }
+    if (gz == 0 && threadIdx.x < 128) {
+        float4 w0 = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (threadIdx.x < A) w0 = w4[(size_t)threadIdx.x * a.F];
+        w0sq[threadIdx.x] = w0.x * w0.x + w0.y * w0.y;
+        w0sq[128 + threadIdx.x] = w0.z * w0.z + w0.w * w0.w;
+    }
+    __syncthreads();
+}
+
+// FP32: the whole (f, beam group) straight into the workgroup's LDS: one round
+// of phasor loads for both pols and all MW * 8 beams (s_w: [2][MW * 8][A]),
+// then every (m, p) part.  Ends with a barrier.
+template <int MW, bool G3>
+__device__ __forceinline__ void bf_pack_lds(const BfArgs& a, const int f, const int gz, float2* s_w,
+                                            unsigned char* dst, float* w0sq) {
+    constexpr int NB = MW * (TILE / 2);
+    const int A = a.A;
+    for (int r = threadIdx.x; r < NB * A; r += blockDim.x) {
+        const int bl_ = r / A, an = r - bl_ * A, b = gz * NB + bl_;
+        float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (b < a.B) w = reinterpret_cast<const float4*>(a.w)[((size_t)b * A + an) * a.F + f];
+        s_w[r] = make_float2(w.x, w.y);
+        s_w[NB * A + r] = make_float2(w.z, w.w);
+    }
+    __syncthreads();
 #pragma unroll
     for (int mp = 0; mp < 2 * MW; mp++) {
         const int p = mp & 1, m = mp >> 1;
-        const float2* sw = s_w + (size_t)p * NB * A + (AR == AR_F16X2 ? 0 : m * (TILE / 2) * A);
-        bf_pack_fill<MW, AR, G3>(a, m, p, sw, scale[p], dst);
+        bf_pack_fill<MW, G3>(a, m, p, s_w + (size_t)p * NB * A + m * (TILE / 2) * A, dst);
     }
     if (gz == 0) {
         bf_pack_w0sq(a, s_w, w0sq);
         bf_pack_w0sq(a, s_w + (size_t)NB * A, w0sq + 128);
     }
-    if (threadIdx.x < 2) unscale[threadIdx.x] = uns[threadIdx.x];
     __syncthreads();
 }
 
@@ -430,15 +393,14 @@ constexpr int EPI_BATCH = EPI_PLAIN | EPI_STAGE_FLAG;
 // Mode-B epilogue through LDS (split variants, 16-beam tiles): the four
 // wavefronts' spectra of one chunk are exchanged so that each store
 // instruction writes 1 KiB of one output row (64 consecutive spectra of one
-// (beam, fine channel)) instead of 256 B pieces of four rows.  Half of the
-// group's 16 beams at a time (a quarter with three BF16 parts, whose operands
-// take more LDS; 3 workgroups still fit a CU): [beams][4 fine channels][64 + 1]
-// float4 in LDS (the staged phasors' space, free once they are packed).
+// (beam, fine channel)) instead of 256 B pieces of four rows.  A quarter of the
+// group's 16 beams at a time, [4 beams][4 fine channels][64 + 1] float4 in LDS
+// behind the operands, so that 3 workgroups fit a CU.
 template <int NT, int AR, int MW, int EPI>
 constexpr bool staged_epilogue() { return ar_split(AR) && MW == 2 && NT == 4 && EPI == EPI_MODEB; }
 constexpr int kStageRow = 65;                                   // float4 per staged row, padded
-constexpr int stage_beams(int ar) { return ar == AR_BF16X3 ? 4 : 8; }
-constexpr size_t stage_bytes(int ar) { return (size_t)stage_beams(ar) * 4 * kStageRow * 16; }
+constexpr int kStageBeams = 4;   // beams per round
+constexpr size_t kStageBytes = (size_t)kStageBeams * 4 * kStageRow * 16;
 
 // Epilogue through LDS within a wavefront (split variants, every other
 // epilogue with 4 samples per lane): a lane's 4 consecutive samples of one beam,
@@ -631,11 +593,10 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
     // ---- This (f, beam group)'s packed phasors into LDS. ---------------------
     // A operands, |w0|^2 per antenna and pol, and the power-of-two unscale of
     // the split-FP16 path.
-    if constexpr (AR == AR_BF16X3)
-        bf_pack_bf16x3<MW>(a, f, gz, lds_raw, &s_w0sq[0][0]);
+    if constexpr (ar_split(AR))
+        bf_pack_split<MW, AR>(a, f, gz, lds_raw, s_max, &s_w0sq[0][0], s_unscale);
     else
-        bf_pack_lds<MW, AR, G3>(a, f, gz, reinterpret_cast<float2*>(lds_raw + a.wbytes), s_max, lds_raw,
-                                &s_w0sq[0][0], s_unscale);
+        bf_pack_lds<MW, G3>(a, f, gz, reinterpret_cast<float2*>(lds_raw + a.wbytes), lds_raw, &s_w0sq[0][0]);
     const float unscale[2] = {AR == AR_F16X2 ? s_unscale[0] : 1.f, AR == AR_F16X2 ? s_unscale[1] : 1.f};
 
     // Three-product FP32 tiles (16 beams): accumulators P1, P2, P3.
@@ -809,34 +770,28 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
             const int s = (cw0 + c * cstride) * (WAVES * TILE) + lane;
             float4* const base = reinterpret_cast<float4*>(a.y);
             float4* const sink = a.sink + lane;
-            // A round stages the beams of one tile (8), or every other one of
-            // them (4: tile m's beams 2g + rr), [beam][fine channel] rows.
-            constexpr int SB = stage_beams(AR);
-            constexpr int RPR = SB / 4;                            // beams per lane and round
+            // A round stages every other beam of a tile (tile m's beams
+            // 2g + rr), [beam][fine channel] rows.
 #pragma unroll
-            for (int h = 0; h < 16 / SB; h++) {
-                const int m = h * SB / 8, r0 = (h * RPR) & 1;
+            for (int h = 0; h < 4; h++) {
+                const int m = h >> 1, rr = h & 1;
                 __syncthreads();   // the previous round's (or chunk's) rows are stored
-#pragma unroll
-                for (int q = 0; q < RPR; q++) {
-                    const int r = 2 * (r0 + q);
+                {
                     float2 v[2][4];
 #pragma unroll
                     for (int p = 0; p < 2; p++)
 #pragma unroll
                         for (int n = 0; n < 4; n++)
-                            v[p][n] = make_float2(acc[m][p][n][r] * unscale[p], acc[m][p][n][r + 1] * unscale[p]);
-                    stage_beam(stg, RPR * g + q, col, v);
+                            v[p][n] = make_float2(acc[m][p][n][2 * rr] * unscale[p], acc[m][p][n][2 * rr + 1] * unscale[p]);
+                    stage_beam(stg, g, col, v);
                 }
                 __syncthreads();
 #pragma unroll
-                for (int j = 0; j < SB; j++) {
-                    const int row = wave * SB + j;
-                    const int b = b_wg + 8 * m + (RPR == 2 ? row >> 2 : 2 * (row >> 2) + r0);
+                for (int j = 0; j < 4; j++) {
+                    const int row = wave * 4 + j;                  // beam 2 wave + rr of the tile, fine channel j
+                    const int b = b_wg + 8 * m + 2 * wave + rr;
                     const float4 q = stg[row * kStageRow + lane];
-                    float4* dst = (s < S && b < a.B)
-                                      ? base + (((size_t)b * a.F + fo) * 4 + (row & 3)) * S + s
-                                      : sink;
+                    float4* dst = (s < S && b < a.B) ? base + (((size_t)b * a.F + fo) * 4 + j) * S + s : sink;
                     store4<NTS>(dst, make_float2(q.x, q.y), make_float2(q.z, q.w));
                 }
             }
@@ -1005,10 +960,10 @@ static size_t operand_bytes(int ar, int mw, int nsteps) {
 
 constexpr size_t kSinkBytes = 64 * sizeof(float4);
 
-// Bytes of the phasors staged behind the A operands: both pols of the group's
-// beams (the three-part BF16 operands are packed without a stage).
+// Bytes of the phasors the FP32 variant stages behind the A operands: both
+// pols of the group's beams (split operands are packed without a stage).
 static size_t staged_bytes(int ar, int mw, int A) {
-    return ar == AR_BF16X3 ? 0 : (size_t)2 * mw * (TILE / 2) * A * sizeof(float2);
+    return ar_split(ar) ? 0 : (size_t)2 * mw * (TILE / 2) * A * sizeof(float2);
 }
 
 constexpr size_t kMaxLds = 150 * 1024;
@@ -1018,10 +973,12 @@ static int nsteps_for(int ar, int A) {
 }
 
 // Antenna limit of a call whose beams are taken `mw` tiles at a time: that of
-// the LDS image of FP32 operands and staged phasors (240 antennas at 16
-// beams, 400 at 8).  Every FP32 variant keeps it, whatever its own LDS need.
-static bool antennas_fit_f32(int mw, int A) {
-    return operand_bytes(AR_F32, mw, nsteps_for(AR_F32, A)) + staged_bytes(AR_F32, mw, A) <= kMaxLds;
+// the LDS image of its operands (FP32 or split FP16) with staged phasors, 240
+// antennas at 16 beams and 400 at 8 for FP32, 192 and 400 for split FP16.  The
+// variants that need less LDS keep it.
+static bool antennas_fit(int ar, int mw, int A) {
+    const int image = ar == AR_F16X2 ? AR_F16X2 : AR_F32;
+    return operand_bytes(image, mw, nsteps_for(image, A)) + staged_bytes(AR_F32, mw, A) <= kMaxLds;
 }
 
 // Beam tiles per wavefront: 16 beams (2 tiles) past 8 beams, where they fit in
@@ -1029,7 +986,7 @@ static bool antennas_fit_f32(int mw, int A) {
 // at 16 beams (up to 176 antennas); above that 8-beam tiles (6 KiB) carry on.
 static int beam_tiles_for(int ar, int A, int B) {
     if (B <= TILE / 2) return 1;
-    if (ar == AR_BF16X3 && operand_bytes(ar, 2, nsteps_for(ar, A)) + stage_bytes(ar) > kMaxLds) return 1;
+    if (ar == AR_BF16X3 && operand_bytes(ar, 2, nsteps_for(ar, A)) + kStageBytes > kMaxLds) return 1;
     return 2;
 }
 
@@ -1082,7 +1039,7 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
     a.wbytes = operand_bytes(AR, MW, a.nsteps);
     // A operands, then the staged phasors of both pols (packed in the kernel).
     size_t lds = a.wbytes + staged_bytes(AR, MW, a.A);
-    if (staged_epilogue<NT, AR, MW, EPI>()) lds = std::max(lds, a.wbytes + stage_bytes(AR));
+    if (staged_epilogue<NT, AR, MW, EPI>()) lds = std::max(lds, a.wbytes + kStageBytes);
     if (wave_stage<NT, AR, MW, EPI>() && (EPI || a.wbytes + kWaveStageBytes <= kMaxLds)) {
         a.stage = 1;
         lds = std::max(lds, a.wbytes + kWaveStageBytes);
@@ -1136,7 +1093,7 @@ static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, h
     if constexpr (NT == 4) {
         // The largest arrays leave no LDS for staged rows: generic variant.
         const size_t wb = operand_bytes(AR, MW, nsteps_for(AR, a.A));
-        if (ar_split(AR) && wb + std::max(stage_bytes(AR), kWaveStageBytes) > kMaxLds)
+        if (ar_split(AR) && wb + std::max(kStageBytes, kWaveStageBytes) > kMaxLds)
             return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
         if (epi == EPI_MODEB) return launch_bf<NT, MW, CI8, AR, D, true, EPI_MODEB>(a, ws, wsb, s);
         // The rate-1 epilogues of CF32 input map a wave onto TILE * NT
@@ -1281,7 +1238,7 @@ static int plan_batch(int ar, const blade_beamform_block* blocks, int n,
         if (!bk.input || !bk.phasors || !bk.output) return fail("batched beamformer: null pointer");
         if ((uintptr_t)bk.input % 16 || (uintptr_t)bk.phasors % 16 || (uintptr_t)bk.output % 16)
             return fail("batched beamformer: buffers must be 16-byte aligned");
-        if (ar == AR_BF16X3 && !antennas_fit_f32(mw_force ? mw_force : (bk.B > TILE / 2 ? 2 : 1), (int)bk.A))
+        if (!antennas_fit(ar, mw_force ? mw_force : (bk.B > TILE / 2 ? 2 : 1), (int)bk.A))
             return fail("batched beamformer: too many antennas");
         BatchBlock& b = ba.blk[k];
         b.mw = tiles_of(bk);
@@ -1385,7 +1342,7 @@ static int run_beamformer(int in_type, int precision, const void* input, const v
     a.stage = 0;
     a.sink = nullptr;
     const int ar = precision == BLADE_PREC_F16X2 ? AR_F16X2 : (in_type == BLADE_CI8 ? AR_BF16X3 : AR_F32);
-    if (ar == AR_BF16X3 && !antennas_fit_f32(a.B > TILE / 2 ? 2 : 1, a.A))
+    if (!antennas_fit(ar, a.B > TILE / 2 ? 2 : 1, a.A))
         return fail("beamformer: too many antennas for the LDS phasor stage");
     const int mw = beam_tiles_for(ar, a.A, a.B);
     const int epi = (int)rate | (polarize ? 8 : 0) | (incoherent ? 16 : 0);

@@ -316,12 +316,14 @@ __device__ __forceinline__ void store4(float4* p, float2 X, float2 Y) {
 __device__ __forceinline__ constexpr int epi_code(int rate, bool pol, bool inc) {
     return rate | (pol ? 8 : 0) | (inc ? 16 : 0);
 }
+constexpr int EPI_ODD_FLAG = 64;
 template <int EPI> __device__ __forceinline__ int epi_rate(const BfArgs& a) { return EPI ? (EPI & 7) : a.rate; }
 template <int NT, int EPI, int AR> constexpr int epi_run() {
-    return (EPI && (EPI & 7) == 1 && !ar_split(AR)) ? 1 : (NT < 4 ? NT : 4);
+    return (EPI && (EPI & 7) == 1 && (!ar_split(AR) || (EPI & EPI_ODD_FLAG))) ? 1 : NT;
 }
-template <int EPI> __device__ __forceinline__ bool epi_pol(const BfArgs& a) { return EPI ? (EPI & 8) != 0 : a.polarize != 0; }
-template <int EPI> __device__ __forceinline__ bool epi_inc(const BfArgs& a) { return EPI ? (EPI & 16) != 0 : a.incoherent != 0; }
+template <int EPI> constexpr bool epi_fixed() { return EPI && !(EPI & EPI_ODD_FLAG); }
+template <int EPI> __device__ __forceinline__ bool epi_pol(const BfArgs& a) { return epi_fixed<EPI>() ? (EPI & 8) != 0 : a.polarize != 0; }
+template <int EPI> __device__ __forceinline__ bool epi_inc(const BfArgs& a) { return epi_fixed<EPI>() ? (EPI & 16) != 0 : a.incoherent != 0; }
 
 template <int NT, bool NTS, int EPI, int AR>
 __device__ __forceinline__ void store_beam(const BfArgs& a, int b, int f, int t0,
@@ -337,7 +339,8 @@ __device__ __forceinline__ void store_beam(const BfArgs& a, int b, int f, int t0
         }
         float4* dst = reinterpret_cast<float4*>(a.y) + ((size_t)b * a.F + f) * a.T + t0;
 #pragma unroll
-        for (int n = 0; n < NT; n++) store4<NTS>(ok ? dst + M::off(n) : sink, v[0][n], v[1][n]);
+        for (int n = 0; n < NT; n++)
+            store4<NTS>(ok && (!(EPI & EPI_ODD_FLAG) || t0 + M::off(n) < a.T) ? dst + M::off(n) : sink, v[0][n], v[1][n]);
         return;
     }
     if constexpr (NT % 4 == 0) {
@@ -389,6 +392,9 @@ constexpr int EPI_PLAIN = 1;              // rate 1
 constexpr int EPI_PLAIN_INC = 1 | 16;     // rate 1, incoherent beam
 constexpr int EPI_STAGE_FLAG = 32;        // with a fixed variant: staged rows only where BfArgs::stage says so
 constexpr int EPI_BATCH = EPI_PLAIN | EPI_STAGE_FLAG;
+// T no multiple of 4 (rate 1): samples one by one, each with its own bound;
+// polarize and incoherent from the arguments.
+constexpr int EPI_ODD = 1 | EPI_ODD_FLAG;
 
 // Mode-B epilogue through LDS (split variants, 16-beam tiles): the four
 // wavefronts' spectra of one chunk are exchanged so that each store
@@ -412,7 +418,9 @@ constexpr size_t kStageBytes = (size_t)kStageBeams * 4 * kStageRow * 16;
 // there is no barrier.  Rows carry one entry of padding per 4, which puts the 16
 // lanes' 64-byte pieces on different banks.
 template <int NT, int AR, int MW, int EPI>
-constexpr bool wave_stage() { return ar_split(AR) && NT == 4 && !staged_epilogue<NT, AR, MW, EPI>(); }
+constexpr bool wave_stage() {
+    return ar_split(AR) && NT == 4 && !staged_epilogue<NT, AR, MW, EPI>() && !(EPI & EPI_ODD_FLAG);
+}
 constexpr int kWaveRow = 80;                                    // float4 per row
 constexpr size_t kWaveStageBytes = (size_t)WAVES * 4 * kWaveRow * 16;
 
@@ -523,8 +531,9 @@ __device__ __forceinline__ void load_words(uint32_t* dst, const uint32_t* src) {
 // antenna and beam row at the same time; with voltages coming from HBM
 // rather than the last-level cache that is ~3% faster than consecutive
 // chunk ranges.  The work item packs its phasors straight into LDS
-// (bf_pack_lds): lds_raw holds the A operands, then the staged phasors
-// [2][MW * 8][A] float2; s_unscale / s_w0sq the split-FP16 unscale and |w0|^2.
+// (bf_pack_split, bf_pack_lds): lds_raw holds the A operands, then the staged
+// phasors (FP32, [2][MW * 8][A] float2) or the epilogue's rows; s_unscale / s_w0sq
+// the split-FP16 unscale and |w0|^2.
 template <int NT, int MW, bool CI8, int AR, int D, bool NTS, int EPI, bool G3 = (AR == AR_F32 && MW == 2)>
 __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int gz, const int cw0,
                                         unsigned char* lds_raw, float* s_unscale, float (*s_w0sq)[128],
@@ -562,6 +571,8 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
         t0 = (t0 < a.T) ? t0 : 0;
         const size_t off = (size_t)f * a.T + t0;
         constexpr int R = M::RUN;
+        // Offset of run h, kept inside the row where T may cut a run.
+        auto run_off = [&](int h) { return (EPI & EPI_ODD_FLAG) ? min(M::off(h * R), a.T - 1 - t0) : M::off(h * R); };
         if constexpr (ar_split(AR)) {
             const uint32_t* x = static_cast<const uint32_t*>(a.x);
 #pragma unroll
@@ -569,17 +580,17 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
                 const int an = min(un * AK + 4 * g + q, a.A - 1);
 #pragma unroll
                 for (int h = 0; h < NT / R; h++)
-                    load_words<R>(u.w + q * NT + h * R, x + an * ant_stride + off + M::off(h * R));
+                    load_words<R>(u.w + q * NT + h * R, x + an * ant_stride + off + run_off(h));
             }
         } else {
             const int an = min(un * KG + g, a.A - 1);
 #pragma unroll
             for (int h = 0; h < NT / R; h++) {
                 if constexpr (CI8) {
-                    load_words<R>(u.w + h * R, static_cast<const uint32_t*>(a.x) + an * ant_stride + off + M::off(h * R));
+                    load_words<R>(u.w + h * R, static_cast<const uint32_t*>(a.x) + an * ant_stride + off + run_off(h));
                 } else {
                     load_words<4 * R>(u.w + 4 * h * R,
-                                      static_cast<const uint32_t*>(a.x) + 4 * (an * ant_stride + off + M::off(h * R)));
+                                      static_cast<const uint32_t*>(a.x) + 4 * (an * ant_stride + off + run_off(h)));
                 }
             }
         }
@@ -1090,32 +1101,38 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
 
 template <int NT, int MW, bool CI8, int AR, int D>
 static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, hipStream_t s) {
-    if constexpr (NT == 4) {
-        // The largest arrays leave no LDS for staged rows: generic variant.
-        const size_t wb = operand_bytes(AR, MW, nsteps_for(AR, a.A));
-        if (ar_split(AR) && wb + std::max(kStageBytes, kWaveStageBytes) > kMaxLds)
-            return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
-        if (epi == EPI_MODEB) return launch_bf<NT, MW, CI8, AR, D, true, EPI_MODEB>(a, ws, wsb, s);
-        // The rate-1 epilogues of CF32 input map a wave onto TILE * NT
-        // consecutive samples (runs of one): T must not cut a wave.  Nontemporal
-        // stores want whole lines besides.
-        if (a.T % (TILE * NT) == 0) {
-            if (epi == EPI_PLAIN) return launch_bf<NT, MW, CI8, AR, D, true, EPI_PLAIN>(a, ws, wsb, s);
-            if (epi == EPI_PLAIN_INC)
-                return launch_bf<NT, MW, CI8, AR, D, true, EPI_PLAIN_INC>(a, ws, wsb, s);
+    if (a.T % 4) {
+        // CF32 takes one sample per lane (chunks of 64 instead of 256 samples)
+        // where chunks of 256 are under four per CU: A20 F192 T511 B8 12.6 against
+        // 13.5 us, A12 F90 T931 B19 16.7 against 18.6; past it 256 are faster (A28
+        // F192 T2047 B8 36.8 against 42.2).  CI8 is faster with 256 at all of these.
+        if constexpr (AR == AR_F32) {
+            if ((long)ceil_div(a.T, WAVES * TILE * NT) * a.F * groups_for(a.B, MW) < 4L * device_cus())
+                return launch_bf<1, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
         }
+        return launch_bf<NT, MW, CI8, AR, D, false, EPI_ODD>(a, ws, wsb, s);
+    }
+    // The largest arrays leave no LDS for staged rows: generic variant.
+    const size_t wb = operand_bytes(AR, MW, nsteps_for(AR, a.A));
+    if (ar_split(AR) && wb + std::max(kStageBytes, kWaveStageBytes) > kMaxLds)
+        return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
+    if (epi == EPI_MODEB) return launch_bf<NT, MW, CI8, AR, D, true, EPI_MODEB>(a, ws, wsb, s);
+    // The rate-1 epilogues of CF32 input map a wave onto TILE * NT
+    // consecutive samples (runs of one): T must not cut a wave.  Nontemporal
+    // stores want whole lines besides.
+    if (a.T % (TILE * NT) == 0) {
+        if (epi == EPI_PLAIN) return launch_bf<NT, MW, CI8, AR, D, true, EPI_PLAIN>(a, ws, wsb, s);
+        if (epi == EPI_PLAIN_INC)
+            return launch_bf<NT, MW, CI8, AR, D, true, EPI_PLAIN_INC>(a, ws, wsb, s);
     }
     return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
 }
 
 template <bool CI8, int AR>
-static int dispatch(const BfArgs& a, int nt, int mw, int epi, unsigned char* ws, size_t wsb, hipStream_t s) {
+static int dispatch(const BfArgs& a, int mw, int epi, unsigned char* ws, size_t wsb, hipStream_t s) {
     constexpr int D = 2;
-    if (nt == 4)
-        return mw == 2 ? launch_epi<4, 2, CI8, AR, D>(a, epi, ws, wsb, s)
-                       : launch_epi<4, 1, CI8, AR, D>(a, epi, ws, wsb, s);
-    return mw == 2 ? launch_epi<1, 2, CI8, AR, D>(a, epi, ws, wsb, s)
-                   : launch_epi<1, 1, CI8, AR, D>(a, epi, ws, wsb, s);
+    return mw == 2 ? launch_epi<4, 2, CI8, AR, D>(a, epi, ws, wsb, s)
+                   : launch_epi<4, 1, CI8, AR, D>(a, epi, ws, wsb, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1346,10 +1363,9 @@ static int run_beamformer(int in_type, int precision, const void* input, const v
         return fail("beamformer: too many antennas for the LDS phasor stage");
     const int mw = beam_tiles_for(ar, a.A, a.B);
     const int epi = (int)rate | (polarize ? 8 : 0) | (incoherent ? 16 : 0);
-    const int nt = T % 4 == 0 ? 4 : 1;
-    if (ar == AR_F16X2) return dispatch<true, AR_F16X2>(a, nt, mw, epi, ws, wsb, s);
-    if (ar == AR_BF16X3) return dispatch<true, AR_BF16X3>(a, nt, mw, epi, ws, wsb, s);
-    return dispatch<false, AR_F32>(a, nt, mw, epi, ws, wsb, s);
+    if (ar == AR_F16X2) return dispatch<true, AR_F16X2>(a, mw, epi, ws, wsb, s);
+    if (ar == AR_BF16X3) return dispatch<true, AR_BF16X3>(a, mw, epi, ws, wsb, s);
+    return dispatch<false, AR_F32>(a, mw, epi, ws, wsb, s);
 }
 
 // Scratch of blade_beamform_chain_noalloc: the store sink of idle lanes as

@@ -134,3 +134,22 @@ def test_stokes_gradient_keeps_nonfinite_values_in_their_beam():
     got = got.cpu().numpy()
     assert np.isfinite(got[[0, 2]]).all() and np.isfinite(got[1, ..., 1]).all()
     assert not np.isfinite(got[1, ..., 0]).any()
+
+
+@pytest.mark.parametrize("kind", ["ci8-f32", "ci8-f16x2", "cf32"])
+@pytest.mark.parametrize("A,F,T,B,inc,polarize", [(3, 2, 1, 2, False, False), (5, 2, 65, 9, True, True),
+                                                  (20, 3, 255, 8, True, False), (7, 300, 1021, 17, False, True)])
+def test_sample_counts_no_multiple_of_four(kind, A, F, T, B, inc, polarize):
+    """Single samples with a bound each (and CF32's one-sample lanes on small
+    grids); normwise, the FP32 bar of the forward bound above."""
+    rng = np.random.default_rng(T)
+    x8 = rng.integers(-128, 128, size=(A, F, T, 2, 2), dtype=np.int8)
+    w = (rng.normal(size=(B, A, F, 1, 2)) + 1j * rng.normal(size=(B, A, F, 1, 2))).astype(np.complex64)
+    ref = O.beamformer_ata(x8, w, inc, False)
+    ref = O.polarizer(ref) if polarize else ref
+    x = torch.from_numpy(x8).cuda() if kind != "cf32" else torch.from_numpy(O.ci8_to_complex(x8).astype(np.complex64)).cuda()
+    y = ops.beamform_chain(x, torch.from_numpy(w).cuda(), inc, False, 1, polarize,
+                           "f16x2" if kind == "ci8-f16x2" else "f32").cpu().numpy()
+    assert O.norm_rel_err(y[:B], ref[:B]) <= 2 * (2 * A + 4) * 2.0 ** -24
+    if inc:
+        assert O.norm_rel_err(y[B], ref[B]) <= 2 * (2 * A + 4) * 2.0 ** -24

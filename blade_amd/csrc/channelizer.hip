@@ -507,30 +507,28 @@ __device__ __forceinline__ void fft16_mid(float2* __restrict__ p0, float2* __res
     float2 tb[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) tb[e] = twl[e * NS + (tl & (NS - 1))];
+    // One polarization's results are written while the other is computed.
     float2 a[16], b[16];
     const int rd = lpad(tl);
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        a[r] = p0[rd + r * (STRIDE + STRIDE / 16)];
-        b[r] = p1[rd + r * (STRIDE + STRIDE / 16)];
-    }
+    for (int r = 0; r < 16; r++) a[r] = p0[rd + r * (STRIDE + STRIDE / 16)];
+#pragma unroll
+    for (int r = 0; r < 16; r++) b[r] = p1[rd + r * (STRIDE + STRIDE / 16)];
     float2 w[16];
     twiddle_powers<16>(tb, w);
 #pragma unroll
-    for (int r = 1; r < 16; r++) {
-        a[r] = cmul(a[r], w[r]);
-        b[r] = cmul(b[r], w[r]);
-    }
+    for (int r = 1; r < 16; r++) a[r] = cmul(a[r], w[r]);
     dft16(a);
-    dft16(b);
-    __syncthreads();
+    __syncthreads();                       // both planes have been read
     const int jm = tl & (NS - 1);
     const int wr = lpad((tl - jm) * 16 + jm);
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        p0[wr + r * (NS + NS / 16)] = a[r];
-        p1[wr + r * (NS + NS / 16)] = b[r];
-    }
+    for (int r = 0; r < 16; r++) p0[wr + r * (NS + NS / 16)] = a[r];
+#pragma unroll
+    for (int r = 1; r < 16; r++) b[r] = cmul(b[r], w[r]);
+    dft16(b);
+#pragma unroll
+    for (int r = 0; r < 16; r++) p1[wr + r * (NS + NS / 16)] = b[r];
     __syncthreads();
 }
 
@@ -726,14 +724,13 @@ __global__ __launch_bounds__(NT, 2) void fft16_kernel(const float4* __restrict__
                     a[r] = make_float2(q[r].x, q[r].y);
                     b[r] = make_float2(q[r].z, q[r].w);
                 }
-                dft16(a);
-                dft16(b);
                 const int wr = tl * 17;
+                dft16(a);
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    p0[wr + r] = a[r];
-                    p1[wr + r] = b[r];
-                }
+                for (int r = 0; r < 16; r++) p0[wr + r] = a[r];
+                dft16(b);
+#pragma unroll
+                for (int r = 0; r < 16; r++) p1[wr + r] = b[r];
                 // Next spectrum into the registers just consumed (a fresh set
                 // would be copied back at the loop latch behind a full wait).
                 // After the last spectrum this re-reads spectrum 0 (an L2 hit)

@@ -56,7 +56,7 @@ class Beamform(torch.autograd.Function):
 class StokesIPower(torch.autograd.Function):
     """``L = -sum_b beam_weights[b] sum_{f,t,p} |y_b|^2`` (FP64 scalar).
 
-    ``precision``: "f32" or "f16x2" (the same kernel, FP32 precision)."""
+    ``precision``: "f32" or "f16x2" (FP16 matrix cores with hi + lo halves)."""
 
     @staticmethod
     def forward(ctx, x, w, beam_weights, precision="f32"):
@@ -196,7 +196,7 @@ def calibrate(x: torch.Tensor, w: torch.Tensor, steps: int = 200, lr: float = 0.
     stay on the device until the end (one read).  With ``graph`` the step
     (steering, fused loss and gradient, chain rule, Adam) is captured once in
     a CUDA graph after a few eager steps on the same stream and replayed.
-    ``precision``: "f32" or "f16x2" (the same loss + gradient kernel).
+    ``precision`` selects the loss + gradient kernel ("f32" or "f16x2").
     With ``fused_adam`` every step is the library's kernels, the Adam updates
     included (``blade_gain_adam``, ``blade_delay_adam``); otherwise
     torch.optim.Adam (capturable) after autograd.

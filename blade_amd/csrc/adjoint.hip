@@ -8,9 +8,16 @@
 // Per (f, p) this is a (B x T)(T x A) product.
 //
 // Fused Stokes-I mode (stokes_grad_kernel): L = -sum_b lambda_b
-// sum_{f,t,p} |y_b|^2, so gy = -lambda_b y_b.  Each wave recomputes y of 64
-// times from the CI8 voltages it holds in registers and runs the adjoint on
-// the same voltages: neither beams nor gy pass through memory.
+// sum_{f,t,p} |y_b|^2, so gy = -lambda_b y_b, which the kernel recomputes from
+// the CI8 voltages, read from memory once.  Both contractions run transposed:
+//     y^T[t][(b,c)]  = sum_a x^T[t][a] . w^T[a][(b,c)]
+//     gw^T[a][(b,c)] = sum_(t,c') x[a][t] . G[(t,c')][(b,c)],
+// so the forward accumulator a lane holds (times 4g..4g+3 of column i) is
+// exactly the adjoint's B operand for K = those four times: gy never passes
+// through LDS.  G's second component block (c' = imaginary part of x) is the
+// neighbouring column's value, one lane swap away.  With at most 4 beams the
+// FP32 form runs stokes_grad_b4_kernel instead, on 4x4-block matrix
+// instructions whose columns are exactly the beams.
 //
 // Plain adjoint (adjoint_kernel): gy from memory.
 //
@@ -29,19 +36,18 @@ constexpr int ADJ_TC = 128;        // adjoint_kernel: time samples per step of a
 constexpr int ADJ_WAVES = 4;
 constexpr int ADJ_MAXAT = 8;       // antenna tiles of 16: A <= 128
 constexpr int ADJ_MAXB = 64;       // beams of the fused loss
-constexpr int SG_TC = 64;          // stokes_grad_kernel: time samples per tile of a wave
-// Words per LDS voltage row of stokes_grad_kernel: 64 times and 4 of padding,
-// which puts the 16 rows a read touches on different banks.
-constexpr int SG_XS = SG_TC + 4;
+constexpr int SG_BATCH = 8;        // stokes_grad_kernel: phasor loads in flight per thread
+constexpr int SG_TC = 64;          // stokes_grad_kernel: time samples per tile, 16 per wave
+constexpr int SG_XPAD = 4;         // its LDS voltage row stride is apad + 4 words (see sg_xs)
 
 struct AdjArgs {
     const uint32_t* x;       // [A,F,T] dwords: CI8 (re0, im0, re1, im1)
     const float2* w;         // [B,A,F,1,P] phasors (fused mode)
     const float2* gy;        // [B,F,T,P] upstream gradient (adjoint mode)
     float* partial;          // [nsplit][F][P][btiles][16][apad]
-    double* loss_part;       // [nsplit][F][btiles]
+    float* loss_part;        // [nsplit][F][btiles]
     int A, F, T, B;
-    int apad, n_at;          // padded antennas, antenna tiles
+    int apad, n_at, nsteps;  // padded antennas, antenna tiles, forward K steps
     int tsplit;              // time samples per workgroup (a multiple of ADJ_TC or SG_TC)
     int btiles;
     float lambda[ADJ_MAXB];  // beam weights of the fused loss
@@ -50,6 +56,14 @@ struct AdjArgs {
 // The value of lane l ^ 1 (DPP quad permutation [1, 0, 3, 2]).
 __device__ __forceinline__ float swap_pairs(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));
+}
+
+__device__ __forceinline__ floatx4 adj_mfma(float a, float b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ float ci8_component(uint32_t d, int idx) {
+    return (float)(int8_t)((d >> (8 * idx)) & 0xFFu);
 }
 
 // Eight consecutive times of byte k of a voltage dword as a BF16 operand.
@@ -212,224 +226,651 @@ __global__ __launch_bounds__(256, (NAT <= 3 ? 3 : NAT <= 5 ? 2 : 1)) void adjoin
     adj_store_partials<NAT>(a, acc, reinterpret_cast<float*>(lds_raw), sp, f, bt);
 }
 
-// Fused Stokes-I loss and phasor gradient of A <= 16 NAT antennas and 8 beams,
-// for either precision (the FP16 split has nothing to gain on it).  A wave
-// takes tiles of 64 times, without barriers:
-//   * voltages: lane (g, i) loads times 4i .. 4i + 3 of antennas 4g .. 4g + 3
-//     of every group of 16 in 16-byte pieces, one tile ahead;
-//   * forward: rows = times (4i + n of four instructions n), K = 16 antennas x
-//     (re, im), columns = (beam, re/im); the phasors are three exact BF16
-//     parts in LDS;
-//   * a lane then holds y of 16 consecutive times of its column, which is, cut
-//     into three BF16 parts, the B operand of the adjoint as it stands:
-//     real products as in adjoint_kernel, K = 32 times;
-//   * the adjoint's A operand (rows = antennas, 8 consecutive times) is the
-//     same voltages turned through 4 KiB of LDS per wave, 16 antennas at a time.
-// Products are exact and accumulate in FP32.  Bound by VALU work (widening the
-// voltages twice, cutting gy) and load latency at 2 waves per SIMD (216 VGPRs
-// at A = 42; 3 waves spill).  A42 F384 T2048 B4 per call: 53 us, where FP32
-// 4x4 and 16x16 matrix instructions took 97 us (B = 4) and 129 us (B = 8), and
-// split FP16 through barriered LDS tiles 69 us; error against FP64 5e-8
-// (FP32 1.1e-7).  VEC: 16-byte loads (T a multiple of 4, aligned voltages).
-template <int NAT, bool VEC>
-__global__ __launch_bounds__(256, (NAT <= 2 ? 3 : NAT <= 4 ? 2 : 1)) void stokes_grad_kernel(AdjArgs a) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    uint4* const s_w = reinterpret_cast<uint4*>(lds_raw);                 // [unit][p][part][64]
-    __shared__ double s_loss[ADJ_WAVES];
+// LDS row stride (words) of stokes_grad_kernel's voltage tile s_x[t][antenna]:
+// apad + 4 puts both read patterns on distinct banks, the forward's (16 lanes
+// read 16 consecutive times of one antenna; lane groups take adjacent
+// antennas) and the adjoint's (16 lanes read 16 consecutive antennas at one
+// time; lane groups take times 4 apart).
+__host__ __device__ constexpr int sg_xs(int apad) { return apad + SG_XPAD; }
 
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+// Fused Stokes-I loss and phasor gradient for A <= 16 NAT antennas.  Each
+// wave takes 16 time rows of every SG_TC-sample tile; the next tile's
+// voltages are loaded into registers while this one is computed and written
+// to the other half of a double-buffered LDS stage: one barrier per tile.
+template <int NAT>
+__global__ __launch_bounds__(256, (NAT <= 4 ? 4 : 2)) void stokes_grad_kernel(AdjArgs a) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int APAD = 16 * NAT;
+    constexpr int XS = sg_xs(APAD);
+    constexpr int PER = SG_TC * APAD / (64 * ADJ_WAVES);     // staged dwords per thread
+    uint32_t* s_x = reinterpret_cast<uint32_t*>(lds_raw);     // [2][SG_TC][XS]
+    float* s_w = reinterpret_cast<float*>(s_x + 2 * SG_TC * XS);   // [2][nsteps][64]
+    __shared__ float s_loss[ADJ_WAVES];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
     const int i = lane & 15;
     const int g = lane >> 4;
     const int sp = blockIdx.x;
     const int f = blockIdx.y;
     const int bt = blockIdx.z;
+    const int b0 = bt * 8;
     const int A = a.A, F = a.F, T = a.T, B = a.B;
+    const int nsteps = a.nsteps;
+    const int n_ag = nsteps / 2;                              // antenna groups of 4
     const int t_begin = sp * a.tsplit;
     const int t_end = min(T, t_begin + a.tsplit);
-    uint32_t* const s_x = reinterpret_cast<uint32_t*>(s_w + NAT * 6 * 64) + wave * 16 * SG_XS;   // this wave's rows
+    const int ntiles = (t_end - t_begin + SG_TC - 1) / SG_TC;
 
-    // Voltages of unit u (antennas 16u + 4g + q, times t0 + 4i .. + 3); rows
-    // past A repeat the last antenna (their phasors are zero, their sums not
-    // stored), times past the split its end (their gy is zeroed).
-    uint4 xd[NAT][4];
-    const uint32_t* const xf = a.x + (size_t)f * T;
-    auto load_unit = [&](int t0, int u) {
-        // Opaque stride: keeps the 4 NAT row addresses from being held in
-        // registers across tiles.
-        size_t st = (size_t)F * T;
-        asm volatile("" : "+s"(st));
+    // Voltage staging: thread (wave, lane) takes antennas wave + 4k at time
+    // lane of the tile (one coalesced 256-byte row per wave and k).
+    uint32_t pre[PER];
+    bool pre_t_ok = true;
+    // Unconditional loads from clamped addresses (no branch per antenna row);
+    // padded antennas and samples past the split are zeroed when the tile is
+    // written to LDS, so the loads stay in flight until then.
+    auto load_tile = [&](int t0) {
+        const int tt = t0 + lane;
+        pre_t_ok = tt < t_end;
+        const int ttc = min(tt, t_end - 1);
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t* const xp = xf + min(16 * u + 4 * g + q, A - 1) * st;
-            const int t = t0 + 4 * i;
-            if constexpr (VEC)
-                xd[u][q] = *reinterpret_cast<const uint4*>(xp + min(t, t_end - 4));
-            else
-                xd[u][q] = make_uint4(xp[min(t, t_end - 1)], xp[min(t + 1, t_end - 1)], xp[min(t + 2, t_end - 1)],
-                                      xp[min(t + 3, t_end - 1)]);
+        for (int k = 0; k < PER; k++)
+            pre[k] = a.x[((size_t)min(wave + ADJ_WAVES * k, A - 1) * F + f) * T + ttc];
+    };
+    auto store_tile = [&](uint32_t* dst) {
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int an = wave + ADJ_WAVES * k;
+            dst[lane * XS + an] = (pre_t_ok && an < A) ? pre[k] : 0u;
         }
     };
-    int t0 = t_begin + wave * SG_TC;
-    if (t0 < t_end) {
-#pragma unroll
-        for (int u = 0; u < NAT; u++) load_unit(t0, u);
-    }
+    load_tile(t_begin);
 
-    // Forward B operand: lane (g, column) of unit u holds k = 8g + 2q + c ->
-    // (antenna 16u + 4g + q, component c of x), column -> (beam, re/im):
-    // y_r = x_r w_r - x_i w_i, y_i = x_r w_i + x_i w_r.
-    for (int e = threadIdx.x; e < NAT * 64; e += 64 * ADJ_WAVES) {
-        const int ln = e & 63, u = e >> 6;
-        const int col = ln & 15, lg = ln >> 4;
-        const int b = bt * 8 + (col >> 1);
-        const bool im = col & 1;
-        float4 w[4];
+    // Forward B operand of beams b0..b0+7, both pols: [p][step][g][col],
+    // step = 2 * antenna group + component of x, col = (beam, re/im).
+    {
+        const int n_w = 2 * nsteps * 64;
+        for (int e0 = tid; e0 < n_w; e0 += SG_BATCH * ADJ_WAVES * 64) {
+            float2 wv[SG_BATCH];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int an = 16 * u + 4 * lg + q;
-            w[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (b < B && an < A) w[q] = reinterpret_cast<const float4*>(a.w)[((size_t)b * A + an) * F + f];
-        }
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            uint32_t h[3][4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float wr = p ? w[q].z : w[q].x, wi = p ? w[q].w : w[q].y;
-                float v0[3], v1[3];
-                split_bf16x3(im ? wi : wr, v0);
-                split_bf16x3(im ? wr : -wi, v1);
-#pragma unroll
-                for (int k = 0; k < 3; k++) h[k][q] = bf16_pair(v0[k], v1[k]);
+            for (int k = 0; k < SG_BATCH; k++) {
+                const int e = e0 + k * ADJ_WAVES * 64;
+                const int p = e / (nsteps * 64);
+                const int r = e - p * nsteps * 64;
+                const int st = r >> 6, kg = (r >> 4) & 3, col = r & 15;
+                const int an = (st >> 1) * 4 + kg, b = b0 + (col >> 1);
+                wv[k] = (e < n_w && b < B && an < A) ? a.w[(((size_t)b * A + an) * F + f) * 2 + p]
+                                                      : make_float2(0.f, 0.f);
             }
 #pragma unroll
-            for (int k = 0; k < 3; k++)
-                s_w[((u * 2 + p) * 3 + k) * 64 + ln] = make_uint4(h[k][0], h[k][1], h[k][2], h[k][3]);
+            for (int k = 0; k < SG_BATCH; k++) {
+                const int e = e0 + k * ADJ_WAVES * 64;
+                if (e < n_w) {
+                    const int r = e % (nsteps * 64);
+                    const int c = (r >> 6) & 1, co = r & 1;
+                    const float2 w = wv[k];
+                    // y_r = x_r w_r - x_i w_i, y_i = x_r w_i + x_i w_r
+                    s_w[e] = (co == 0) ? (c == 0 ? w.x : -w.y) : (c == 0 ? w.y : w.x);
+                }
+            }
         }
     }
+    store_tile(s_x);
+    if (ntiles > 1) load_tile(t_begin + SG_TC);
     __syncthreads();
 
-    const int bcol = bt * 8 + (i >> 1);
+    const int bcol = b0 + (i >> 1);
     const float lam = bcol < B ? a.lambda[bcol] : 0.f;
-    const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    floatx4 acc[2][NAT][2];
+    const float swap_sign = (i & 1) ? -1.f : 1.f;
+    floatx4 acc2[2][NAT];
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int at = 0; at < NAT; at++) acc2[p][at] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float loss = 0.f;
+
+    for (int k = 0; k < ntiles; k++) {
+        const uint32_t* sx = s_x + (k & 1) * SG_TC * XS;
+        const int trow = wave * 16;
+        // Forward: y^T rows = this wave's 16 times, both pols from one dword.
+        floatx4 y[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int ag = 0; ag < 4 * NAT; ag++) {
+            if (ag < n_ag) {                       // uniform
+                const uint32_t d = sx[(trow + i) * XS + ag * 4 + g];
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    const float w0 = s_w[(p * nsteps + 2 * ag) * 64 + lane];
+                    const float w1 = s_w[(p * nsteps + 2 * ag + 1) * 64 + lane];
+                    y[p] = adj_mfma(ci8_component(d, 2 * p), w0, y[p]);
+                    y[p] = adj_mfma(ci8_component(d, 2 * p + 1), w1, y[p]);
+                }
+            }
+        }
+        // Lane (g, i), register r: y at time trow + 4g + r, column i.  Its
+        // gradient is gy = -lambda y; the imaginary-x block of G takes the
+        // neighbouring column (re <-> im) with the sign of conj(x).
+        float gyo[2][4], gys[2][4];
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float v = y[p][r];
+                loss += lam * v * v;
+                gyo[p][r] = -lam * v;
+                gys[p][r] = swap_sign * swap_pairs(gyo[p][r]);
+            }
+        // Adjoint: K = times trow + 4g + r (g = k index), both x components.
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const uint32_t* row = sx + (trow + 4 * g + r) * XS + i;
+#pragma unroll
+            for (int at = 0; at < NAT; at++) {
+                const uint32_t d = row[at * 16];
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    acc2[p][at] = adj_mfma(ci8_component(d, 2 * p), gyo[p][r], acc2[p][at]);
+                    acc2[p][at] = adj_mfma(ci8_component(d, 2 * p + 1), gys[p][r], acc2[p][at]);
+                }
+            }
+        }
+        if (k + 1 < ntiles) {
+            // Tile k + 1 into the other buffer (last read in iteration k - 1,
+            // before the barrier that ended it), then tile k + 2's loads.
+            store_tile(s_x + ((k + 1) & 1) * SG_TC * XS);
+            if (k + 2 < ntiles) load_tile(t_begin + (k + 2) * SG_TC);
+        }
+        __syncthreads();
+    }
+
+    // Partials of the four waves into LDS (the voltage stage is free now),
+    // [wave][p][col][antenna], then summed in wave order.
+    float* s_part = reinterpret_cast<float*>(lds_raw);
 #pragma unroll
     for (int p = 0; p < 2; p++)
 #pragma unroll
         for (int at = 0; at < NAT; at++)
 #pragma unroll
-            for (int c = 0; c < 2; c++) acc[p][at][c] = zero4;
-    double loss = 0.0;      // FP64 past the 32 squares of a lane's tile
+            for (int r = 0; r < 4; r++)
+                s_part[((wave * 2 + p) * 16 + i) * APAD + at * 16 + 4 * g + r] = acc2[p][at][r];
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
+    if (lane == 0) s_loss[wave] = loss;
+    __syncthreads();
+    constexpr int NPART = 2 * 16 * APAD;
+    float* out = a.partial + ((((size_t)sp * F + f) * 2) * a.btiles + bt) * 16 * APAD;
+    const size_t pstride = (size_t)a.btiles * 16 * APAD;   // between pols
+    for (int e = tid; e < NPART; e += blockDim.x) {
+        const float v = ((s_part[e] + s_part[NPART + e]) + s_part[2 * NPART + e]) + s_part[3 * NPART + e];
+        const int p = e / (16 * APAD), r = e - p * 16 * APAD;
+        out[p * pstride + r] = v;
+    }
+    if (tid == 0)
+        a.loss_part[((size_t)sp * F + f) * a.btiles + bt] = ((s_loss[0] + s_loss[1]) + s_loss[2]) + s_loss[3];
+}
 
-    for (; t0 < t_end; t0 += ADJ_WAVES * SG_TC) {
-        // ---- forward: y[p][n], register r of lane (g, column): time
-        // t0 + 16g + 4r + n.
-        floatx4 y[2][4];
+// ---------------------------------------------------------------------------
+// Stokes-I loss and gradient for at most 4 beams (FP32), on
+// v_mfma_f32_4x4x1_16b_f32: 16 independent 4x4 blocks with K = 1.  Lane
+// 4 blk + c holds row c of block blk's A operand, column c of its B operand,
+// and column c of its result (register r = row r).  With 4 beams the columns
+// are exactly the beams, so no matrix work goes to absent beams (the 16x16
+// tiles of stokes_grad_kernel are half empty there).  Complex products take
+// three real products (P3 - P1 - P2 form).
+//   Forward, blocks = groups of 4 times, K = one antenna per instruction:
+//     lane (blk, c) feeds x[a][t0 + 4 blk + c] and w[a][beam c]; register r
+//     of the result is y at time t0 + 4 blk + r, beam c.
+//   Adjoint, blocks = groups of 4 antennas, K = one time per instruction:
+//     lane (blk, c) feeds conj(x)[4 blk + c][t] and gy[beam c][t]; register r
+//     is gw of antenna 4 blk + r, beam c.  gy passes through a per-wave LDS
+//     tile [p][product][beam][time], read as broadcasts (all blocks read the
+//     same four addresses).
+// Each wave takes 64-time tiles; partial sums are added across waves in LDS
+// in wave order and across time splits by adjoint_reduce_kernel, whose
+// partial layout this kernel writes (rows 2 b and 2 b + 1, beam tile 0).
+// Needs A <= 64, T % 4 == 0, A F T < 2^31 and 16-byte aligned voltages.
+// ---------------------------------------------------------------------------
+constexpr int SG4_TC = 64;            // times per wave tile
+constexpr int SG4_WS = 8;             // LDS floats per (antenna, beam): (wr, wi, wr + wi) per pol, padded
+// gy tile rows ([p][product][beam], SG4_TC times each) are padded by 4
+// floats, so the four beams' rows that a read instruction broadcasts start
+// on different LDS banks (unpadded, their 256-byte stride put all four on the
+// same banks: 7 conflict cycles per LDS instruction).
+constexpr int SG4_GS = SG4_TC + 4;
+constexpr int SG4_GY = 2 * 3 * 4 * SG4_GS;   // floats of one wave's gy tile
+constexpr int SG4_WGS = 3;            // resident workgroups per CU (launch bounds)
+
+__device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+}
+
+template <int NAT>
+__global__ __launch_bounds__(256, SG4_WGS) void stokes_grad_b4_kernel(AdjArgs a) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int AMAX = 16 * NAT;
+    float* const s_w = reinterpret_cast<float*>(lds_raw);            // [A][4][SG4_WS]
+    float* const s_gy = s_w + (size_t)a.A * 4 * SG4_WS;               // [wave][SG4_GY]
+    __shared__ float s_loss[ADJ_WAVES];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int blk = lane >> 2;
+    const int c = lane & 3;
+    const int sp = blockIdx.x;
+    const int f = blockIdx.y;
+    const int A = a.A, F = a.F, T = a.T, B = a.B;
+    const int t_begin = sp * a.tsplit;
+    const int t_end = min(T, t_begin + a.tsplit);
+    const int ntiles = (t_end - t_begin + SG4_TC - 1) / SG4_TC;
+    const unsigned ant_stride = (unsigned)F * (unsigned)T;   // A F T < 2^31 (host check)
+
+    // Phasors of (antenna, beam): wr, wi, wr + wi of pol 0, then of pol 1.
+    for (int e = tid; e < A * 4; e += blockDim.x) {
+        const int an = e >> 2, b = e & 3;
+        float v[6];
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const float2 w = b < B ? a.w[(((size_t)b * A + an) * F + f) * 2 + p] : make_float2(0.f, 0.f);
+            v[3 * p] = w.x;
+            v[3 * p + 1] = w.y;
+            v[3 * p + 2] = w.x + w.y;
+        }
+        float4* dst = reinterpret_cast<float4*>(s_w + (size_t)e * SG4_WS);
+        dst[0] = make_float4(v[0], v[1], v[2], v[3]);
+        dst[1] = make_float4(v[4], v[5], 0.f, 0.f);
+    }
+    __syncthreads();
+
+    const float lam = c < B ? a.lambda[c] : 0.f;
+    // Adjoint sums per pol: Q1 = sum gr xr, Q2 = sum gi xi, Q3 = sum (gr + gi)(xr - xi);
+    // gw = (Q1 + Q2) + j (Q3 - Q1 + Q2).
+    floatx4 q[2][3];
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) q[p][k] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float loss = 0.f;
+    float* const gyw = s_gy + wave * SG4_GY;
+    // This lane's adjoint antenna row (clamped: rows past A are never stored).
+    const uint4* const xa = reinterpret_cast<const uint4*>(a.x + min(4 * blk + c, A - 1) * ant_stride + f * T);
+
+    // Forward voltages of tile kk at this lane's time, antennas 8 g .. 8 g + 7
+    // (group g + 1 is in flight while group g is computed: 3% faster than
+    // all antennas at once, with 136 instead of 168 VGPRs).  The stride and
+    // count are opaque to the compiler, which would otherwise keep one
+    // offset and one guard mask per antenna in scalar registers across tiles
+    // (and spill them).
+    uint32_t xd[2][8];
+    auto load_fwd = [&](int kk, int g, uint32_t (&dst)[8]) {
+        const int tl = t_begin + kk * SG4_TC + 4 * blk + c;
+        const uint32_t* const xf = a.x + (f * T + min(tl, t_end - 1));
+        unsigned st = ant_stride;
+        int na = A;
+        asm volatile("" : "+s"(st), "+s"(na));
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (8 * g + j < na) dst[j] = xf[(8 * g + j) * st];     // uniform
+    };
+    // Adjoint voltages of 16 times from t: this lane's antenna row (times
+    // past tn re-read the last 4 in bounds; their gy is not used).
+    auto load_adj = [&](int t0, int tn, int t, uint4 (&xv)[4]) {
+#pragma unroll
+        for (int s4 = 0; s4 < 4; s4++) xv[s4] = xa[(t0 + min(t + 4 * s4, tn - 4)) >> 2];
+    };
+
+    for (int k = wave; k < ntiles; k += ADJ_WAVES) {
+        const int t0 = t_begin + k * SG4_TC;
+        const int tn = min(SG4_TC, t_end - t0);            // a multiple of 4
+        uint4 xv[2][4];
+        load_adj(t0, tn, 0, xv[0]);                        // in flight during the forward
+        load_fwd(k, 0, xd[0]);
+        // ---- forward: this lane feeds time t0 + 4 blk + c (clamped to the
+        // split; results for times past it are zeroed below).  The antenna
+        // count is opaque here too: 48 hoisted guard masks would not fit in
+        // scalar registers.
+        int na = A;
+        asm volatile("" : "+s"(na));
+        floatx4 y[2][3];
 #pragma unroll
         for (int p = 0; p < 2; p++)
 #pragma unroll
-            for (int n = 0; n < 4; n++) y[p][n] = zero4;
+            for (int m = 0; m < 3; m++) y[p][m] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int u = 0; u < NAT; u++)
+        for (int an = 0; an < AMAX; an++) {
+            if (an % 8 == 0 && an + 8 < AMAX) load_fwd(k, an / 8 + 1, xd[(an / 8 + 1) & 1]);
+            if (an < na) {                                        // uniform
+                const uint32_t d = xd[(an / 8) & 1][an % 8];
+                const float* wv = s_w + (an * 4 + c) * SG4_WS;
+                const float4 w0 = *reinterpret_cast<const float4*>(wv);
+                const float2 w1 = *reinterpret_cast<const float2*>(wv + 4);
+                const float wp[2][3] = {{w0.x, w0.y, w0.z}, {w0.w, w1.x, w1.y}};
 #pragma unroll
-            for (int p = 0; p < 2; p++) {
-                uint4 xo[4];
-#pragma unroll
-                for (int n = 0; n < 4; n++) {
-                    auto dw = [&](int q) { return n == 0 ? xd[u][q].x : n == 1 ? xd[u][q].y : n == 2 ? xd[u][q].z : xd[u][q].w; };
-                    xo[n] = make_uint4(ci8_to_bf16(dw(0), p), ci8_to_bf16(dw(1), p), ci8_to_bf16(dw(2), p),
-                                       ci8_to_bf16(dw(3), p));
+                for (int p = 0; p < 2; p++) {
+                    const float xr = ci8_component(d, 2 * p), xi = ci8_component(d, 2 * p + 1);
+                    y[p][0] = mfma4(xr, wp[p][0], y[p][0]);
+                    y[p][1] = mfma4(xi, wp[p][1], y[p][1]);
+                    y[p][2] = mfma4(xr + xi, wp[p][2], y[p][2]);
                 }
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    const uint4 wk = s_w[((u * 2 + p) * 3 + k) * 64 + lane];
-#pragma unroll
-                    for (int n = 0; n < 4; n++) y[p][n] = mfma_bf16(xo[n], wk, y[p][n]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
             }
-        // ---- loss and gy = -lambda y in three parts; the 8 times
-        // 16g + 8h + (0 .. 7) are one K = 32 operand.
-        if (t0 + SG_TC > t_end) {              // uniform: the split's last tile
-#pragma unroll
-            for (int p = 0; p < 2; p++)
-#pragma unroll
-                for (int n = 0; n < 4; n++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (t0 + 16 * g + 4 * r + n >= t_end) y[p][n][r] = 0.f;
         }
-        float tl = 0.f;
+        // ---- gy = -lambda y at (time t0 + 4 blk + r, beam c): gr, gi, gr + gi
+        // into this wave's LDS tile [p][product][beam][time].  Times past the
+        // split read clamped voltages: their y, and so gy and the loss, are
+        // set to 0.
 #pragma unroll
-        for (int n = 0; n < 4; n++) {
-            float e = 0.f;
+        for (int p = 0; p < 2; p++) {
+            float g[3][4];
 #pragma unroll
-            for (int p = 0; p < 2; p++)
+            for (int r = 0; r < 4; r++) {
+                const bool ok = 4 * blk + r < tn;
+                const float yr = ok ? y[p][0][r] - y[p][1][r] : 0.f;
+                const float yi = ok ? (y[p][2][r] - y[p][0][r]) - y[p][1][r] : 0.f;
+                loss += lam * (yr * yr + yi * yi);
+                const float gr = -lam * yr, gi = -lam * yi;
+                g[0][r] = gr;
+                g[1][r] = gi;
+                g[2][r] = gr + gi;
+            }
 #pragma unroll
-                for (int r = 0; r < 4; r++) e += y[p][n][r] * y[p][n][r];
-            tl += e;
+            for (int m = 0; m < 3; m++)
+                *reinterpret_cast<float4*>(gyw + ((p * 3 + m) * 4 + c) * SG4_GS + 4 * blk) =
+                    make_float4(g[m][0], g[m][1], g[m][2], g[m][3]);
         }
-        loss += (double)lam * (double)tl;
-        // Infinities and NaN (they show in tl) take the split that keeps them.
-        const bool plain = __all(fabsf(tl) <= 3.0e38f);
-        // ---- adjoint, half of the times at a time (half the operands of gy
-        // live): per antenna tile, the unit's rows turned through this wave's
-        // LDS rows (LDS operations of a wave complete in order); after the
-        // second half the next tile's loads go into the registers just read.
-        const bool more = t0 + ADJ_WAVES * SG_TC < t_end;
+        // ---- adjoint: this lane feeds antenna 4 blk + c and gy of beam c;
+        // one instruction per (time, pol, product).  The wave reads back its
+        // own LDS writes (LDS operations of a wave complete in order).  The
+        // next 16 times' voltages load while these are computed.
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            uint4 gb[2][3];
-            auto parts = [&](auto checked) {
+        for (int h = 0; h < SG4_TC / 16; h++) {
+            if (h + 1 < SG4_TC / 16) load_adj(t0, tn, 16 * (h + 1), xv[(h + 1) & 1]);
+            if (16 * h < tn) {                                    // uniform
 #pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    uint32_t w[3][4];
+                for (int s4 = 0; s4 < 4; s4++) {
+                    const int tt = 16 * h + 4 * s4;
+                    if (tt < tn) {                                // uniform
+                        float4 gv[2][3];
 #pragma unroll
-                    for (int m = 0; m < 4; m++) {
-                        const int r = 2 * h + (m >> 1), n = 2 * (m & 1);
-                        float u0[3], u1[3];
-                        split_bf16x3<decltype(checked)::value>(-lam * y[p][n][r], u0);
-                        split_bf16x3<decltype(checked)::value>(-lam * y[p][n + 1][r], u1);
+                        for (int p = 0; p < 2; p++)
 #pragma unroll
-                        for (int k = 0; k < 3; k++) w[k][m] = bf16_pair(u0[k], u1[k]);
+                            for (int m = 0; m < 3; m++)
+                                gv[p][m] = *reinterpret_cast<const float4*>(gyw + ((p * 3 + m) * 4 + c) * SG4_GS + tt);
+                        const uint4 xq = xv[h & 1][s4];
+                        const uint32_t dw[4] = {xq.x, xq.y, xq.z, xq.w};
+#pragma unroll
+                        for (int s = 0; s < 4; s++) {
+#pragma unroll
+                            for (int p = 0; p < 2; p++) {
+                                const float xr = ci8_component(dw[s], 2 * p), xi = ci8_component(dw[s], 2 * p + 1);
+                                q[p][0] = mfma4(xr, gv[p][0][s], q[p][0]);
+                                q[p][1] = mfma4(xi, gv[p][1][s], q[p][1]);
+                                q[p][2] = mfma4(xr - xi, gv[p][2][s], q[p][2]);
+                            }
+                        }
                     }
-#pragma unroll
-                    for (int k = 0; k < 3; k++) gb[p][k] = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
                 }
-            };
-            if (plain)
-                parts(std::false_type{});
-            else
-                parts(std::true_type{});
-#pragma unroll
-            for (int at = 0; at < NAT; at++) {
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    *reinterpret_cast<uint4*>(s_x + (4 * g + q) * SG_XS + 4 * i) = xd[at][q];
-                if (h == 1 && more) load_unit(t0 + ADJ_WAVES * SG_TC, at);
-                const uint32_t* const row = s_x + i * SG_XS + 16 * g + 8 * h;
-                const uint4 lo = *reinterpret_cast<const uint4*>(row), hi = *reinterpret_cast<const uint4*>(row + 4);
-#pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    uint4 xo[2];
-#pragma unroll
-                    for (int c = 0; c < 2; c++) xo[c] = ci8_times_bf16(lo, hi, 2 * p + c);
-#pragma unroll
-                    for (int k = 0; k < 3; k++)
-#pragma unroll
-                        for (int c = 0; c < 2; c++) acc[p][at][c] = mfma_bf16(xo[c], gb[p][k], acc[p][at][c]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
 
+    // This wave's sums into its own gy tile (its last reads of it are done):
+    // [p][row = 2 beam + re/im][antenna 64], then summed over waves in order.
+    float* const pw = gyw;
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int an = 4 * blk + r;
+            pw[(p * 8 + 2 * c) * 64 + an] = q[p][0][r] + q[p][1][r];
+            pw[(p * 8 + 2 * c + 1) * 64 + an] = (q[p][2][r] - q[p][0][r]) + q[p][1][r];
+        }
     for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
     if (lane == 0) s_loss[wave] = loss;
-    __syncthreads();                          // every wave is done with the LDS operands
-    adj_store_partials<NAT>(a, acc, reinterpret_cast<float*>(lds_raw), sp, f, bt);
-    if (threadIdx.x == 0)
+    __syncthreads();
+    const int apad = a.apad;
+    float* out = a.partial + ((size_t)sp * F + f) * 2 * a.btiles * 16 * apad;
+    const size_t pstride = (size_t)a.btiles * 16 * apad;   // between pols
+    for (int e = tid; e < 2 * 8 * A; e += blockDim.x) {
+        const int an = e % A, pr = e / A;                   // pr = p * 8 + row
+        const float* src = s_gy + pr * 64 + an;
+        const float v = ((src[0] + src[SG4_GY]) + src[2 * SG4_GY]) + src[3 * SG4_GY];
+        out[(pr >> 3) * pstride + (pr & 7) * apad + an] = v;
+    }
+    if (tid == 0) a.loss_part[((size_t)sp * F + f) * a.btiles] = ((s_loss[0] + s_loss[1]) + s_loss[2]) + s_loss[3];
+}
+
+// Power-of-two scale s with m * s in [0.5, 1) for m > 0 (1 for m = 0), and 1/s.
+__device__ __forceinline__ void pow2_scale(float m, float& s, float& inv) {
+    int ex = 0;
+    frexpf(m, &ex);
+    s = m > 0.f ? ldexpf(1.0f, -ex) : 1.f;
+    inv = m > 0.f ? ldexpf(1.0f, ex) : 1.f;
+}
+
+// v (|v| < 1) as hi + lo FP16 halves, into element j of two vectors.
+__device__ __forceinline__ void split_f16(float v, halfx8& hi, halfx8& lo, int j) {
+    const _Float16 h = (_Float16)v;
+    hi[j] = h;
+    lo[j] = (_Float16)(v - (float)h);
+}
+
+// Split-FP16 form of stokes_grad_kernel: the same transposed contractions and
+// tiles on v_mfma_f32_16x16x32_f16 (K = 32 per instruction), FP32
+// accumulation.  CI8 voltages are exact in FP16.
+//   * Forward B operand: the phasor embedding times a power-of-two scale per
+//     pol (every component below 1), as hi + lo FP16 halves; K = 16
+//     antennas x (re, im) of x per instruction.
+//   * Adjoint B operand: the wave's gy of the tile, K = 16 times x (re, im)
+//     -- exactly the forward outputs the lane holds (times 4g..4g+3 and the
+//     neighbouring column) -- scaled by a power of two from the wave's
+//     largest |gy| and split the same way; each tile's product is unscaled
+//     into the FP32 sums.
+// Error against FP64 is that of FP32 arithmetic (hi + lo carry ~22 bits).
+template <int NAT>
+__global__ __launch_bounds__(256, (NAT <= 3 ? 3 : 2)) void stokes_grad_f16_kernel(AdjArgs a) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int APAD = 16 * NAT;
+    constexpr int XS = sg_xs(APAD);
+    constexpr int PER = SG_TC * APAD / (64 * ADJ_WAVES);
+    uint32_t* s_x = reinterpret_cast<uint32_t*>(lds_raw);                 // [2][SG_TC][XS]
+    halfx8* s_wh = reinterpret_cast<halfx8*>(s_x + 2 * SG_TC * XS);       // [p][blk][hl][64]
+    __shared__ float s_loss[ADJ_WAVES];
+    __shared__ unsigned int s_wmax[2];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int i = lane & 15;
+    const int g = lane >> 4;
+    const int sp = blockIdx.x;
+    const int f = blockIdx.y;
+    const int bt = blockIdx.z;
+    const int b0 = bt * 8;
+    const int A = a.A, F = a.F, T = a.T, B = a.B;
+    const int t_begin = sp * a.tsplit;
+    const int t_end = min(T, t_begin + a.tsplit);
+    const int ntiles = (t_end - t_begin + SG_TC - 1) / SG_TC;
+
+    uint32_t pre[PER];
+    bool pre_t_ok = true;
+    // Unconditional loads from clamped addresses (no branch per antenna row);
+    // padded antennas and samples past the split are zeroed when the tile is
+    // written to LDS, so the loads stay in flight until then.
+    auto load_tile = [&](int t0) {
+        const int tt = t0 + lane;
+        pre_t_ok = tt < t_end;
+        const int ttc = min(tt, t_end - 1);
+#pragma unroll
+        for (int k = 0; k < PER; k++)
+            pre[k] = a.x[((size_t)min(wave + ADJ_WAVES * k, A - 1) * F + f) * T + ttc];
+    };
+    auto store_tile = [&](uint32_t* dst) {
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int an = wave + ADJ_WAVES * k;
+            dst[lane * XS + an] = (pre_t_ok && an < A) ? pre[k] : 0u;
+        }
+    };
+    load_tile(t_begin);
+
+    // Phasor scale per pol: the largest component magnitude of this
+    // workgroup's beams (an exact maximum, so the order of the atomics does
+    // not matter).
+    if (tid < 2) s_wmax[tid] = 0u;
+    __syncthreads();
+    {
+        float mx[2] = {0.f, 0.f};
+        for (int e = tid; e < 2 * 8 * A; e += blockDim.x) {
+            const int p = e / (8 * A), r = e - p * 8 * A;
+            const int bb = r / A, an = r - bb * A, b = b0 + bb;
+            if (b < B) {
+                const float2 w = a.w[(((size_t)b * A + an) * F + f) * 2 + p];
+                mx[p] = fmaxf(mx[p], fmaxf(fabsf(w.x), fabsf(w.y)));
+            }
+        }
+        atomicMax(&s_wmax[0], __float_as_uint(mx[0]));
+        atomicMax(&s_wmax[1], __float_as_uint(mx[1]));
+    }
+    __syncthreads();
+    float wsc[2], wuns[2];
+    pow2_scale(__uint_as_float(s_wmax[0]), wsc[0], wuns[0]);
+    pow2_scale(__uint_as_float(s_wmax[1]), wsc[1], wuns[1]);
+    // Forward B operand: lane (g, i) of block blk holds k = 8g + 2q + c ->
+    // (antenna 16 blk + 4g + q, component c of x), column i -> (beam
+    // b0 + i/2, re/im).  y_r = x_r w_r - x_i w_i, y_i = x_r w_i + x_i w_r.
+    for (int e = tid; e < 2 * NAT * 64; e += blockDim.x) {
+        const int ln = e & 63, pb = e >> 6;
+        const int p = pb / NAT, blk = pb - p * NAT;
+        const int li = ln & 15, lg = ln >> 4;
+        const int b = b0 + (li >> 1), co = li & 1;
+        halfx8 hi, lo;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int an = blk * 16 + 4 * lg + q;
+            float2 w = make_float2(0.f, 0.f);
+            if (b < B && an < A) w = a.w[(((size_t)b * A + an) * F + f) * 2 + p];
+            const float v0 = (co == 0 ? w.x : w.y) * wsc[p];     // multiplies Re x
+            const float v1 = (co == 0 ? -w.y : w.x) * wsc[p];    // multiplies Im x
+            split_f16(v0, hi, lo, 2 * q);
+            split_f16(v1, hi, lo, 2 * q + 1);
+        }
+        s_wh[(pb * 2 + 0) * 64 + ln] = hi;
+        s_wh[(pb * 2 + 1) * 64 + ln] = lo;
+    }
+    store_tile(s_x);
+    if (ntiles > 1) load_tile(t_begin + SG_TC);
+    __syncthreads();
+
+    const int bcol = b0 + (i >> 1);
+    const float lam = bcol < B ? a.lambda[bcol] : 0.f;
+    const float swap_sign = (i & 1) ? -1.f : 1.f;
+    floatx4 acc2[2][NAT];
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int at = 0; at < NAT; at++) acc2[p][at] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float loss = 0.f;
+    const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
+
+    for (int k = 0; k < ntiles; k++) {
+        const uint32_t* sx = s_x + (k & 1) * SG_TC * XS;
+        const int trow = wave * 16;
+        // Forward: rows = this wave's 16 times; one 16-byte LDS read gives
+        // 4 antennas x both pols.  The phasor operands are re-read from LDS
+        // every tile (an opaque offset keeps the compiler from holding all
+        // 4 NAT of them in registers across the loop).
+        int woff = lane;
+        asm volatile("" : "+v"(woff));
+        const halfx8* wh = s_wh + woff;
+        floatx4 y[2] = {zero4, zero4};
+#pragma unroll
+        for (int blk = 0; blk < NAT; blk++) {
+            const uint4 d = *reinterpret_cast<const uint4*>(sx + (trow + i) * XS + blk * 16 + 4 * g);
+            halfx8 xa[2];
+            const uint32_t dw[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                halfx2 h0, h1;
+                ci8_to_half2x2(dw[q], h0, h1);
+                xa[0][2 * q] = h0[0]; xa[0][2 * q + 1] = h0[1];
+                xa[1][2 * q] = h1[0]; xa[1][2 * q + 1] = h1[1];
+            }
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                y[p] = mfma_f16(xa[p], wh[((p * NAT + blk) * 2 + 0) * 64], y[p]);
+                y[p] = mfma_f16(xa[p], wh[((p * NAT + blk) * 2 + 1) * 64], y[p]);
+            }
+        }
+        // gy = -lambda y (unscaled), its wave maximum, and the B operands.
+        halfx8 gh[2], gl[2];
+        float gsc_inv[2];
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            float gyo[4], gys[4], m = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float v = y[p][r] * wuns[p];
+                loss += lam * v * v;
+                gyo[r] = -lam * v;
+                gys[r] = swap_sign * swap_pairs(gyo[r]);
+                m = fmaxf(m, fabsf(gyo[r]));
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+            float sc;
+            pow2_scale(m, sc, gsc_inv[p]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                split_f16(gyo[r] * sc, gh[p], gl[p], 2 * r);
+                split_f16(gys[r] * sc, gh[p], gl[p], 2 * r + 1);
+            }
+        }
+        // Adjoint: rows = antennas 16 at + i, K = times trow + 4g + q (x re, im).
+#pragma unroll
+        for (int at = 0; at < NAT; at++) {
+            halfx8 xa[2];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                halfx2 h0, h1;
+                ci8_to_half2x2(sx[(trow + 4 * g + q) * XS + at * 16 + i], h0, h1);
+                xa[0][2 * q] = h0[0]; xa[0][2 * q + 1] = h0[1];
+                xa[1][2 * q] = h1[0]; xa[1][2 * q + 1] = h1[1];
+            }
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                floatx4 t = mfma_f16(xa[p], gh[p], zero4);
+                t = mfma_f16(xa[p], gl[p], t);
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc2[p][at][r] = fmaf(t[r], gsc_inv[p], acc2[p][at][r]);
+            }
+        }
+        if (k + 1 < ntiles) {
+            store_tile(s_x + ((k + 1) & 1) * SG_TC * XS);
+            if (k + 2 < ntiles) load_tile(t_begin + (k + 2) * SG_TC);
+        }
+        __syncthreads();
+    }
+
+    float* s_part = reinterpret_cast<float*>(lds_raw);
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int at = 0; at < NAT; at++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                s_part[((wave * 2 + p) * 16 + i) * APAD + at * 16 + 4 * g + r] = acc2[p][at][r];
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
+    if (lane == 0) s_loss[wave] = loss;
+    __syncthreads();
+    constexpr int NPART = 2 * 16 * APAD;
+    float* out = a.partial + ((((size_t)sp * F + f) * 2) * a.btiles + bt) * 16 * APAD;
+    const size_t pstride = (size_t)a.btiles * 16 * APAD;
+    for (int e = tid; e < NPART; e += blockDim.x) {
+        const float v = ((s_part[e] + s_part[NPART + e]) + s_part[2 * NPART + e]) + s_part[3 * NPART + e];
+        const int p = e / (16 * APAD), r = e - p * 16 * APAD;
+        out[p * pstride + r] = v;
+    }
+    if (tid == 0)
         a.loss_part[((size_t)sp * F + f) * a.btiles + bt] = ((s_loss[0] + s_loss[1]) + s_loss[2]) + s_loss[3];
 }
 
@@ -444,7 +885,7 @@ __global__ __launch_bounds__(256) void adjoint_reduce_kernel(AdjArgs a, int nspl
     if (loss && blockIdx.x == gridDim.x - 1) {
         __shared__ double s[256];
         double v = 0.0;
-        for (size_t e = threadIdx.x; e < n_loss; e += blockDim.x) v += a.loss_part[e];
+        for (size_t e = threadIdx.x; e < n_loss; e += blockDim.x) v += (double)a.loss_part[e];
         s[threadIdx.x] = v;
         __syncthreads();
         for (int off = 128; off > 0; off >>= 1) {
@@ -477,7 +918,7 @@ __global__ __launch_bounds__(256) void adjoint_reduce_kernel(AdjArgs a, int nspl
     gw[(((size_t)b * a.A + an) * a.F + f) * 2 + p] = make_float2(re, im);
 }
 
-static int run_adjoint(bool fused, const void* input, const void* phasors, const void* grad_out,
+static int run_adjoint(bool fused, bool f16, const void* input, const void* phasors, const void* grad_out,
                        const float* beam_weights, double* loss, void* grad_phasors, uint64_t A,
                        uint64_t F, uint64_t T, uint64_t P, uint64_t B, hipStream_t s) {
     const char* who = fused ? "stokes-i gradient" : "beamformer adjoint";
@@ -499,26 +940,32 @@ static int run_adjoint(bool fused, const void* input, const void* phasors, const
     a.A = (int)A; a.F = (int)F; a.T = (int)T; a.B = (int)B;
     a.n_at = (int)ceil_div(A, 16);
     a.apad = 16 * a.n_at;
+    a.nsteps = 2 * (int)ceil_div(A, 4);
     a.btiles = (int)ceil_div(B, 8);
     if (fused)
         for (uint64_t b = 0; b < B; b++) a.lambda[b] = beam_weights[b];
-    // Time splits, each a whole number of tiles.  Both kernels fill a CU's
-    // SIMDs with one or two workgroups, so a launch costs its workgroups per
-    // CU times the tiles of a wave plus about one tile time of set-up (packing
-    // the phasors, summing the waves); a single workgroup per CU hides its
+    // FP32 loss + gradient with at most 4 beams: the 4x4-block kernel.
+    const bool b4 = fused && !f16 && B <= 4 && A <= 64 && T % 4 == 0 && (uintptr_t)input % 16 == 0 &&
+                    A * F * T < (1ull << 31);
+    // Time splits, each a whole number of tiles.  Fused: the split length that
+    // minimises rounds of resident workgroups (per CU: 4 FP32 or 3 split FP16
+    // up to 64 or 48 antennas, else 2; the 4x4-block kernel SG4_WGS) x tiles
+    // per wave.  Plain adjoint: one or two workgroups fill a CU's SIMDs, so a
+    // launch costs its workgroups per CU times the tiles of a wave plus about
+    // one tile time to sum the waves; a single workgroup per CU hides its
     // loads worse (1.3x a tile).  Ties take the longest split (fewest partial
-    // sums).  A42 F384 T2048 B4 (loss + gradient): 2 splits 53 us, 1 or 4
-    // splits 56 us, 8 splits 70 us.
-    const int tc = fused ? SG_TC : ADJ_TC;
+    // sums).
+    const int tc = b4 ? SG4_TC : fused ? SG_TC : ADJ_TC;
     const long tiles = (long)ceil_div(std::max<uint64_t>(T, 1), (uint64_t)tc);
     const long per_split = (long)F * a.btiles;
     const long cus = device_cus();
+    const long slots = !fused ? cus : cus * (b4 ? SG4_WGS : f16 ? (a.n_at <= 3 ? 3 : 2) : (a.n_at <= 4 ? 4 : 2));
     long tiles_per = tiles;
     double best = -1;
     for (long tp = tiles; tp >= 1; tp--) {
-        const long rounds = ((tiles + tp - 1) / tp * per_split + cus - 1) / cus;
-        const long per_wave = fused ? (tp + ADJ_WAVES - 1) / ADJ_WAVES : tp;   // fused: waves take tiles in turn
-        const double cost = (double)rounds * (per_wave + 1) * (rounds == 1 ? 1.3 : 1.0);
+        const long rounds = ((tiles + tp - 1) / tp * per_split + slots - 1) / slots;
+        const long per_wave = b4 ? (tp + ADJ_WAVES - 1) / ADJ_WAVES : tp;   // b4: waves take tiles in turn
+        const double cost = fused ? (double)rounds * per_wave : (double)rounds * (per_wave + 1) * (rounds == 1 ? 1.3 : 1.0);
         if (best < 0 || cost < best) { best = cost; tiles_per = tp; }
     }
     const long nsplit = (tiles + tiles_per - 1) / tiles_per;
@@ -527,25 +974,28 @@ static int run_adjoint(bool fused, const void* input, const void* phasors, const
     const size_t part_floats = (size_t)nsplit * F * 2 * a.btiles * 16 * a.apad;
     const size_t n_loss = (size_t)nsplit * F * a.btiles;
     unsigned char* ws = nullptr;
-    const size_t ws_bytes = part_floats * sizeof(float) + n_loss * sizeof(double);
+    const size_t ws_bytes = (part_floats + n_loss) * sizeof(float);
     if (F == 0) return BLADE_SUCCESS;
     int rc = library_workspace(WS_ADJOINT, ws_bytes, s, &ws);
     if (rc) return rc;
     a.partial = reinterpret_cast<float*>(ws);
-    a.loss_part = reinterpret_cast<double*>(a.partial + part_floats);     // part_floats is even
+    a.loss_part = a.partial + part_floats;
 
     const size_t lds_sum = (size_t)ADJ_WAVES * 2 * 16 * a.apad * 4;
-    const size_t lds = fused ? std::max(lds_sum, (size_t)a.n_at * 6 * 64 * 16 + ADJ_WAVES * 16 * SG_XS * 4) : lds_sum;
+    const size_t lds = !fused ? lds_sum
+                       : b4    ? ((size_t)a.A * 4 * SG4_WS + (size_t)ADJ_WAVES * SG4_GY) * 4
+                       : f16   ? (size_t)2 * SG_TC * sg_xs(a.apad) * 4 + (size_t)2 * a.n_at * 2 * 64 * 16
+                               : ((size_t)2 * SG_TC * sg_xs(a.apad) + 2 * (size_t)a.nsteps * 64) * 4;
 #define ADJ_FN(...) reinterpret_cast<const void*>(&__VA_ARGS__)
     static const void* const fn_adj[2][ADJ_MAXAT] = {
         {ADJ_FN(adjoint_kernel<1, false>), ADJ_FN(adjoint_kernel<2, false>), ADJ_FN(adjoint_kernel<3, false>), ADJ_FN(adjoint_kernel<4, false>), ADJ_FN(adjoint_kernel<5, false>), ADJ_FN(adjoint_kernel<6, false>), ADJ_FN(adjoint_kernel<7, false>), ADJ_FN(adjoint_kernel<8, false>)},
         {ADJ_FN(adjoint_kernel<1, true>), ADJ_FN(adjoint_kernel<2, true>), ADJ_FN(adjoint_kernel<3, true>), ADJ_FN(adjoint_kernel<4, true>), ADJ_FN(adjoint_kernel<5, true>), ADJ_FN(adjoint_kernel<6, true>), ADJ_FN(adjoint_kernel<7, true>), ADJ_FN(adjoint_kernel<8, true>)}};
-    static const void* const fn_grad[2][ADJ_MAXAT] = {
-        {ADJ_FN(stokes_grad_kernel<1, false>), ADJ_FN(stokes_grad_kernel<2, false>), ADJ_FN(stokes_grad_kernel<3, false>), ADJ_FN(stokes_grad_kernel<4, false>), ADJ_FN(stokes_grad_kernel<5, false>), ADJ_FN(stokes_grad_kernel<6, false>), ADJ_FN(stokes_grad_kernel<7, false>), ADJ_FN(stokes_grad_kernel<8, false>)},
-        {ADJ_FN(stokes_grad_kernel<1, true>), ADJ_FN(stokes_grad_kernel<2, true>), ADJ_FN(stokes_grad_kernel<3, true>), ADJ_FN(stokes_grad_kernel<4, true>), ADJ_FN(stokes_grad_kernel<5, true>), ADJ_FN(stokes_grad_kernel<6, true>), ADJ_FN(stokes_grad_kernel<7, true>), ADJ_FN(stokes_grad_kernel<8, true>)}};
+    static const void* const fn_f32[ADJ_MAXAT] = {ADJ_FN(stokes_grad_kernel<1>), ADJ_FN(stokes_grad_kernel<2>), ADJ_FN(stokes_grad_kernel<3>), ADJ_FN(stokes_grad_kernel<4>), ADJ_FN(stokes_grad_kernel<5>), ADJ_FN(stokes_grad_kernel<6>), ADJ_FN(stokes_grad_kernel<7>), ADJ_FN(stokes_grad_kernel<8>)};
+    static const void* const fn_f16[ADJ_MAXAT] = {ADJ_FN(stokes_grad_f16_kernel<1>), ADJ_FN(stokes_grad_f16_kernel<2>), ADJ_FN(stokes_grad_f16_kernel<3>), ADJ_FN(stokes_grad_f16_kernel<4>), ADJ_FN(stokes_grad_f16_kernel<5>), ADJ_FN(stokes_grad_f16_kernel<6>), ADJ_FN(stokes_grad_f16_kernel<7>), ADJ_FN(stokes_grad_f16_kernel<8>)};
+    static const void* const fn_b4[4] = {ADJ_FN(stokes_grad_b4_kernel<1>), ADJ_FN(stokes_grad_b4_kernel<2>), ADJ_FN(stokes_grad_b4_kernel<3>), ADJ_FN(stokes_grad_b4_kernel<4>)};
 #undef ADJ_FN
     const bool vec = T % 4 == 0 && (uintptr_t)input % 16 == 0 && (uintptr_t)grad_out % 16 == 0;
-    const void* fn = fused ? fn_grad[vec][a.n_at - 1] : fn_adj[vec][a.n_at - 1];
+    const void* fn = b4 ? fn_b4[a.n_at - 1] : !fused ? fn_adj[vec][a.n_at - 1] : (f16 ? fn_f16 : fn_f32)[a.n_at - 1];
     if (lds > 65536) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) {
@@ -569,7 +1019,7 @@ using namespace bl;
 extern "C" int blade_beamformer_adjoint(const void* input, const void* grad_output,
                                         void* grad_phasors, uint64_t A, uint64_t F, uint64_t T,
                                         uint64_t P, uint64_t B, blade_stream_t stream) {
-    return run_adjoint(false, input, nullptr, grad_output, nullptr, nullptr, grad_phasors, A, F, T,
+    return run_adjoint(false, false, input, nullptr, grad_output, nullptr, nullptr, grad_phasors, A, F, T,
                        P, B, reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -580,6 +1030,6 @@ extern "C" int blade_beamformer_stokes_i_grad(int precision, const void* input, 
                                               blade_stream_t stream) {
     if (precision != BLADE_PREC_F32 && precision != BLADE_PREC_F16X2)
         return fail("stokes-i gradient: unknown precision");
-    return run_adjoint(true, input, phasors, nullptr, beam_weights, loss, grad_phasors, A, F, T, P,
+    return run_adjoint(true, precision == BLADE_PREC_F16X2, input, phasors, nullptr, beam_weights, loss, grad_phasors, A, F, T, P,
                        B, reinterpret_cast<hipStream_t>(stream));
 }

@@ -190,8 +190,8 @@ def stokes_i_loss_and_grad(x: torch.Tensor, phasors: torch.Tensor, beam_weights,
                            stream=None, precision: str = "f32") -> tuple[torch.Tensor, torch.Tensor]:
     """L = -sum_b beam_weights[b] sum |y_b|^2 (FP64 device scalar) and dL/dconj(w) CF32.
 
-    ``precision``: "f32" or "f16x2"; both run the FP32-precision kernel, the
-    faster one."""
+    ``precision``: "f32" (FP32 matrix cores) or "f16x2" (FP16 matrix cores,
+    hi + lo split phasors and gradients, FP32 accumulation)."""
     A, F, T, P = _shape4(x, "ci8")
     B = phasors.shape[0]
     if tuple(phasors.shape) != (B, A, F, 1, P) or phasors.dtype != torch.complex64:

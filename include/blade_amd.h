@@ -179,9 +179,9 @@ int blade_beamformer_adjoint(const void* input, const void* grad_output, void* g
  * loss: one FP64 value in device memory; grad_phasors = dL/dconj(w) CF32
  * [B,A,F,1,P] (PyTorch's gradient is twice this).  The beams are recomputed
  * tile by tile and never stored.  beam_weights: host array of B floats,
- * B <= 64; P = 2, A <= 128.  precision: BLADE_PREC_F32 or BLADE_PREC_F16X2;
- * one kernel serves both (phasors and gradients as three exact BF16 parts,
- * FP32 accumulation), since it is faster than either FP32 or FP16 matrix work.
+ * B <= 64; P = 2, A <= 128.  precision: BLADE_PREC_F32 (FP32 matrix cores)
+ * or BLADE_PREC_F16X2 (FP16 matrix cores with hi + lo phasors and
+ * gradients, FP32 accumulation; error at the FP32 level).
  */
 int blade_beamformer_stokes_i_grad(int precision, const void* input, const void* phasors,
                                    const float* beam_weights, double* loss, void* grad_phasors,

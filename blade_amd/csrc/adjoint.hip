@@ -233,12 +233,74 @@ __global__ __launch_bounds__(256, (NAT <= 3 ? 3 : NAT <= 5 ? 2 : 1)) void adjoin
 // time; lane groups take times 4 apart).
 __host__ __device__ constexpr int sg_xs(int apad) { return apad + SG_XPAD; }
 
+// Adjoint of one wave's 16 times (rows trow .. + 15 of the LDS voltage tile)
+// and the gy = gy[pol][time 4g + r] its lanes hold: K = 16 times x (re, im) of
+// x, which are the lane's own values and, for Im x, the neighbouring column's
+// (re <-> im) with the sign of conj(x).  gy as three BF16 parts, CI8 exact:
+// exact products, accumulated in FP32 from the smallest part up.  TILE: the 16
+// times are summed by themselves, one rounding into the long sum, as the split
+// FP16 form always did (error 1.1e-7 at A42 T2048 B16; 1.7e-7 without).  The
+// FP32 form's was one chain of 8 instructions, so 3 are below it without.
+template <int NAT, int XS, bool TILE>
+__device__ __forceinline__ void sg_adjoint(const uint32_t* rows, const float (&gy)[2][4], float swap_sign, int i, int g,
+                                           floatx4 (&acc)[2][NAT]) {
+    uint4 gb[2][3];
+    float mag = 0.f;
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) mag += fabsf(gy[p][r]);
+    auto parts = [&](auto checked) {
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            uint32_t w[3][4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                float u[3], v[3];
+                split_bf16x3<decltype(checked)::value>(gy[p][r], u);
+#pragma unroll
+                for (int m = 0; m < 3; m++) {
+                    v[m] = swap_sign * swap_pairs(u[m]);
+                    w[m][r] = bf16_pair(u[m], v[m]);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < 3; m++) gb[p][m] = make_uint4(w[m][0], w[m][1], w[m][2], w[m][3]);
+        }
+    };
+    // Infinities and NaN (they show in mag) take the split that keeps them.
+    if (__all(mag <= 3.0e38f))
+        parts(std::false_type{});
+    else
+        parts(std::true_type{});
+#pragma unroll
+    for (int at = 0; at < NAT; at++) {
+        uint32_t d[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) d[q] = rows[(4 * g + q) * XS + at * 16 + i];
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const uint4 xo = make_uint4(ci8_to_bf16(d[0], p), ci8_to_bf16(d[1], p), ci8_to_bf16(d[2], p),
+                                        ci8_to_bf16(d[3], p));
+            floatx4 t = TILE ? floatx4{0.f, 0.f, 0.f, 0.f} : acc[p][at];
+#pragma unroll
+            for (int m = 2; m >= 0; m--) t = mfma_bf16(xo, gb[p][m], t);
+            acc[p][at] = TILE ? acc[p][at] + t : t;
+        }
+        __builtin_amdgcn_sched_barrier(0);     // one tile's operands live at a time (7 and 8 tiles spilled)
+    }
+}
+
 // Fused Stokes-I loss and phasor gradient for A <= 16 NAT antennas.  Each
 // wave takes 16 time rows of every SG_TC-sample tile; the next tile's
 // voltages are loaded into registers while this one is computed and written
 // to the other half of a double-buffered LDS stage: one barrier per tile.
+// The forward stays on FP32 instructions: the loss is returned in FP64, and
+// callers follow its history.  Bound by them (32 cycles per K = 4): A42 F384
+// T2048 B16 213 us with an FP32 adjoint of 8 instructions per antenna tile and
+// pol, 167 us with sg_adjoint's 3 of half the length.
 template <int NAT>
-__global__ __launch_bounds__(256, (NAT <= 4 ? 4 : 2)) void stokes_grad_kernel(AdjArgs a) {
+__global__ __launch_bounds__(256, (NAT <= 4 ? 4 : NAT <= 6 ? 3 : 2)) void stokes_grad_kernel(AdjArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     constexpr int APAD = 16 * NAT;
     constexpr int XS = sg_xs(APAD);
@@ -274,9 +336,14 @@ __global__ __launch_bounds__(256, (NAT <= 4 ? 4 : 2)) void stokes_grad_kernel(Ad
         const int tt = t0 + lane;
         pre_t_ok = tt < t_end;
         const int ttc = min(tt, t_end - 1);
+        // Opaque stride and a uniform wave number: otherwise the PER row
+        // addresses are held in registers across tiles.
+        size_t st = (size_t)F * T;
+        asm volatile("" : "+s"(st));
+        const int w0 = __builtin_amdgcn_readfirstlane(wave);
+        const uint32_t* const xf = a.x + (size_t)f * T + ttc;
 #pragma unroll
-        for (int k = 0; k < PER; k++)
-            pre[k] = a.x[((size_t)min(wave + ADJ_WAVES * k, A - 1) * F + f) * T + ttc];
+        for (int k = 0; k < PER; k++) pre[k] = xf[min(w0 + ADJ_WAVES * k, A - 1) * st];
     };
     auto store_tile = [&](uint32_t* dst) {
 #pragma unroll
@@ -348,33 +415,17 @@ __global__ __launch_bounds__(256, (NAT <= 4 ? 4 : 2)) void stokes_grad_kernel(Ad
                 }
             }
         }
-        // Lane (g, i), register r: y at time trow + 4g + r, column i.  Its
-        // gradient is gy = -lambda y; the imaginary-x block of G takes the
-        // neighbouring column (re <-> im) with the sign of conj(x).
-        float gyo[2][4], gys[2][4];
+        // Lane (g, i), register r: y at time trow + 4g + r, column i.
+        float gy[2][4];
 #pragma unroll
         for (int p = 0; p < 2; p++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const float v = y[p][r];
                 loss += lam * v * v;
-                gyo[p][r] = -lam * v;
-                gys[p][r] = swap_sign * swap_pairs(gyo[p][r]);
+                gy[p][r] = -lam * v;
             }
-        // Adjoint: K = times trow + 4g + r (g = k index), both x components.
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const uint32_t* row = sx + (trow + 4 * g + r) * XS + i;
-#pragma unroll
-            for (int at = 0; at < NAT; at++) {
-                const uint32_t d = row[at * 16];
-#pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    acc2[p][at] = adj_mfma(ci8_component(d, 2 * p), gyo[p][r], acc2[p][at]);
-                    acc2[p][at] = adj_mfma(ci8_component(d, 2 * p + 1), gys[p][r], acc2[p][at]);
-                }
-            }
-        }
+        sg_adjoint<NAT, XS, false>(sx + trow * XS, gy, swap_sign, i, g, acc2);
         if (k + 1 < ntiles) {
             // Tile k + 1 into the other buffer (last read in iteration k - 1,
             // before the barrier that ended it), then tile k + 2's loads.
@@ -420,11 +471,13 @@ __global__ __launch_bounds__(256, (NAT <= 4 ? 4 : 2)) void stokes_grad_kernel(Ad
 //   Forward, blocks = groups of 4 times, K = one antenna per instruction:
 //     lane (blk, c) feeds x[a][t0 + 4 blk + c] and w[a][beam c]; register r
 //     of the result is y at time t0 + 4 blk + r, beam c.
-//   Adjoint, blocks = groups of 4 antennas, K = one time per instruction:
-//     lane (blk, c) feeds conj(x)[4 blk + c][t] and gy[beam c][t]; register r
-//     is gw of antenna 4 blk + r, beam c.  gy passes through a per-wave LDS
-//     tile [p][product][beam][time], read as broadcasts (all blocks read the
-//     same four addresses).
+//   Adjoint: gy, cut into three BF16 parts, passes through a per-wave LDS
+//     tile into the operand layout of adjoint_kernel, and so does the rest: the
+//     voltages as 16-byte pieces of memory (they were just read, so from L2),
+//     K = 32 times per instruction.  On 4x4 FP32 blocks as well it took 384
+//     instructions of 8 cycles and 96 LDS reads a tile instead of 24 NAT of 16
+//     and 12, and a call 101 us instead of 76 us (A42 F384 T2048 B4; A28 76
+//     and 50 us).
 // Each wave takes 64-time tiles; partial sums are added across waves in LDS
 // in wave order and across time splits by adjoint_reduce_kernel, whose
 // partial layout this kernel writes (rows 2 b and 2 b + 1, beam tile 0).
@@ -432,12 +485,10 @@ __global__ __launch_bounds__(256, (NAT <= 4 ? 4 : 2)) void stokes_grad_kernel(Ad
 // ---------------------------------------------------------------------------
 constexpr int SG4_TC = 64;            // times per wave tile
 constexpr int SG4_WS = 8;             // LDS floats per (antenna, beam): (wr, wi, wr + wi) per pol, padded
-// gy tile rows ([p][product][beam], SG4_TC times each) are padded by 4
-// floats, so the four beams' rows that a read instruction broadcasts start
-// on different LDS banks (unpadded, their 256-byte stride put all four on the
-// same banks: 7 conflict cycles per LDS instruction).
-constexpr int SG4_GS = SG4_TC + 4;
-constexpr int SG4_GY = 2 * 3 * 4 * SG4_GS;   // floats of one wave's gy tile
+// gy tile rows ([p][part][beam][re/im], SG4_TC BF16 times each) are padded by
+// 16 bytes, which puts the rows of a read on different banks.
+constexpr int SG4_GS = 2 * SG4_TC + 16;      // bytes
+constexpr int SG4_GY = 2 * 3 * 8 * SG4_GS;   // bytes of one wave's gy tile
 constexpr int SG4_WGS = 3;            // resident workgroups per CU (launch bounds)
 
 __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
@@ -445,11 +496,11 @@ __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
 }
 
 template <int NAT>
-__global__ __launch_bounds__(256, SG4_WGS) void stokes_grad_b4_kernel(AdjArgs a) {
+__global__ __launch_bounds__(256, (NAT <= 3 ? SG4_WGS : 2)) void stokes_grad_b4_kernel(AdjArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     constexpr int AMAX = 16 * NAT;
     float* const s_w = reinterpret_cast<float*>(lds_raw);            // [A][4][SG4_WS]
-    float* const s_gy = s_w + (size_t)a.A * 4 * SG4_WS;               // [wave][SG4_GY]
+    unsigned char* const gyw = lds_raw + (size_t)a.A * 4 * SG4_WS * 4 + (threadIdx.x >> 6) * SG4_GY;   // this wave's gy
     __shared__ float s_loss[ADJ_WAVES];
 
     const int tid = threadIdx.x;
@@ -483,17 +534,15 @@ __global__ __launch_bounds__(256, SG4_WGS) void stokes_grad_b4_kernel(AdjArgs a)
     __syncthreads();
 
     const float lam = c < B ? a.lambda[c] : 0.f;
-    // Adjoint sums per pol: Q1 = sum gr xr, Q2 = sum gi xi, Q3 = sum (gr + gi)(xr - xi);
-    // gw = (Q1 + Q2) + j (Q3 - Q1 + Q2).
-    floatx4 q[2][3];
+    const int i = lane & 15, g = lane >> 4;                  // adjoint operand row and K group
+    floatx4 acc[2][NAT][2];    // [pol][antenna tile][component of x]
 #pragma unroll
     for (int p = 0; p < 2; p++)
 #pragma unroll
-        for (int k = 0; k < 3; k++) q[p][k] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int at = 0; at < NAT; at++)
+#pragma unroll
+            for (int k = 0; k < 2; k++) acc[p][at][k] = floatx4{0.f, 0.f, 0.f, 0.f};
     float loss = 0.f;
-    float* const gyw = s_gy + wave * SG4_GY;
-    // This lane's adjoint antenna row (clamped: rows past A are never stored).
-    const uint4* const xa = reinterpret_cast<const uint4*>(a.x + min(4 * blk + c, A - 1) * ant_stride + f * T);
 
     // Forward voltages of tile kk at this lane's time, antennas 8 g .. 8 g + 7
     // (group g + 1 is in flight while group g is computed: 3% faster than
@@ -512,18 +561,23 @@ __global__ __launch_bounds__(256, SG4_WGS) void stokes_grad_b4_kernel(AdjArgs a)
         for (int j = 0; j < 8; j++)
             if (8 * g + j < na) dst[j] = xf[(8 * g + j) * st];     // uniform
     };
-    // Adjoint voltages of 16 times from t: this lane's antenna row (times
-    // past tn re-read the last 4 in bounds; their gy is not used).
-    auto load_adj = [&](int t0, int tn, int t, uint4 (&xv)[4]) {
+    // Adjoint voltages: times t + 8 g .. + 7 of this lane's row of tile at
+    // (antennas past A repeat the last one, never stored; times past the split
+    // its end, their gy is 0).
+    uint4 xq[NAT][2];
+    auto load_adj = [&](int t, int at) {
+        unsigned st = ant_stride;
+        asm volatile("" : "+s"(st));
+        const uint32_t* const xp = a.x + (min(16 * at + i, A - 1) * st + f * T);
 #pragma unroll
-        for (int s4 = 0; s4 < 4; s4++) xv[s4] = xa[(t0 + min(t + 4 * s4, tn - 4)) >> 2];
+        for (int h = 0; h < 2; h++) xq[at][h] = *reinterpret_cast<const uint4*>(xp + min(t + 8 * g + 4 * h, t_end - 4));
     };
 
     for (int k = wave; k < ntiles; k += ADJ_WAVES) {
         const int t0 = t_begin + k * SG4_TC;
         const int tn = min(SG4_TC, t_end - t0);            // a multiple of 4
-        uint4 xv[2][4];
-        load_adj(t0, tn, 0, xv[0]);                        // in flight during the forward
+#pragma unroll
+        for (int at = 0; at < NAT; at++) load_adj(t0, at);   // in flight during the forward
         load_fwd(k, 0, xd[0]);
         // ---- forward: this lane feeds time t0 + 4 blk + c (clamped to the
         // split; results for times past it are zeroed below).  The antenna
@@ -554,89 +608,75 @@ __global__ __launch_bounds__(256, SG4_WGS) void stokes_grad_b4_kernel(AdjArgs a)
                 }
             }
         }
-        // ---- gy = -lambda y at (time t0 + 4 blk + r, beam c): gr, gi, gr + gi
-        // into this wave's LDS tile [p][product][beam][time].  Times past the
-        // split read clamped voltages: their y, and so gy and the loss, are
-        // set to 0.
+        // ---- gy = -lambda y at (time t0 + 4 blk + r, beam c), in parts, into
+        // this wave's LDS tile.  Times past the split read clamped voltages:
+        // their y, and so gy and the loss, are set to 0.
+        float gr[2][4], gi[2][4], mag = 0.f;
 #pragma unroll
-        for (int p = 0; p < 2; p++) {
-            float g[3][4];
+        for (int p = 0; p < 2; p++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const bool ok = 4 * blk + r < tn;
                 const float yr = ok ? y[p][0][r] - y[p][1][r] : 0.f;
                 const float yi = ok ? (y[p][2][r] - y[p][0][r]) - y[p][1][r] : 0.f;
                 loss += lam * (yr * yr + yi * yi);
-                const float gr = -lam * yr, gi = -lam * yi;
-                g[0][r] = gr;
-                g[1][r] = gi;
-                g[2][r] = gr + gi;
+                gr[p][r] = -lam * yr;
+                gi[p][r] = -lam * yi;
+                mag += fabsf(gr[p][r]) + fabsf(gi[p][r]);
             }
+        auto parts = [&](auto checked) {
 #pragma unroll
-            for (int m = 0; m < 3; m++)
-                *reinterpret_cast<float4*>(gyw + ((p * 3 + m) * 4 + c) * SG4_GS + 4 * blk) =
-                    make_float4(g[m][0], g[m][1], g[m][2], g[m][3]);
-        }
-        // ---- adjoint: this lane feeds antenna 4 blk + c and gy of beam c;
-        // one instruction per (time, pol, product).  The wave reads back its
-        // own LDS writes (LDS operations of a wave complete in order).  The
-        // next 16 times' voltages load while these are computed.
+            for (int p = 0; p < 2; p++)
 #pragma unroll
-        for (int h = 0; h < SG4_TC / 16; h++) {
-            if (h + 1 < SG4_TC / 16) load_adj(t0, tn, 16 * (h + 1), xv[(h + 1) & 1]);
-            if (16 * h < tn) {                                    // uniform
+                for (int co = 0; co < 2; co++) {
+                    float v[4][3];
 #pragma unroll
-                for (int s4 = 0; s4 < 4; s4++) {
-                    const int tt = 16 * h + 4 * s4;
-                    if (tt < tn) {                                // uniform
-                        float4 gv[2][3];
+                    for (int r = 0; r < 4; r++) split_bf16x3<decltype(checked)::value>(co ? gi[p][r] : gr[p][r], v[r]);
 #pragma unroll
-                        for (int p = 0; p < 2; p++)
-#pragma unroll
-                            for (int m = 0; m < 3; m++)
-                                gv[p][m] = *reinterpret_cast<const float4*>(gyw + ((p * 3 + m) * 4 + c) * SG4_GS + tt);
-                        const uint4 xq = xv[h & 1][s4];
-                        const uint32_t dw[4] = {xq.x, xq.y, xq.z, xq.w};
-#pragma unroll
-                        for (int s = 0; s < 4; s++) {
-#pragma unroll
-                            for (int p = 0; p < 2; p++) {
-                                const float xr = ci8_component(dw[s], 2 * p), xi = ci8_component(dw[s], 2 * p + 1);
-                                q[p][0] = mfma4(xr, gv[p][0][s], q[p][0]);
-                                q[p][1] = mfma4(xi, gv[p][1][s], q[p][1]);
-                                q[p][2] = mfma4(xr - xi, gv[p][2][s], q[p][2]);
-                            }
-                        }
-                    }
+                    for (int m = 0; m < 3; m++)
+                        *reinterpret_cast<uint2*>(gyw + ((p * 3 + m) * 8 + 2 * c + co) * SG4_GS + 8 * blk) =
+                            make_uint2(bf16_pair(v[0][m], v[1][m]), bf16_pair(v[2][m], v[3][m]));
                 }
+        };
+        // Infinities and NaN (they show in mag) take the split that keeps them.
+        if (__all(mag <= 3.0e38f))
+            parts(std::false_type{});
+        else
+            parts(std::true_type{});
+        // ---- adjoint, 32 times at a time.  The wave reads back its own LDS
+        // writes (LDS operations of a wave complete in order); columns 8 to 15
+        // repeat 0 to 7 and are not used.
+#pragma unroll
+        for (int h = 0; h < SG4_TC / 32; h++) {
+            uint4 gb[2][3];
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int m = 0; m < 3; m++)
+                    gb[p][m] = *reinterpret_cast<const uint4*>(gyw + ((p * 3 + m) * 8 + (i & 7)) * SG4_GS + 64 * h + 16 * g);
+#pragma unroll
+            for (int at = 0; at < NAT; at++) {
+                uint4 xo[2][2];
+#pragma unroll
+                for (int p = 0; p < 2; p++)
+#pragma unroll
+                    for (int k2 = 0; k2 < 2; k2++) xo[p][k2] = ci8_times_bf16(xq[at][0], xq[at][1], 2 * p + k2);
+                if (h + 1 < SG4_TC / 32) load_adj(t0 + 32 * (h + 1), at);
+#pragma unroll
+                for (int m = 0; m < 3; m++)
+#pragma unroll
+                    for (int p = 0; p < 2; p++)
+#pragma unroll
+                        for (int k2 = 0; k2 < 2; k2++) acc[p][at][k2] = mfma_bf16(xo[p][k2], gb[p][m], acc[p][at][k2]);
             }
         }
     }
 
-    // This wave's sums into its own gy tile (its last reads of it are done):
-    // [p][row = 2 beam + re/im][antenna 64], then summed over waves in order.
-    float* const pw = gyw;
-#pragma unroll
-    for (int p = 0; p < 2; p++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int an = 4 * blk + r;
-            pw[(p * 8 + 2 * c) * 64 + an] = q[p][0][r] + q[p][1][r];
-            pw[(p * 8 + 2 * c + 1) * 64 + an] = (q[p][2][r] - q[p][0][r]) + q[p][1][r];
-        }
     for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
     if (lane == 0) s_loss[wave] = loss;
-    __syncthreads();
-    const int apad = a.apad;
-    float* out = a.partial + ((size_t)sp * F + f) * 2 * a.btiles * 16 * apad;
-    const size_t pstride = (size_t)a.btiles * 16 * apad;   // between pols
-    for (int e = tid; e < 2 * 8 * A; e += blockDim.x) {
-        const int an = e % A, pr = e / A;                   // pr = p * 8 + row
-        const float* src = s_gy + pr * 64 + an;
-        const float v = ((src[0] + src[SG4_GY]) + src[2 * SG4_GY]) + src[3 * SG4_GY];
-        out[(pr >> 3) * pstride + (pr & 7) * apad + an] = v;
-    }
-    if (tid == 0) a.loss_part[((size_t)sp * F + f) * a.btiles] = ((s_loss[0] + s_loss[1]) + s_loss[2]) + s_loss[3];
+    __syncthreads();                          // every wave is done with the LDS operands
+    adj_store_partials<NAT>(a, acc, reinterpret_cast<float*>(lds_raw), sp, f, 0);
+    if (tid == 0) a.loss_part[(size_t)sp * F + f] = ((s_loss[0] + s_loss[1]) + s_loss[2]) + s_loss[3];
 }
 
 // Power-of-two scale s with m * s in [0.5, 1) for m > 0 (1 for m = 0), and 1/s.
@@ -660,11 +700,9 @@ __device__ __forceinline__ void split_f16(float v, halfx8& hi, halfx8& lo, int j
 //   * Forward B operand: the phasor embedding times a power-of-two scale per
 //     pol (every component below 1), as hi + lo FP16 halves; K = 16
 //     antennas x (re, im) of x per instruction.
-//   * Adjoint B operand: the wave's gy of the tile, K = 16 times x (re, im)
-//     -- exactly the forward outputs the lane holds (times 4g..4g+3 and the
-//     neighbouring column) -- scaled by a power of two from the wave's
-//     largest |gy| and split the same way; each tile's product is unscaled
-//     into the FP32 sums.
+//   * Adjoint: sg_adjoint, where gy needs no scale: as hi + lo FP16 halves it
+//     took the wave's largest |gy| over 6 lane exchanges per pol and tile.
+//     A42 F384 T2048 B4 67 -> 60 us, A28 56 -> 47 us, A16 B8 44 -> 34 us.
 // Error against FP64 is that of FP32 arithmetic (hi + lo carry ~22 bits).
 template <int NAT>
 __global__ __launch_bounds__(256, (NAT <= 3 ? 3 : 2)) void stokes_grad_f16_kernel(AdjArgs a) {
@@ -700,9 +738,18 @@ __global__ __launch_bounds__(256, (NAT <= 3 ? 3 : 2)) void stokes_grad_f16_kerne
         const int tt = t0 + lane;
         pre_t_ok = tt < t_end;
         const int ttc = min(tt, t_end - 1);
+        size_t st = (size_t)F * T;
+        int w0 = wave;
+        if constexpr (NAT == ADJ_MAXAT) {
+            // Opaque stride, uniform wave number: otherwise the row addresses
+            // are held in registers across tiles, which spilled here (A128 F64
+            // T2048 B8 80 -> 64 us; with fewer tiles they fit and cost nothing).
+            asm volatile("" : "+s"(st));
+            w0 = __builtin_amdgcn_readfirstlane(wave);
+        }
+        const uint32_t* const xf = a.x + (size_t)f * T + ttc;
 #pragma unroll
-        for (int k = 0; k < PER; k++)
-            pre[k] = a.x[((size_t)min(wave + ADJ_WAVES * k, A - 1) * F + f) * T + ttc];
+        for (int k = 0; k < PER; k++) pre[k] = xf[min(w0 + ADJ_WAVES * k, A - 1) * st];
     };
     auto store_tile = [&](uint32_t* dst) {
 #pragma unroll
@@ -801,49 +848,16 @@ __global__ __launch_bounds__(256, (NAT <= 3 ? 3 : 2)) void stokes_grad_f16_kerne
                 y[p] = mfma_f16(xa[p], wh[((p * NAT + blk) * 2 + 1) * 64], y[p]);
             }
         }
-        // gy = -lambda y (unscaled), its wave maximum, and the B operands.
-        halfx8 gh[2], gl[2];
-        float gsc_inv[2];
+        float gy[2][4];
 #pragma unroll
-        for (int p = 0; p < 2; p++) {
-            float gyo[4], gys[4], m = 0.f;
+        for (int p = 0; p < 2; p++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const float v = y[p][r] * wuns[p];
                 loss += lam * v * v;
-                gyo[r] = -lam * v;
-                gys[r] = swap_sign * swap_pairs(gyo[r]);
-                m = fmaxf(m, fabsf(gyo[r]));
+                gy[p][r] = -lam * v;
             }
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-            float sc;
-            pow2_scale(m, sc, gsc_inv[p]);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                split_f16(gyo[r] * sc, gh[p], gl[p], 2 * r);
-                split_f16(gys[r] * sc, gh[p], gl[p], 2 * r + 1);
-            }
-        }
-        // Adjoint: rows = antennas 16 at + i, K = times trow + 4g + q (x re, im).
-#pragma unroll
-        for (int at = 0; at < NAT; at++) {
-            halfx8 xa[2];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                halfx2 h0, h1;
-                ci8_to_half2x2(sx[(trow + 4 * g + q) * XS + at * 16 + i], h0, h1);
-                xa[0][2 * q] = h0[0]; xa[0][2 * q + 1] = h0[1];
-                xa[1][2 * q] = h1[0]; xa[1][2 * q + 1] = h1[1];
-            }
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                floatx4 t = mfma_f16(xa[p], gh[p], zero4);
-                t = mfma_f16(xa[p], gl[p], t);
-#pragma unroll
-                for (int r = 0; r < 4; r++) acc2[p][at][r] = fmaf(t[r], gsc_inv[p], acc2[p][at][r]);
-            }
-        }
+        sg_adjoint<NAT, XS, true>(sx + trow * XS, gy, swap_sign, i, g, acc2);
         if (k + 1 < ntiles) {
             store_tile(s_x + ((k + 1) & 1) * SG_TC * XS);
             if (k + 2 < ntiles) load_tile(t_begin + (k + 2) * SG_TC);
@@ -983,7 +997,7 @@ static int run_adjoint(bool fused, bool f16, const void* input, const void* phas
 
     const size_t lds_sum = (size_t)ADJ_WAVES * 2 * 16 * a.apad * 4;
     const size_t lds = !fused ? lds_sum
-                       : b4    ? ((size_t)a.A * 4 * SG4_WS + (size_t)ADJ_WAVES * SG4_GY) * 4
+                       : b4    ? std::max(lds_sum, (size_t)a.A * 4 * SG4_WS * 4 + ADJ_WAVES * SG4_GY)
                        : f16   ? (size_t)2 * SG_TC * sg_xs(a.apad) * 4 + (size_t)2 * a.n_at * 2 * 64 * 16
                                : ((size_t)2 * SG_TC * sg_xs(a.apad) + 2 * (size_t)a.nsteps * 64) * 4;
 #define ADJ_FN(...) reinterpret_cast<const void*>(&__VA_ARGS__)

@@ -93,12 +93,15 @@ def test_adjoint_matches_oracle_elementwise(A, B, T, offset):
     assert (again == got).all()
 
 
+@pytest.mark.parametrize("precision", ["f32", "f16x2"])
 @pytest.mark.parametrize("A,B", [(1, 1), (16, 8), (17, 9), (42, 4), (48, 3), (64, 5), (65, 2), (96, 2), (128, 17)])
 @pytest.mark.parametrize("T,offset", [(1, 0), (63, 0), (64, 0), (68, 0), (260, 0), (261, 0), (512, 1)])
-def test_stokes_gradient_matches_oracle_elementwise(A, B, T, offset):
+def test_stokes_gradient_matches_oracle_elementwise(A, B, T, offset, precision):
     """y as in the forward test (error ey); gy = -lambda y rounds once; the
     adjoint accumulates 2T terms and the partial sums.  ``offset`` shifts the
-    voltages off 16-byte alignment (single loads)."""
+    voltages off 16-byte alignment (single loads).  Split FP16 phasors are
+    off by 2^-22 of themselves, or by half the smallest FP16 step (2^-25) of
+    a scale below twice the largest of the pol and beam group of 8."""
     rng = np.random.default_rng(A + 10 * T)
     x8 = rng.integers(-128, 128, size=(A, 2, T, 2, 2), dtype=np.int8)
     w = (10.0 ** rng.uniform(-4, 4, size=(B, 1, 1, 1, 1)) *
@@ -107,7 +110,7 @@ def test_stokes_gradient_matches_oracle_elementwise(A, B, T, offset):
     buf = torch.empty(x8.size + 4 * offset, dtype=torch.int8, device="cuda")
     xd = buf[4 * offset:].view(x8.shape)
     xd.copy_(torch.from_numpy(x8))
-    loss, got = ops.stokes_i_loss_and_grad(xd, torch.from_numpy(w).cuda(), lam)
+    loss, got = ops.stokes_i_loss_and_grad(xd, torch.from_numpy(w).cuda(), lam, precision=precision)
     got = got.cpu().numpy()[:, :, :, 0]
     x = x8[..., 0].astype(np.float64) + 1j * x8[..., 1]
     y = np.einsum("bafp,aftp->bftp", w[:, :, :, 0].astype(np.complex128), x)
@@ -117,6 +120,12 @@ def test_stokes_gradient_matches_oracle_elementwise(A, B, T, offset):
     w1 = np.abs(w.real[:, :, :, 0].astype(np.float64)) + np.abs(w.imag[:, :, :, 0].astype(np.float64))
     u = 2.0 ** -24
     ey = 2 * (2 * A + 2) * u * np.einsum("bafp,aftp->bftp", w1, x1)
+    if precision == "f16x2":
+        ew = 2.0 ** -22 * w1
+        for b in range(0, B, 8):
+            top = np.maximum(np.abs(w.real[b:b + 8]), np.abs(w.imag[b:b + 8])).astype(np.float64)[:, :, :, 0]
+            ew[b:b + 8] += 2 * 2.0 ** -25 * 2 * top.max((0, 1))
+        ey += np.einsum("bafp,aftp->bftp", ew, x1)
     y1 = np.abs(y.real) + np.abs(y.imag) + 2 * ey
     bound = np.einsum("bftp,aftp->bafp", L * (2 * ey + (2 * (2 * T + 16) + 2) * u * y1), x1)
     d = got - ref

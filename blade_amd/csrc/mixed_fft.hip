@@ -31,9 +31,12 @@
 #include "mixed_fft.hh"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <vector>
 
 namespace bl {
 
@@ -439,55 +442,41 @@ static bool mix_plan(int C, MixPlan* pl) {
     return true;
 }
 
+// The search takes microseconds, as long as a small launch: answered once per
+// rate (0: not yet, 1: no, 2: yes).
 bool mixed_fft_covers(uint64_t rate) {
-    MixPlan pl;
-    return rate <= (uint64_t)kMixMaxC && mix_plan((int)rate, &pl);
-}
-
-static std::mutex g_mix_mutex;
-static std::map<std::pair<int, int>, float2*> g_mix_tw;
-
-static int mix_table(const MixPlan& pl, hipStream_t s, const float2** out) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return fail("channelizer: hipGetDevice failed");
-    std::lock_guard<std::mutex> lock(g_mix_mutex);
-    float2*& slot = g_mix_tw[{dev, pl.C}];
-    if (!slot) {
-        float2* p = nullptr;
-        hipError_t e = hipMalloc(&p, sizeof(float2) * (size_t)pl.C);   // sum of (R - 1) Ns = C - R_0
-        if (e != hipSuccess) {
-            set_error(std::string("channelizer: twiddle allocation: ") + hipGetErrorString(e));
-            return BLADE_HIP_ERROR;
-        }
-        hipLaunchKernelGGL(mixed_twiddle_kernel, dim3(8), dim3(256), 0, s, p, pl);
-        int rc = check_launch("channelizer twiddles");
-        if (rc) return rc;
-        slot = p;
+    static std::atomic<unsigned char> known[kMixMaxC + 1];
+    if (rate > (uint64_t)kMixMaxC) return false;
+    unsigned char k = known[rate].load(std::memory_order_relaxed);
+    if (!k) {
+        MixPlan pl;
+        k = mix_plan((int)rate, &pl) ? 2 : 1;
+        known[rate].store(k, std::memory_order_relaxed);
     }
-    *out = slot;
-    return BLADE_SUCCESS;
+    return k == 2;
 }
 
-int mixed_fft_plan(int C, hipStream_t s) {
+// A launch shape, rated by the lanes its passes keep busy and the points in
+// flight per CU (short of ~8000 the loads are not hidden).
+struct MixShape {
+    unsigned spw, threads;                 // spectra per workgroup and step
+    double score;
+};
+
+// What a rate keeps per device: it depends on the rate alone.  Found anew on
+// each call it cost 5-7 us of host time (6 x 74 channels of one 64-sample
+// spectrum 12.7 us a call, 7.1 us so).
+struct MixTable {
     MixPlan pl;
-    if (!mix_plan(C, &pl)) return fail("channelizer: no mixed-radix plan");
-    const float2* tw = nullptr;
-    return mix_table(pl, s, &tw);
-}
+    unsigned CS;                           // LDS row stride, float4
+    std::vector<MixShape> shapes;
+    float2* tw;
+};
 
-// Spectra per workgroup and threads.  A choice is rated by the lanes its
-// passes keep busy, the points in flight per CU (short of ~8000 the loads are
-// not hidden), the run of neighbouring output samples its stores write
-// (`run_of`) and whether the grid fills the chip.
-template <typename RunOf>
-static void mix_shape(const MixPlan& pl, uint64_t units, unsigned unit, RunOf run_of, unsigned* spw, unsigned* threads,
-                      unsigned* CS) {
-    const unsigned C = (unsigned)pl.C;
-    *CS = (C + C / 8 + 1) | 1;
-    double best = -1;
-    for (unsigned m = 1; m * unit <= 64; m++) {
-        const unsigned s = m * unit;
-        const size_t lds = (size_t)s * *CS * 16;
+static std::vector<MixShape> mix_shapes(const MixPlan& pl, unsigned CS) {
+    std::vector<MixShape> out;
+    for (unsigned s = 1; s <= 64; s++) {
+        const size_t lds = (size_t)s * CS * 16;
         if (lds > kMixLds) break;
         unsigned one = 0, two = 0;                   // threads with one butterfly each, and with two where allowed
         for (int i = 0; i < pl.n; i++) {
@@ -504,15 +493,61 @@ static void mix_shape(const MixPlan& pl, uint64_t units, unsigned unit, RunOf ru
                 busy += (double)nb / (nt * ((nb + nt - 1) / nt)) / pl.n;
             }
             const double wgs = std::min<double>({std::floor(160.0 * 1024 / lds), std::floor(1024.0 / nt), 16.0});
-            const double points = wgs * s * C;
-            const double grid = (double)((units + m - 1) / m) / (2.0 * device_cus());
-            const double score = busy * std::min(1.0, points / 8192) * (wgs < 2 ? 0.7 : 1.0) * run_of(s) *
-                                 std::min(1.0, 0.25 + 0.75 * grid);
-            if (score > best) {
-                best = score;
-                *spw = s;
-                *threads = nt;
-            }
+            const double points = wgs * s * pl.C;
+            out.push_back({s, nt, busy * std::min(1.0, points / 8192) * (wgs < 2 ? 0.7 : 1.0)});
+        }
+    }
+    return out;
+}
+
+static std::mutex g_mix_mutex;
+static std::map<std::pair<int, int>, std::unique_ptr<MixTable>> g_mix_tables;
+
+static int mix_table(int C, hipStream_t s, const MixTable** out) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return fail("channelizer: hipGetDevice failed");
+    std::lock_guard<std::mutex> lock(g_mix_mutex);
+    std::unique_ptr<MixTable>& slot = g_mix_tables[{dev, C}];
+    if (!slot) {
+        std::unique_ptr<MixTable> t(new MixTable);
+        if (!mix_plan(C, &t->pl)) return fail("channelizer: no mixed-radix plan");
+        t->CS = ((unsigned)C + C / 8 + 1) | 1;
+        t->shapes = mix_shapes(t->pl, t->CS);
+        hipError_t e = hipMalloc(&t->tw, sizeof(float2) * (size_t)C);   // sum of (R - 1) Ns = C - R_0
+        if (e != hipSuccess) {
+            set_error(std::string("channelizer: twiddle allocation: ") + hipGetErrorString(e));
+            return BLADE_HIP_ERROR;
+        }
+        hipLaunchKernelGGL(mixed_twiddle_kernel, dim3(8), dim3(256), 0, s, t->tw, t->pl);
+        int rc = check_launch("channelizer twiddles");
+        if (rc) return rc;
+        slot = std::move(t);
+    }
+    *out = slot.get();
+    return BLADE_SUCCESS;
+}
+
+int mixed_fft_plan(int C, hipStream_t s) {
+    const MixTable* t = nullptr;
+    return mix_table(C, s, &t);
+}
+
+// Spectra per workgroup (a multiple of `unit`) and threads: the rate's shapes
+// rated besides by the run of neighbouring output samples their stores write
+// (`run_of`) and whether the grid of `units` fills the chip.
+template <typename RunOf>
+static void mix_shape(const MixTable& t, uint64_t units, unsigned unit, RunOf run_of, unsigned* spw, unsigned* threads) {
+    const double full = 2.0 * device_cus();
+    double best = -1;
+    for (const MixShape& c : t.shapes) {
+        if (c.spw % unit || c.score <= best) continue;
+        const unsigned m = c.spw / unit;
+        const double grid = (double)((units + m - 1) / m) / full;
+        const double score = c.score * run_of(c.spw) * std::min(1.0, 0.25 + 0.75 * grid);
+        if (score > best) {
+            best = score;
+            *spw = c.spw;
+            *threads = c.threads;
         }
     }
 }
@@ -530,14 +565,17 @@ static int mix_launch(MixArgs& a, uint64_t blocks, unsigned threads, hipStream_t
 
 int mixed_fft(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec, hipStream_t s) {
     MixArgs a = {};
-    if (!mix_plan(C, &a.pl)) return fail("channelizer: no mixed-radix plan");
-    int rc = mix_table(a.pl, s, &a.tw);
+    const MixTable* t = nullptr;
+    int rc = mix_table(C, s, &t);
     if (rc) return rc;
+    a.pl = t->pl;
+    a.CS = t->CS;
+    a.tw = t->tw;
     unsigned threads = 0;
-    mix_shape(a.pl, n_spec, 1, [&](unsigned w) {
+    mix_shape(*t, n_spec, 1, [&](unsigned w) {
         const uint64_t run = S == 1 ? 16 : gcd(S, w);
         return run >= 8 ? 1.0 : run >= 4 ? 0.9 : run >= 2 ? 0.7 : 0.5;
-    }, &a.spw, &threads, &a.CS);
+    }, &a.spw, &threads);
     a.in = reinterpret_cast<const float4*>(in);
     a.out = out;
     a.S = (unsigned)S;
@@ -552,13 +590,15 @@ int mixed_fft(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec,
 int mixed_fft_detect(int C, const float2* in, float* out, uint64_t Sg, int groups, uint64_t n_groups, int out_pols,
                      int flags, hipStream_t s) {
     MixArgs a = {};
-    if (!mix_plan(C, &a.pl)) return fail("channelizer: no mixed-radix plan");
-    int rc = mix_table(a.pl, s, &a.tw);
+    const MixTable* t = nullptr;
+    int rc = mix_table(C, s, &t);
     if (rc) return rc;
+    a.pl = t->pl;
+    a.CS = t->CS;
+    a.tw = t->tw;
     unsigned threads = 0;
     // Whole integrations per workgroup where they fit, otherwise one
     // integration in steps of (about) equal numbers of spectra.
-    a.CS = ((unsigned)C + C / 8 + 1) | 1;
     unsigned most = 1;
     for (unsigned w = 2; w <= 32; w++) {
         bool ok = (size_t)w * a.CS * 16 <= kMixLds / 2;
@@ -568,12 +608,12 @@ int mixed_fft_detect(int C, const float2* in, float* out, uint64_t Sg, int group
     a.steps = (unsigned)ceil_div(Sg, most);
     a.sub = (unsigned)ceil_div(Sg, a.steps);
     if (a.steps > 1) {
-        mix_shape(a.pl, n_groups, a.sub, [&](unsigned w) { return w == a.sub ? 1.0 : 0.0; }, &a.spw, &threads, &a.CS);
+        mix_shape(*t, n_groups, a.sub, [&](unsigned w) { return w == a.sub ? 1.0 : 0.0; }, &a.spw, &threads);
     } else {
-        mix_shape(a.pl, n_groups, a.sub, [&](unsigned w) {
+        mix_shape(*t, n_groups, a.sub, [&](unsigned w) {
             const uint64_t run = groups == 1 ? 64 : out_pols * gcd((uint64_t)groups, w / a.sub);   // floats
             return run >= 16 ? 1.0 : run >= 8 ? 0.9 : run >= 4 ? 0.75 : 0.6;
-        }, &a.spw, &threads, &a.CS);
+        }, &a.spw, &threads);
     }
     a.in = reinterpret_cast<const float4*>(in);
     a.out = out;

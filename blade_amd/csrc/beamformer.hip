@@ -1115,6 +1115,13 @@ static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, h
     const size_t wb = operand_bytes(AR, MW, nsteps_for(AR, a.A));
     if (ar_split(AR) && wb + std::max(kStageBytes, kWaveStageBytes) > kMaxLds)
         return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
+    // CF32 rows off 64-byte sectors: ordinary stores (A28 F192 T8188 B16 267
+    // against 305 us nontemporal, T3004 104 against 116, A42 F384 T1004 B5 64
+    // against 78).  CI8 stays nontemporal, its stores go out in longer runs
+    // (same sizes: 136 against 145, 57 against 60, 22 against 25).
+    if constexpr (AR == AR_F32) {
+        if (epi == EPI_MODEB && a.T % 16) return launch_bf<NT, MW, CI8, AR, D, false, EPI_MODEB>(a, ws, wsb, s);
+    }
     if (epi == EPI_MODEB) return launch_bf<NT, MW, CI8, AR, D, true, EPI_MODEB>(a, ws, wsb, s);
     // The rate-1 epilogues of CF32 input map a wave onto TILE * NT
     // consecutive samples (runs of one): T must not cut a wave.  Nontemporal

@@ -465,7 +465,7 @@ struct MixShape {
 
 // What a rate keeps per device: it depends on the rate alone.  Found anew on
 // each call it cost 5-7 us of host time (6 x 74 channels of one 64-sample
-// spectrum 12.7 us a call, 7.1 us so).
+// spectrum 12.7 us a call, 5.1 us so).
 struct MixTable {
     MixPlan pl;
     unsigned CS;                           // LDS row stride, float4

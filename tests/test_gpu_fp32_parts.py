@@ -162,3 +162,21 @@ def test_sample_counts_no_multiple_of_four(kind, A, F, T, B, inc, polarize):
     assert O.norm_rel_err(y[:B], ref[:B]) <= 2 * (2 * A + 4) * 2.0 ** -24
     if inc:
         assert O.norm_rel_err(y[B], ref[B]) <= 2 * (2 * A + 4) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("kind", ["ci8-f32", "ci8-f16x2", "cf32"])
+@pytest.mark.parametrize("rate,polarize,B,inc", [(4, True, 5, False), (4, True, 16, False), (2, False, 9, True)])
+@pytest.mark.parametrize("T", [4, 8, 12, 260, 264, 268, 272])
+def test_integrated_rows_at_every_alignment(kind, rate, polarize, B, inc, T):
+    """Rows of T / rate samples on and off 64-byte sectors take different
+    stores; normwise, the same bar."""
+    rng = np.random.default_rng(T)
+    A, F = 6, 3
+    x8 = rng.integers(-128, 128, size=(A, F, T, 2, 2), dtype=np.int8)
+    w = (rng.normal(size=(B, A, F, 1, 2)) + 1j * rng.normal(size=(B, A, F, 1, 2))).astype(np.complex64)
+    ref = O.channelizer(O.beamformer_ata(x8, w, inc, False), rate)
+    ref = O.polarizer(ref) if polarize else ref
+    x = torch.from_numpy(x8).cuda() if kind != "cf32" else torch.from_numpy(O.ci8_to_complex(x8).astype(np.complex64)).cuda()
+    got = ops.beamform_chain(x, torch.from_numpy(w).cuda(), inc, False, rate, polarize,
+                             "f16x2" if kind == "ci8-f16x2" else "f32").cpu().numpy()
+    assert got.shape == ref.shape and O.norm_rel_err(got, ref) <= 1e-6

@@ -1007,11 +1007,14 @@ static int groups_for(int B, int mw) { return (B + mw * (TILE / 2) - 1) / (mw * 
 // grid in rounds, and a round takes cpw chunk times, so the estimated time is
 // ceil(workgroups / resident) * cpw chunk times.  The chosen cpw is the
 // largest one within 2% of the best estimate: fewer, longer workgroups pack
-// their phasors fewer times.  Measured at the production shapes: the Mode-B
-// kernels (3 per CU) get one round of 768 workgroups, cpw = 8; the Mode-A
-// kernel (4 per CU) gets three rounds of 1024, cpw = 4 (146 against 150 us
-// with one round of 768).
-static int pick_chunks_per_wg(const void* fn, size_t lds, int n_tchunks, long per_chunk) {
+// their phasors fewer times.  CI8 sample counts that are no multiple of 4 count
+// the packing as `pack` samples of a round besides (A14 F380 T1587 B16, split
+// FP16: 39 us, with one chunk per workgroup 51); elsewhere it hides behind the
+// other workgroups, and counting it cost 4% (Mode A) to 7% (CF32).  At the
+// production shapes the Mode-B kernels (3 per CU) get one round of 768
+// workgroups, cpw = 8; the Mode-A kernel (4 per CU) gets three rounds of 1024,
+// cpw = 4 (146 against 150 us with one round of 768).
+static int pick_chunks_per_wg(const void* fn, size_t lds, int n_tchunks, long per_chunk, long span, long pack) {
     // Occupancy per (kernel, LDS bytes), cached in a fixed table (no heap
     // allocation on the launch path; past 64 entries it is recomputed).
     struct Occ { const void* fn; size_t lds; int occ; };
@@ -1033,7 +1036,7 @@ static int pick_chunks_per_wg(const void* fn, size_t lds, int n_tchunks, long pe
     const int cmax = std::min(n_tchunks, 4096);
     auto est = [&](int c) {
         const long wgs = (long)((n_tchunks + c - 1) / c) * per_chunk;
-        return ((wgs + resident - 1) / resident) * c;
+        return ((wgs + resident - 1) / resident) * (c * span + pack);
     };
     long best_t = est(1);
     for (int c = 2; c <= cmax; c++) best_t = std::min(best_t, est(c));
@@ -1081,7 +1084,8 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
         }
     }
     int cpw = env_int("BLADE_BF_CHUNKS_PER_WG", 0);
-    if (cpw <= 0) cpw = pick_chunks_per_wg(fn, lds, a.n_tchunks, (long)a.F * groups);
+    if (cpw <= 0) cpw = pick_chunks_per_wg(fn, lds, a.n_tchunks, (long)a.F * groups, span,
+                                           ar_split(AR) && a.T % 4 ? 128 : 0);
     cpw = std::min(cpw, a.n_tchunks);
     a.chunks_per_wg = cpw;
     dim3 grid((unsigned)((a.n_tchunks + cpw - 1) / cpw), (unsigned)a.F, (unsigned)groups);
@@ -1098,18 +1102,24 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
 // (the fixed epilogues, staged rows); otherwise ordinary stores let L2 merge the
 // lines before they go out.
 
+// T no multiple of 4, CI8: whether chunks of 256 samples beat chunks of 64 (four
+// samples a lane, or one).  They need beams to amortise the wider tile and a
+// tail that wastes little of the last chunk.  256 against 64 (us, FP32; split
+// FP16): A28 F192 T2047 B8 18.6, 20.9; 22.2, 23.7; B16 26.7, 31.0; 30.9, 33.7;
+// B33 83, 80; 99, 86; B2 27.3, 25.8.  A42 F60 T4097 (6% waste) B16 27.6, 26.3;
+// 35.5, 29.7.  A59 F52 T5433 B33 74, 81; 70, 80.  A20 F64 T511 B8 6.9, 6.7.
+static bool odd_wide(int B, long T) {
+    const bool full = 20 * (long)ceil_div(T, 256) * 256 <= 21 * T;
+    return B > 4 && (B <= 8 ? T >= 768 : full && T >= (B <= 16 ? 768 : 5000));
+}
+
 template <int NT, int MW, bool CI8, int AR, int D>
 static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, hipStream_t s) {
     if (a.T % 4) {
-        // CF32 takes one sample per lane (chunks of 64 instead of 256 samples)
-        // where chunks of 256 are under four per CU: A20 F192 T511 B8 12.6 against
-        // 13.5 us, A12 F90 T931 B19 16.7 against 18.6; past it 256 are faster (A28
-        // F192 T2047 B8 36.8 against 42.2).  CI8 is faster with 256 at all of these.
-        if constexpr (AR == AR_F32) {
-            if ((long)ceil_div(a.T, WAVES * TILE * NT) * a.F * groups_for(a.B, MW) < 4L * device_cus())
-                return launch_bf<1, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
+        if constexpr (ar_split(AR)) {
+            if (odd_wide(a.B, a.T)) return launch_bf<NT, MW, CI8, AR, D, false, EPI_ODD>(a, ws, wsb, s);
         }
-        return launch_bf<NT, MW, CI8, AR, D, false, EPI_ODD>(a, ws, wsb, s);
+        return launch_bf<1, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
     }
     // The largest arrays leave no LDS for staged rows: generic variant.
     const size_t wb = operand_bytes(AR, MW, nsteps_for(AR, a.A));

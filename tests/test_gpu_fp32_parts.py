@@ -147,10 +147,11 @@ def test_stokes_gradient_keeps_nonfinite_values_in_their_beam():
 
 @pytest.mark.parametrize("kind", ["ci8-f32", "ci8-f16x2", "cf32"])
 @pytest.mark.parametrize("A,F,T,B,inc,polarize", [(3, 2, 1, 2, False, False), (5, 2, 65, 9, True, True),
-                                                  (20, 3, 255, 8, True, False), (7, 300, 1021, 17, False, True)])
+                                                  (20, 3, 255, 8, True, False), (7, 300, 1021, 17, False, True),
+                                                  (6, 3, 1023, 6, True, True), (18, 2, 2046, 12, True, False)])
 def test_sample_counts_no_multiple_of_four(kind, A, F, T, B, inc, polarize):
-    """Single samples with a bound each (and CF32's one-sample lanes on small
-    grids); normwise, the FP32 bar of the forward bound above."""
+    """Lanes of one sample, and lanes of four with a bound each; normwise, the
+    FP32 bar of the forward bound above."""
     rng = np.random.default_rng(T)
     x8 = rng.integers(-128, 128, size=(A, F, T, 2, 2), dtype=np.int8)
     w = (rng.normal(size=(B, A, F, 1, 2)) + 1j * rng.normal(size=(B, A, F, 1, 2))).astype(np.complex64)

@@ -476,8 +476,11 @@ __global__ __launch_bounds__(256, (NAT <= 4 ? 4 : NAT <= 6 ? 3 : 2)) void stokes
 //     voltages as 16-byte pieces of memory (they were just read, so from L2),
 //     K = 32 times per instruction.  On 4x4 FP32 blocks as well it took 384
 //     instructions of 8 cycles and 96 LDS reads a tile instead of 24 NAT of 16
-//     and 12, and a call 101 us instead of 76 us (A42 F384 T2048 B4; A28 76
-//     and 50 us).
+//     and 12, and a call 95 us instead of 70 us (A42 F384 T2048 B4; A28 77
+//     and 49 us).  One pol at a time, and with 4 antenna tiles the voltages
+//     after the forward, keep 3 workgroups per CU; A49-64 still spill 72 bytes,
+//     with 2 workgroups none (A64 F384 T1024 B2 56 against 68 us, F128 T2048 B4
+//     47 against 42 us).
 // Each wave takes 64-time tiles; partial sums are added across waves in LDS
 // in wave order and across time splits by adjoint_reduce_kernel, whose
 // partial layout this kernel writes (rows 2 b and 2 b + 1, beam tile 0).
@@ -496,7 +499,7 @@ __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
 }
 
 template <int NAT>
-__global__ __launch_bounds__(256, (NAT <= 3 ? SG4_WGS : 2)) void stokes_grad_b4_kernel(AdjArgs a) {
+__global__ __launch_bounds__(256, SG4_WGS) void stokes_grad_b4_kernel(AdjArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     constexpr int AMAX = 16 * NAT;
     float* const s_w = reinterpret_cast<float*>(lds_raw);            // [A][4][SG4_WS]
@@ -576,8 +579,11 @@ __global__ __launch_bounds__(256, (NAT <= 3 ? SG4_WGS : 2)) void stokes_grad_b4_
     for (int k = wave; k < ntiles; k += ADJ_WAVES) {
         const int t0 = t_begin + k * SG4_TC;
         const int tn = min(SG4_TC, t_end - t0);            // a multiple of 4
+        // In flight during the forward (4 tiles: after it).
+        if constexpr (NAT < 4) {
 #pragma unroll
-        for (int at = 0; at < NAT; at++) load_adj(t0, at);   // in flight during the forward
+            for (int at = 0; at < NAT; at++) load_adj(t0, at);
+        }
         load_fwd(k, 0, xd[0]);
         // ---- forward: this lane feeds time t0 + 4 blk + c (clamped to the
         // split; results for times past it are zeroed below).  The antenna
@@ -607,6 +613,11 @@ __global__ __launch_bounds__(256, (NAT <= 3 ? SG4_WGS : 2)) void stokes_grad_b4_
                     y[p][2] = mfma4(xr + xi, wp[p][2], y[p][2]);
                 }
             }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (NAT == 4) {
+#pragma unroll
+            for (int at = 0; at < NAT; at++) load_adj(t0, at);
         }
         // ---- gy = -lambda y at (time t0 + 4 blk + r, beam c), in parts, into
         // this wave's LDS tile.  Times past the split read clamped voltages:
@@ -648,26 +659,24 @@ __global__ __launch_bounds__(256, (NAT <= 3 ? SG4_WGS : 2)) void stokes_grad_b4_
         // repeat 0 to 7 and are not used.
 #pragma unroll
         for (int h = 0; h < SG4_TC / 32; h++) {
-            uint4 gb[2][3];
 #pragma unroll
-            for (int p = 0; p < 2; p++)
-#pragma unroll
-                for (int m = 0; m < 3; m++)
-                    gb[p][m] = *reinterpret_cast<const uint4*>(gyw + ((p * 3 + m) * 8 + (i & 7)) * SG4_GS + 64 * h + 16 * g);
-#pragma unroll
-            for (int at = 0; at < NAT; at++) {
-                uint4 xo[2][2];
-#pragma unroll
-                for (int p = 0; p < 2; p++)
-#pragma unroll
-                    for (int k2 = 0; k2 < 2; k2++) xo[p][k2] = ci8_times_bf16(xq[at][0], xq[at][1], 2 * p + k2);
-                if (h + 1 < SG4_TC / 32) load_adj(t0 + 32 * (h + 1), at);
+            for (int p = 0; p < 2; p++) {
+                uint4 gb[3];
 #pragma unroll
                 for (int m = 0; m < 3; m++)
+                    gb[m] = *reinterpret_cast<const uint4*>(gyw + ((p * 3 + m) * 8 + (i & 7)) * SG4_GS + 64 * h + 16 * g);
 #pragma unroll
-                    for (int p = 0; p < 2; p++)
+                for (int at = 0; at < NAT; at++) {
+                    uint4 xo[2];
 #pragma unroll
-                        for (int k2 = 0; k2 < 2; k2++) acc[p][at][k2] = mfma_bf16(xo[p][k2], gb[p][m], acc[p][at][k2]);
+                    for (int k2 = 0; k2 < 2; k2++) xo[k2] = ci8_times_bf16(xq[at][0], xq[at][1], 2 * p + k2);
+                    if (p == 1 && h + 1 < SG4_TC / 32) load_adj(t0 + 32 * (h + 1), at);
+#pragma unroll
+                    for (int m = 0; m < 3; m++)
+#pragma unroll
+                        for (int k2 = 0; k2 < 2; k2++) acc[p][at][k2] = mfma_bf16(xo[k2], gb[m], acc[p][at][k2]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     }

@@ -1461,7 +1461,11 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     // interleave: its stores write runs of them ([8,.,4 C,2]: 123 us against
     // 156 us at S = 4, 102 against 108 at S = 2; 512 to 2048 are staged there
     // and 10-30% faster, 8192 106 against 129 us).
-    if (P == 2 && (!use_fft16(C) || (C == 4096 && S > 1)) && T < (1ull << 31) && mixed_fft_covers(rate))
+    // Between 513 and 1535 spectra in all, up to 5 per channel, that kernel's one
+    // to three rounds of workgroups lose up to 6% ([4,64,4 C,2] 44.0 against 41.5
+    // us; 512 spectra 19.4 against 22.3, [16,30,6 C,2] 110 against 166).
+    const bool runs4096 = C == 4096 && S > 1 && (S > 5 || n_spec <= 512 || n_spec >= 1536);
+    if (P == 2 && (!use_fft16(C) || runs4096) && T < (1ull << 31) && mixed_fft_covers(rate))
         return mixed_fft(C, in, out, S, n_spec, s);
     const float2* tw = nullptr;
     int rc = get_twiddles(C, s, &tw);

@@ -103,3 +103,10 @@ def test_integrations_of_a_block(C, A, F, S, N, pols):
         ops.channelizer_detector(x, C, 2 * N, pols, out=y)
         ops.channelizer_detector(x, C, 2 * N, pols, out=y, accumulate=True)
         assert _err(y, 2 * ref) <= 2 * bar
+
+
+@pytest.mark.parametrize("F,S", [(256, 2), (257, 2), (384, 4), (383, 4), (103, 5), (103, 6)])
+def test_4096_by_number_of_spectra(F, S):
+    """Both kernels of the rate, on each side of their bounds."""
+    x = _rand(F + S, 1, F, S * 4096, 2)
+    assert _err(ops.channelizer(x, 4096), _spectra(x, 4096)) <= _bar(4096)

@@ -1060,8 +1060,10 @@ constexpr uint64_t NT_MAX_SPECTRA = 32;    // spectra per workgroup at C = 256, 
 template <int MODE>
 static int launch_fft16(int C, const float2* in, void* out, uint64_t S, uint64_t n_items, int groups, int accumulate,
                         const float2* tw, hipStream_t s, int* rc) {
-    // Lane offsets within a workgroup's spectra are 32-bit.
+    // Lane offsets within a workgroup's spectra are 32-bit, and so are the
+    // detector's from an item's first output (C rows of `groups` integrations).
     if ((uint64_t)(NT_MAX_SPECTRA + 2) * S * (uint64_t)C >= (1ull << 31)) return 0;
+    if (MODE != 0 && (uint64_t)C * (uint64_t)groups * MODE >= (1ull << 32)) return 0;
     switch (C) {
         case 1 << 8: *rc = launch_fft16_lc<8, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
         case 1 << 9: *rc = launch_fft16_lc<9, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;

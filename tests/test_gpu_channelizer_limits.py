@@ -1,0 +1,66 @@
+"""Channelizer and detector at the bounds of their kernels' index types.
+
+Blocks of zeros with a few spectra of noise: every other output must be zero
+(the buffer starts as NaN, so an output that nothing wrote shows too).
+"""
+
+import math
+
+import pytest
+import torch
+
+from blade_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _powers(spec, pols):
+    """FP64 powers of spectra [n, C, 2], fftshifted: [C, n, pols]."""
+    X = torch.fft.fftshift(torch.fft.fft(spec.to(torch.complex128), dim=1), dim=1)
+    a, b = X[..., 0], X[..., 1]
+    if pols == 1:
+        return (a.abs().square() + b.abs().square()).T[..., None]
+    xy = a * b.conj()
+    return torch.stack((a.abs().square(), b.abs().square(), xy.real, xy.imag), -1).transpose(0, 1)
+
+
+def _needs(gib):
+    free, _ = torch.cuda.mem_get_info()
+    if free < gib * 2 ** 30:
+        pytest.skip(f"needs {gib} GiB of device memory")
+
+
+def _sparse_block(C, S, at, seed):
+    """One channel of S spectra, zero but for those numbered `at`."""
+    x = torch.zeros((1, 1, S * C, 2), dtype=torch.complex64, device="cuda")
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    noise = torch.randn((len(at), C, 2), dtype=torch.complex64, device="cuda", generator=gen)
+    for i, s in enumerate(at):
+        x[0, 0, s * C:(s + 1) * C] = noise[i]
+    return x, noise
+
+
+def _check_single_spectra(C, S, pols, at):
+    """Integrations of one spectrum."""
+    x, noise = _sparse_block(C, S, at, 1)
+    out = torch.full((1, C, S, pols), float("nan"), dtype=torch.float32, device="cuda")
+    ops.channelizer_detector(x, C, 1, pols, out=out)
+    del x
+    ref = _powers(noise, pols)
+    got = out[0][:, at].double()
+    err = float((got - ref).norm() / ref.norm())
+    assert err <= (4 * math.log2(max(C, 2)) + 5) * 2.0 ** -24
+    out[0][:, at] = 0
+    for k in range(C):
+        row = out[0, k].view(-1)
+        for i in range(0, row.numel(), 1 << 28):
+            assert not (row[i:i + (1 << 28)] != 0).any(), f"channel {k}"
+    del out
+    torch.cuda.empty_cache()
+
+
+def test_outputs_past_32_bits_of_a_channel():
+    """C * integrations * 4 past 2^32: the last rows' offsets."""
+    C, S = 256, 4_600_000
+    _needs(48)
+    _check_single_spectra(C, S, 4, [0, 1, S // 2, S - 1])

@@ -376,7 +376,7 @@ __global__ __launch_bounds__(1024) void chan_big_pass2(const float2* __restrict_
 template <int NPOL, int KPT>
 __global__ __launch_bounds__(1024) void chan_detect_kernel(const float2* __restrict__ in,
                                                            float* __restrict__ out, int C,
-                                                           int S, int groups, uint64_t n_items,
+                                                           uint64_t S, uint64_t groups, uint64_t n_items,
                                                            const float2* __restrict__ tw,
                                                            Radices rad, int flags) {
     extern __shared__ float2 data[];
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(1024) void chan_detect_kernel(const float2* __restr
         for (int j = 0; j < KPT; j++)
 #pragma unroll
             for (int q = 0; q < NPOL; q++) acc[j][q] = 0.f;
-        for (int s = 0; s < S; s++) {
+        for (uint64_t s = 0; s < S; s++) {
             const float4* src = reinterpret_cast<const float4*>(in + ((item * S + s) * (uint64_t)C) * 2);
             for (int n = threadIdx.x; n < C; n += blockDim.x) {
                 const float4 q = src[n];
@@ -426,8 +426,7 @@ __global__ __launch_bounds__(1024) void chan_detect_kernel(const float2* __restr
             }
             __syncthreads();
             if (s == S - 1) {
-                const uint64_t af = item / (unsigned)groups;
-                const unsigned grp = (unsigned)(item - af * (unsigned)groups);
+                const uint64_t af = item / groups, grp = item - af * groups;
                 if (circular) {
 #pragma unroll
                     for (int j = 0; j < KPT; j++) circular_sums<NPOL>(acc[j]);
@@ -1559,9 +1558,10 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     const int flags = (accumulate ? 1 : 0) | (polarize ? 2 : 0);
     // An item is one integration: Sg spectra in a row of one (antenna, channel)
     // (all S of the block when the integration spans blocks), whose sums stay
-    // in one thread's registers.  Every (antenna, channel) gives `groups`.
+    // in one thread's registers.  Every (antenna, channel) gives `groups`; only
+    // the kernels behind `small` may count them in an int.
     const uint64_t Sg = std::min(integration, S);
-    const int groups = (int)(S / Sg);
+    const uint64_t groups = S / Sg;
     const uint64_t n_items = A * F * groups;
     Radices rad;
     if (!factorize(C, &rad)) return fail("channelizer-detector: rate must factor into 2, 3, 5 and 7");
@@ -1572,16 +1572,16 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     const bool small = n_items < (1ull << 31);      // these kernels count items in 32 bits
     const bool runs = out_pols == 4 && groups > 1 && (C == 2048 || C == 4096);
     if (small && Sg < (1ull << 31) && (!use_fft16(C) || runs) && mixed_fft_covers(rate))
-        return mixed_fft_detect(C, static_cast<const float2*>(input), static_cast<float*>(output), Sg, groups, n_items,
-                                (int)out_pols, flags, s);
+        return mixed_fft_detect(C, static_cast<const float2*>(input), static_cast<float*>(output), Sg, (int)groups,
+                                n_items, (int)out_pols, flags, s);
     const float2* tw = nullptr;
     int rc = get_twiddles(C, s, &tw);
     if (rc) return rc;
     if (small && use_fft16(C)) {
         int rc16 = 0;
         const float2* in16 = static_cast<const float2*>(input);
-        if (out_pols == 1 ? launch_fft16<1>(C, in16, output, Sg, n_items, groups, flags, tw, s, &rc16)
-                          : launch_fft16<4>(C, in16, output, Sg, n_items, groups, flags, tw, s, &rc16))
+        if (out_pols == 1 ? launch_fft16<1>(C, in16, output, Sg, n_items, (int)groups, flags, tw, s, &rc16)
+                          : launch_fft16<4>(C, in16, output, Sg, n_items, (int)groups, flags, tw, s, &rc16))
             return rc16;
     }
     int threads = 64;
@@ -1602,9 +1602,9 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     float* out = static_cast<float*>(output);
     if (out_pols == 1)
         hipLaunchKernelGGL((chan_detect_kernel<1, 8>), dim3((unsigned)blocks), dim3(threads), lds, s, in, out, C,
-                           (int)Sg, groups, n_items, tw, rad, flags);
+                           Sg, groups, n_items, tw, rad, flags);
     else
         hipLaunchKernelGGL((chan_detect_kernel<4, 8>), dim3((unsigned)blocks), dim3(threads), lds, s, in, out, C,
-                           (int)Sg, groups, n_items, tw, rad, flags);
+                           Sg, groups, n_items, tw, rad, flags);
     return check_launch("channelizer-detector");
 }

@@ -64,3 +64,10 @@ def test_outputs_past_32_bits_of_a_channel():
     C, S = 256, 4_600_000
     _needs(48)
     _check_single_spectra(C, S, 4, [0, 1, S // 2, S - 1])
+
+
+def test_integrations_past_31_bits():
+    """More than 2^31 integrations of one channel."""
+    S = 2 ** 31 + 8
+    _needs(64)
+    _check_single_spectra(1, S, 1, [0, 1, 2 ** 31 - 1, 2 ** 31, S - 1])

@@ -50,7 +50,7 @@ static std::mutex g_tw_mutex;
 static std::map<std::pair<int, int>, float2*> g_tw;
 
 // The table of rate C, or with N2 > 0 the matrix of C = N1 N2.
-static int get_twiddles(int C, hipStream_t s, const float2** out, int N2 = 0) {
+static int get_twiddles(int C, const float2** out, int N2 = 0) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fail("channelizer: hipGetDevice failed");
     std::lock_guard<std::mutex> lock(g_tw_mutex);
@@ -60,20 +60,16 @@ static int get_twiddles(int C, hipStream_t s, const float2** out, int N2 = 0) {
         *out = it->second;
         return BLADE_SUCCESS;
     }
-    float2* p = nullptr;
-    hipError_t e = hipMalloc(&p, sizeof(float2) * C + kTwiddleSinkBytes);
-    if (e != hipSuccess) {
-        set_error(std::string("channelizer: twiddle allocation: ") + hipGetErrorString(e));
-        return BLADE_HIP_ERROR;
-    }
-    if (N2 > 0)
-        hipLaunchKernelGGL(twiddle_matrix_kernel, dim3((C + 255) / 256), dim3(256), 0, s, p, C, N2);
-    else
-        hipLaunchKernelGGL(twiddle_kernel, dim3((C + 255) / 256), dim3(256), 0, s, p, C);
-    int rc = check_launch("channelizer twiddles");
+    void* p = nullptr;
+    const int rc = device_table("channelizer twiddles", sizeof(float2) * C + kTwiddleSinkBytes, &p,
+                                [&](void* t, hipStream_t ts) {
+        if (N2 > 0)
+            hipLaunchKernelGGL(twiddle_matrix_kernel, dim3((C + 255) / 256), dim3(256), 0, ts, static_cast<float2*>(t), C, N2);
+        else
+            hipLaunchKernelGGL(twiddle_kernel, dim3((C + 255) / 256), dim3(256), 0, ts, static_cast<float2*>(t), C);
+    });
     if (rc) return rc;
-    g_tw[key] = p;
-    *out = p;
+    *out = g_tw[key] = static_cast<float2*>(p);
     return BLADE_SUCCESS;
 }
 
@@ -1225,9 +1221,9 @@ static int launch_four_step(int C, const float2* in, float2* out, uint64_t S, ui
     four_step_lengths(C, &ln1, &ln2);
     int N1 = 1 << ln1, N2 = 1 << ln2;
     const float2 *twm = nullptr, *tw1 = nullptr, *tw2 = nullptr;
-    int rc = get_twiddles(C, s, &twm, N2);
-    if (!rc) rc = get_twiddles(N1, s, &tw1);
-    if (!rc) rc = get_twiddles(N2, s, &tw2);
+    int rc = get_twiddles(C, &twm, N2);
+    if (!rc) rc = get_twiddles(N1, &tw1);
+    if (!rc) rc = get_twiddles(N2, &tw2);
     if (rc) return rc;
     // Spectra per group.  In place, a group's output must not reach input that
     // is still to be read: whole (antenna, channel)s when input and output are
@@ -1354,9 +1350,9 @@ template <int P>
 static int launch_big(const BigPlan& pl, int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec,
                       hipStream_t s) {
     const float2 *twC = nullptr, *tw1 = nullptr, *tw2 = nullptr;
-    int rc = get_twiddles(C, s, &twC);
-    if (!rc) rc = get_twiddles(pl.N1, s, &tw1);
-    if (!rc) rc = get_twiddles(pl.N2, s, &tw2);
+    int rc = get_twiddles(C, &twC);
+    if (!rc) rc = get_twiddles(pl.N1, &tw1);
+    if (!rc) rc = get_twiddles(pl.N2, &tw2);
     if (rc) return rc;
     unsigned char* scratch = nullptr;
     rc = library_workspace(WS_CHANNELIZER_BIG, sizeof(float2) * (size_t)n_spec * C * P, s, &scratch);
@@ -1469,7 +1465,7 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     if (P == 2 && (!use_fft16(C) || runs4096) && T < (1ull << 31) && mixed_fft_covers(rate))
         return mixed_fft(C, in, out, S, n_spec, s);
     const float2* tw = nullptr;
-    int rc = get_twiddles(C, s, &tw);
+    int rc = get_twiddles(C, &tw);
     if (rc) return rc;
     if (P == 2 && use_fft16(C)) {
         int rc16 = 0;
@@ -1515,24 +1511,24 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
 extern "C" int blade_channelizer_plan(uint64_t rate, blade_stream_t stream) {
     if (rate == 0 || (rate % 2 && rate != 1)) return fail("channelizer: invalid rate");
     if (rate > (uint64_t)kMaxBigRate) return fail("channelizer: rate above 2^20 is not supported");
+    (void)stream;                           // the tables are filled on a stream of their own
     if (rate <= 16) return BLADE_SUCCESS;   // register kernels carry their twiddles as arguments
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const float2* tw = nullptr;
-    int rc = get_twiddles((int)rate, s, &tw);
-    if (!rc && mixed_fft_covers(rate)) rc = mixed_fft_plan((int)rate, s);
+    int rc = get_twiddles((int)rate, &tw);
+    if (!rc && mixed_fft_covers(rate)) rc = mixed_fft_plan((int)rate);
     if (rc) return rc;
     if (use_four_step((int)rate, 2)) {
         int ln1, ln2;
         four_step_lengths((int)rate, &ln1, &ln2);
-        rc = get_twiddles((int)rate, s, &tw, 1 << ln2);
-        if (!rc) rc = get_twiddles(1 << ln1, s, &tw);
-        if (!rc) rc = get_twiddles(1 << ln2, s, &tw);
+        rc = get_twiddles((int)rate, &tw, 1 << ln2);
+        if (!rc) rc = get_twiddles(1 << ln1, &tw);
+        if (!rc) rc = get_twiddles(1 << ln2, &tw);
         if (rc) return rc;
     }
     BigPlan pl;   // the two-pass FFT's tables (for two polarizations)
     if (rate * 2 > (uint64_t)kMaxLdsComplex && big_plan((int)rate, 2, &pl)) {
-        rc = get_twiddles(pl.N1, s, &tw);
-        if (!rc) rc = get_twiddles(pl.N2, s, &tw);
+        rc = get_twiddles(pl.N1, &tw);
+        if (!rc) rc = get_twiddles(pl.N2, &tw);
     }
     return rc;
 }
@@ -1575,7 +1571,7 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
         return mixed_fft_detect(C, static_cast<const float2*>(input), static_cast<float*>(output), Sg, (int)groups,
                                 n_items, (int)out_pols, flags, s);
     const float2* tw = nullptr;
-    int rc = get_twiddles(C, s, &tw);
+    int rc = get_twiddles(C, &tw);
     if (rc) return rc;
     if (small && use_fft16(C)) {
         int rc16 = 0;

@@ -58,6 +58,33 @@ inline int device_cus() {
 enum WorkspaceUser { WS_BEAMFORMER_SINK = 0, WS_ADJOINT = 1, WS_CHANNELIZER_BIG = 2 };
 int library_workspace(int user, size_t bytes, hipStream_t s, unsigned char** out);
 
+// A library-owned table of the current device, whole when this returns: `fill`
+// queues its kernels on a stream of their own, which is waited for.  Filled on
+// the caller's stream it would be ready there only, while calls on other
+// streams find the same pointer; and a stream under capture would record the
+// fill instead of running it.  Once per table, so the wait costs nothing later.
+template <typename Fill>
+int device_table(const char* what, size_t bytes, void** out, Fill fill) {
+    void* p = nullptr;
+    hipStream_t s = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    if (e == hipSuccess) {
+        fill(p, s);
+        e = hipGetLastError();
+        const hipError_t w = hipStreamSynchronize(s);
+        if (e == hipSuccess) e = w;
+        (void)hipStreamDestroy(s);
+    }
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        set_error(std::string(what) + ": " + hipGetErrorString(e));
+        return BLADE_HIP_ERROR;
+    }
+    *out = p;
+    return BLADE_SUCCESS;
+}
+
 // Number of scalar components and bytes per element of a blade_type.
 inline int type_components(int t) {
     switch (t) {

@@ -10,7 +10,7 @@ bool mixed_fft_covers(uint64_t rate);
 
 // Build the rate's twiddle table (once per device), so that later launches
 // allocate nothing.
-int mixed_fft_plan(int C, hipStream_t s);
+int mixed_fft_plan(int C);
 
 // CF32 [n_spec spectra of C samples][2] -> [n_spec / S, C, S, 2], fftshifted.
 int mixed_fft(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec, hipStream_t s);

@@ -503,7 +503,7 @@ static std::vector<MixShape> mix_shapes(const MixPlan& pl, unsigned CS) {
 static std::mutex g_mix_mutex;
 static std::map<std::pair<int, int>, std::unique_ptr<MixTable>> g_mix_tables;
 
-static int mix_table(int C, hipStream_t s, const MixTable** out) {
+static int mix_table(int C, const MixTable** out) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fail("channelizer: hipGetDevice failed");
     std::lock_guard<std::mutex> lock(g_mix_mutex);
@@ -513,23 +513,22 @@ static int mix_table(int C, hipStream_t s, const MixTable** out) {
         if (!mix_plan(C, &t->pl)) return fail("channelizer: no mixed-radix plan");
         t->CS = ((unsigned)C + C / 8 + 1) | 1;
         t->shapes = mix_shapes(t->pl, t->CS);
-        hipError_t e = hipMalloc(&t->tw, sizeof(float2) * (size_t)C);   // sum of (R - 1) Ns = C - R_0
-        if (e != hipSuccess) {
-            set_error(std::string("channelizer: twiddle allocation: ") + hipGetErrorString(e));
-            return BLADE_HIP_ERROR;
-        }
-        hipLaunchKernelGGL(mixed_twiddle_kernel, dim3(8), dim3(256), 0, s, t->tw, t->pl);
-        int rc = check_launch("channelizer twiddles");
+        void* p = nullptr;                            // sum of (R - 1) Ns = C - R_0 entries
+        const int rc = device_table("channelizer twiddles", sizeof(float2) * (size_t)C, &p,
+                                    [&](void* tw, hipStream_t ts) {
+            hipLaunchKernelGGL(mixed_twiddle_kernel, dim3(8), dim3(256), 0, ts, static_cast<float2*>(tw), t->pl);
+        });
         if (rc) return rc;
+        t->tw = static_cast<float2*>(p);
         slot = std::move(t);
     }
     *out = slot.get();
     return BLADE_SUCCESS;
 }
 
-int mixed_fft_plan(int C, hipStream_t s) {
+int mixed_fft_plan(int C) {
     const MixTable* t = nullptr;
-    return mix_table(C, s, &t);
+    return mix_table(C, &t);
 }
 
 // Spectra per workgroup (a multiple of `unit`) and threads: the rate's shapes
@@ -566,7 +565,7 @@ static int mix_launch(MixArgs& a, uint64_t blocks, unsigned threads, hipStream_t
 int mixed_fft(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec, hipStream_t s) {
     MixArgs a = {};
     const MixTable* t = nullptr;
-    int rc = mix_table(C, s, &t);
+    int rc = mix_table(C, &t);
     if (rc) return rc;
     a.pl = t->pl;
     a.CS = t->CS;
@@ -591,7 +590,7 @@ int mixed_fft_detect(int C, const float2* in, float* out, uint64_t Sg, int group
                      int flags, hipStream_t s) {
     MixArgs a = {};
     const MixTable* t = nullptr;
-    int rc = mix_table(C, s, &t);
+    int rc = mix_table(C, &t);
     if (rc) return rc;
     a.pl = t->pl;
     a.CS = t->CS;

@@ -261,8 +261,9 @@ int blade_channelizer(const void* input, void* output, uint64_t A, uint64_t F, u
                       uint64_t P, uint64_t rate, blade_stream_t stream);
 
 /*
- * Build (once per device and rate) the twiddle table blade_channelizer uses,
- * so that later calls allocate nothing (e.g. inside hipGraph capture).
+ * Build (once per device and rate) the twiddle tables blade_channelizer uses,
+ * so that later calls allocate nothing (e.g. inside hipGraph capture).  They
+ * are ready on every stream when this returns; `stream` is not used.
  * Replaces the cuFFT plan creation of the Channelizer constructor
  * (src/modules/channelizer/base.cc:58-93).
  */

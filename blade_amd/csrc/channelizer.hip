@@ -1512,7 +1512,8 @@ extern "C" int blade_channelizer_plan(uint64_t rate, blade_stream_t stream) {
     if (rate == 0 || (rate % 2 && rate != 1)) return fail("channelizer: invalid rate");
     if (rate > (uint64_t)kMaxBigRate) return fail("channelizer: rate above 2^20 is not supported");
     (void)stream;                           // the tables are filled on a stream of their own
-    if (rate <= 16) return BLADE_SUCCESS;   // register kernels carry their twiddles as arguments
+    // Rates up to 16 too: only the channelizer's register kernels (out of place)
+    // carry their twiddles as arguments.
     const float2* tw = nullptr;
     int rc = get_twiddles((int)rate, &tw);
     if (!rc && mixed_fft_covers(rate)) rc = mixed_fft_plan((int)rate);

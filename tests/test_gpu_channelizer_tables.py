@@ -69,8 +69,32 @@ for C, P in ((1000, 2), (512, 2), (1000, 1)):
         check(C, yg, ref, "replay")
 """
 
+# After a plan, the first call of a small rate may be captured (nothing is
+# allocated): the detector, and in place (rate == number of samples).
+PLANNED = """
+from blade_amd import _lib
+for C in (1, 2, 4, 6, 14, 16, 32):
+    _lib.call("blade_channelizer_plan", C, None)
+    x, ref, _ = block(C, 2)
+    z, zref, _ = block(C, 2, S=1)
+    y = torch.zeros((2, 5 * C, 3, 1), device="cuda")
+    zin = z.clone()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ops.channelizer_detector(x, C, 1, 1, out=y)
+        ops.channelizer(z, C, out=z)
+    for _ in range(3):
+        y.zero_()
+        z.copy_(zin)
+        g.replay()
+        torch.cuda.synchronize()
+        check(max(C, 2) ** 2, y, power(ref), "detector")
+        check(max(C, 2), z.view(zref.shape), zref, "in place")
+"""
 
-@pytest.mark.parametrize("script", [TWO_STREAMS, IN_CAPTURE], ids=["two_streams", "in_capture"])
+
+@pytest.mark.parametrize("script", [TWO_STREAMS, IN_CAPTURE, PLANNED], ids=["two_streams", "in_capture", "planned"])
 def test_first_use(script):
     r = subprocess.run([sys.executable, "-u", "-c", PRELUDE + script], cwd=ROOT, stdout=subprocess.PIPE,
                        stderr=subprocess.STDOUT, text=True, timeout=110)

@@ -49,8 +49,9 @@ __global__ void twiddle_matrix_kernel(float2* tw, int C, int N2) {
 static std::mutex g_tw_mutex;
 static std::map<std::pair<int, int>, float2*> g_tw;
 
-// The table of rate C, or with N2 > 0 the matrix of C = N1 N2.
-static int get_twiddles(int C, const float2** out, int N2 = 0) {
+// The table of rate C, or with N2 > 0 the matrix of C = N1 N2.  `made` is set
+// when this call built it.
+static int get_twiddles(int C, const float2** out, int N2 = 0, bool* made = nullptr) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fail("channelizer: hipGetDevice failed");
     std::lock_guard<std::mutex> lock(g_tw_mutex);
@@ -70,7 +71,17 @@ static int get_twiddles(int C, const float2** out, int N2 = 0) {
     });
     if (rc) return rc;
     *out = g_tw[key] = static_cast<float2*>(p);
+    if (made) *made = true;
     return BLADE_SUCCESS;
+}
+
+// The table of rate C, and with it on first use the mixed-radix kernel's: which
+// of them a call reads depends on its shape, and a call at any shape prepares
+// its rate for captures at every other.
+static int rate_twiddles(int C, const float2** out) {
+    bool made = false;
+    const int rc = get_twiddles(C, out, 0, &made);
+    return !rc && made && mixed_fft_covers((uint64_t)C) ? mixed_fft_plan(C) : rc;
 }
 
 // ---------------------------------------------------------------------------
@@ -1437,10 +1448,14 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     }
     const float2* in = static_cast<const float2*>(input);
     float2* out = static_cast<float2*>(output);
+    const float2* tw = nullptr;
     if ((uint64_t)C * P > (uint64_t)kMaxLdsComplex) {
         // Past one workgroup's LDS: two passes through a scratch buffer (which
         // also makes any in-place call safe).
-        if (use_four_step(C, (int)P)) return launch_four_step(C, in, out, S, n_spec, s);
+        if (use_four_step(C, (int)P)) {
+            const int rc = rate_twiddles(C, &tw);     // one polarization's, at 2^14
+            return rc ? rc : launch_four_step(C, in, out, S, n_spec, s);
+        }
         BigPlan pl;
         if (!big_plan(C, (int)P, &pl))
             return fail("channelizer: rate must be even, at most 2^20, and factor into 2, 3, 5 and 7");
@@ -1453,6 +1468,8 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
                                 : dispatch_small<1>(C, in, out, n_spec, S, s);
         if (ok) return check_launch("channelizer");
     }
+    int rc = rate_twiddles(C, &tw);
+    if (rc) return rc;
     // Mixed-radix kernel: every rate made of 2, 3, 5 and 7 but the powers of two
     // of the radix-16 kernel, and of these C = 4096 where several spectra
     // interleave: its stores write runs of them ([8,.,4 C,2]: 123 us against
@@ -1464,9 +1481,6 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     const bool runs4096 = C == 4096 && S > 1 && (S > 5 || n_spec <= 512 || n_spec >= 1536);
     if (P == 2 && (!use_fft16(C) || runs4096) && T < (1ull << 31) && mixed_fft_covers(rate))
         return mixed_fft(C, in, out, S, n_spec, s);
-    const float2* tw = nullptr;
-    int rc = get_twiddles(C, &tw);
-    if (rc) return rc;
     if (P == 2 && use_fft16(C)) {
         int rc16 = 0;
         if (launch_fft16<0>(C, in, out, S, n_spec, 1, 0, tw, s, &rc16)) return rc16;
@@ -1515,8 +1529,7 @@ extern "C" int blade_channelizer_plan(uint64_t rate, blade_stream_t stream) {
     // Rates up to 16 too: only the channelizer's register kernels (out of place)
     // carry their twiddles as arguments.
     const float2* tw = nullptr;
-    int rc = get_twiddles((int)rate, &tw);
-    if (!rc && mixed_fft_covers(rate)) rc = mixed_fft_plan((int)rate);
+    int rc = rate_twiddles((int)rate, &tw);
     if (rc) return rc;
     if (use_four_step((int)rate, 2)) {
         int ln1, ln2;
@@ -1562,6 +1575,9 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     const uint64_t n_items = A * F * groups;
     Radices rad;
     if (!factorize(C, &rad)) return fail("channelizer-detector: rate must factor into 2, 3, 5 and 7");
+    const float2* tw = nullptr;
+    int rc = rate_twiddles(C, &tw);
+    if (rc) return rc;
     // Mixed-radix kernel: as for the channelizer, and full Stokes at 2048 and
     // 4096 with several integrations per channel, whose 16-byte outputs it writes
     // in runs (one spectrum each: 117 against 151 and 136 against 190 us for
@@ -1571,9 +1587,6 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     if (small && Sg < (1ull << 31) && (!use_fft16(C) || runs) && mixed_fft_covers(rate))
         return mixed_fft_detect(C, static_cast<const float2*>(input), static_cast<float*>(output), Sg, (int)groups,
                                 n_items, (int)out_pols, flags, s);
-    const float2* tw = nullptr;
-    int rc = get_twiddles(C, &tw);
-    if (rc) return rc;
     if (small && use_fft16(C)) {
         int rc16 = 0;
         const float2* in16 = static_cast<const float2*>(input);

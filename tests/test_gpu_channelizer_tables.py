@@ -93,8 +93,36 @@ for C in (1, 2, 4, 6, 14, 16, 32):
         check(max(C, 2), z.view(zref.shape), zref, "in place")
 """
 
+# An eager call at one shape warms its rate for every other shape, number of
+# polarizations and the detector, whichever kernels these take.
+WARMED = """
+def captured(run, y, ref, C, what):
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        run()
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        check(C, y, ref, what)
+for C, P, S in ((4096, 2, 1), (2048, 2, 3), (1000, 1, 3), (1024, 2, 2), (64, 1, 2), (16384, 2, 1)):
+    x, ref, (y, _) = block(C, P, S)
+    ops.channelizer(x, C, out=y)
+    check(C, y, ref, "warm")
+    for P, S in ((1, 3), (2, 8)) if C < 16384 else ((1, 3),):
+        x, ref, (y, _) = block(C, P, S)
+        captured(lambda: ops.channelizer(x, C, out=y), y, ref, C, f"P {P} S {S}")
+    if C <= 8192:
+        ab = ref[..., 0] * ref[..., 1].conj()
+        four = torch.stack((ref[..., 0].abs() ** 2, ref[..., 1].abs() ** 2, ab.real, ab.imag), -1)
+        d = torch.zeros(four.shape, device="cuda")
+        captured(lambda: ops.channelizer_detector(x, C, 1, 4, out=d), d, four, C * C, "detector")
+"""
 
-@pytest.mark.parametrize("script", [TWO_STREAMS, IN_CAPTURE, PLANNED], ids=["two_streams", "in_capture", "planned"])
+
+@pytest.mark.parametrize("script", [TWO_STREAMS, IN_CAPTURE, PLANNED, WARMED],
+                         ids=["two_streams", "in_capture", "planned", "warmed"])
 def test_first_use(script):
     r = subprocess.run([sys.executable, "-u", "-c", PRELUDE + script], cwd=ROOT, stdout=subprocess.PIPE,
                        stderr=subprocess.STDOUT, text=True, timeout=110)

@@ -1584,9 +1584,10 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     // 200 MB; Stokes I 95 against 82 and 109 against 71 us the other way).
     const bool small = n_items < (1ull << 31);      // these kernels count items in 32 bits
     const bool runs = out_pols == 4 && groups > 1 && (C == 2048 || C == 4096);
-    if (small && Sg < (1ull << 31) && (!use_fft16(C) || runs) && mixed_fft_covers(rate))
-        return mixed_fft_detect(C, static_cast<const float2*>(input), static_cast<float*>(output), Sg, (int)groups,
-                                n_items, (int)out_pols, flags, s);
+    if (small && Sg < (1ull << 31) && (!use_fft16(C) || runs) && mixed_fft_covers(rate) &&
+        mixed_fft_detect(C, static_cast<const float2*>(input), static_cast<float*>(output), Sg, (int)groups, n_items,
+                         (int)out_pols, flags, s, &rc))
+        return rc;
     if (small && use_fft16(C)) {
         int rc16 = 0;
         const float2* in16 = static_cast<const float2*>(input);

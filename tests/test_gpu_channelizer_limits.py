@@ -71,3 +71,20 @@ def test_integrations_past_31_bits():
     S = 2 ** 31 + 8
     _needs(64)
     _check_single_spectra(1, S, 1, [0, 1, 2 ** 31 - 1, 2 ** 31, S - 1])
+
+
+@pytest.mark.parametrize("C", [1, 4, 64, 96, 256, 1000, 4096, 4374, 4802, 8100, 8192])
+@pytest.mark.parametrize("S", [3, 70])
+@pytest.mark.parametrize("pols", [1, 4])
+def test_adding_a_block_rounds_once(C, S, pols):
+    """An integration over several blocks: each call adds its block's sums in one
+    FP32 addition.  On outputs 2^20 times the block's, adding them in parts
+    rounds by many times more than half a unit in the last place."""
+    gen = torch.Generator(device="cuda").manual_seed(C + S)
+    x = torch.randn((1, 5, S * C, 2), dtype=torch.complex64, device="cuda", generator=gen)
+    y = ops.channelizer_detector(x, C, S, pols)
+    start = 2.0 ** (20 + round(math.log2(4 * C * S)))
+    out = torch.full_like(y, start)
+    ops.channelizer_detector(x, C, 3 * S, pols, out=out, accumulate=True)
+    err = float((out.double() - (start + y.double())).abs().max())
+    assert err <= start * 2.0 ** -24 * (1 + 2.0 ** -10)

@@ -1060,25 +1060,27 @@ static int launch_fft16_lc(const float2* in, void* out, uint64_t S, uint64_t n_i
         return launch_fft16_t<LC, 512, MODE, 0>(in, out, S, n_items, groups, accumulate, tw, s);
 }
 
-constexpr uint64_t NT_MAX_SPECTRA = 32;    // spectra per workgroup at C = 256, 512 threads
+// Whether a detector call keeps to fft16_kernel's 32-bit offsets: a lane's
+// within its workgroup's items (up to 8192 / C, of S spectra each), and from an item's first output
+// (C rows of `groups` integrations).  Spectra have none: items are single
+// spectra, outputs are indexed in 64 bits.
+static bool fft16_fits(int C, uint64_t S, uint64_t groups, uint64_t out_pols) {
+    return (8192 / C + 2) * S * (uint64_t)C < (1ull << 31) && (uint64_t)C * groups * out_pols < (1ull << 32);
+}
 
-// Returns 1 and launches when fft16_kernel covers C, else 0.
+// Launches fft16_kernel for a rate that use_fft16 admits.
 template <int MODE>
 static int launch_fft16(int C, const float2* in, void* out, uint64_t S, uint64_t n_items, int groups, int accumulate,
-                        const float2* tw, hipStream_t s, int* rc) {
-    // Lane offsets within a workgroup's spectra are 32-bit, and so are the
-    // detector's from an item's first output (C rows of `groups` integrations).
-    if ((uint64_t)(NT_MAX_SPECTRA + 2) * S * (uint64_t)C >= (1ull << 31)) return 0;
-    if (MODE != 0 && (uint64_t)C * (uint64_t)groups * MODE >= (1ull << 32)) return 0;
+                        const float2* tw, hipStream_t s) {
     switch (C) {
-        case 1 << 8: *rc = launch_fft16_lc<8, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
-        case 1 << 9: *rc = launch_fft16_lc<9, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
-        case 1 << 10: *rc = launch_fft16_lc<10, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
-        case 1 << 11: *rc = launch_fft16_lc<11, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
-        case 1 << 12: *rc = launch_fft16_lc<12, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
-        case 1 << 13: *rc = launch_fft16_lc<13, MODE>(in, out, S, n_items, groups, accumulate, tw, s); return 1;
+        case 1 << 8: return launch_fft16_lc<8, MODE>(in, out, S, n_items, groups, accumulate, tw, s);
+        case 1 << 9: return launch_fft16_lc<9, MODE>(in, out, S, n_items, groups, accumulate, tw, s);
+        case 1 << 10: return launch_fft16_lc<10, MODE>(in, out, S, n_items, groups, accumulate, tw, s);
+        case 1 << 11: return launch_fft16_lc<11, MODE>(in, out, S, n_items, groups, accumulate, tw, s);
+        case 1 << 12: return launch_fft16_lc<12, MODE>(in, out, S, n_items, groups, accumulate, tw, s);
+        case 1 << 13: return launch_fft16_lc<13, MODE>(in, out, S, n_items, groups, accumulate, tw, s);
     }
-    return 0;
+    return fail("channelizer: no radix-16 kernel for this rate");
 }
 
 // ---------------------------------------------------------------------------
@@ -1481,10 +1483,7 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     const bool runs4096 = C == 4096 && S > 1 && (S > 5 || n_spec <= 512 || n_spec >= 1536);
     if (P == 2 && (!use_fft16(C) || runs4096) && T < (1ull << 31) && mixed_fft_covers(rate))
         return mixed_fft(C, in, out, S, n_spec, s);
-    if (P == 2 && use_fft16(C)) {
-        int rc16 = 0;
-        if (launch_fft16<0>(C, in, out, S, n_spec, 1, 0, tw, s, &rc16)) return rc16;
-    }
+    if (P == 2 && use_fft16(C)) return launch_fft16<0>(C, in, out, S, n_spec, 1, 0, tw, s);
     Radices rad;
     const size_t lds = sizeof(float2) * (size_t)C * P;
     uint64_t blocks = n_spec;
@@ -1584,17 +1583,14 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     // 200 MB; Stokes I 95 against 82 and 109 against 71 us the other way).
     const bool small = n_items < (1ull << 31);      // these kernels count items in 32 bits
     const bool runs = out_pols == 4 && groups > 1 && (C == 2048 || C == 4096);
-    if (small && Sg < (1ull << 31) && (!use_fft16(C) || runs) && mixed_fft_covers(rate) &&
+    const bool fft16 = small && use_fft16(C) && fft16_fits(C, Sg, groups, out_pols);
+    if (small && Sg < (1ull << 31) && (!fft16 || runs) && mixed_fft_covers(rate) &&
         mixed_fft_detect(C, static_cast<const float2*>(input), static_cast<float*>(output), Sg, (int)groups, n_items,
                          (int)out_pols, flags, s, &rc))
         return rc;
-    if (small && use_fft16(C)) {
-        int rc16 = 0;
-        const float2* in16 = static_cast<const float2*>(input);
-        if (out_pols == 1 ? launch_fft16<1>(C, in16, output, Sg, n_items, (int)groups, flags, tw, s, &rc16)
-                          : launch_fft16<4>(C, in16, output, Sg, n_items, (int)groups, flags, tw, s, &rc16))
-            return rc16;
-    }
+    if (fft16)
+        return out_pols == 1 ? launch_fft16<1>(C, static_cast<const float2*>(input), output, Sg, n_items, (int)groups, flags, tw, s)
+                             : launch_fft16<4>(C, static_cast<const float2*>(input), output, Sg, n_items, (int)groups, flags, tw, s);
     int threads = 64;
     while (threads < 1024 && threads * 8 < 2 * C) threads *= 2;
     const size_t lds = sizeof(float2) * 2 * (size_t)C;

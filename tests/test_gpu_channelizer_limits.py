@@ -88,3 +88,22 @@ def test_adding_a_block_rounds_once(C, S, pols):
     ops.channelizer_detector(x, C, 3 * S, pols, out=out, accumulate=True)
     err = float((out.double() - (start + y.double())).abs().max())
     assert err <= start * 2.0 ** -24 * (1 + 2.0 ** -10)
+
+
+@pytest.mark.parametrize("C", [64, 256, 2048, 4096, 8192])
+def test_channels_past_63_million_samples(C):
+    """Spectra of one long channel, and their powers in integrations of one."""
+    S = 2 ** 26 // C + 16
+    _needs(8)
+    at = [0, 7, S // 2, S - 1]
+    x, noise = _sparse_block(C, S, at, C)
+    y = torch.full((1, C, S, 2), complex("nan"), dtype=torch.complex64, device="cuda")
+    ops.channelizer(x, C, out=y)
+    X = torch.fft.fftshift(torch.fft.fft(noise.to(torch.complex128), dim=1), dim=1).transpose(0, 1)
+    err = float((y[0][:, at] - X).norm() / X.norm())
+    assert err <= 2 * math.log2(C) * 2.0 ** -24
+    y[0][:, at] = 0
+    assert not (y != 0).any()
+    del x, y
+    for pols in (1, 4):
+        _check_single_spectra(C, S, pols, at)

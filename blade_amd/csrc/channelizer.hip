@@ -77,7 +77,8 @@ static int get_twiddles(int C, const float2** out, int N2 = 0, bool* made = null
 
 // The table of rate C, and with it on first use the mixed-radix kernel's: which
 // of them a call reads depends on its shape, and a call at any shape prepares
-// its rate for captures at every other.
+// its rate for captures at every other.  Calls of the mixed-radix kernel build
+// this one beside theirs (one lookup per call: 0.2 us of 7).
 static int rate_twiddles(int C, const float2** out) {
     bool made = false;
     const int rc = get_twiddles(C, out, 0, &made);
@@ -1470,8 +1471,8 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
                                 : dispatch_small<1>(C, in, out, n_spec, S, s);
         if (ok) return check_launch("channelizer");
     }
-    int rc = rate_twiddles(C, &tw);
-    if (rc) return rc;
+    int rc = BLADE_SUCCESS;
+    bool made = false;
     // Mixed-radix kernel: every rate made of 2, 3, 5 and 7 but the powers of two
     // of the radix-16 kernel, and of these C = 4096 where several spectra
     // interleave: its stores write runs of them ([8,.,4 C,2]: 123 us against
@@ -1481,8 +1482,12 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     // to three rounds of workgroups lose up to 6% ([4,64,4 C,2] 44.0 against 41.5
     // us; 512 spectra 19.4 against 22.3, [16,30,6 C,2] 110 against 166).
     const bool runs4096 = C == 4096 && S > 1 && (S > 5 || n_spec <= 512 || n_spec >= 1536);
-    if (P == 2 && (!use_fft16(C) || runs4096) && T < (1ull << 31) && mixed_fft_covers(rate))
-        return mixed_fft(C, in, out, S, n_spec, s);
+    if (P == 2 && (!use_fft16(C) || runs4096) && T < (1ull << 31) && mixed_fft_covers(rate)) {
+        rc = mixed_fft(C, in, out, S, n_spec, s, &made);
+        return !rc && made ? get_twiddles(C, &tw) : rc;
+    }
+    rc = rate_twiddles(C, &tw);
+    if (rc) return rc;
     if (P == 2 && use_fft16(C)) return launch_fft16<0>(C, in, out, S, n_spec, 1, 0, tw, s);
     Radices rad;
     const size_t lds = sizeof(float2) * (size_t)C * P;
@@ -1575,8 +1580,8 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     Radices rad;
     if (!factorize(C, &rad)) return fail("channelizer-detector: rate must factor into 2, 3, 5 and 7");
     const float2* tw = nullptr;
-    int rc = rate_twiddles(C, &tw);
-    if (rc) return rc;
+    int rc = BLADE_SUCCESS;
+    bool made = false;
     // Mixed-radix kernel: as for the channelizer, and full Stokes at 2048 and
     // 4096 with several integrations per channel, whose 16-byte outputs it writes
     // in runs (one spectrum each: 117 against 151 and 136 against 190 us for
@@ -1586,8 +1591,10 @@ extern "C" int blade_channelizer_detector(const void* input, void* output, uint6
     const bool fft16 = small && use_fft16(C) && fft16_fits(C, Sg, groups, out_pols);
     if (small && Sg < (1ull << 31) && (!fft16 || runs) && mixed_fft_covers(rate) &&
         mixed_fft_detect(C, static_cast<const float2*>(input), static_cast<float*>(output), Sg, (int)groups, n_items,
-                         (int)out_pols, flags, s, &rc))
-        return rc;
+                         (int)out_pols, flags, s, &rc, &made))
+        return !rc && made ? get_twiddles(C, &tw) : rc;
+    rc = rate_twiddles(C, &tw);
+    if (rc) return rc;
     if (fft16)
         return out_pols == 1 ? launch_fft16<1>(C, static_cast<const float2*>(input), output, Sg, n_items, (int)groups, flags, tw, s)
                              : launch_fft16<4>(C, static_cast<const float2*>(input), output, Sg, n_items, (int)groups, flags, tw, s);

@@ -67,9 +67,9 @@ struct MixArgs {
     unsigned Sg, groups;                   // detector: spectra per integration, integrations per channel
     unsigned S;                            // spectra per (antenna, channel)
     unsigned m_spw, m_sub, m_per, m_gpw;   // division multipliers of spw, sub, S or groups, spw / sub
-    unsigned sums;                         // detector: running sums in LDS from this float on (0: in `out`)
     uint64_t n_spec, n_groups;
     int flags;
+    unsigned sums;                         // detector, KEEP: running sums in LDS from this float on
 };
 
 // n / d from m = ceil(2^32 / d), d > 1; exact for n d < 2^32.  m = 0 stands
@@ -290,14 +290,15 @@ __device__ __forceinline__ void mix_last(const MixArgs& a, unsigned t, uint64_t 
 // owns an output in every step.  Where the integration is added to earlier
 // blocks', the steps are summed in LDS first: added one by one, each would round
 // at the size of the long sum (64 blocks of 128 spectra at rate 1000: error
-// 6.0e-7 against 1.2e-7).
-template <int MODE>
+// 6.0e-7 against 1.2e-7).  KEEP: in a kernel of its own, its registers and branches
+// cost the others up to 7%.
+template <int MODE, bool KEEP>
 __device__ __forceinline__ void mix_sum(const MixArgs& a, unsigned t, uint64_t wg, unsigned step, float4* lds) {
     const unsigned C = (unsigned)a.pl.C, gpw = a.gpw, half = C / 2;
     const uint64_t g0 = wg * gpw, af0 = a.groups == 1 ? g0 : g0 / a.groups;
     const unsigned r0 = (unsigned)(g0 - af0 * a.groups);
     const unsigned cnt = min(a.sub, a.Sg - step * a.sub);
-    const bool add = (step > 0 && !a.sums) || (a.flags & 1), circular = a.flags & 2;
+    const bool add = KEEP || step > 0 || (a.flags & 1), circular = a.flags & 2;
     for (unsigned e = t; e < C * gpw; e += blockDim.x) {
         const unsigned k = mix_div1(e, a.m_gpw), gl = e - k * gpw;
         if (g0 + gl >= a.n_groups) continue;
@@ -316,7 +317,7 @@ __device__ __forceinline__ void mix_sum(const MixArgs& a, unsigned t, uint64_t w
                 v[MODE > 3 ? 3 : 0] += q.w;
             }
         }
-        if (a.sums) {                              // one integration per workgroup: e is its output
+        if constexpr (KEEP) {                      // one integration per workgroup: e is its output
             float* const sum = reinterpret_cast<float*>(lds) + a.sums + e * MODE;
             if (step > 0) {
 #pragma unroll
@@ -350,8 +351,9 @@ __device__ __forceinline__ void mix_sum(const MixArgs& a, unsigned t, uint64_t w
 
 #define MIX_RADICES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(14) X(15) X(16)
 
-// MODE 0: spectra; 1: Stokes I; 4: XX*, YY*, Re XY*, Im XY*.
-template <int MODE>
+// MODE 0: spectra; 1: Stokes I; 4: XX*, YY*, Re XY*, Im XY*.  KEEP: the steps of
+// an integration are summed in LDS (mix_sum).
+template <int MODE, bool KEEP = false>
 __global__ __launch_bounds__(kMixThreads) void mixed_fft_kernel(MixArgs a) {
     extern __shared__ __align__(16) float4 lds[];
     // Outputs of neighbouring workgroups that share lines are written on one XCD.
@@ -382,7 +384,7 @@ __global__ __launch_bounds__(kMixThreads) void mixed_fft_kernel(MixArgs a) {
         }
         if constexpr (MODE != 0) {
             __syncthreads();
-            mix_sum<MODE>(a, t, wg, step, lds);
+            mix_sum<MODE, KEEP>(a, t, wg, step, lds);
             if (step + 1 < steps) __syncthreads();     // LDS is rewritten by the next step
         }
     }
@@ -519,7 +521,7 @@ static std::vector<MixShape> mix_shapes(const MixPlan& pl, unsigned CS) {
 static std::mutex g_mix_mutex;
 static std::map<std::pair<int, int>, std::unique_ptr<MixTable>> g_mix_tables;
 
-static int mix_table(int C, const MixTable** out) {
+static int mix_table(int C, const MixTable** out, bool* made = nullptr) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fail("channelizer: hipGetDevice failed");
     std::lock_guard<std::mutex> lock(g_mix_mutex);
@@ -537,6 +539,7 @@ static int mix_table(int C, const MixTable** out) {
         if (rc) return rc;
         t->tw = static_cast<float2*>(p);
         slot = std::move(t);
+        if (made) *made = true;
     }
     *out = slot.get();
     return BLADE_SUCCESS;
@@ -567,10 +570,10 @@ static void mix_shape(const MixTable& t, uint64_t units, unsigned unit, RunOf ru
     }
 }
 
-template <int MODE>
+template <int MODE, bool KEEP = false>
 static int mix_launch(MixArgs& a, uint64_t blocks, unsigned threads, hipStream_t s) {
-    const void* fn = reinterpret_cast<const void*>(&mixed_fft_kernel<MODE>);
-    const size_t lds = (size_t)a.spw * a.CS * 16 + (a.sums ? (size_t)a.pl.C * MODE * 4 : 0);
+    const void* fn = reinterpret_cast<const void*>(&mixed_fft_kernel<MODE, KEEP>);
+    const size_t lds = (size_t)a.spw * a.CS * 16 + (KEEP ? (size_t)a.pl.C * MODE * 4 : 0);
     if (lds > 65536 && hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return fail("channelizer: LDS attribute of the mixed-radix FFT");
     void* args[] = {&a};
@@ -578,10 +581,10 @@ static int mix_launch(MixArgs& a, uint64_t blocks, unsigned threads, hipStream_t
     return check_launch("channelizer");
 }
 
-int mixed_fft(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec, hipStream_t s) {
+int mixed_fft(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec, hipStream_t s, bool* made) {
     MixArgs a = {};
     const MixTable* t = nullptr;
-    int rc = mix_table(C, &t);
+    int rc = mix_table(C, &t, made);
     if (rc) return rc;
     a.pl = t->pl;
     a.CS = t->CS;
@@ -603,10 +606,10 @@ int mixed_fft(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec,
 }
 
 bool mixed_fft_detect(int C, const float2* in, float* out, uint64_t Sg, int groups, uint64_t n_groups, int out_pols,
-                      int flags, hipStream_t s, int* rc) {
+                      int flags, hipStream_t s, int* rc, bool* made) {
     MixArgs a = {};
     const MixTable* t = nullptr;
-    *rc = mix_table(C, &t);
+    *rc = mix_table(C, &t, made);
     if (*rc) return true;
     a.pl = t->pl;
     a.CS = t->CS;
@@ -654,7 +657,10 @@ bool mixed_fft_detect(int C, const float2* in, float* out, uint64_t Sg, int grou
     a.m_per = mix_magic((uint64_t)groups);
     uint64_t blocks = ceil_div(n_groups, a.gpw);
     if (groups > 1) blocks = ceil_div(blocks, 8) * 8;    // xcd_order needs G % 8 == 0
-    *rc = out_pols == 1 ? mix_launch<1>(a, blocks, threads, s) : mix_launch<4>(a, blocks, threads, s);
+    if (keep)
+        *rc = out_pols == 1 ? mix_launch<1, true>(a, blocks, threads, s) : mix_launch<4, true>(a, blocks, threads, s);
+    else
+        *rc = out_pols == 1 ? mix_launch<1>(a, blocks, threads, s) : mix_launch<4>(a, blocks, threads, s);
     return true;
 }
 

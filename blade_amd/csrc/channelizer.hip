@@ -1482,7 +1482,7 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     // to three rounds of workgroups lose up to 6% ([4,64,4 C,2] 44.0 against 41.5
     // us; 512 spectra 19.4 against 22.3, [16,30,6 C,2] 110 against 166).
     const bool runs4096 = C == 4096 && S > 1 && (S > 5 || n_spec <= 512 || n_spec >= 1536);
-    if (P == 2 && (!use_fft16(C) || runs4096) && T < (1ull << 31) && mixed_fft_covers(rate)) {
+    if (P == 2 && (!use_fft16(C) || runs4096) && mixed_fft_covers(rate)) {
         rc = mixed_fft(C, in, out, S, n_spec, s, &made);
         return !rc && made ? get_twiddles(C, &tw) : rc;
     }

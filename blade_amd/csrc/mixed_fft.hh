@@ -19,7 +19,8 @@ int mixed_fft(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec,
 // Powers summed over Sg consecutive spectra, `groups` integrations per
 // (antenna, channel): F32 [n_groups / groups, C, groups, out_pols].
 // flags: 1 adds into out, 2 XY -> LR first.  False if it does not take the
-// call (adding to earlier blocks, where LDS has no room for the block's sums).
+// call (adding to earlier blocks, where LDS has no room for the block's sums, or
+// more threads than a launch holds).
 bool mixed_fft_detect(int C, const float2* in, float* out, uint64_t Sg, int groups, uint64_t n_groups, int out_pols,
                       int flags, hipStream_t s, int* rc, bool* made);
 

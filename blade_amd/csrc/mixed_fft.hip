@@ -36,6 +36,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace bl {
@@ -70,6 +71,7 @@ struct MixArgs {
     uint64_t n_spec, n_groups;
     int flags;
     unsigned sums;                         // detector, KEEP: running sums in LDS from this float on
+    unsigned wg0;                          // MODE 0, OPT: first workgroup of this launch
 };
 
 // n / d from m = ceil(2^32 / d), d > 1; exact for n d < 2^32.  m = 0 stands
@@ -191,7 +193,7 @@ __device__ __forceinline__ void mix_mid(const MixArgs& a, unsigned t, const MixP
     __syncthreads();
 }
 
-template <int R, int MODE>
+template <int R, int MODE, bool OPT>
 __device__ __forceinline__ void mix_last(const MixArgs& a, unsigned t, uint64_t wg, float4* lds) {
     const MixPass& p = a.pl.p[a.pl.n - 1];       // Ns = nb: butterfly j holds bins j + r nb
     constexpr int G = mix_per_thread<R>();
@@ -219,6 +221,7 @@ __device__ __forceinline__ void mix_last(const MixArgs& a, unsigned t, uint64_t 
                 mix_dft<R>(x, y);
                 const unsigned q = s0 + slot, af = mix_div_wide(q, a.S, a.m_per), s = q - af * a.S;
                 float4* const dst = out + (uint64_t)af * ((uint64_t)C * a.S) + s;
+                typedef std::conditional_t<OPT, uint64_t, unsigned> Offset;      // within C S outputs
                 unsigned ko = j + half;
                 if (ko >= C) ko -= C;
                 // Two loops: with the branch inside, the compiler merges both
@@ -234,7 +237,7 @@ __device__ __forceinline__ void mix_last(const MixArgs& a, unsigned t, uint64_t 
                 } else {
 #pragma unroll
                     for (int r = 0; r < R; r++) {
-                        dst[ko * a.S] = make_float4(x[r].x, x[r].y, y[r].x, y[r].y);   // C S < 2^31 (host check)
+                        dst[Offset(ko) * a.S] = make_float4(x[r].x, x[r].y, y[r].x, y[r].y);
                         ko += p.nb;
                         if (ko >= C) ko -= C;
                     }
@@ -351,13 +354,15 @@ __device__ __forceinline__ void mix_sum(const MixArgs& a, unsigned t, uint64_t w
 
 #define MIX_RADICES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(14) X(15) X(16)
 
-// MODE 0: spectra; 1: Stokes I; 4: XX*, YY*, Re XY*, Im XY*.  KEEP: the steps of
-// an integration are summed in LDS (mix_sum).
-template <int MODE, bool KEEP = false>
+// MODE 0: spectra; 1: Stokes I; 4: XX*, YY*, Re XY*, Im XY*.  OPT: channels of
+// 2^31 outputs or more and 2^32 threads or more in several launches (MODE 0; the
+// 64-bit arithmetic costs small calls 2%); the steps of an integration are summed in LDS (detector, mix_sum).
+template <int MODE, bool OPT = false>
 __global__ __launch_bounds__(kMixThreads) void mixed_fft_kernel(MixArgs a) {
     extern __shared__ __align__(16) float4 lds[];
     // Outputs of neighbouring workgroups that share lines are written on one XCD.
-    const uint64_t wg = (MODE == 0 ? a.S > 1 : a.groups > 1) ? xcd_order(blockIdx.x, gridDim.x) : blockIdx.x;
+    const unsigned wgi = (MODE == 0 ? a.S > 1 : a.groups > 1) ? xcd_order(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint64_t wg = MODE == 0 && OPT ? a.wg0 + (uint64_t)wgi : wgi;
     const unsigned steps = MODE == 0 ? 1 : a.steps;
     for (unsigned step = 0; step < steps; step++) {
         // Opaque: keeps every radix's index arithmetic from being hoisted out
@@ -378,13 +383,13 @@ __global__ __launch_bounds__(kMixThreads) void mixed_fft_kernel(MixArgs a) {
             }
         }
         switch (a.pl.p[a.pl.n - 1].R) {
-#define X(R) case R: mix_last<R, MODE>(a, t, wg, lds); break;
+#define X(R) case R: mix_last<R, MODE, OPT>(a, t, wg, lds); break;
             MIX_RADICES(X)
 #undef X
         }
         if constexpr (MODE != 0) {
             __syncthreads();
-            mix_sum<MODE, KEEP>(a, t, wg, step, lds);
+            mix_sum<MODE, OPT>(a, t, wg, step, lds);
             if (step + 1 < steps) __syncthreads();     // LDS is rewritten by the next step
         }
     }
@@ -570,14 +575,18 @@ static void mix_shape(const MixTable& t, uint64_t units, unsigned unit, RunOf ru
     }
 }
 
-template <int MODE, bool KEEP = false>
+template <int MODE, bool OPT = false>
 static int mix_launch(MixArgs& a, uint64_t blocks, unsigned threads, hipStream_t s) {
-    const void* fn = reinterpret_cast<const void*>(&mixed_fft_kernel<MODE, KEEP>);
-    const size_t lds = (size_t)a.spw * a.CS * 16 + (KEEP ? (size_t)a.pl.C * MODE * 4 : 0);
+    const void* fn = reinterpret_cast<const void*>(&mixed_fft_kernel<MODE, OPT>);
+    const size_t lds = (size_t)a.spw * a.CS * 16 + (OPT ? (size_t)a.pl.C * MODE * 4 : 0);
     if (lds > 65536 && hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return fail("channelizer: LDS attribute of the mixed-radix FFT");
-    void* args[] = {&a};
-    (void)hipLaunchKernel(fn, dim3((unsigned)blocks), dim3(threads), args, lds, s);
+    const uint64_t most = 0xffffffffull / threads & ~7ull;          // a launch holds less than 2^32 threads
+    for (uint64_t wg0 = 0; wg0 < blocks; wg0 += most) {             // once unless MODE 0, OPT
+        a.wg0 = (unsigned)wg0;
+        void* args[] = {&a};
+        (void)hipLaunchKernel(fn, dim3((unsigned)std::min(most, blocks - wg0)), dim3(threads), args, lds, s);
+    }
     return check_launch("channelizer");
 }
 
@@ -602,7 +611,8 @@ int mixed_fft(int C, const float2* in, float2* out, uint64_t S, uint64_t n_spec,
     a.m_per = mix_magic(S);
     uint64_t blocks = ceil_div(n_spec, a.spw);
     if (S > 1) blocks = ceil_div(blocks, 8) * 8;         // xcd_order needs G % 8 == 0
-    return mix_launch<0>(a, blocks, threads, s);
+    const bool wide = (uint64_t)C * S >= (1ull << 31) || blocks * threads >= (1ull << 32);
+    return wide ? mix_launch<0, true>(a, blocks, threads, s) : mix_launch<0>(a, blocks, threads, s);
 }
 
 bool mixed_fft_detect(int C, const float2* in, float* out, uint64_t Sg, int groups, uint64_t n_groups, int out_pols,
@@ -657,6 +667,7 @@ bool mixed_fft_detect(int C, const float2* in, float* out, uint64_t Sg, int grou
     a.m_per = mix_magic((uint64_t)groups);
     uint64_t blocks = ceil_div(n_groups, a.gpw);
     if (groups > 1) blocks = ceil_div(blocks, 8) * 8;    // xcd_order needs G % 8 == 0
+    if (blocks * threads >= (1ull << 32)) return false;
     if (keep)
         *rc = out_pols == 1 ? mix_launch<1, true>(a, blocks, threads, s) : mix_launch<4, true>(a, blocks, threads, s);
     else

@@ -90,12 +90,7 @@ def test_adding_a_block_rounds_once(C, S, pols):
     assert err <= start * 2.0 ** -24 * (1 + 2.0 ** -10)
 
 
-@pytest.mark.parametrize("C", [64, 256, 2048, 4096, 8192])
-def test_channels_past_63_million_samples(C):
-    """Spectra of one long channel, and their powers in integrations of one."""
-    S = 2 ** 26 // C + 16
-    _needs(8)
-    at = [0, 7, S // 2, S - 1]
+def _check_sparse_spectra(C, S, at):
     x, noise = _sparse_block(C, S, at, C)
     y = torch.full((1, C, S, 2), complex("nan"), dtype=torch.complex64, device="cuda")
     ops.channelizer(x, C, out=y)
@@ -103,7 +98,23 @@ def test_channels_past_63_million_samples(C):
     err = float((y[0][:, at] - X).norm() / X.norm())
     assert err <= 2 * math.log2(C) * 2.0 ** -24
     y[0][:, at] = 0
-    assert not (y != 0).any()
-    del x, y
+    for k in range(C):
+        assert not (y[0, k] != 0).any(), f"channel {k}"
+
+
+@pytest.mark.parametrize("C", [64, 256, 2048, 4096, 8192])
+def test_channels_past_63_million_samples(C):
+    """Spectra of one long channel, and their powers in integrations of one."""
+    S = 2 ** 26 // C + 16
+    _needs(8)
+    at = [0, 7, S // 2, S - 1]
+    _check_sparse_spectra(C, S, at)
     for pols in (1, 4):
         _check_single_spectra(C, S, pols, at)
+
+
+def test_channel_past_31_bits_of_samples():
+    S = 2 ** 31 // 64 + 24
+    _needs(80)
+    _check_sparse_spectra(64, S, [0, S // 2, S - 2, S - 1])
+    torch.cuda.empty_cache()

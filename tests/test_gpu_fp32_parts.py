@@ -181,3 +181,31 @@ def test_integrated_rows_at_every_alignment(kind, rate, polarize, B, inc, T):
     got = ops.beamform_chain(x, torch.from_numpy(w).cuda(), inc, False, rate, polarize,
                              "f16x2" if kind == "ci8-f16x2" else "f32").cpu().numpy()
     assert got.shape == ref.shape and O.norm_rel_err(got, ref) <= 1e-6
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16x2", "adjoint"])
+@pytest.mark.parametrize("A,B", [(1, 1), (16, 2), (42, 4), (64, 3), (17, 9), (128, 17)])
+@pytest.mark.parametrize("T", [4, 8, 64, 260])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -100])
+def test_gradients_keep_the_third_part(kind, A, B, T, scale):
+    """Normwise per beam.  Without their third part the operands are cut at 16
+    bits: each is off by up to 2^-16 of itself, 7e-6 in the norm.  FP32
+    accumulation (and the 22 bits of split-FP16 phasors) leave 16 units of
+    2^-24."""
+    rng = np.random.default_rng(A + 10 * T)
+    x8 = rng.integers(-128, 128, size=(A, 2, T, 2, 2), dtype=np.int8)
+    x = x8[..., 0].astype(np.float64) + 1j * x8[..., 1]
+    xd = torch.from_numpy(x8).cuda()
+    if kind == "adjoint":
+        gy = (scale * (rng.normal(size=(B, 2, T, 2)) + 1j * rng.normal(size=(B, 2, T, 2)))).astype(np.complex64)
+        got = ops.beamformer_adjoint(xd, torch.from_numpy(gy).cuda())
+        ref = np.einsum("bftp,aftp->bafp", gy.astype(np.complex128), x.conj())
+    else:
+        w = (scale * (rng.normal(size=(B, A, 2, 1, 2)) + 1j * rng.normal(size=(B, A, 2, 1, 2)))).astype(np.complex64)
+        lam = [float(np.float32(v)) for v in rng.uniform(0.5, 1.0, size=B)]
+        _, got = ops.stokes_i_loss_and_grad(xd, torch.from_numpy(w).cuda(), lam, precision=kind)
+        y = np.einsum("bafp,aftp->bftp", w[:, :, :, 0].astype(np.complex128), x)
+        ref = np.einsum("bftp,aftp->bafp", -np.array(lam)[:, None, None, None] * y, x.conj())
+    got = got.cpu().numpy()[:, :, :, 0].astype(np.complex128)
+    for b in range(B):
+        assert np.linalg.norm(got[b] - ref[b]) <= 16 * 2.0 ** -24 * np.linalg.norm(ref[b]), b

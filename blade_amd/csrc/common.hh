@@ -127,8 +127,9 @@ __device__ __forceinline__ uint32_t ci8_to_bf16(uint32_t d, int p) {
 
 // v = part[0] + part[1] + part[2] exactly, each part with the 8 significant
 // bits of BF16 (in the high half of its float): an FP32 value has 24, so
-// cutting 8 off the top three times leaves nothing (parts below FP32's normal
-// range aside).  Infinities and NaN stay in part 0 (CHECKED; otherwise they
+// cutting 8 off the top three times leaves nothing.  As BF16 pairs the parts end
+// at 2^-133, so this holds from |v| = 2^-110 on; smaller values lose what they
+// hold below 2^-133 (relative error 2^-15 at 2^-118).  Infinities and NaN stay in part 0 (CHECKED; otherwise they
 // become NaN).
 template <bool CHECKED = true>
 __device__ __forceinline__ void split_bf16x3(float v, float (&part)[3]) {

@@ -42,7 +42,8 @@ enum blade_type {
 /* Beamformer arithmetic. */
 enum blade_precision {
     BLADE_PREC_F32 = 0,     /* FP32 phasors and accumulation: FP32 MFMA, or for CI8 input BF16 MFMA on
-                               phasors split exactly into three BF16 parts */
+                               phasors split into three BF16 parts: exact for components from 2^-110
+                               (7.7e-34) on; what smaller ones hold below 2^-133 is cut off */
     BLADE_PREC_F16X2 = 1,   /* split FP16: phasor = hi + lo, 2 FP16 MFMAs, FP32 accumulate (CI8 input only) */
 };
 
@@ -167,6 +168,7 @@ int blade_beamform_batched(int precision, const blade_beamform_block* blocks, ui
  *     grad_phasors[b,a,f,p] = sum_t grad_output[b,f,t,p] * conj(x[a,f,t,p]).
  * input: CI8 [A,F,T,P]; P = 2, A <= 128.  This is also the gradient in
  * PyTorch's convention when grad_output is PyTorch's gradient of y.
+ * grad_output is multiplied as three BF16 parts, exact as above (from 2^-110 on).
  */
 int blade_beamformer_adjoint(const void* input, const void* grad_output, void* grad_phasors,
                              uint64_t A, uint64_t F, uint64_t T, uint64_t P, uint64_t B,
@@ -180,8 +182,9 @@ int blade_beamformer_adjoint(const void* input, const void* grad_output, void* g
  * [B,A,F,1,P] (PyTorch's gradient is twice this).  The beams are recomputed
  * tile by tile and never stored.  beam_weights: host array of B floats,
  * B <= 64; P = 2, A <= 128.  precision: BLADE_PREC_F32 (FP32 matrix cores)
- * or BLADE_PREC_F16X2 (FP16 matrix cores with hi + lo phasors and
- * gradients, FP32 accumulation; error at the FP32 level).
+ * or BLADE_PREC_F16X2 (FP16 matrix cores with hi + lo phasors, FP32
+ * accumulation; error at the FP32 level).  In both, the beams' gradient is
+ * multiplied as three BF16 parts (exact from 2^-110 on).
  */
 int blade_beamformer_stokes_i_grad(int precision, const void* input, const void* phasors,
                                    const float* beam_weights, double* loss, void* grad_phasors,

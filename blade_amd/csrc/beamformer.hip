@@ -415,13 +415,17 @@ constexpr size_t kStageBytes = (size_t)kStageBeams * 4 * kStageRow * 16;
 // 256 bytes instead of 16 bytes of every 64, 32 or 256.  The loads keep runs of
 // 4 samples (16 bytes per lane).  4 rows (every other beam of a tile) at a time,
 // private to the wavefront: LDS operations of a wavefront complete in order, so
-// there is no barrier.  Rows carry one entry of padding per 4, which puts the 16
-// lanes' 64-byte pieces on different banks.
+// there is no barrier.  A column's place within its four turns with the column's
+// sixteen (wave_col), which puts what 16 lanes write at once on different banks
+// at every rate.  16 KiB for the workgroup: with a float4 of padding per 4 the
+// rows took 20 KiB and, from A = 64 (16 beams) or 128 (8 beams) on, a workgroup
+// per CU (split FP16 A128 F134 T2304 B8 rate 4 57.7 us, 47.2 so).
 template <int NT, int AR, int MW, int EPI>
 constexpr bool wave_stage() {
     return ar_split(AR) && NT == 4 && !staged_epilogue<NT, AR, MW, EPI>() && !(EPI & EPI_ODD_FLAG);
 }
-constexpr int kWaveRow = 80;                                    // float4 per row
+constexpr int kWaveRow = 64;                                    // float4 per row
+__device__ __forceinline__ int wave_col(int c) { return c ^ ((c >> 4) & 3); }
 constexpr size_t kWaveStageBytes = (size_t)WAVES * 4 * kWaveRow * 16;
 
 // One beam's 4 consecutive samples (lane i of its group) into its row.
@@ -463,7 +467,7 @@ __device__ __forceinline__ void wave_stage_beam(float4* row, int i, int rate, bo
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         if (pol) polarize2(o[0][j], o[1][j]);
-        row[c[j] + (c[j] >> 2)] = make_float4(o[0][j].x, o[0][j].y, o[1][j].x, o[1][j].y);
+        row[wave_col(c[j])] = make_float4(o[0][j].x, o[0][j].y, o[1][j].x, o[1][j].y);
     }
 }
 
@@ -821,7 +825,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
             float4* const base = reinterpret_cast<float4*>(a.y) + ((size_t)fo * rate + kp) * S + sc;
             const size_t bstride = (size_t)a.F * a.T;
             float4* const sink = a.sink + lane;
-            const int rd = lane + (lane >> 2);
+            const int rd = wave_col(lane);
 #pragma unroll
             for (int m = 0; m < MW; m++)
 #pragma unroll
@@ -1199,7 +1203,7 @@ __device__ __forceinline__ BfArgs batch_block_args(const BatchArgs& ba, int k) {
 }
 
 template <int NT, int AR, int D>
-__global__ __launch_bounds__(256, 2) void beamform_batched_kernel(BatchArgs ba) {
+__global__ __launch_bounds__(256, (AR == AR_BF16X3 ? 3 : 2)) void beamform_batched_kernel(BatchArgs ba) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     __shared__ float s_unscale[2];
     __shared__ float s_w0sq[2][128];

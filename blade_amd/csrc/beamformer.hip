@@ -956,8 +956,21 @@ __global__ __launch_bounds__(256, (staged_epilogue<NT, AR, MW, EPI>() ? 3 : 2)) 
     __shared__ float s_unscale[2];
     __shared__ float s_w0sq[2][128];
     __shared__ unsigned int s_max[2];
-    bf_body<NT, MW, CI8, AR, D, NTS, EPI, (AR == AR_F32 && MW == 2)>(a, blockIdx.y, blockIdx.z, blockIdx.x, lds_raw,
-                                                                s_unscale, s_w0sq, s_max, gridDim.x);
+    unsigned x = blockIdx.x, f = blockIdx.y, gz = blockIdx.z;
+    if constexpr (ar_split(AR) && EPI == EPI_MODEB && !NTS) {
+        // Rows off memory lines: the workgroups of neighbouring chunks share the
+        // lines at their ends.  Consecutive ones on one XCD (the dispatcher deals
+        // them out b mod 8), whose L2 merges the pieces.
+        const unsigned G = gridDim.x, N = G * gridDim.y * gridDim.z;
+        unsigned b = x + G * (f + gridDim.y * gz);
+        if (b < (N & ~7u)) b = (b & 7u) * (N >> 3) + (b >> 3);
+        const unsigned fg = b / G, g = fg / gridDim.y;
+        x = __builtin_amdgcn_readfirstlane(b - fg * G);
+        f = __builtin_amdgcn_readfirstlane(fg - g * gridDim.y);
+        gz = __builtin_amdgcn_readfirstlane(g);
+    }
+    bf_body<NT, MW, CI8, AR, D, NTS, EPI, (AR == AR_F32 && MW == 2)>(a, f, gz, x, lds_raw, s_unscale, s_w0sq, s_max,
+                                                                gridDim.x);
 }
 
 static int env_int(const char* name, int dflt) {
@@ -1117,6 +1130,28 @@ static bool odd_wide(int B, long T) {
     return B > 4 && (B <= 8 ? T >= 768 : full && T >= (B <= 16 ? 768 : 5000));
 }
 
+constexpr double kL2Bytes = 32.0 * 1024 * 1024;      // of all XCDs
+
+// Mode-B rows (T / 4 samples) off 64-byte sectors: whether ordinary stores beat
+// nontemporal ones, which write the lines at the ends of rows and chunks in
+// parts.  Measured over A 6-64, F 16-384, T 256-16384, B 1-40.
+//  * CI8, staged rows of 16-beam tiles: outputs past the L2s with few idle beams.
+//    A8 F259 T2740 B16 171 us nontemporal, 60 ordinary; A7 F176 T5756 B40 536
+//    against 206; A41 F278 T3132 B25 300 against 184.  Below, and up to 12 beams
+//    (the other lanes store to the sink), nontemporal: A10 F105 T6232 B10 39
+//    against 50.
+//  * CF32, stored from registers: nontemporal only where the last chunk leaves
+//    wavefronts without samples and the data or the outputs are small: A9 F195
+//    T3876 B6 40 us against 59 ordinary, but A8 F128 T1220 B14 87 against 17.
+static bool modeb_plain(bool split, const BfArgs& a) {
+    if (a.T % 16 == 0) return false;
+    const double samples = (double)a.F * a.T, out = samples * a.B * 16;
+    if (split) return a.B > 12 && out > kL2Bytes;
+    const double in = samples * a.A * 16;
+    const int last = a.T % (WAVES * TILE * 4);
+    return !(last > 0 && last <= (WAVES - 1) * TILE * 4 && in <= 146e6 && (out <= kL2Bytes || out <= in));
+}
+
 template <int NT, int MW, bool CI8, int AR, int D>
 static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, hipStream_t s) {
     if (a.T % 4) {
@@ -1129,12 +1164,9 @@ static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, h
     const size_t wb = operand_bytes(AR, MW, nsteps_for(AR, a.A));
     if (ar_split(AR) && wb + std::max(kStageBytes, kWaveStageBytes) > kMaxLds)
         return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
-    // CF32 rows off 64-byte sectors: ordinary stores (A28 F192 T8188 B16 267
-    // against 305 us nontemporal, T3004 104 against 116, A42 F384 T1004 B5 64
-    // against 78).  CI8 stays nontemporal, its stores go out in longer runs
-    // (same sizes: 136 against 145, 57 against 60, 22 against 25).
-    if constexpr (AR == AR_F32) {
-        if (epi == EPI_MODEB && a.T % 16) return launch_bf<NT, MW, CI8, AR, D, false, EPI_MODEB>(a, ws, wsb, s);
+    if constexpr (!ar_split(AR) || MW == 2) {
+        if (epi == EPI_MODEB && modeb_plain(ar_split(AR), a))
+            return launch_bf<NT, MW, CI8, AR, D, false, EPI_MODEB>(a, ws, wsb, s);
     }
     if (epi == EPI_MODEB) return launch_bf<NT, MW, CI8, AR, D, true, EPI_MODEB>(a, ws, wsb, s);
     // The rate-1 epilogues of CF32 input map a wave onto TILE * NT

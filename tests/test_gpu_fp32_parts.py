@@ -209,3 +209,19 @@ def test_gradients_keep_the_third_part(kind, A, B, T, scale):
     got = got.cpu().numpy()[:, :, :, 0].astype(np.complex128)
     for b in range(B):
         assert np.linalg.norm(got[b] - ref[b]) <= 16 * 2.0 ** -24 * np.linalg.norm(ref[b]), b
+
+
+@pytest.mark.parametrize("precision", ["f32", "f16x2"])
+@pytest.mark.parametrize("A,F,T,B", [(6, 37, 4100, 16), (5, 41, 4108, 13), (3, 19, 8204, 33), (4, 50, 2052, 24)])
+def test_mode_b_rows_off_sectors_past_the_caches(A, F, T, B, precision):
+    """Outputs past 32 MiB with rows off 64-byte sectors: workgroups in XCD order,
+    their number a multiple of 8 and not."""
+    rng = np.random.default_rng(F)
+    x8 = rng.integers(-128, 128, size=(A, F, T, 2, 2), dtype=np.int8)
+    w = (rng.normal(size=(B, A, F, 1, 2)) + 1j * rng.normal(size=(B, A, F, 1, 2))).astype(np.complex64)
+    assert T % 16 and B * F * T * 16 > 2 ** 25
+    out = torch.full((B, F * 4, T // 4, 2), complex("nan"), dtype=torch.complex64, device="cuda")
+    ops.beamform_chain(torch.from_numpy(x8).cuda(), torch.from_numpy(w).cuda(), False, False, 4, True, precision, out=out)
+    ref = O.polarizer(O.channelizer(O.beamformer_ata(x8, w, False, False), 4))
+    for b in range(B):
+        assert O.norm_rel_err(out[b].cpu().numpy(), ref[b]) <= 1e-6

@@ -1478,10 +1478,14 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     // interleave: its stores write runs of them ([8,.,4 C,2]: 123 us against
     // 156 us at S = 4, 102 against 108 at S = 2; 512 to 2048 are staged there
     // and 10-30% faster, 8192 106 against 129 us).
-    // Between 513 and 1535 spectra in all, up to 5 per channel, that kernel's one
-    // to three rounds of workgroups lose up to 6% ([4,64,4 C,2] 44.0 against 41.5
-    // us; 512 spectra 19.4 against 22.3, [16,30,6 C,2] 110 against 166).
-    const bool runs4096 = C == 4096 && S > 1 && (S > 5 || n_spec <= 512 || n_spec >= 1536);
+    // The radix-16 kernel keeps one workgroup of two such spectra on a CU.  Where it
+    // needs little more than one round, the mixed-radix kernel's spread of spectra
+    // over the chip is worse: 520 to 800 spectra on 256 CUs 1 to 16% in its favour at
+    // S = 2 to 8 (800 of S = 4 36.2 against 38.8 us, buffers in turn); up to one round
+    // (480 of S = 2: 21.3 against 17.6) and from 1.75 on (896 of S = 4: 47.4 against
+    // 42.8) the runs win.
+    const uint64_t cus = (uint64_t)device_cus();
+    const bool runs4096 = C == 4096 && S > 1 && (n_spec <= 2 * cus || 4 * n_spec > 13 * cus);
     if (P == 2 && (!use_fft16(C) || runs4096) && mixed_fft_covers(rate)) {
         rc = mixed_fft(C, in, out, S, n_spec, s, &made);
         return !rc && made ? get_twiddles(C, &tw) : rc;

@@ -118,3 +118,14 @@ def test_channel_past_31_bits_of_samples():
     _needs(80)
     _check_sparse_spectra(64, S, [0, S // 2, S - 2, S - 1])
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("F,S", [(256, 2), (257, 2), (416, 2), (417, 2), (208, 4), (209, 4)])
+def test_4096_by_rounds_of_workgroups(F, S):
+    """512 and 832 spectra on 256 compute units: both kernels, on each side."""
+    gen = torch.Generator(device="cuda").manual_seed(F)
+    x = torch.randn((1, F, S * 4096, 2), dtype=torch.complex64, device="cuda", generator=gen)
+    v = x.to(torch.complex128).reshape(1, F, S, 4096, 2)
+    ref = torch.fft.fftshift(torch.fft.fft(v, dim=3), dim=3).permute(0, 1, 3, 2, 4).reshape(1, F * 4096, S, 2)
+    err = float((ops.channelizer(x, 4096) - ref).norm() / ref.norm())
+    assert err <= 2 * 12 * 2.0 ** -24

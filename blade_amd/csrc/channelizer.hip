@@ -1049,11 +1049,14 @@ static int launch_fft16_lc(const float2* in, void* out, uint64_t S, uint64_t n_i
     // C = 256 56 / 60 us, 512 60 / 69, 1024 72 / 90; Stokes I 512 55 / 57,
     // 1024 51 / 57, but 256 53 / 47 and C = 4096 109 / 103 (178 / 155 with 4
     // pols), which keep 512.
-    // At C = 8192 (one spectrum per workgroup) items are whole (antenna,
-    // channel)s where these fill the chip: 2.5% faster in the Mode-A case.
-    if constexpr (MODE != 0 && LC == 13) {
-        if (n_items / groups >= (uint64_t)device_cus() || groups == 1)
-            return launch_fft16_t<LC, 512, MODE, 3>(in, out, S * groups, n_items / groups, (int)S, accumulate, tw, s);
+    // At C = 8192, Stokes I and one integration per channel: the same items through
+    // SM 3, whose flush inside the spectrum loop compiles to a loop 2-5% faster
+    // ([8,192,4 C,2] 206 against 212 us, [1,40,8 C,2] 55.5 against 58.4).  With 4
+    // polarizations it is 2-3% slower, with several integrations per channel, which
+    // it would walk one after the other, up to 20% ([1,300,6 C,2], two spectra each,
+    // 107 against 86 us).
+    if constexpr (MODE == 1 && LC == 13) {
+        if (groups == 1) return launch_fft16_t<LC, 512, MODE, 3>(in, out, S, n_items, (int)S, accumulate, tw, s);
     }
     if constexpr ((MODE == 4 && LC <= 11) || (MODE == 1 && LC >= 9 && LC <= 11))
         return launch_fft16_t<LC, 256, MODE, 0>(in, out, S, n_items, groups, accumulate, tw, s);

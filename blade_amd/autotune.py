@@ -2,8 +2,9 @@
 
 For a list of block shapes it times each candidate ``blade_batch_tuning``
 on the device with HIP events (after a warm-up), keeps the fastest, and
-caches it in a JSON file keyed by the precision and the multiset of block
-shapes, so later runs of the same workload start from the tuned shape.
+caches it in a JSON file keyed by the precision, the multiset of block
+shapes and the generation of the kernels, so later runs of the same workload
+start from the tuned shape.
 
 Candidates span the knobs of the launch:
 
@@ -34,6 +35,11 @@ from . import ops
 __all__ = ["candidates", "signature", "tune_batched", "cached_tuning"]
 
 
+# Raised when work items, tiles or the grid change meaning or cost: a shape tuned
+# for the kernels before is not applied to these.
+KERNELS = 2
+
+
 def candidates():
     for bt, cpi, wpc in itertools.product((0, 1, 2), (0, 1, 2, 4, 8), (2, 3, 4, 8, 16, 64)):
         yield {"time_samples_per_lane": 4, "beam_tiles": bt, "chunks_per_item": cpi,
@@ -41,7 +47,7 @@ def candidates():
 
 
 def signature(shapes, precision):
-    key = json.dumps({"precision": precision, "shapes": sorted(list(map(list, shapes)))})
+    key = json.dumps({"kernels": KERNELS, "precision": precision, "shapes": sorted(list(map(list, shapes)))})
     return hashlib.sha1(key.encode()).hexdigest()
 
 

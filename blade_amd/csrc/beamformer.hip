@@ -72,10 +72,6 @@ __device__ __forceinline__ floatx4 mfma_f32(float a, float b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float ci8_byte(uint32_t d, int idx) {
-    return (float)(int8_t)((d >> (8 * idx)) & 0xFFu);
-}
-
 struct BfArgs {
     const void* x;          // [A,F,T,P] CI8 or CF32
     const float2* w;        // [B,A,F,1,P] CF32
@@ -276,9 +272,10 @@ __device__ __forceinline__ void polarize2(float2& X, float2& Y) {
 // Time sample of a lane's n-th column: lanes own runs of RUN consecutive
 // samples, the runs of one lane TILE * RUN samples apart, so a 16-lane group
 // reads and writes TILE * RUN contiguous samples per access.  RUN = 4 gives
-// 16-byte voltage loads and keeps the 4 samples of a DFT-4 in one lane; the
-// plain (rate 1) epilogues use RUN = 1, where each store instruction writes
-// 16 lanes x 16 contiguous bytes instead of 16 bytes of every 64.
+// 16-byte voltage loads and keeps the 4 samples of a DFT-4 in one lane.  The
+// plain (rate 1) epilogues of CF32 input and the sample-by-sample one (EPI_ODD)
+// use RUN = 1, where each store instruction writes 16 lanes x 16 contiguous bytes
+// instead of 16 bytes of every 64; CI8 rows go through LDS (wave_stage).
 template <int NT, int RUN_ = (NT < 4 ? NT : 4)>
 struct TimeMap {
     static constexpr int RUN = RUN_;
@@ -496,13 +493,11 @@ __device__ __forceinline__ void stage_beam(float4* stg, int lb, int col, float2 
 }
 
 // One "unit" of voltage loads: what a lane needs for one K block.
-//  FP32, CI8  : one antenna x NT samples          -> NT words
-//  FP32, CF32 : one antenna x NT samples x 16 B   -> 4 NT words
-//  split      : four antennas x NT samples        -> 4 NT words
-template <int NT, bool CI8, int AR>
+//  FP32 (CF32) : one antenna x NT samples x 16 B   -> 4 NT words
+//  split (CI8) : four antennas x NT samples        -> 4 NT words
+template <int NT>
 struct Unit {
-    static constexpr int WORDS = (ar_split(AR) || !CI8) ? 4 * NT : NT;
-    uint32_t w[WORDS];
+    uint32_t w[4 * NT];
 };
 
 template <int NW>
@@ -543,7 +538,8 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
                                         unsigned char* lds_raw, float* s_unscale, float (*s_w0sq)[128],
                                         unsigned int* s_max, const int cstride = 1) {
     constexpr int AK = ar_split(AR) ? 4 * KG : KG;       // antennas per unit
-    typedef Unit<NT, CI8, AR> U_t;
+    static_assert(CI8 == ar_split(AR), "CI8 voltages take the split variants, CF32 the FP32 one");
+    typedef Unit<NT> U_t;
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -590,12 +586,8 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
             const int an = min(un * KG + g, a.A - 1);
 #pragma unroll
             for (int h = 0; h < NT / R; h++) {
-                if constexpr (CI8) {
-                    load_words<R>(u.w + h * R, static_cast<const uint32_t*>(a.x) + an * ant_stride + off + run_off(h));
-                } else {
-                    load_words<4 * R>(u.w + 4 * h * R,
-                                      static_cast<const uint32_t*>(a.x) + 4 * (an * ant_stride + off + run_off(h)));
-                }
+                load_words<4 * R>(u.w + 4 * h * R,
+                                  static_cast<const uint32_t*>(a.x) + 4 * (an * ant_stride + off + run_off(h)));
             }
         }
     };
@@ -716,17 +708,10 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
             float xv[2][3][NT];   // [p][c][n]: Re x, Im x and (three-product tiles) Re x + Im x
 #pragma unroll
             for (int n = 0; n < NT; n++) {
-                if constexpr (CI8) {
 #pragma unroll
-                    for (int p = 0; p < 2; p++)
+                for (int p = 0; p < 2; p++)
 #pragma unroll
-                        for (int c = 0; c < 2; c++) xv[p][c][n] = ci8_byte(u.w[n], 2 * p + c);
-                } else {
-#pragma unroll
-                    for (int p = 0; p < 2; p++)
-#pragma unroll
-                        for (int c = 0; c < 2; c++) xv[p][c][n] = __uint_as_float(u.w[4 * n + 2 * p + c]);
-                }
+                    for (int c = 0; c < 2; c++) xv[p][c][n] = __uint_as_float(u.w[4 * n + 2 * p + c]);
 #pragma unroll
                 for (int p = 0; p < 2; p++) xv[p][2][n] = xv[p][0][n] + xv[p][1][n];
             }

@@ -58,23 +58,26 @@ inline int device_cus() {
 enum WorkspaceUser { WS_BEAMFORMER_SINK = 0, WS_ADJOINT = 1, WS_CHANNELIZER_BIG = 2 };
 int library_workspace(int user, size_t bytes, hipStream_t s, unsigned char** out);
 
+// The library's own stream on the current device, for filling tables: created on
+// first use, kept for the life of the process.
+hipError_t table_stream(hipStream_t* out);
+
 // A library-owned table of the current device, whole when this returns: `fill`
-// queues its kernels on a stream of their own, which is waited for.  Filled on
-// the caller's stream it would be ready there only, while calls on other
-// streams find the same pointer; and a stream under capture would record the
-// fill instead of running it.  Once per table, so the wait costs nothing later.
+// queues its kernels on the library's stream, which is waited for.  Filled on the
+// caller's stream it would be ready there only, while calls on other streams find
+// the same pointer; and a stream under capture would record the fill instead of
+// running it.  Once per table, so the wait costs nothing later.
 template <typename Fill>
 int device_table(const char* what, size_t bytes, void** out, Fill fill) {
     void* p = nullptr;
     hipStream_t s = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    if (e == hipSuccess) e = table_stream(&s);
     if (e == hipSuccess) {
         fill(p, s);
         e = hipGetLastError();
         const hipError_t w = hipStreamSynchronize(s);
         if (e == hipSuccess) e = w;
-        (void)hipStreamDestroy(s);
     }
     if (e != hipSuccess) {
         (void)hipFree(p);

@@ -46,6 +46,24 @@ int library_workspace(int user, size_t bytes, hipStream_t s, unsigned char** out
     return BLADE_SUCCESS;
 }
 
+hipError_t table_stream(hipStream_t* out) {
+    static std::mutex mutex;
+    static std::map<int, hipStream_t> streams;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    std::lock_guard<std::mutex> lock(mutex);
+    auto it = streams.find(dev);
+    if (it == streams.end()) {
+        hipStream_t s = nullptr;
+        e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+        if (e != hipSuccess) return e;
+        it = streams.emplace(dev, s).first;
+    }
+    *out = it->second;
+    return hipSuccess;
+}
+
 }  // namespace bl
 
 extern "C" const char* blade_amd_version(void) {

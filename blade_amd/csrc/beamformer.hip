@@ -412,20 +412,30 @@ constexpr size_t kStageBytes = (size_t)kStageBeams * 4 * kStageRow * 16;
 // 256 bytes instead of 16 bytes of every 64, 32 or 256.  The loads keep runs of
 // 4 samples (16 bytes per lane).  4 rows (every other beam of a tile) at a time,
 // private to the wavefront: LDS operations of a wavefront complete in order, so
-// there is no barrier.  A column's place within its four turns with the column's
-// sixteen (wave_col), which puts what 16 lanes write at once on different banks
-// at every rate.  16 KiB for the workgroup: with a float4 of padding per 4 the
-// rows took 20 KiB and, from A = 64 (16 beams) or 128 (8 beams) on, a workgroup
-// per CU (split FP16 A128 F134 T2304 B8 rate 4 57.7 us, 47.2 so).
+// there is no barrier.  What 16 lanes write at once has to lie on different
+// banks, in one of two ways (wave_col):
+//  - an entry of padding per 4, 20 KiB for the workgroup;
+//  - wave_turned: a column's place within its four turns with the column's
+//    sixteen, 16 KiB.  From 64 antennas (16 beams) or 128 (8 beams) on that
+//    keeps another workgroup on a CU: split FP16 A128 F134 T2304 B8 rate 4 57.7
+//    us padded, 47.2 so.  Not at FP32 precision, where the third workgroup that
+//    it admits (16 beams of 33-48 antennas) costs up to 30% (A39 F33 T13184 B13
+//    29.7 us padded, 37.7 so), and not for 8 beams with the incoherent one, where
+//    it takes 4 more VGPRs and 1.6% more time on average.
 template <int NT, int AR, int MW, int EPI>
 constexpr bool wave_stage() {
     return ar_split(AR) && NT == 4 && !staged_epilogue<NT, AR, MW, EPI>() && !(EPI & EPI_ODD_FLAG);
 }
-constexpr int kWaveRow = 64;                                    // float4 per row
-__device__ __forceinline__ int wave_col(int c) { return c ^ ((c >> 4) & 3); }
-constexpr size_t kWaveStageBytes = (size_t)WAVES * 4 * kWaveRow * 16;
+constexpr bool wave_turned(int ar, int mw, int epi) { return ar == AR_F16X2 && !(mw == 1 && epi == EPI_PLAIN_INC); }
+constexpr int wave_row(bool turned) { return turned ? 64 : 80; }         // float4 per row
+constexpr size_t wave_stage_bytes(bool turned) { return (size_t)WAVES * 4 * wave_row(turned) * 16; }
+template <bool TURNED>
+__device__ __forceinline__ int wave_col(int c) {
+    return TURNED ? c ^ ((c >> 4) & 3) : c + (c >> 2);
+}
 
 // One beam's 4 consecutive samples (lane i of its group) into its row.
+template <bool TURNED>
 __device__ __forceinline__ void wave_stage_beam(float4* row, int i, int rate, bool pol, float2 (&v)[2][4]) {
     float2 o[2][4];
     int c[4];           // column of result j: (fine channel, spectrum)
@@ -464,7 +474,7 @@ __device__ __forceinline__ void wave_stage_beam(float4* row, int i, int rate, bo
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         if (pol) polarize2(o[0][j], o[1][j]);
-        row[wave_col(c[j])] = make_float4(o[0][j].x, o[0][j].y, o[1][j].x, o[1][j].y);
+        row[wave_col<TURNED>(c[j])] = make_float4(o[0][j].x, o[0][j].y, o[1][j].x, o[1][j].y);
     }
 }
 
@@ -799,7 +809,8 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
         }
         if constexpr (wave_stage<NT, AR, MW, EPI>()) {
             if ((EPI && !(EPI & EPI_STAGE_FLAG)) || a.stage) {
-            float4* const stg = reinterpret_cast<float4*>(lds_raw + a.wbytes) + wave * 4 * kWaveRow;
+            constexpr bool TURNED = wave_turned(AR, MW, EPI);
+            float4* const stg = reinterpret_cast<float4*>(lds_raw + a.wbytes) + wave * 4 * wave_row(TURNED);
             const int rate = epi_rate<EPI>(a), lr = rate >> 1;       // log2 of 1, 2, 4
             const bool pol = epi_pol<EPI>(a);
             // This lane's result of a row: fine channel k, spectrum s.
@@ -810,7 +821,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
             float4* const base = reinterpret_cast<float4*>(a.y) + ((size_t)fo * rate + kp) * S + sc;
             const size_t bstride = (size_t)a.F * a.T;
             float4* const sink = a.sink + lane;
-            const int rd = wave_col(lane);
+            const int rd = wave_col<TURNED>(lane);
 #pragma unroll
             for (int m = 0; m < MW; m++)
 #pragma unroll
@@ -821,12 +832,12 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
 #pragma unroll
                         for (int n = 0; n < 4; n++)
                             v[p][n] = make_float2(acc[m][p][n][2 * rr] * unscale[p], acc[m][p][n][2 * rr + 1] * unscale[p]);
-                    wave_stage_beam(stg + g * kWaveRow, i, rate, pol, v);
+                    wave_stage_beam<TURNED>(stg + g * wave_row(TURNED), i, rate, pol, v);
                     __builtin_amdgcn_wave_barrier();
 #pragma unroll
                     for (int q = 0; q < 4; q++) {
                         const int b = b_wg + 8 * m + 2 * q + rr;
-                        const float4 z = stg[q * kWaveRow + rd];
+                        const float4 z = stg[q * wave_row(TURNED) + rd];
                         store4<NTS>(s_ok && b < a.B ? base + b * bstride : sink, make_float2(z.x, z.y),
                                     make_float2(z.z, z.w));
                     }
@@ -843,7 +854,7 @@ __device__ __forceinline__ void bf_body(const BfArgs& a, const int f, const int 
                         e += __shfl_xor(e, 32, 64);
                         v[p][n] = make_float2(a.inc_sqrt ? sqrtf(e) : e, 0.f);
                     }
-                wave_stage_beam(stg + g * kWaveRow, i, rate, pol, v);     // four equal rows
+                wave_stage_beam<TURNED>(stg + g * wave_row(TURNED), i, rate, pol, v);     // four equal rows
                 __builtin_amdgcn_wave_barrier();
                 const float4 z = stg[rd];
                 store4<NTS>(do_inc && s_ok ? base + a.B * bstride : sink, make_float2(z.x, z.y), make_float2(z.z, z.w));
@@ -1056,9 +1067,10 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
     // A operands, then the staged phasors of both pols (packed in the kernel).
     size_t lds = a.wbytes + staged_bytes(AR, MW, a.A);
     if (staged_epilogue<NT, AR, MW, EPI>()) lds = std::max(lds, a.wbytes + kStageBytes);
-    if (wave_stage<NT, AR, MW, EPI>() && (EPI || a.wbytes + kWaveStageBytes <= kMaxLds)) {
+    const size_t rows = wave_stage_bytes(wave_turned(AR, MW, EPI));
+    if (wave_stage<NT, AR, MW, EPI>() && (EPI || a.wbytes + rows <= kMaxLds)) {
         a.stage = 1;
-        lds = std::max(lds, a.wbytes + kWaveStageBytes);
+        lds = std::max(lds, a.wbytes + rows);
     }
     const int span = WAVES * TILE * NT;
     const int groups = groups_for(a.B, MW);
@@ -1147,7 +1159,7 @@ static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, h
     }
     // The largest arrays leave no LDS for staged rows: generic variant.
     const size_t wb = operand_bytes(AR, MW, nsteps_for(AR, a.A));
-    if (ar_split(AR) && wb + std::max(kStageBytes, kWaveStageBytes) > kMaxLds)
+    if (ar_split(AR) && wb + std::max(kStageBytes, wave_stage_bytes(AR == AR_F16X2)) > kMaxLds)
         return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
     if constexpr (!ar_split(AR) || MW == 2) {
         if (epi == EPI_MODEB && modeb_plain(ar_split(AR), a))
@@ -1220,7 +1232,7 @@ __device__ __forceinline__ BfArgs batch_block_args(const BatchArgs& ba, int k) {
 }
 
 template <int NT, int AR, int D>
-__global__ __launch_bounds__(256, (AR == AR_BF16X3 ? 3 : 2)) void beamform_batched_kernel(BatchArgs ba) {
+__global__ __launch_bounds__(256, 2) void beamform_batched_kernel(BatchArgs ba) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     __shared__ float s_unscale[2];
     __shared__ float s_w0sq[2][128];
@@ -1315,8 +1327,9 @@ static int plan_batch(int ar, const blade_beamform_block* blocks, int n,
         b.item_base = (int)items;
         items += (long)ceil_div(b.n_tchunks, b.cpw) * b.F * b.groups;
         // A operands, then the staged phasors of both pols and the group's beams
-        b.stage = b.wbytes + kWaveStageBytes <= kMaxLds;
-        lds = std::max(lds, b.wbytes + std::max(staged_bytes(ar, b.mw, b.A), b.stage ? kWaveStageBytes : 0));
+        const size_t rows = wave_stage_bytes(wave_turned(ar, b.mw, EPI_BATCH));
+        b.stage = b.wbytes + rows <= kMaxLds;
+        lds = std::max(lds, b.wbytes + std::max(staged_bytes(ar, b.mw, b.A), b.stage ? rows : 0));
     }
     if (items > (1L << 30)) return fail("batched beamformer: too many work items");
     if (lds > kMaxLds) return fail("batched beamformer: too many antennas");

@@ -1016,18 +1016,8 @@ static int beam_tiles_for(int ar, int A, int B) {
 
 static int groups_for(int B, int mw) { return (B + mw * (TILE / 2) - 1) / (mw * (TILE / 2)); }
 
-// Chunks per workgroup.  The resident workgroups (occupancy x CUs) run the
-// grid in rounds, and a round takes cpw chunk times, so the estimated time is
-// ceil(workgroups / resident) * cpw chunk times.  The chosen cpw is the
-// largest one within 2% of the best estimate: fewer, longer workgroups pack
-// their phasors fewer times.  CI8 sample counts that are no multiple of 4 count
-// the packing as `pack` samples of a round besides (A14 F380 T1587 B16, split
-// FP16: 39 us, with one chunk per workgroup 51); elsewhere it hides behind the
-// other workgroups, and counting it cost 4% (Mode A) to 7% (CF32).  At the
-// production shapes the Mode-B kernels (3 per CU) get one round of 768
-// workgroups, cpw = 8; the Mode-A kernel (4 per CU) gets three rounds of 1024,
-// cpw = 4 (146 against 150 us with one round of 768).
-static int pick_chunks_per_wg(const void* fn, size_t lds, int n_tchunks, long per_chunk, long span, long pack) {
+// Workgroups the device holds at once.
+static long resident_wgs(const void* fn, size_t lds) {
     // Occupancy per (kernel, LDS bytes), cached in a fixed table (no heap
     // allocation on the launch path; past 64 entries it is recomputed).
     struct Occ { const void* fn; size_t lds; int occ; };
@@ -1045,7 +1035,21 @@ static int pick_chunks_per_wg(const void* fn, size_t lds, int n_tchunks, long pe
             if (n_cached < 64) cache[n_cached++] = {fn, lds, occ};
         }
     }
-    const long resident = (long)occ * device_cus();
+    return (long)occ * device_cus();
+}
+
+// Chunks per workgroup.  The resident workgroups (occupancy x CUs) run the
+// grid in rounds, and a round takes cpw chunk times, so the estimated time is
+// ceil(workgroups / resident) * cpw chunk times.  The chosen cpw is the
+// largest one within 2% of the best estimate: fewer, longer workgroups pack
+// their phasors fewer times.  CI8 sample counts that are no multiple of 4 count
+// the packing as `pack` samples of a round besides (A14 F380 T1587 B16, split
+// FP16: 39 us, with one chunk per workgroup 51); elsewhere it hides behind the
+// other workgroups, and counting it cost 4% (Mode A) to 7% (CF32).  At the
+// production shapes the Mode-B kernels (3 per CU) get one round of 768
+// workgroups, cpw = 8; the Mode-A kernel (4 per CU) gets three rounds of 1024,
+// cpw = 4 (146 against 150 us with one round of 768).
+static int pick_chunks_per_wg(long resident, int n_tchunks, long per_chunk, long span, long pack) {
     const int cmax = std::min(n_tchunks, 4096);
     auto est = [&](int c) {
         const long wgs = (long)((n_tchunks + c - 1) / c) * per_chunk;
@@ -1057,6 +1061,32 @@ static int pick_chunks_per_wg(const void* fn, size_t lds, int n_tchunks, long pe
     for (int c = 1; c <= cmax; c++)
         if (est(c) * 100 <= best_t * 102) best = c;
     return best;
+}
+
+constexpr double kL2Bytes = 32.0 * 1024 * 1024;      // of all XCDs
+
+// Mode-B rows (T / 4 samples) off 64-byte sectors: whether ordinary stores beat
+// nontemporal ones, which write the lines at the ends of rows and chunks in
+// parts.  Measured over A 6-64, F 16-384, T 256-16384, B 9-40 (B 1-40 for CF32).
+//  * CI8, staged rows of 16-beam tiles, ordinary in XCD order: outputs past the
+//    L2s where no beam of a tile is idle (A8 F259 T2740 B16 171 us nontemporal, 60
+//    ordinary), the workgroups take more than a round (A41 F278 T3132 B25 300
+//    against 184) or the outputs are over 8 times the voltages (A7 F176 T5756 B40
+//    536 against 206).  Otherwise, and below 16 beams (the idle lanes store to the
+//    sink), nontemporal: A10 F105 T6232 B10 39 against 50, A62 F44 T6104 B14 30
+//    against 37, A35 F41 T14636 B33 127 against 152.
+//  * CF32, stored from registers: nontemporal only where the last chunk leaves
+//    wavefronts without samples and the data or the outputs are small: A9 F195
+//    T3876 B6 40 us against 59 ordinary, but A8 F128 T1220 B14 87 against 17.
+static bool modeb_plain_ci8(const BfArgs& a, bool rounds) {
+    const double out = (double)a.F * a.T * a.B * 16;
+    return a.T % 16 && a.B >= 16 && out > kL2Bytes && (a.B % 16 == 0 || rounds || a.B > 2 * a.A);
+}
+
+static bool modeb_plain_cf32(const BfArgs& a) {
+    const double samples = (double)a.F * a.T, out = samples * a.B * 16, in = samples * a.A * 16;
+    const int last = a.T % (WAVES * TILE * 4);
+    return a.T % 16 && !(last > 0 && last <= (WAVES - 1) * TILE * 4 && in <= 146e6 && (out <= kL2Bytes || out <= in));
 }
 
 template <int NT, int MW, bool CI8, int AR, int D, bool NTS, int EPI = 0>
@@ -1088,22 +1118,30 @@ static int launch_bf(const BfArgs& args, unsigned char* ws, size_t ws_bytes, hip
     }
     a.sink = reinterpret_cast<float4*>(sink_mem);
     a.n_tchunks = (a.T + span - 1) / span;
-    const void* fn = reinterpret_cast<const void*>(&beamform_kernel<NT, MW, CI8, AR, D, NTS, EPI>);
+    auto kernel = &beamform_kernel<NT, MW, CI8, AR, D, NTS, EPI>;
     if (lds > kMaxLds) return fail("beamformer: too many antennas for the LDS phasor stage");
-    if (lds > 65536) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) {
-            set_error(std::string("beamformer: LDS attribute: ") + hipGetErrorString(e));
-            return BLADE_HIP_ERROR;
-        }
-    }
+    auto allow_lds = [&] {
+        if (lds <= 65536) return hipSuccess;
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) set_error(std::string("beamformer: LDS attribute: ") + hipGetErrorString(e));
+        return e;
+    };
+    if (allow_lds() != hipSuccess) return BLADE_HIP_ERROR;
+    const long resident = resident_wgs(reinterpret_cast<const void*>(kernel), lds);
     int cpw = env_int("BLADE_BF_CHUNKS_PER_WG", 0);
-    if (cpw <= 0) cpw = pick_chunks_per_wg(fn, lds, a.n_tchunks, (long)a.F * groups, span,
+    if (cpw <= 0) cpw = pick_chunks_per_wg(resident, a.n_tchunks, (long)a.F * groups, span,
                                            ar_split(AR) && a.T % 4 ? 128 : 0);
     cpw = std::min(cpw, a.n_tchunks);
     a.chunks_per_wg = cpw;
     dim3 grid((unsigned)((a.n_tchunks + cpw - 1) / cpw), (unsigned)a.F, (unsigned)groups);
-    hipLaunchKernelGGL((beamform_kernel<NT, MW, CI8, AR, D, NTS, EPI>), grid, dim3(64 * WAVES), lds, s, a);
+    if constexpr (ar_split(AR) && MW == 2 && EPI == EPI_MODEB) {
+        if (modeb_plain_ci8(a, (long)grid.x * grid.y * grid.z > resident)) {
+            kernel = &beamform_kernel<NT, MW, CI8, AR, D, false, EPI>;
+            if (allow_lds() != hipSuccess) return BLADE_HIP_ERROR;
+        }
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * WAVES), lds, s, a);
     return check_launch("beamformer");
 }
 
@@ -1127,28 +1165,6 @@ static bool odd_wide(int B, long T) {
     return B > 4 && (B <= 8 ? T >= 768 : full && T >= (B <= 16 ? 768 : 5000));
 }
 
-constexpr double kL2Bytes = 32.0 * 1024 * 1024;      // of all XCDs
-
-// Mode-B rows (T / 4 samples) off 64-byte sectors: whether ordinary stores beat
-// nontemporal ones, which write the lines at the ends of rows and chunks in
-// parts.  Measured over A 6-64, F 16-384, T 256-16384, B 1-40.
-//  * CI8, staged rows of 16-beam tiles: outputs past the L2s with few idle beams.
-//    A8 F259 T2740 B16 171 us nontemporal, 60 ordinary; A7 F176 T5756 B40 536
-//    against 206; A41 F278 T3132 B25 300 against 184.  Below, and up to 12 beams
-//    (the other lanes store to the sink), nontemporal: A10 F105 T6232 B10 39
-//    against 50.
-//  * CF32, stored from registers: nontemporal only where the last chunk leaves
-//    wavefronts without samples and the data or the outputs are small: A9 F195
-//    T3876 B6 40 us against 59 ordinary, but A8 F128 T1220 B14 87 against 17.
-static bool modeb_plain(bool split, const BfArgs& a) {
-    if (a.T % 16 == 0) return false;
-    const double samples = (double)a.F * a.T, out = samples * a.B * 16;
-    if (split) return a.B > 12 && out > kL2Bytes;
-    const double in = samples * a.A * 16;
-    const int last = a.T % (WAVES * TILE * 4);
-    return !(last > 0 && last <= (WAVES - 1) * TILE * 4 && in <= 146e6 && (out <= kL2Bytes || out <= in));
-}
-
 template <int NT, int MW, bool CI8, int AR, int D>
 static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, hipStream_t s) {
     if (a.T % 4) {
@@ -1161,8 +1177,8 @@ static int launch_epi(const BfArgs& a, int epi, unsigned char* ws, size_t wsb, h
     const size_t wb = operand_bytes(AR, MW, nsteps_for(AR, a.A));
     if (ar_split(AR) && wb + std::max(kStageBytes, wave_stage_bytes(AR == AR_F16X2)) > kMaxLds)
         return launch_bf<NT, MW, CI8, AR, D, false, 0>(a, ws, wsb, s);
-    if constexpr (!ar_split(AR) || MW == 2) {
-        if (epi == EPI_MODEB && modeb_plain(ar_split(AR), a))
+    if constexpr (!ar_split(AR)) {
+        if (epi == EPI_MODEB && modeb_plain_cf32(a))
             return launch_bf<NT, MW, CI8, AR, D, false, EPI_MODEB>(a, ws, wsb, s);
     }
     if (epi == EPI_MODEB) return launch_bf<NT, MW, CI8, AR, D, true, EPI_MODEB>(a, ws, wsb, s);

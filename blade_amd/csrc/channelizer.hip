@@ -1487,7 +1487,7 @@ extern "C" int blade_channelizer(const void* input, void* output, uint64_t A, ui
     // S = 2 to 8 (800 of S = 4 36.2 against 38.8 us, buffers in turn); up to one round
     // (480 of S = 2: 21.3 against 17.6) and from 1.75 on (896 of S = 4: 47.4 against
     // 42.8) the runs win.
-    const uint64_t cus = (uint64_t)device_cus();
+    const uint64_t cus = C == 4096 ? (uint64_t)device_cus() : 0;
     const bool runs4096 = C == 4096 && S > 1 && (n_spec <= 2 * cus || 4 * n_spec > 13 * cus);
     if (P == 2 && (!use_fft16(C) || runs4096) && mixed_fft_covers(rate)) {
         rc = mixed_fft(C, in, out, S, n_spec, s, &made);

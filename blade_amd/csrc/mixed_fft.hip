@@ -70,8 +70,10 @@ struct MixArgs {
     unsigned m_spw, m_sub, m_per, m_gpw;   // division multipliers of spw, sub, S or groups, spw / sub
     uint64_t n_spec, n_groups;
     int flags;
-    unsigned sums;                         // detector, KEEP: running sums in LDS from this float on
-    unsigned wg0;                          // MODE 0, OPT: first workgroup of this launch
+    union {                                // one word: the arguments stay 248 bytes (past it calls of 4 us take 0.2 us more)
+        unsigned sums;                     // detector, KEEP: running sums in LDS from this float on
+        unsigned wg0;                      // MODE 0, OPT: first workgroup of this launch
+    };
 };
 
 // n / d from m = ceil(2^32 / d), d > 1; exact for n d < 2^32.  m = 0 stands
@@ -583,7 +585,7 @@ static int mix_launch(MixArgs& a, uint64_t blocks, unsigned threads, hipStream_t
         return fail("channelizer: LDS attribute of the mixed-radix FFT");
     const uint64_t most = 0xffffffffull / threads & ~7ull;          // a launch holds less than 2^32 threads
     for (uint64_t wg0 = 0; wg0 < blocks; wg0 += most) {             // once unless MODE 0, OPT
-        a.wg0 = (unsigned)wg0;
+        if (MODE == 0) a.wg0 = (unsigned)wg0;
         void* args[] = {&a};
         (void)hipLaunchKernel(fn, dim3((unsigned)std::min(most, blocks - wg0)), dim3(threads), args, lds, s);
     }

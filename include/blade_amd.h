@@ -256,8 +256,10 @@ int blade_delay_adam(const void* steered, const void* grad_phasors, const double
  *   out[a, f*C+k, s, p] = fftshift(fft(in[a, f, s*C:(s+1)*C, p]))[k]
  * CF32 [A,F,T,P] -> CF32 [A,F*C,T/C,P]; rate 1 copies; C up to 2^20 and,
  * when C * P > 16384, factoring into 2, 3, 5 and 7 (two passes through a
- * library-owned scratch buffer, of at most 192 MiB at powers of two up to
- * 65536 with two polarizations, otherwise of the data's size).  in == out (in-place) is
+ * library-owned scratch buffer: at powers of two up to 65536 with two
+ * polarizations 192 MiB or one channel's 16 T bytes, whichever is more, or
+ * the data's size where in and out overlap at different addresses; otherwise
+ * of the data's size).  in == out (in-place) is
  * supported when C == T, or when C * P > 16384.
  */
 int blade_channelizer(const void* input, void* output, uint64_t A, uint64_t F, uint64_t T,
